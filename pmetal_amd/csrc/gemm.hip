@@ -36,47 +36,10 @@
 // fragment for a second group of weight rows without doubling the dequantization work per matrix instruction,
 // which measured slower, as did one wave per SIMD with a 128 x 64 tile), so a 128-row workgroup is bound by the
 // LDS read rate at about 60 % of the matrix peak.
-#include "internal.hpp"
+#include "gemm_common.hpp"
 
 namespace {
 
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kGroups = 18;    // 16-byte items per activation row and half super-block
-constexpr int kBlockBytes = 144;
-// FMT 0: Q4_K (144 bytes: d, dmin, 12 scale bytes, 128 quant bytes); FMT 1: Q5_K (176 bytes: the same header, then 32 bytes
-// qh with the fifth bits, then the 128 quant bytes; crates/pmetal-gguf/src/k_quants.rs:407-462)
-template <int FMT>
-struct BlockFmt {
-    static constexpr int kBytes = FMT ? 176 : 144, kQs = FMT ? 48 : 16;
-};
-
-#define PMH_GPTR(p) ((const __attribute__((address_space(1))) void *)(p))
-#define PMH_LPTR(p) ((__attribute__((address_space(3))) void *)(p))
-
-// 16 bytes per lane from global memory to LDS: lane l lands at dst + 16 l (dst is wave-uniform).
-__device__ __forceinline__ void dma16(const void *src, uint4 *dst) {
-    __builtin_amdgcn_global_load_lds(PMH_GPTR(src), PMH_LPTR(dst), 16, 0, 0);
-}
-
-// Workgroup barrier that leaves the newest `keep` vector-memory requests in flight.  (__syncthreads() carries a
-// release fence, which waits for every direct-to-LDS copy.)  The copies that the other waves will read are older
-// than those, and this wave's own LDS reads have returned (lgkmcnt(0)) before another wave may refill a stage.
-template <int KEEP>
-__device__ __forceinline__ void barrier_keep() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0070 | KEEP);  // vmcnt(KEEP) lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-__device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
-}
-__device__ __forceinline__ float bf16_to_f32(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
 
 // ------------------------------------------------------------------------------------------------
 // Pre-pass: a workgroup takes R activation rows m < Mp (R = 1: 512 threads on one row, for few rows; R = 4: 256 threads
@@ -94,7 +57,7 @@ template <bool XF32, int ORDER, int R>
 __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__restrict__ xg, int64_t k, int M, int Mp,
                                                                   float *__restrict__ rowscale, uint4 *__restrict__ xs) {
     constexpr int NT = R == 1 ? 512 : 1024, JN = NT / R, NWV = NT / 64;
-    constexpr int kGroups = ORDER == 5 ? 20 : 18;  // items per half super-block and row (shadows the Q4_K constant)
+    constexpr int kGroups = ORDER == 5 ? 20 : (ORDER == 2 || ORDER == 3 ? 16 : 18);  // items per half super-block and row (shadows the Q4_K constant)
     const int tid = threadIdx.x, lane = tid & 63, r = tid % R, j = tid / R;
     const int m = blockIdx.x * R + r;
     const bool live = m < M;
@@ -237,10 +200,6 @@ constexpr size_t tile_lds_bytes() {
     return (size_t)32 * MB * (32 * NW * 4 + kTilePad);
 }
 
-__device__ __forceinline__ uint32_t bf16_rne_bits(const float v) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, v);
-    return ((u & 0x7FFFFFFFu) > 0x7F800000u) ? ((u >> 16) | 0x40u) : ((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
 
 template <int MB, int NW = 8>
 __device__ __forceinline__ void store_tile(const float16_t (&acc)[MB], uint4 *smem, const int wave, const int col, const int g,
@@ -316,53 +275,6 @@ struct Acc {
     uint32_t qh[NR][8];  // Q5_K: the 32 qh bytes of the current super-block of this lane's row
 };
 
-// 8 quants of one dword (low nibbles, then high nibbles) times their integer scales -> 8 exact f16 values:
-// 0x6400 | q is the f16 1024 + q, and (1024 + q) * sc - 1024 * sc is exact in a packed f16 fma.  Built in four
-// pieces, so that the pieces can be placed between matrix instructions.  k-step t selects the
-// scales: GGML order multiplies the low nibbles by the first and the high nibbles by the second sub-block scale,
-// REF order both by the scale of sub-block t / 4.
-struct Dq {
-    uint32_t lo, hi;
-    half2_t r[4];
-    __device__ __forceinline__ half8_t value() const { return half8_t{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]}; }
-};
-// Q5_K (FMT 1): bit 4 of every quant comes from `hq`.  GGML order: hq is the qh dword of the same four bytes, shifted so
-// that bits 0 and 1 of each of its bytes belong to the low and the high nibble of the quant byte at the same place.  REF
-// order: hq is the one qh byte whose bits 0..7 belong to the eight consecutive elements of this k-step (even elements =
-// low nibbles): a multiplication spreads bits 0, 2, 4, 6 to bit 4 of bytes 0..3 (bit 2 i lands on 2 i + 4 + 6 i; the
-// other partial products meet at most in pairs on bits that the mask drops, and their carries stop there).  Values up to
-// 31 times scales up to 63 stay below 2048: exact in f16 like Q4_K's.
-template <int ORDER, int FMT = 0>
-__device__ __forceinline__ void dq_chunk(const int c, const int t, const uint32_t w, const half2_t (&sc2)[2], const half2_t (&off2)[2], Dq &d,
-                                         const uint32_t hq = 0) {
-    const int lo_s = ORDER == 0 ? (t >> 2) : 0, hi_s = ORDER == 0 ? (t >> 2) : 1;
-    if (FMT == 1 && c == 0) {
-        const uint32_t bit = ORDER == 0 ? ((hq & 0x55u) * 0x00410410u) & 0x10101010u : (hq & 0x01010101u) << 4;
-        d.lo = (w & 0x0F0F0F0Fu) | bit;
-        d.r[0] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04010400u)), sc2[lo_s], off2[lo_s]);
-    } else if (FMT == 1 && c == 1) {
-        d.r[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04030402u)), sc2[lo_s], off2[lo_s]);
-        const uint32_t bit = ORDER == 0 ? (((hq >> 1) & 0x55u) * 0x00410410u) & 0x10101010u : (hq & 0x02020202u) << 3;
-        d.hi = ((w >> 4) & 0x0F0F0F0Fu) | bit;
-    } else if (c == 0) {
-        d.lo = w & 0x0F0F0F0Fu;
-        d.r[0] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04010400u)), sc2[lo_s], off2[lo_s]);
-    } else if (c == 1) {
-        d.r[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04030402u)), sc2[lo_s], off2[lo_s]);
-        d.hi = (w >> 4) & 0x0F0F0F0Fu;
-    } else if (c == 2) {
-        d.r[2] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.hi, 0x04010400u)), sc2[hi_s], off2[hi_s]);
-    } else {
-        d.r[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.hi, 0x04030402u)), sc2[hi_s], off2[hi_s]);
-    }
-}
-
-// -(dmin * mn) split exactly into an f16 head and tail (dmin has 11 significant bits, mn 6).
-__device__ __forceinline__ void neg_min_split(const float dmin, const uint32_t mn, _Float16 &h, _Float16 &l) {
-    const float p = -(dmin * (float)mn);  // exact in fp32
-    h = (_Float16)p;
-    l = (_Float16)(p - (float)h);
-}
 
 // One half super-block H of one wave.  The restrict qualifiers say what the copies in flight cannot touch:
 // operand reads from a_cur / q_cur need not wait for the direct loads into a_nxt / q_nxt / hb.
@@ -636,15 +548,6 @@ __global__ __launch_bounds__(64 * NW, MB * NR <= 1 && NW <= 8 ? 2 : 1) void k_qg
 //     header pieces of a row are Q2_K: bytes 0..15 (scales) and 68..83 (d, dmin in the last dword); Q3_K: 0..31 (hmask) and
 //     94..109 (scales in bytes 2..13 of the piece, d in 14..15).
 // ------------------------------------------------------------------------------------------------
-constexpr int kGroups16 = 20;  // activation items per row and half super-block: 16 operands and four of sub-block sums
-template <int FMT>
-struct Block16 {  // FMT 2: Q3_K, 3: Q2_K
-    static constexpr int kBytes = FMT == 3 ? 84 : 110, kQs = FMT == 3 ? 16 : 32;
-    static constexpr int kHdrPieces = FMT == 3 ? 2 : 3;           // per row and super-block
-    static constexpr int kHdrRounds = (32 * kHdrPieces + 63) / 64;  // whole-wave copies
-    static constexpr int kHdrStage = 64 * kHdrRounds;              // items of a wave's header stage
-    static __device__ __forceinline__ uint32_t piece_off(int p) { return FMT == 3 ? (p == 0 ? 0u : 68u) : (p == 2 ? 94u : 16u * (uint32_t)p); }
-};
 
 template <int FMT, int MB, int H>
 __device__ __forceinline__ void rw16_half(const uint4 *__restrict__ a_cur, uint4 *__restrict__ a_nxt, const uint4 *__restrict__ q_cur,
@@ -875,7 +778,6 @@ constexpr size_t rw16_lds_bytes() {
 //     4 t + e (two-bit field g for the low, 2 + g for the high nibbles);
 //   * super-blocks are only 2-byte aligned; the direct-to-LDS loads take such addresses.
 // ------------------------------------------------------------------------------------------------
-constexpr int kQ6Bytes = 210, kQ6Groups = 16, kQ6Stage = 192;  // LDS items of a wave's quant stage: 128 ql + 64 qh
 
 template <int MB>
 struct LaneQ6 {
@@ -894,31 +796,6 @@ struct AccQ6 {
     uint32_t d;  // f16 bits of d
 };
 
-// The two operands of one k-step, built in eight pieces that are placed between matrix instructions.
-struct Dq6 {
-    uint32_t nlo, nhi, hlo, hhi;
-    half2_t r1[4], r2[4];
-    __device__ __forceinline__ half8_t b1() const { return half8_t{r1[0][0], r1[0][1], r1[1][0], r1[1][1], r1[2][0], r1[2][1], r1[3][0], r1[3][1]}; }
-    __device__ __forceinline__ half8_t b2() const { return half8_t{r2[0][0], r2[0][1], r2[1][0], r2[1][1], r2[2][0], r2[2][1], r2[3][0], r2[3][1]}; }
-};
-// qlw: the ql dword of the k-step; qhw: its qh dword already shifted by 2 g; s2 / s1: (sc, sc) and (16 sc, 16 sc)
-// of the low-nibble and of the high-nibble elements.  0x6400 | v is the f16 1024 + v; both steps of each value are exact.
-__device__ __forceinline__ void dq6_chunk(const int c, const uint32_t qlw, const uint32_t qhw, const half2_t (&s2)[2],
-                                          const half2_t (&s1)[2], Dq6 &d) {
-    const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f}, m1026 = {(_Float16)-1026.0f, (_Float16)-1026.0f};
-    const uint32_t sel = (c & 1) ? 0x04030402u : 0x04010400u;  // bytes (b0, b1) resp. (b2, b3) -> 0x64bb pairs
-    if (c == 0) d.nlo = qlw & 0x0F0F0F0Fu;
-    if (c == 2) d.nhi = (qlw >> 4) & 0x0F0F0F0Fu;
-    if (c == 4) d.hlo = qhw & 0x03030303u;
-    if (c == 6) d.hhi = (qhw >> 4) & 0x03030303u;
-    if (c < 4) {
-        const uint32_t v = c < 2 ? d.nlo : d.nhi;
-        d.r2[c] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + m1024) * s2[c >> 1];
-    } else {
-        const uint32_t v = c < 6 ? d.hlo : d.hhi;
-        d.r1[c - 4] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + m1026) * s1[(c - 4) >> 1];
-    }
-}
 
 template <int MB, int H>
 __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint4 *__restrict__ a_nxt,
@@ -1067,7 +944,7 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q6(const uint8_t *__restric
         }
         dma16(blk + L.qh_off, qa + 128);
         dma16(blk + 32 + L.qh_off, qb + 128);
-        const uint4 *xa = xs + (size_t)(sb0 * 2 * kGroups) * Mp + m0;
+        const uint4 *xa = xs + (size_t)(sb0 * 2 * kQ6Groups) * Mp + m0;
 #pragma unroll
         for (int i = 0; i < LaneQ6<MB>::kARounds; i++) dma16(xa + L.a_off[i], a0 + i * kThreads + L.wave * 64);
     }
@@ -1078,9 +955,9 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q6(const uint8_t *__restric
         const int sb = sb0 + s;
         const int sbn = sb + 1 < spr ? sb + 1 : spr - 1;
         const uint8_t *blkn = wblk + (size_t)sbn * kQ6Bytes;
-        rw_half_q6<MB, 0>(a0, a1, qa, qc, hw, xs + (size_t)((sb * 2 + 1) * kGroups) * Mp + m0, blkn, blkn, L, R);
+        rw_half_q6<MB, 0>(a0, a1, qa, qc, hw, xs + (size_t)((sb * 2 + 1) * kQ6Groups) * Mp + m0, blkn, blkn, L, R);
         barrier_keep<3>();
-        rw_half_q6<MB, 1>(a1, a0, qb, qa, hw, xs + (size_t)(sbn * 2 * kGroups) * Mp + m0, blkn, nullptr, L, R);
+        rw_half_q6<MB, 1>(a1, a0, qb, qa, hw, xs + (size_t)(sbn * 2 * kQ6Groups) * Mp + m0, blkn, nullptr, L, R);
         barrier_keep<3>();
         uint4 *t = qc;
         qc = qb, qb = qa, qa = t;
@@ -1122,16 +999,6 @@ __device__ __forceinline__ void q8_load(const uint8_t *p, const int g, Q8Half &h
     }
 }
 
-// 8 int8 -> 8 exact f16: q + 128 as an unsigned byte b, 0x6400 | b is the f16 1024 + b, minus 1152.
-__device__ __forceinline__ half8_t q8_operand(const uint32_t w0, const uint32_t w1) {
-    const half2_t m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u;
-    const half2_t r0 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u0, 0x04010400u)) + m1152;
-    const half2_t r1 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u0, 0x04030402u)) + m1152;
-    const half2_t r2 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u1, 0x04010400u)) + m1152;
-    const half2_t r3 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u1, 0x04030402u)) + m1152;
-    return half8_t{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
-}
 
 template <int MB>
 __device__ __forceinline__ void rw_half_q8(const uint4 *__restrict__ a_cur, uint4 *__restrict__ a_nxt,
@@ -1219,7 +1086,7 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restric
     Q8Half ha, hb;
     q8_load(wp, L.g, ha);
     {
-        const uint4 *xa = xs + (size_t)(sb0 * 2 * kGroups) * Mp + m0;
+        const uint4 *xa = xs + (size_t)(sb0 * 2 * kQ6Groups) * Mp + m0;
 #pragma unroll
         for (int i = 0; i < LaneQ6<MB>::kARounds; i++) dma16(xa + L.a_off[i], a0 + i * kThreads + L.wave * 64);
     }
@@ -1230,9 +1097,9 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restric
         const int sb = sb0 + s;
         const int sbn = sb + 1 < spr ? sb + 1 : spr - 1;  // the copies for "the next super-block" stay inside the matrix
         const uint8_t *w1 = wp + 136, *w2 = wp + 272;
-        rw_half_q8<MB>(a0, a1, xs + (size_t)((sb * 2 + 1) * kGroups) * Mp + m0, w1, ha, hb, L, acc);
+        rw_half_q8<MB>(a0, a1, xs + (size_t)((sb * 2 + 1) * kQ6Groups) * Mp + m0, w1, ha, hb, L, acc);
         barrier_keep<12>();
-        rw_half_q8<MB>(a1, a0, xs + (size_t)(sbn * 2 * kGroups) * Mp + m0, w2 < wlast ? w2 : wlast, hb, ha, L, acc);
+        rw_half_q8<MB>(a1, a0, xs + (size_t)(sbn * 2 * kQ6Groups) * Mp + m0, w2 < wlast ? w2 : wlast, hb, ha, L, acc);
         barrier_keep<12>();
         wp = w2;
     }
@@ -1265,7 +1132,6 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restric
 //     by the rows' powers of two.  No store and no other load is issued inside the streaming loop: on this target stores
 //     share the loads' counter, and one of them in flight turns every counted wait into a wait for everything.
 // ------------------------------------------------------------------------------------------------
-typedef float float4_t __attribute__((ext_vector_type(4)));
 constexpr int kSmallWaves = 8;  // waves per workgroup (fewer when a row has fewer super-blocks); 16 waves of one super-block each run alike
 constexpr int kSmallDepth = 2;  // row tiles in flight per wave (four are slower: 16.5 against 12.7 us at 14336 x 4096)
 constexpr int kSmallMaxM = 16, kSmallMaxSpr = 16;
@@ -1549,7 +1415,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
         for (int mb = 0; mb < MT; mb++)
 #pragma unroll
             for (int b = 0; b < 8; b++) {
-                const uint4 *item = xs + (size_t)((2 * sbi[i] + (b >> 2)) * kGroups + 4 * (b & 3) + kg) * Mp + 16 * mb + nl;
+                const uint4 *item = xs + (size_t)((2 * sbi[i] + (b >> 2)) * kQ6Groups + 4 * (b & 3) + kg) * Mp + 16 * mb + nl;
                 af[i][mb][b] = __builtin_bit_cast(half8_t, *item);
                 if (!sbv[i]) af[i][mb][b] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
             }
@@ -1703,7 +1569,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
             for (int lh = 0; lh < 2; lh++)
 #pragma unroll
                 for (int gp = 0; gp < 2; gp++) {
-                    const uint4 *item = xs + (size_t)((2 * (sbv[i] ? sb0 + i : 0) + hh) * kGroups + 2 * (4 * lh + kg) + gp) * Mp + nl;
+                    const uint4 *item = xs + (size_t)((2 * (sbv[i] ? sb0 + i : 0) + hh) * kQ6Groups + 2 * (4 * lh + kg) + gp) * Mp + nl;
                     af[i][hh][lh][gp] = __builtin_bit_cast(half8_t, *item);
                     if (!sbv[i]) af[i][hh][lh][gp] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
                 }
@@ -1890,7 +1756,7 @@ struct SmallRun16 {  // what a lane holds of a row tile
     u32x4 sc[NSB];         // Q3_K: scales and d; Q2_K: x, y = scale bytes 8 h .., z = d | dmin << 16
 };
 
-template <int FMT, int NSB, int MT = 1>
+template <int FMT, int NSB>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                                      const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                      int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
@@ -1905,7 +1771,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
     const uint32_t h = (uint32_t)(kg >> 1), g = (uint32_t)(kg & 1);
     const int rounds = (tiles_per_wg + kSmallDepth - 1) / kSmallDepth;
     float4_t *out_tiles = dyn;
-    float4_t *keep = tiles_per_wg * MT <= kSmallKeepTiles ? dyn + rounds * kSmallDepth * MT * 64 : nullptr;
+    float4_t *keep = tiles_per_wg <= kSmallKeepTiles ? dyn + rounds * kSmallDepth * 64 : nullptr;
     int sbi[NSB];
     bool sbv[NSB];  // wave-uniform
 #pragma unroll
@@ -1914,23 +1780,21 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         sbv[i] = sbi[i] < spr;
         sbi[i] = sbv[i] ? sbi[i] : 0;
     }
-    half8_t af[NSB][MT][8], asum[NSB][MT][2];  // (MT 16-row blocks of activations: rows nl, 16 + nl)
+    half8_t af[NSB][8], asum[NSB][2];
 #pragma unroll
-    for (int i = 0; i < NSB; i++)
+    for (int i = 0; i < NSB; i++) {
+        const uint4 *base = xs + (size_t)((2 * sbi[i] + (int)h) * kGroups16) * Mp + nl;
 #pragma unroll
-        for (int mb = 0; mb < MT; mb++) {
-            const uint4 *base = xs + (size_t)((2 * sbi[i] + (int)h) * kGroups16) * Mp + 16 * mb + nl;
+        for (int t = 0; t < 8; t++) af[i][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (int)g) * Mp]);
+        asum[i][0] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (int)g) * Mp]);
+        asum[i][1] = __builtin_bit_cast(half8_t, base[(size_t)(18 + (int)g) * Mp]);
+        if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
+            const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-            for (int t = 0; t < 8; t++) af[i][mb][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (int)g) * Mp]);
-            asum[i][mb][0] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (int)g) * Mp]);
-            asum[i][mb][1] = __builtin_bit_cast(half8_t, base[(size_t)(18 + (int)g) * Mp]);
-            if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
-                const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-                for (int t = 0; t < 8; t++) af[i][mb][t] = z;
-                asum[i][mb][0] = z, asum[i][mb][1] = z;
-            }
+            for (int t = 0; t < 8; t++) af[i][t] = z;
+            asum[i][0] = z, asum[i][1] = z;
         }
+    }
     const int t0 = (int)blockIdx.x * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;  // t1 > t0 by the launch geometry
     const uint32_t row_bytes = (uint32_t)spr * (uint32_t)B::kBytes;
@@ -1961,9 +1825,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         }
     };
     auto consume = [&](int ti, const SmallRun16<FMT, NSB> &w) __attribute__((always_inline)) {
-        float4_t acc[MT];
-#pragma unroll
-        for (int mb = 0; mb < MT; mb++) acc[mb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < NSB; i++) {
             uint32_t qd[4], hm[4] = {0, 0, 0, 0}, s8[3], dbits;
@@ -2005,9 +1867,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
                     const _Float16 s16 = (_Float16)scf, o16 = (_Float16)(-1024.0f * scf);  // exact: |sc| <= 32
                     sc2[2 * sp + lh] = half2_t{s16, s16}, off2[2 * sp + lh] = half2_t{o16, o16};
                 }
-            float4_t part[MT];
-#pragma unroll
-            for (int mb = 0; mb < MT; mb++) part[mb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            float4_t part = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int t = 0; t < 8; t++) {
                 const int dw = t >> 1, sp = t & 1;
@@ -2021,24 +1881,19 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
                 const half2_t r2 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u)), sc2[2 * sp + 1], off2[2 * sp + 1]);
                 const half2_t r3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u)), sc2[2 * sp + 1], off2[2 * sp + 1]);
                 const half8_t b = half8_t{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
-#pragma unroll
-                for (int mb = 0; mb < MT; mb++) part[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i][mb][t], b, part[mb], 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i][t], b, part, 0, 0, 0);
             }
 #pragma unroll
             for (int sp = 0; sp < 2; sp++) {
                 const _Float16 h0 = (_Float16)nm[2 * sp], h1 = (_Float16)nm[2 * sp + 1];
                 const _Float16 l0 = (_Float16)(nm[2 * sp] - (float)h0), l1 = (_Float16)(nm[2 * sp + 1] - (float)h1);
                 const half8_t br = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
-#pragma unroll
-                for (int mb = 0; mb < MT; mb++) acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(asum[i][mb][sp], br, acc[mb], 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(asum[i][sp], br, acc, 0, 0, 0);
             }
 #pragma unroll
-            for (int mb = 0; mb < MT; mb++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) acc[mb][r] = __builtin_fmaf(d, part[mb][r], acc[mb][r]);
+            for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(d, part[r], acc[r]);
         }
-#pragma unroll
-        for (int mb = 0; mb < MT; mb++) small_add_waves(red, keep, ti * MT + mb, wave, nwaves, lane, acc[mb], out_tiles);
+        small_add_waves(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRun16<FMT, NSB> ring0, ring1;
@@ -2050,8 +1905,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         consume(2 * rd + 1, ring1);
         issue(2 * rd + 3, ring1);
     }
-    small_add_kept(keep, rounds * kSmallDepth * MT, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rowscale, yg, ybf16, partial, MT);
+    small_add_kept(keep, rounds * kSmallDepth, wave, nwaves, lane, out_tiles);
+    small_store(out_tiles, t0, t1, M, Mp, N, rowscale, yg, ybf16, partial);
 }
 
 }  // namespace
@@ -2064,14 +1919,13 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // workgroup row of the grid each, whose partial tiles k_rw_reduce adds (qgemm_plan sets splits and chunk to match).
 constexpr int kSmallMaxRuns = 8;  // k <= 32768
 // Super-blocks of a row that one short-batch workgroup takes (a longer row goes in runs of that many); 0: no such kernel.
-// Up to 16 rows: eight waves of two super-blocks.  17 to 32 rows (two 16-row blocks of activations per weight operand): the
-// Q4_K / Q5_K and Q2_K kernels still hold two super-blocks' activations per wave, the Q8_0 kernel one (43.4 -> 27.1 us at 14336 x 4096);
-// the Q6_K kernel in that form, with its rows in runs of eight, is no faster than the large kernel (32.2 against 29.9 us).
+// Up to 16 rows: eight waves of two super-blocks.  17 to 32 rows (two 16-row blocks of activations per weight operand), where
+// the tile kernel does not take them: Q4_K / Q5_K hold two super-blocks' activations per wave, Q8_0 one.
 static int small_run_spr(uint32_t type, int64_t m) {
     const bool any = type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ6K || type == kTypeQ8_0 || type == kTypeQ3K || type == kTypeQ2K;
     if (m <= kSmallMaxM) return any ? kSmallMaxSpr : 0;
     if (m > kSmallMaxM2) return 0;
-    if (type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ2K) return kSmallMaxSpr;
+    if (type == kTypeQ4K || type == kTypeQ5K) return kSmallMaxSpr;
     if (type == kTypeQ8_0) return kSmallWaves;
     return 0;
 }
@@ -2103,8 +1957,38 @@ bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
     return (type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ6K || type == kTypeQ8_0 || type == kTypeQ3K || type == kTypeQ2K) && m >= 1 && m <= (int64_t)1 << 22 && n >= 1 && k >= 256 && k % 256 == 0 && k <= (int64_t)1 << 22 && n <= 0x7FFFFF00;
 }
 
+// The tile kernel's best tile and K split for a shape, and the microseconds it is expected to take behind the pre-pass.  Fitted
+// to 1400 measured times (rms 12 %): per round of 256 workgroups a wave's super-blocks cost 1/113 us per KB of activations and
+// 1/41 us per KB of weights the workgroup takes in, plus 0.7 us per 32 x 32 tile (twice the matrix instructions for Q6_K).
+struct KwChoice {
+    int mb, nr, splits;
+    double us, rounds;
+};
+static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
+    const double block = type == kTypeQ4K ? 144 : type == kTypeQ5K ? 176 : type == kTypeQ6K ? 210 : type == kTypeQ8_0 ? 272 : type == kTypeQ3K ? 110 : 84;
+    const double items = type == kTypeQ3K || type == kTypeQ2K ? 40 : type == kTypeQ6K || type == kTypeQ8_0 ? 32 : 36;  // per row and super-block
+    const double cost = type == kTypeQ6K ? 2.0 : type == kTypeQ8_0 ? 1.5 : 1.0;
+    KwChoice best = {1, 1, 1, 0.0, 0.0};
+    bool have = false;
+    for (int mb = 1; mb <= (m <= 32 ? 1 : 2); mb++)
+        for (int nr = 1; nr <= 2; nr++) {
+            if (m > 32 && mb == 1 && nr == 2) continue;  // never the best tile
+            const int64_t tiles = ((n + 32 * nr - 1) / (32 * nr)) * ((m + 32 * mb - 1) / (32 * mb));
+            for (int splits = 1; splits <= 4 && splits <= spr; splits *= 2) {
+                if (splits > 1 && (tiles * splits > 288 || (m <= 32 && nr == 2))) break;  // only to fill the machine
+                const int64_t chunk = (spr + splits - 1) / splits, per = (chunk + 7) / 8, wgs = tiles * splits;
+                double rounds = ((double)wgs / 256.0 + (double)((wgs + 255) / 256)) / 2;
+                const double one = (double)per * 8.0 * (mb * 32 * items * 16 / 1e3 / 113.0 + nr * 32 * block / 1e3 / 41.0) + 0.7 * cost * mb * nr * per;
+                const double us = 6.0 + (1.0 + (rounds - 1.0) * 0.77) * one + (splits > 1 ? 2.2 + splits * (double)m * (double)n * 8.0 * 0.7 / 4.0e6 : 0.0);
+                if (!have || us < best.us) best = {mb, nr, splits, us, (double)wgs / 256.0}, have = true;
+            }
+        }
+    return best;
+}
+
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     GemmPlan p;
+    p.kernel = GemmKernel::kRows, p.nr = 1;
     // 32, 64 or 128 activation rows per workgroup; up to 192 rows 64-row blocks beat 128-row blocks (fewer K splits
     // for the same number of workgroups: 36.9 against 38.3 us at M = 128, 51.7 against 53.8 at M = 192, 14336x4096;
     // equal at 256, and from 320 rows on the larger block wins)
@@ -2134,20 +2018,51 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
                          (splits > 1 ? (double)splits * (double)m * (double)n * 8.0 / 4.0e12 + 3.0e-6 : 0.0);
         if (want == 1 || t < best) best = t, p.splits = (int)splits, p.chunk = (int)chunk;
     }
-    // short batches against long rows: runs of 16 (or 8) super-blocks, the fused kernels' K split (a shape they do not take
-    // keeps the split chosen above)
+    // The tile kernel (gemm_kw.hip) needs no second pass over partial tiles and no barrier per step, but reads the activations
+    // once per 32 or 64 weight rows: the better one for few activation rows and for narrow weights.
+    const KwChoice kw = kw_choice(m, n, spr, type);
     const int run = small_run_spr(type, m);
-    if (run && spr > run && qgemm_small_applies(type, m, n, k)) p.chunk = run, p.splits = (int)((spr + run - 1) / run);
+    const bool small = qgemm_small_applies(type, m, n, k);
+    bool waves;
+    if (m <= kSmallMaxM) {
+        waves = false;
+    } else if (m <= kSmallMaxM2) {
+        // 17 to 32 rows, against the short-batch kernels with two blocks of activations or, for the types without them, the
+        // 32-row blocks: ahead up to four rounds of workgroups (Q4_K 4096 x 4096 12.8 -> 10.9 us, Q6_K 21.9 -> 13.4, 14336 x 4096
+        // 29.2 -> 26.1; behind at 128256 x 4096: Q4_K 87 -> 103, Q6_K 141 -> 154) and where a row is not whole runs (32000 x 5120:
+        // Q4_K 50.8 -> 40.5)
+        waves = n * k < ((int64_t)96 << 20) || (small && spr > run && spr % run != 0 && type != kTypeQ8_0);
+        waves = waves || (type == kTypeQ2K);  // (no short-batch form for two blocks; ahead at every size: 128256 x 4096 98 -> 90 us)
+    } else {
+        // against the row kernels, by the times fitted to both over 1000...14336 weight rows of 1536...14336 elements and
+        // 64...256 activation rows (the chosen kernel is within 2 % of the best one on average)
+        const double half = type == kTypeQ4K ? 0.96 : type == kTypeQ5K ? 1.2 : type == kTypeQ6K ? 1.83 : type == kTypeQ8_0 ? 3.2 : type == kTypeQ3K ? 1.35 : 1.03;
+        const double rounds = (double)((base * p.splits + 255) / 256);
+        const double t_rows = rounds * 2.0 * p.chunk * half * (p.mb == 4 ? 1.33 : 1.0) +
+                              (p.splits > 1 ? 13.2 + (double)p.splits * (double)m * (double)n * 8.0 * 0.9 / 4.0e6 : 0.0);
+        waves = kw.rounds <= 3.0 && kw.us - 6.0 < t_rows;
+    }
+    if (waves) {
+        p.kernel = GemmKernel::kWaves;
+        p.mb = kw.mb, p.nr = kw.nr, p.splits = kw.splits, p.chunk = (int)((spr + kw.splits - 1) / kw.splits);
+        // (one padding for both block heights, so that weights of one batch share their converted activations)
+        p.mp = (int)(m <= 32 ? 32 : (m + 63) / 64 * 64);
+    } else if (small) {
+        // short batches: rows longer than a run are cut into runs of 16 (or 8) super-blocks, these kernels' K split
+        p.kernel = GemmKernel::kSmall;
+        p.chunk = spr > run ? run : (int)spr, p.splits = (int)((spr + p.chunk - 1) / p.chunk);
+    }
     return p;
 }
+
+// the tile kernel requests up to six k-steps of items past the last one (32 bytes per row each): they lie in the workspace
+static size_t kw_slack(const GemmPlan &p) { return p.kernel == GemmKernel::kWaves ? (size_t)p.mp * 256 : 0; }
 
 size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k) {
     const GemmPlan p = qgemm_plan(m, n, k, type);
     const size_t xs = align256((size_t)(k / 256) * 2 * (type == kTypeQ3K || type == kTypeQ2K ? kGroups16 : kGroups) * p.mp * 16);
-    // the short-batch kernels take a row of up to kSmallMaxSpr super-blocks whole: the plan's K split is not used there
-    const bool unsplit = qgemm_small_applies(type, m, n, k) && k / 256 <= small_run_spr(type, m);
-    const size_t part = p.splits > 1 && !unsplit ? align256((size_t)p.splits * p.mp * n * 4) : 0;
-    return xs + align256((size_t)p.mp * 4) + part;
+    const size_t part = p.splits > 1 ? align256((size_t)p.splits * p.mp * n * 4) : 0;
+    return xs + align256((size_t)p.mp * 4) + part + kw_slack(p);
 }
 
 template <int ORDER, int MB, int NR, int NW, int FMT = 0>
@@ -2250,13 +2165,16 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const bool ybf = y_dtype == kDtypeBf16;
-    if (qgemm_small_applies(type, m, n, k)) {
+    if (p.kernel == GemmKernel::kWaves) {
+        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, s);
+        if (e != hipSuccess || p.splits == 1) return e;
+    } else if (p.kernel == GemmKernel::kSmall) {
         const int nwaves = spr < kSmallWaves ? spr : kSmallWaves;
         const int tiles = (int)((n + 15) / 16);
         // one workgroup per compute unit over all runs of a long row: each then walks several row tiles with its activation
         // operands in registers (one tile per workgroup and four times the workgroups: 35 against 27 us at M = 16, 4096 x 14336)
         const int run = small_run_spr(type, m);
-        const int runs_of_row = spr > run ? p.splits : 1;
+        const int runs_of_row = p.splits;
         int64_t slots = (int64_t)compute_units_gemm() * (kSmallWaves / nwaves) / runs_of_row;
         slots = slots < 1 ? 1 : slots;
         const int n_wg = (int)(tiles < slots ? tiles : slots);
@@ -2265,8 +2183,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         // the finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and the 16 KiB of the
         // reduction buffers: 64 of them keep the workgroup within 160 KiB for every type
         tiles_per_wg = tiles_per_wg < 64 / mt ? tiles_per_wg : 64 / mt;
-        // a long row: p.splits runs of 16 super-blocks, one workgroup row of the grid each, partial tiles for k_rw_reduce
-        // (for rows of up to 16 super-blocks the plan's split belongs to the large kernel and is not used here)
+        // a long row: p.splits runs, one workgroup row of the grid each, partial tiles for k_rw_reduce
         const int runs = runs_of_row;
         float *const part_out = runs > 1 ? partial : nullptr;
         const int nsb = run > kSmallWaves && spr > kSmallWaves ? 2 : 1;
@@ -2296,24 +2213,22 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         else PMH_SMALL_F(O, S, 0);    \
     } while (0)
         if (q23) {
-#define PMH_SMALL16(F, S, T)                                                                                                     \
+#define PMH_SMALL16(F, S)                                                                                                     \
     do {                                                                                                                         \
         if (lds > 48 * 1024) {                                                                                                   \
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_qgemm_small16<F, S, T>), hipFuncAttributeMaxDynamicSharedMemorySize, \
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_qgemm_small16<F, S>), hipFuncAttributeMaxDynamicSharedMemorySize, \
                                     (int)lds);                                                                                   \
             if (e != hipSuccess) return e;                                                                                       \
         }                                                                                                                        \
-        hipLaunchKernelGGL((k_qgemm_small16<F, S, T>), grid, block, lds, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
+        hipLaunchKernelGGL((k_qgemm_small16<F, S>), grid, block, lds, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
                            tiles_per_wg, ybf ? 1 : 0, part_out);                                                                 \
     } while (0)
             if (type == kTypeQ2K) {
-                if (mt == 2 && nsb == 2) PMH_SMALL16(3, 2, 2);
-                else if (mt == 2) PMH_SMALL16(3, 1, 2);
-                else if (nsb == 2) PMH_SMALL16(3, 2, 1);
-                else PMH_SMALL16(3, 1, 1);
+                if (nsb == 2) PMH_SMALL16(3, 2);
+                else PMH_SMALL16(3, 1);
             } else {
-                if (nsb == 2) PMH_SMALL16(2, 2, 1);
-                else PMH_SMALL16(2, 1, 1);
+                if (nsb == 2) PMH_SMALL16(2, 2);
+                else PMH_SMALL16(2, 1);
             }
 #undef PMH_SMALL16
         } else if (q6) {

@@ -1,0 +1,151 @@
+// Device code shared by the dequant-fused GEMM kernels (gemm.hip, gemm_kw.hip): operand types, direct global -> LDS copies,
+// and the exact f16 operands built from the packed quants of each format.
+#pragma once
+
+#include "internal.hpp"
+
+namespace {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kGroups = 18;    // 16-byte items per activation row and half super-block
+constexpr int kBlockBytes = 144;
+// FMT 0: Q4_K (144 bytes: d, dmin, 12 scale bytes, 128 quant bytes); FMT 1: Q5_K (176 bytes: the same header, then 32 bytes
+// qh with the fifth bits, then the 128 quant bytes; crates/pmetal-gguf/src/k_quants.rs:407-462)
+template <int FMT>
+struct BlockFmt {
+    static constexpr int kBytes = FMT ? 176 : 144, kQs = FMT ? 48 : 16;
+};
+
+#define PMH_GPTR(p) ((const __attribute__((address_space(1))) void *)(p))
+#define PMH_LPTR(p) ((__attribute__((address_space(3))) void *)(p))
+
+// 16 bytes per lane from global memory to LDS: lane l lands at dst + 16 l (dst is wave-uniform).
+__device__ __forceinline__ void dma16(const void *src, uint4 *dst) {
+    __builtin_amdgcn_global_load_lds(PMH_GPTR(src), PMH_LPTR(dst), 16, 0, 0);
+}
+
+// Workgroup barrier that leaves the newest `keep` vector-memory requests in flight.  (__syncthreads() carries a
+// release fence, which waits for every direct-to-LDS copy.)  The copies that the other waves will read are older
+// than those, and this wave's own LDS reads have returned (lgkmcnt(0)) before another wave may refill a stage.
+template <int KEEP>
+__device__ __forceinline__ void barrier_keep() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | KEEP);  // vmcnt(KEEP) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
+}
+__device__ __forceinline__ float bf16_to_f32(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
+
+__device__ __forceinline__ uint32_t bf16_rne_bits(const float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    return ((u & 0x7FFFFFFFu) > 0x7F800000u) ? ((u >> 16) | 0x40u) : ((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+}
+
+// 8 quants of one dword (low nibbles, then high nibbles) times their integer scales -> 8 exact f16 values:
+// 0x6400 | q is the f16 1024 + q, and (1024 + q) * sc - 1024 * sc is exact in a packed f16 fma.  Built in four
+// pieces, so that the pieces can be placed between matrix instructions.  k-step t selects the
+// scales: GGML order multiplies the low nibbles by the first and the high nibbles by the second sub-block scale,
+// REF order both by the scale of sub-block t / 4.
+struct Dq {
+    uint32_t lo, hi;
+    half2_t r[4];
+    __device__ __forceinline__ half8_t value() const { return half8_t{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]}; }
+};
+// Q5_K (FMT 1): bit 4 of every quant comes from `hq`.  GGML order: hq is the qh dword of the same four bytes, shifted so
+// that bits 0 and 1 of each of its bytes belong to the low and the high nibble of the quant byte at the same place.  REF
+// order: hq is the one qh byte whose bits 0..7 belong to the eight consecutive elements of this k-step (even elements =
+// low nibbles): a multiplication spreads bits 0, 2, 4, 6 to bit 4 of bytes 0..3 (bit 2 i lands on 2 i + 4 + 6 i; the
+// other partial products meet at most in pairs on bits that the mask drops, and their carries stop there).  Values up to
+// 31 times scales up to 63 stay below 2048: exact in f16 like Q4_K's.
+template <int ORDER, int FMT = 0>
+__device__ __forceinline__ void dq_chunk(const int c, const int t, const uint32_t w, const half2_t (&sc2)[2], const half2_t (&off2)[2], Dq &d,
+                                         const uint32_t hq = 0) {
+    const int lo_s = ORDER == 0 ? (t >> 2) : 0, hi_s = ORDER == 0 ? (t >> 2) : 1;
+    if (FMT == 1 && c == 0) {
+        const uint32_t bit = ORDER == 0 ? ((hq & 0x55u) * 0x00410410u) & 0x10101010u : (hq & 0x01010101u) << 4;
+        d.lo = (w & 0x0F0F0F0Fu) | bit;
+        d.r[0] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04010400u)), sc2[lo_s], off2[lo_s]);
+    } else if (FMT == 1 && c == 1) {
+        d.r[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04030402u)), sc2[lo_s], off2[lo_s]);
+        const uint32_t bit = ORDER == 0 ? (((hq >> 1) & 0x55u) * 0x00410410u) & 0x10101010u : (hq & 0x02020202u) << 3;
+        d.hi = ((w >> 4) & 0x0F0F0F0Fu) | bit;
+    } else if (c == 0) {
+        d.lo = w & 0x0F0F0F0Fu;
+        d.r[0] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04010400u)), sc2[lo_s], off2[lo_s]);
+    } else if (c == 1) {
+        d.r[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.lo, 0x04030402u)), sc2[lo_s], off2[lo_s]);
+        d.hi = (w >> 4) & 0x0F0F0F0Fu;
+    } else if (c == 2) {
+        d.r[2] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.hi, 0x04010400u)), sc2[hi_s], off2[hi_s]);
+    } else {
+        d.r[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d.hi, 0x04030402u)), sc2[hi_s], off2[hi_s]);
+    }
+}
+
+// -(dmin * mn) split exactly into an f16 head and tail (dmin has 11 significant bits, mn 6).
+__device__ __forceinline__ void neg_min_split(const float dmin, const uint32_t mn, _Float16 &h, _Float16 &l) {
+    const float p = -(dmin * (float)mn);  // exact in fp32
+    h = (_Float16)p;
+    l = (_Float16)(p - (float)h);
+}
+
+constexpr int kGroups16 = 20;  // activation items per row and half super-block: 16 operands and four of sub-block sums
+template <int FMT>
+struct Block16 {  // FMT 2: Q3_K, 3: Q2_K
+    static constexpr int kBytes = FMT == 3 ? 84 : 110, kQs = FMT == 3 ? 16 : 32;
+    static constexpr int kHdrPieces = FMT == 3 ? 2 : 3;           // per row and super-block
+    static constexpr int kHdrRounds = (32 * kHdrPieces + 63) / 64;  // whole-wave copies
+    static constexpr int kHdrStage = 64 * kHdrRounds;              // items of a wave's header stage
+    static __device__ __forceinline__ uint32_t piece_off(int p) { return FMT == 3 ? (p == 0 ? 0u : 68u) : (p == 2 ? 94u : 16u * (uint32_t)p); }
+};
+
+constexpr int kQ6Bytes = 210, kQ6Groups = 16, kQ6Stage = 192;  // LDS items of a wave's quant stage: 128 ql + 64 qh
+
+// The two operands of one k-step, built in eight pieces that are placed between matrix instructions.
+struct Dq6 {
+    uint32_t nlo, nhi, hlo, hhi;
+    half2_t r1[4], r2[4];
+    __device__ __forceinline__ half8_t b1() const { return half8_t{r1[0][0], r1[0][1], r1[1][0], r1[1][1], r1[2][0], r1[2][1], r1[3][0], r1[3][1]}; }
+    __device__ __forceinline__ half8_t b2() const { return half8_t{r2[0][0], r2[0][1], r2[1][0], r2[1][1], r2[2][0], r2[2][1], r2[3][0], r2[3][1]}; }
+};
+// qlw: the ql dword of the k-step; qhw: its qh dword already shifted by 2 g; s2 / s1: (sc, sc) and (16 sc, 16 sc)
+// of the low-nibble and of the high-nibble elements.  0x6400 | v is the f16 1024 + v; both steps of each value are exact.
+__device__ __forceinline__ void dq6_chunk(const int c, const uint32_t qlw, const uint32_t qhw, const half2_t (&s2)[2],
+                                          const half2_t (&s1)[2], Dq6 &d) {
+    const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f}, m1026 = {(_Float16)-1026.0f, (_Float16)-1026.0f};
+    const uint32_t sel = (c & 1) ? 0x04030402u : 0x04010400u;  // bytes (b0, b1) resp. (b2, b3) -> 0x64bb pairs
+    if (c == 0) d.nlo = qlw & 0x0F0F0F0Fu;
+    if (c == 2) d.nhi = (qlw >> 4) & 0x0F0F0F0Fu;
+    if (c == 4) d.hlo = qhw & 0x03030303u;
+    if (c == 6) d.hhi = (qhw >> 4) & 0x03030303u;
+    if (c < 4) {
+        const uint32_t v = c < 2 ? d.nlo : d.nhi;
+        d.r2[c] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + m1024) * s2[c >> 1];
+    } else {
+        const uint32_t v = c < 6 ? d.hlo : d.hhi;
+        d.r1[c - 4] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + m1026) * s1[(c - 4) >> 1];
+    }
+}
+
+// 8 int8 -> 8 exact f16: q + 128 as an unsigned byte b, 0x6400 | b is the f16 1024 + b, minus 1152.
+__device__ __forceinline__ half8_t q8_operand(const uint32_t w0, const uint32_t w1) {
+    const half2_t m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u;
+    const half2_t r0 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u0, 0x04010400u)) + m1152;
+    const half2_t r1 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u0, 0x04030402u)) + m1152;
+    const half2_t r2 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u1, 0x04010400u)) + m1152;
+    const half2_t r3 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u1, 0x04030402u)) + m1152;
+    return half8_t{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
+}
+
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+}  // namespace

@@ -1,0 +1,542 @@
+// Dequant-fused GEMM  Y[m,n] = sum_k X[m,k] * W[n,k]  for a few dozen activation rows, or few weight rows: the waves of a
+// workgroup split K between them.
+//
+// The kernels of gemm.hip give every wave its own weight rows and fill the machine with a K split over workgroups, whose
+// partial tiles a second launch adds: at M = 64 their loop has 0.5 us of matrix work per step and waits for memory in each,
+// and prepare + multiply + add are three dependent launches.  Here a workgroup owns a tile of 32 MB activation rows x 32 NR
+// weight rows for the whole of K.  Its (up to) eight waves take consecutive runs of super-blocks, run without a barrier from
+// start to end, and their fp32 tiles are added through LDS in wave order: no partial tiles in memory, no third launch, and
+// the result does not depend on scheduling.
+//   * Weights: a wave copies a unit of its rows (one or half a super-block of 32 NR rows) directly global -> LDS, one unit
+//     ahead, into LDS of its own; a lane (row n = lane % 32, half g = lane / 32) reads its quants and scales back and
+//     makes the exact f16 operands of gemm_common.hpp.
+//   * Activations: the items of the pre-pass (k_prep_rw) are matrix operands as they lie in memory, so they are loaded
+//     straight into registers, a ring of kDepth k-steps ahead.  Nothing is shared between waves, so LDS would not help.
+//   * Requests return in order, so waiting for a fragment waits for the copies requested before it: the wait in front of a
+//     unit is never longer than that for its first fragments.
+//   * The operands of k-step s + 1 are made between the matrix instructions of step s.
+//
+// What bounds it: a compute unit takes in cold data at about 50 bytes per clock behind a fixed 3800 clocks (a plain
+// read of data that another kernel wrote), and a tile needs (32 MB * 2.25 + 32 NR * bytes per weight) * K of it.
+#include "gemm_common.hpp"
+
+namespace {
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {  // at most N vector-memory requests outstanding
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+
+// p + off with the offset kept in one 32-bit register: a uniform base and a lane offset are one address operand of a load.
+// (Otherwise the compiler widens loop-invariant offsets to 64-bit pairs ahead of the loop: twice the registers.)
+__device__ __forceinline__ const uint8_t *at(const uint8_t *p, uint32_t off) {
+    asm("" : "+v"(off));
+    return p + off;
+}
+
+// 16 bytes per lane from a buffer to LDS (lane l lands at dst + 16 l).  The buffer form and not dma16(): the compiler takes a
+// global load into LDS for an access to either memory and waits for everything outstanding at the next use of any load.
+__device__ __forceinline__ void buf16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint4 *dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, PMH_LPTR(dst), 16, voff, soff, 0, 0);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Formats.  kUnitHalves: halves of a super-block that a unit of copies holds; kPieces: its 16-byte pieces per row, piece p
+// at piece_off(p), moved by half_delta(p) for the second half; slot(p, row): where piece p of a row lies in the staged row
+// (rows whose stride would put them on the same LDS banks are swizzled).  kSums: operand items of sub-block sums per half;
+// kTiles: matrix instructions per fragment (Q6_K's exact split); kFlush: k-steps between two additions of scale * partial
+// sum.
+// ------------------------------------------------------------------------------------------------
+template <int ORDER, int FMT>
+struct KwQ45 {  // FMT 0: Q4_K, 1: Q5_K
+    static constexpr int kBytes = BlockFmt<FMT>::kBytes, kUnitHalves = FMT ? 1 : 2, kPieces = FMT ? 7 : 9, kSums = 1, kTiles = 1,
+                         kFlush = 16;
+    static __device__ __forceinline__ uint32_t piece_off(int p) { return 16u * (uint32_t)p; }
+    static __device__ __forceinline__ uint32_t half_delta(int p) { return FMT && p >= 3 ? 64u : 0u; }
+    static __device__ __forceinline__ int slot(int p, int) { return p; }
+    const uint4 *row_;
+    int g_;
+    uint32_t q[4], qh[4];  // of four k-steps
+    half2_t sc2[2], off2[2];
+    half8_t br;
+    float d;
+    template <int H>
+    __device__ __forceinline__ void load(const uint4 *st, int, const int g) {
+        row_ = st, g_ = g;
+        const uint4 hdr = st[0];
+        // scales and mins of sub-blocks j0 = 4 H + 2 g and j0 + 1 (6-bit fields, crates/pmetal/src/commands/quantize.rs:844-855)
+        const uint32_t sh = 16u * (uint32_t)g;
+        const uint32_t yv = hdr.y >> sh, zv = hdr.z >> sh, wv = hdr.w >> sh;
+        uint32_t sc0, sc1, mn0, mn1;
+        if (H == 0) {
+            sc0 = yv & 63u, sc1 = (yv >> 8) & 63u;
+            mn0 = zv & 63u, mn1 = (zv >> 8) & 63u;
+        } else {
+            sc0 = (wv & 0xFu) | ((yv >> 2) & 0x30u), sc1 = ((wv >> 8) & 0xFu) | ((yv >> 10) & 0x30u);
+            mn0 = ((wv >> 4) & 0xFu) | ((zv >> 2) & 0x30u), mn1 = ((wv >> 12) & 0xFu) | ((zv >> 10) & 0x30u);
+        }
+        const _Float16 s0 = (_Float16)(float)sc0, s1 = (_Float16)(float)sc1;
+        const _Float16 o0 = (_Float16)(-1024.0f * (float)sc0), o1 = (_Float16)(-1024.0f * (float)sc1);  // exact: sc <= 63
+        sc2[0] = half2_t{s0, s0}, sc2[1] = half2_t{s1, s1};
+        off2[0] = half2_t{o0, o0}, off2[1] = half2_t{o1, o1};
+        d = f16_bits_to_f32(hdr.x & 0xFFFFu);
+        const float dmin = f16_bits_to_f32(hdr.x >> 16);
+        _Float16 h0, l0, h1, l1;
+        neg_min_split(dmin, mn0, h0, l0);
+        neg_min_split(dmin, mn1, h1, l1);
+        br = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
+    }
+    template <int H>
+    __device__ __forceinline__ void operands(const int t, half8_t (&b)[1]) {
+        if (t % 4 == 0) {
+            const uint4 v = row_[(FMT ? 3 : 1 + 4 * H) + 2 * g_ + t / 4];
+            q[0] = v.x, q[1] = v.y, q[2] = v.z, q[3] = v.w;
+            if (FMT && ORDER) {  // qh dword t: the same four bytes as quant dword t
+                const uint4 h = row_[1 + t / 4];
+                const uint32_t sh = (uint32_t)(4 * H + 2 * g_);
+                qh[0] = h.x >> sh, qh[1] = h.y >> sh, qh[2] = h.z >> sh, qh[3] = h.w >> sh;
+            } else if (FMT) {  // qh byte 4 (4 H + 2 g) + t
+                qh[0] = reinterpret_cast<const uint32_t *>(row_ + 1)[4 * H + 2 * g_ + t / 4];
+            }
+        }
+        const uint32_t hq = !FMT ? 0u : ORDER ? qh[t % 4] : qh[0] >> (8 * (t & 3));
+        Dq v;
+#pragma unroll
+        for (int c = 0; c < 4; c++) dq_chunk<ORDER, FMT>(c, t, q[t % 4], sc2, off2, v, hq);
+        b[0] = v.value();
+    }
+    __device__ __forceinline__ half8_t sums(int) const { return br; }
+    __device__ __forceinline__ float scale(int) const { return d; }
+};
+
+struct KwQ6 {
+    static constexpr int kBytes = kQ6Bytes, kUnitHalves = 1, kPieces = 8, kSums = 0, kTiles = 2, kFlush = 16;
+    // pieces 0..3: ql, 4, 5: qh, 6: bytes 192..207 (scales), 7: bytes 194..209 (d in the last two)
+    static __device__ __forceinline__ uint32_t piece_off(int p) { return p < 4 ? 16u * (uint32_t)p : p < 6 ? 64u + 16u * (uint32_t)p : 180u + 2u * (uint32_t)p; }
+    static __device__ __forceinline__ uint32_t half_delta(int p) { return p < 4 ? 64u : p < 6 ? 32u : 0u; }
+    static __device__ __forceinline__ int slot(int p, int row) { return p ^ ((row >> 1) & 7); }
+    const uint4 *row_;
+    int i_, g_;
+    uint32_t q[4], h[4];  // of four k-steps
+    half2_t s2[2][2], s1[2][2];
+    float d;
+    template <int H>
+    __device__ __forceinline__ void load(const uint4 *st, const int row, const int g) {
+        row_ = st, i_ = row, g_ = g;
+        const uint4 sv = st[slot(6, row)];
+        d = f16_bits_to_f32(reinterpret_cast<const uint32_t *>(st + slot(7, row))[3] >> 16);
+        // scales 8 H + 2 g + t / 4 (low nibbles) and 8 H + 4 + 2 g + t / 4 (high nibbles)
+        const uint32_t wlo = (H == 0 ? sv.x : sv.z) >> (16u * (uint32_t)g), whi = (H == 0 ? sv.y : sv.w) >> (16u * (uint32_t)g);
+#pragma unroll
+        for (int th = 0; th < 2; th++) {
+            const float fl = (float)(int)(int8_t)(wlo >> (8 * th)), fh = (float)(int)(int8_t)(whi >> (8 * th));
+            const _Float16 l2 = (_Float16)fl, h2 = (_Float16)fh, l1 = (_Float16)(16.0f * fl), h1 = (_Float16)(16.0f * fh);  // exact: |sc| <= 128
+            s2[th][0] = half2_t{l2, l2}, s2[th][1] = half2_t{h2, h2};
+            s1[th][0] = half2_t{l1, l1}, s1[th][1] = half2_t{h1, h1};
+        }
+    }
+    template <int H>
+    __device__ __forceinline__ void operands(const int t, half8_t (&b)[2]) {
+        if (t % 4 == 0) {
+            const uint4 v = row_[slot(2 * g_ + t / 4, i_)], w = row_[slot(4 + t / 4, i_)];
+            const uint32_t hs = 2u * (uint32_t)g_;
+            q[0] = v.x, q[1] = v.y, q[2] = v.z, q[3] = v.w;
+            h[0] = w.x >> hs, h[1] = w.y >> hs, h[2] = w.z >> hs, h[3] = w.w >> hs;
+        }
+        Dq6 v;
+#pragma unroll
+        for (int c = 0; c < 8; c++) dq6_chunk(c, q[t % 4], h[t % 4], s2[t >> 2], s1[t >> 2], v);
+        b[0] = v.b1(), b[1] = v.b2();
+    }
+    __device__ __forceinline__ half8_t sums(int) const { return half8_t{0, 0, 0, 0, 0, 0, 0, 0}; }
+    __device__ __forceinline__ float scale(int) const { return d; }
+};
+
+struct KwQ8 {  // eight 34-byte blocks stand for a super-block; a half (136 bytes) begins 8 bytes into its first piece when it is the second
+    static constexpr int kBytes = 272, kUnitHalves = 1, kPieces = 9, kSums = 0, kTiles = 1, kFlush = 2;
+    static __device__ __forceinline__ uint32_t piece_off(int p) { return 16u * (uint32_t)p; }
+    static __device__ __forceinline__ uint32_t half_delta(int) { return 128u; }
+    static __device__ __forceinline__ int slot(int p, int) { return p; }
+    const uint32_t *p_;
+    int g_;
+    float ds[2];
+    template <int H>
+    __device__ __forceinline__ void load(const uint4 *st, int, const int g) { p_ = reinterpret_cast<const uint32_t *>(st) + 2 * H, g_ = g; }
+    template <int H>
+    __device__ __forceinline__ void operands(const int t, half8_t (&b)[1]) {
+        const int blk = t >> 1, w0 = (34 * blk) / 4;  // block blk starts at this dword (blk even) or two bytes into it
+        const uint32_t *v = p_ + w0 + 4 * (t & 1) + 2 * g_;
+        if (t % 2 == 0) ds[blk % 2] = f16_bits_to_f32((blk & 1 ? p_[w0] >> 16 : p_[w0]) & 0xFFFFu);
+        if (blk & 1) b[0] = q8_operand(v[1], v[2]);
+        else b[0] = q8_operand(__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16));
+    }
+    __device__ __forceinline__ half8_t sums(int) const { return half8_t{0, 0, 0, 0, 0, 0, 0, 0}; }
+    __device__ __forceinline__ float scale(int t) const { return ds[(t >> 1) % 2]; }
+};
+
+template <int FMT>
+struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
+    static constexpr int kBytes = Block16<FMT>::kBytes, kUnitHalves = 2, kPieces = FMT == 3 ? 6 : 7, kSums = 2, kTiles = 1, kFlush = 16;
+    // Q2_K: scales, four of quants, bytes 68..83 (d, dmin in the last dword); Q3_K: two of hmask, four of quants, bytes 94..109
+    static __device__ __forceinline__ uint32_t piece_off(int p) {
+        return FMT == 3 ? (p < 5 ? 16u * (uint32_t)p : 68u) : (p < 6 ? 16u * (uint32_t)p : 94u);
+    }
+    static __device__ __forceinline__ uint32_t half_delta(int) { return 0; }
+    static __device__ __forceinline__ int slot(int p, int) { return p; }
+    uint32_t qd[4], hm[4];
+    half2_t sc2[4], off2[4];
+    half8_t br[2];
+    float d;
+    template <int H>
+    __device__ __forceinline__ void load(const uint4 *st, int, const int g) {
+        const uint4 qv = st[(FMT == 3 ? 1 : 2) + 2 * H + g];
+        qd[0] = qv.x, qd[1] = qv.y, qd[2] = qv.z, qd[3] = qv.w;
+        uint32_t hdr[4], dbits;
+        if (FMT == 3) {
+            const uint4 sc = st[0], dd = st[5];
+            hdr[0] = sc.x, hdr[1] = sc.y, hdr[2] = sc.z, hdr[3] = sc.w;
+            dbits = dd.w;  // d | dmin << 16
+        } else {
+            const uint4 m = st[g], sd = st[6];
+            hm[0] = m.x, hm[1] = m.y, hm[2] = m.z, hm[3] = m.w;  // hmask bytes 16 g ..
+            // the twelve scale bytes as three dwords (they start two bytes into the piece), d behind them
+            hdr[0] = __builtin_amdgcn_alignbit(sd.y, sd.x, 16), hdr[1] = __builtin_amdgcn_alignbit(sd.z, sd.y, 16);
+            hdr[2] = __builtin_amdgcn_alignbit(sd.w, sd.z, 16), hdr[3] = 0;
+            dbits = sd.w >> 16;
+        }
+        d = f16_bits_to_f32(dbits & 0xFFFFu);
+        // scales (and what a sub-block subtracts per unit of its activation sum) of sub-blocks 8 H + 4 sp + 2 lh + g
+        float nm[4];
+#pragma unroll
+        for (int sp = 0; sp < 2; sp++)
+#pragma unroll
+            for (int lh = 0; lh < 2; lh++) {
+                float scf;
+                if (FMT == 3) {
+                    const uint32_t b = (hdr[2 * H + sp] >> (8u * (uint32_t)g + 16u * lh)) & 0xFFu;
+                    scf = (float)(b & 15u);
+                    nm[2 * sp + lh] = -(f16_bits_to_f32(dbits >> 16) * (float)(b >> 4));
+                } else {
+                    const uint32_t lo4 = (hdr[sp] >> (8u * (uint32_t)g + 16u * lh + 4u * H)) & 15u;
+                    const uint32_t hi2 = (hdr[2] >> (8u * (uint32_t)g + 16u * lh + 2u * (2 * H + sp))) & 3u;
+                    scf = (float)((int)(lo4 | (hi2 << 4)) - 32);
+                    nm[2 * sp + lh] = -(d * (4.0f * scf));
+                }
+                const _Float16 sh = (_Float16)scf, oh = (_Float16)(-1024.0f * scf);  // exact: |sc| <= 32
+                sc2[2 * sp + lh] = half2_t{sh, sh}, off2[2 * sp + lh] = half2_t{oh, oh};
+            }
+#pragma unroll
+        for (int sp = 0; sp < 2; sp++) {
+            const _Float16 h0 = (_Float16)nm[2 * sp], h1 = (_Float16)nm[2 * sp + 1];
+            const _Float16 l0 = (_Float16)(nm[2 * sp] - (float)h0), l1 = (_Float16)(nm[2 * sp + 1] - (float)h1);
+            br[sp] = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
+        }
+        if (FMT == 2) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) hm[i] >>= 4 * H;
+        }
+    }
+    template <int H>
+    __device__ __forceinline__ void operands(const int t, half8_t (&b)[1]) {
+        const int dw = t >> 1, sp = t & 1;
+        uint32_t lo = (qd[dw] >> (4 * sp)) & 0x03030303u, hi = (qd[dw] >> (4 * sp + 2)) & 0x03030303u;
+        if (FMT == 2) {
+            const uint32_t m = hm[dw] >> (2 * sp);
+            lo |= (m & 0x01010101u) << 2, hi |= (m & 0x02020202u) << 1;
+        }
+        const half2_t r0 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u)), sc2[2 * sp], off2[2 * sp]);
+        const half2_t r1 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u)), sc2[2 * sp], off2[2 * sp]);
+        const half2_t r2 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u)), sc2[2 * sp + 1], off2[2 * sp + 1]);
+        const half2_t r3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u)), sc2[2 * sp + 1], off2[2 * sp + 1]);
+        b[0] = half8_t{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
+    }
+    __device__ __forceinline__ half8_t sums(int i) const { return br[i]; }
+    __device__ __forceinline__ float scale(int) const { return d; }
+};
+
+// ------------------------------------------------------------------------------------------------
+constexpr int kKwWaves = 8;
+
+template <class F, int MB, int NR>
+struct Kw {
+    static constexpr int kItems = 32 * NR * F::kPieces, kCopies = (kItems + 63) / 64;  // 16-byte pieces of a unit, whole-wave copies
+    static constexpr int kSteps = 8 + F::kSums;                                        // k-steps and sum steps of a half
+    // k-steps of activation fragments in flight: a divisor of the steps of a super-block
+    static constexpr int kDepth = F::kSums == 1 ? 6 : F::kSums == 2 ? (MB * NR == 4 ? 4 : 5) : (MB * NR == 4 ? 2 : 4);
+    static constexpr int kTile = MB * NR * 4 * 64;                                     // 16-byte slots of a wave's fp32 tile
+    static_assert((2 * kSteps) % kDepth == 0, "the ring's slots are picked at compile time");
+    static_assert(kDepth <= 8, "a unit's copies must be older than the fragments in flight when it is used");
+};
+
+template <class F, int MB, int NR>
+struct KwCopy {  // a wave's copies of one unit
+    uint32_t off[Kw<F, MB, NR>::kCopies];
+    uint32_t by64 = 0, by32 = 0;  // bit j: copy j of this lane moves by 64, by 32 bytes for the second half (Q8_0: all by 128)
+    template <int H>
+    __device__ __forceinline__ void issue(const __amdgpu_buffer_rsrc_t r, const uint32_t sb_off, uint4 *dst, const int lane) const {
+        using K = Kw<F, MB, NR>;
+#pragma unroll
+        for (int j = 0; j < K::kCopies; j++)
+            if (64 * j + 64 <= K::kItems || 64 * j + lane < K::kItems) {
+                uint32_t o = off[j];
+                if (H && F::kFlush > 2) {
+                    uint32_t a = by64, b = by32;
+                    asm("" : "+v"(a), "+v"(b));  // (made anew for each unit: kept sums would be a second set of offsets in registers)
+                    o += ((a >> j & 1u) << 6) + ((b >> j & 1u) << 5);
+                }
+                buf16(r, o, H && F::kFlush == 2 ? sb_off + 128u : sb_off, dst + 64 * j);
+            }
+    }
+};
+
+// Half H of a super-block.  cur: the staged unit; nxt: where the copies of the next unit go (half HN of the super-block at
+// sb_next of every row); xa: the items of the k-step whose fragments are requested next.
+template <class F, int MB, int NR, int H, bool NEXT>
+__device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__restrict__ nxt, const __amdgpu_buffer_rsrc_t r, const uint32_t sb_next,
+                                        const KwCopy<F, MB, NR> &C, const uint8_t *__restrict__ &xa, const uint32_t step, const uint32_t a_off,
+                                        half8_t (&af)[Kw<F, MB, NR>::kDepth][MB], const int lane, float16_t (&acc)[NR][MB], float16_t (&part)[NR][MB]) {
+    using K = Kw<F, MB, NR>;
+    const int col = lane & 31, g = lane >> 5;
+    constexpr bool kNewUnit = F::kUnitHalves == 1 || H == 0;
+    if (kNewUnit) wait_vm<K::kDepth * MB>();  // what is newer than this unit's copies is in the ring of fragments
+    F op[NR];
+#pragma unroll
+    for (int rg = 0; rg < NR; rg++) op[rg].template load<H>(cur + (32 * rg + col) * F::kPieces, 32 * rg + col, g);
+    if (kNewUnit && NEXT) {
+        __builtin_amdgcn_sched_barrier(0);
+        C.template issue<F::kUnitHalves == 1 && H == 0 ? 1 : 0>(r, sb_next, nxt, lane);
+    }
+    half8_t b[NR][F::kTiles];
+#pragma unroll
+    for (int rg = 0; rg < NR; rg++) op[rg].template operands<H>(0, b[rg]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < K::kSteps; s++) {
+        const int slot = (H * K::kSteps + s) % K::kDepth;
+        half8_t bn[NR][F::kTiles];
+        if (s + 1 < K::kSteps) {
+#pragma unroll
+            for (int rg = 0; rg < NR; rg++) {
+                if (s + 1 < 8) op[rg].template operands<H>(s + 1, bn[rg]);
+                else bn[rg][0] = op[rg].sums(s + 1 - 8);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int rg = 0; rg < NR; rg++) {
+                const half8_t a = af[slot][i];
+                if (s >= 8) {
+                    acc[rg][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[rg][0], acc[rg][i], 0, 0, 0);
+                } else {
+#pragma unroll
+                    for (int tl = 0; tl < F::kTiles; tl++) {
+                        if ((8 * H + s) % F::kFlush == 0 && tl == 0) {  // the first product behind a flush starts from zero
+                            float16_t z;
+#pragma unroll
+                            for (int e = 0; e < 16; e++) z[e] = 0.0f;
+                            part[rg][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[rg][tl], z, 0, 0, 0);
+                        } else {
+                            part[rg][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[rg][tl], part[rg][i], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+        // the slot takes the fragments of kDepth steps on (past the last step: items of another wave, or the slack behind them)
+#pragma unroll
+        for (int i = 0; i < MB; i++) af[slot][i] = *reinterpret_cast<const half8_t *>(at(xa, a_off) + 512 * i);
+        xa += step;
+        if (s + 1 < 8) {  // issue order: a matrix instruction, then the vector instructions that fit behind it
+#pragma unroll
+            for (int e = 0; e < MB * NR * F::kTiles; e++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, F::kTiles == 2 ? (16 + MB - 1) / MB : (11 + MB - 1) / MB, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (s < 8 && (8 * H + s + 1) % F::kFlush == 0) {
+#pragma unroll
+            for (int rg = 0; rg < NR; rg++) {
+                const float d = op[rg].scale(s);
+#pragma unroll
+                for (int i = 0; i < MB; i++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[rg][i][e] = __builtin_fmaf(d, part[rg][i][e], acc[rg][i][e]);
+                if (F::kFlush < 16)  // (added here and not where the sums are next used: the partial sums would stay in registers until then)
+#pragma unroll
+                    for (int i = 0; i < MB; i++) asm volatile("" : "+v"(acc[rg][i]));
+            }
+        }
+#pragma unroll
+        for (int rg = 0; rg < NR; rg++)
+#pragma unroll
+            for (int tl = 0; tl < F::kTiles; tl++) b[rg][tl] = bn[rg][tl];
+    }
+}
+
+// grid (8, blocks of activation rows x splits of K, groups of eight tiles of weight rows), up to eight waves; wave w of split z
+// takes super-blocks [z * chunk + w * per, + per) below min(spr, (z + 1) * chunk).  The blocks of activation rows of one tile of weights are eight workgroups apart, so on one die.
+template <class F, int MB, int NR>
+__global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
+                                                             const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
+                                                             int spr, int per, int chunk, int mblocks, int tiles, int ybf16,
+                                                             float *__restrict__ partial) {
+    using K = Kw<F, MB, NR>;
+    extern __shared__ uint4 smem[];
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = (int)(blockDim.x >> 6);
+    const int nt = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / mblocks, m0 = ((int)blockIdx.y - z * mblocks) * (32 * MB);
+    if (nt >= tiles) return;  // (the whole workgroup)
+    const int n0 = nt * (32 * NR);
+    int sb0 = z * chunk + wave * per, cnt = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - sb0;
+    const bool idle = cnt < 1;  // the last split is the shortest: a wave left without work multiplies one super-block for nothing
+    sb0 = idle ? 0 : sb0, cnt = idle ? 1 : cnt < per ? cnt : per;
+    const uint32_t row_bytes = (uint32_t)spr * F::kBytes;
+    KwCopy<F, MB, NR> C;
+#pragma unroll
+    for (int j = 0; j < K::kCopies; j++) {
+        int idx = lane + 64 * j;
+        idx = idx < K::kItems ? idx : K::kItems - 1;
+        const int row = idx / F::kPieces, p = F::slot(idx % F::kPieces, row);  // (the swizzle is its own inverse)
+        int n = n0 + row;
+        n = n < N ? n : N - 1;  // rows past the last repeat it
+        C.off[j] = (uint32_t)(n - n0) * row_bytes + F::piece_off(p);
+        C.by64 |= (F::half_delta(p) >> 6 & 1u) << j, C.by32 |= (F::half_delta(p) >> 5 & 1u) << j;
+    }
+    uint4 *st0 = smem + wave * (2 * K::kItems), *st1 = st0 + K::kItems;
+    uint32_t sb_off = (uint32_t)sb0 * F::kBytes;
+    const size_t left = (size_t)(N - n0) * row_bytes;
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W + (size_t)n0 * row_bytes), 0, (int)(left < 0xFFFFFFF0u ? left : 0xFFFFFFF0u), 0x00027000);
+    const uint32_t step = 32u * (uint32_t)Mp, a_off = (uint32_t)(g * Mp + m0 + col) * 16u;
+    const uint8_t *xa = reinterpret_cast<const uint8_t *>(xs) + (size_t)(sb0 * 2 * K::kSteps) * step;
+    C.template issue<0>(r, sb_off, st0, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    half8_t af[Kw<F, MB, NR>::kDepth][MB];
+#pragma unroll
+    for (int s = 0; s < K::kDepth; s++) {
+#pragma unroll
+        for (int i = 0; i < MB; i++) af[s][i] = *reinterpret_cast<const half8_t *>(at(xa, a_off) + 512 * i);
+        xa += step;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const float rs_mine = lane < 32 * MB ? rowscale[m0 + lane] : 0.0f;
+    float16_t acc[NR][MB], part[NR][MB];
+#pragma unroll
+    for (int rg = 0; rg < NR; rg++)
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[rg][i][e] = 0.0f, part[rg][i][e] = 0.0f;
+    for (int s = 0; s + 1 < cnt; s++) {
+        if (F::kUnitHalves == 1) {
+            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+            sb_off += F::kBytes;
+            kw_half<F, MB, NR, 1, true>(st1, st0, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+        } else {
+            sb_off += F::kBytes;
+            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+            kw_half<F, MB, NR, 1, true>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+            uint4 *t = st0;
+            st0 = st1, st1 = t;
+        }
+    }
+    kw_half<F, MB, NR, 0, F::kUnitHalves == 1>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+    kw_half<F, MB, NR, 1, false>(F::kUnitHalves == 1 ? st1 : st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+
+    // The waves' tiles are added in wave order: slot (rg, block i, quarter q, lane) holds rows 8 q + 4 g .. + 3 of block i
+    wait_vm<0>();
+    __syncthreads();
+    float4_t *red = reinterpret_cast<float4_t *>(smem);
+    float *rs = reinterpret_cast<float *>(smem) + (size_t)nwaves * K::kTile * 4;
+#pragma unroll
+    for (int rg = 0; rg < NR; rg++)
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                red[wave * K::kTile + ((rg * MB + i) * 4 + q) * 64 + lane] =
+                    idle ? float4_t{0.0f, 0.0f, 0.0f, 0.0f}
+                         : float4_t{acc[rg][i][4 * q], acc[rg][i][4 * q + 1], acc[rg][i][4 * q + 2], acc[rg][i][4 * q + 3]};
+    if (wave == 0 && lane < 32 * MB) rs[lane] = rs_mine;
+    __syncthreads();
+    constexpr int kTrips = (K::kTile + 64 * kKwWaves - 1) / (64 * kKwWaves);  // with all eight waves
+    for (int base = tid; base < K::kTile; base += kTrips * (int)blockDim.x) {
+#pragma unroll
+        for (int j = 0; j < kTrips; j++) {
+            const int idx = base + j * (int)blockDim.x;
+            if (idx >= K::kTile) break;
+            const int l = idx & 63, t = idx >> 6, q = t & 3, i = (t >> 2) % MB, rg = (t >> 2) / MB;
+            const int n = n0 + 32 * rg + (l & 31), ml = 32 * i + 8 * q + 4 * (l >> 5), m = m0 + ml;
+            float4_t u[kKwWaves];
+#pragma unroll
+            for (int w = 0; w < kKwWaves; w++) u[w] = red[(w < nwaves ? w : 0) * K::kTile + idx];
+            float4_t v = u[0];
+#pragma unroll
+            for (int w = 1; w < kKwWaves; w++)
+                if (w < nwaves) v += u[w];
+            if (!partial) v *= *reinterpret_cast<const float4_t *>(rs + ml);
+            if (n < N) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (m + e >= M) continue;
+                    if (partial) partial[((size_t)z * Mp + m + e) * N + n] = v[e];
+                    else if (ybf16) reinterpret_cast<uint16_t *>(yg)[(size_t)(m + e) * N + n] = (uint16_t)bf16_rne_bits(v[e]);
+                    else reinterpret_cast<float *>(yg)[(size_t)(m + e) * N + n] = v[e];
+                }
+            }
+        }
+    }
+}
+
+}  // namespace
+
+namespace pmh {
+
+template <class F, int MB, int NR>
+static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n, int spr,
+                            float *partial, hipStream_t s) {
+    using K = Kw<F, MB, NR>;
+    auto kern = k_qgemm_kw<F, MB, NR>;
+    const int per = (p.chunk + kKwWaves - 1) / kKwWaves, nwaves = (p.chunk + per - 1) / per;
+    const size_t stage = (size_t)nwaves * 2 * K::kItems * 16, red = (size_t)nwaves * K::kTile * 16 + 32 * MB * 4, lds = stage > red ? stage : red;
+    static_assert((size_t)kKwWaves * 2 * K::kItems * 16 <= 160 * 1024 && (size_t)kKwWaves * K::kTile * 16 + 32 * MB * 4 <= 160 * 1024, "LDS");
+    if (lds > 64 * 1024) {
+        hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (a != hipSuccess) return a;
+    }
+    const int tiles = (int)((n + 32 * NR - 1) / (32 * NR)), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
+    const dim3 grid(8, (unsigned)(mblocks * p.splits), (unsigned)((tiles + 7) / 8));
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, per, p.chunk, mblocks, tiles, y_bf16 ? 1 : 0,
+                       p.splits > 1 ? partial : nullptr);
+    return hipGetLastError();
+}
+
+template <class F>
+static hipError_t launch_kw_tile(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n,
+                                 int spr, float *partial, hipStream_t s) {
+    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
+    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
+    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
+    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
+}
+
+hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &p, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
+                           int64_t n, int spr, uint32_t order, float *partial, hipStream_t s) {
+    const uint4 *x4 = reinterpret_cast<const uint4 *>(xs);
+    const bool ref = order == kOrderRef;
+    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, s); };
+    switch (type) {
+    case kTypeQ4K: return ref ? go(KwQ45<0, 0>{}) : go(KwQ45<1, 0>{});
+    case kTypeQ5K: return ref ? go(KwQ45<0, 1>{}) : go(KwQ45<1, 1>{});
+    case kTypeQ6K: return go(KwQ6{});
+    case kTypeQ8_0: return go(KwQ8{});
+    case kTypeQ3K: return go(KwQ23<2>{});
+    case kTypeQ2K: return go(KwQ23<3>{});
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace pmh

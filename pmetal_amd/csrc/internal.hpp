@@ -60,11 +60,18 @@ hipError_t launch_qgemv_q4k_q6k_group(const uint8_t *const *w, const int64_t *n,
 hipError_t launch_qgemv_q4k_group(const uint8_t *const *w, const int64_t *n, float *const *y, int count, int64_t k,
                                   const void *x, uint32_t x_dtype, uint32_t order, hipStream_t s);
 
-// ---- gemm.hip: dequant-fused Y = X W^T for Q4_K and Q6_K (every wave owns 32 weight rows) ----
+// ---- gemm.hip, gemm_kw.hip: dequant-fused Y = X W^T ----
+enum class GemmKernel {
+    kSmall,  // gemm.hip, k_qgemm_small*: the weights stream past activations held in registers (at most 32 rows)
+    kWaves,  // gemm_kw.hip: a tile of Y per workgroup, K split between its waves
+    kRows,   // gemm.hip, k_qgemm_rw*: every wave owns 32 weight rows, activations shared through LDS
+};
 struct GemmPlan {
-    int mb;      // 32-row activation blocks per workgroup (1, 2 or 4)
-    int mp;      // activation rows padded to a multiple of 32 mb
-    int nw;      // waves per workgroup
+    GemmKernel kernel;
+    int mb;      // 32-row activation blocks per workgroup (kRows: 1, 2 or 4; kWaves: 1 or 2)
+    int nr;      // kWaves: 32-row blocks of weights per workgroup (1 or 2)
+    int mp;      // padded activation rows, a multiple of 32 mb
+    int nw;      // kRows: waves per workgroup
     int splits;  // workgroups along K (more than one: partial tiles plus a reduction kernel)
     int chunk;   // super-blocks per split
 };
@@ -78,6 +85,10 @@ size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k);
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,
                         int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s,
                         bool reuse_prepass = false);
+
+// gemm_kw.hip (spr: super-blocks per row; partial: fp32 tiles [splits][mp][n] when plan.splits > 1, not scaled by rowscale)
+hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &plan, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
+                           int64_t n, int spr, uint32_t order, float *partial, hipStream_t s);
 
 // ---- q8k.hip: Q8_K activation blocks and the integer dot products over them ----
 hipError_t launch_quantize_q8k(const float *x, size_t n, uint8_t *dst, hipStream_t s);

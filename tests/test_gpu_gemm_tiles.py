@@ -1,0 +1,48 @@
+"""GPU parity of the tile GEMM (gemm_kw.hip): a workgroup owns a tile of Y and its waves split K."""
+import numpy as np
+import pytest
+
+import pmetal_amd as pm
+from gpu_util import Q4K, Q6K, Q8_0
+from test_gpu_gemm import gpu_qgemm, reference
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = {Q4K: 144, Q6K: 210, Q8_0: 34, 13: 176, 11: 110, 10: 84}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    pm.init(0)
+
+
+def random_blocks(rng, t, n, k):
+    """Every scale, min and quant pattern; d (and dmin) of ordinary size and, where the format allows it, of both signs."""
+    raw = rng.integers(0, 256, size=(n * (k // (32 if t == Q8_0 else 256)), BLOCK[t]), dtype=np.uint8)
+    d = (rng.uniform(0.5, 2.0, (raw.shape[0], 2)) * 0.01 * rng.choice([-1.0, 1.0], (raw.shape[0], 2))).astype(np.float16).view(np.uint8)
+    at = {Q4K: 0, 13: 0, Q6K: 208, Q8_0: 0, 11: 108, 10: 80}[t]
+    width = 4 if t in (Q4K, 13, 10) else 2
+    raw[:, at:at + width] = d[:, :width]
+    return raw.reshape(-1)
+
+
+# (m, n, k): one weight row, one super-block; edges of the 32- and 64-row blocks of both sides; rows of 7, 8, 9 and 17
+# super-blocks (waves of equal and of different length); a narrow weight with long rows (K split over workgroups, the last
+# split shorter than the others); enough tiles for more than one round of workgroups
+@pytest.mark.parametrize("m,n,k", [(17, 1, 256), (32, 31, 1792), (33, 33, 2048), (64, 64, 2304), (65, 65, 4352), (63, 97, 512),
+                                   (48, 40, 18688), (29, 70, 33024), (130, 1000, 1024), (200, 4100, 768)])
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k):
+    rng = np.random.default_rng(7 * t + m + n + k)
+    raw = random_blocks(rng, t, n, k)
+    bits = oracle.f32_to_bf16_bits(rng.standard_normal(m * k).astype(np.float32)).reshape(m, k)
+    x = oracle.bf16_bits_to_f32(bits.reshape(-1)).reshape(m, k)
+    for order in (0, 1) if t in (Q4K, 13) else (0,):
+        want = reference(oracle, t, raw, n, k, x, order)
+        got = gpu_qgemm(t, raw, n, k, bits, m, order=order)
+        # bf16 activations and the integer weight tiles are exact; what is left are at most k / 16 + 16 additions in f32 on
+        # partial sums within four times the largest result
+        bound = (k / 16 + 16) * 2.0 ** -24 * 4
+        assert np.max(np.abs(got - want)) <= bound * np.max(np.abs(want)), order
+        got16 = gpu_qgemm(t, raw, n, k, bits, m, y_dtype=pm.DTYPE_BF16, order=order)
+        assert np.max(np.abs(got16 - want)) <= (2.0 ** -8 + bound) * np.max(np.abs(want)), order
