@@ -33,7 +33,7 @@ EXTRA = {
     "gemv_q5k.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "gemv_q6k.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "gemv_q8_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
-    "gemm.hip": [],
+    "gemm.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "gemm_kw.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "q8k.hip": ["-ffp-contract=off", "-fno-gpu-flush-denormals-to-zero"],
     "util.hip": [],

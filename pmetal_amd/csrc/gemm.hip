@@ -201,6 +201,10 @@ constexpr size_t tile_lds_bytes() {
 }
 
 
+struct __attribute__((packed, aligned(2))) u32x4_a2 {
+    uint32_t x, y, z, w;
+};
+
 template <int MB, int NW = 8>
 __device__ __forceinline__ void store_tile(const float16_t (&acc)[MB], uint4 *smem, const int wave, const int col, const int g,
                                            const int m0, const int n0, const int M, const int N, const int Mp,
@@ -247,6 +251,8 @@ __device__ __forceinline__ void store_tile(const float16_t (&acc)[MB], uint4 *sm
             // other row blocks' weights out of the caches (a partial tile is read back by the reduction: an ordinary store)
             if (mode == 2) *reinterpret_cast<uint4 *>(dst) = pack;
             else __builtin_nontemporal_store(u32x4{pack.x, pack.y, pack.z, pack.w}, reinterpret_cast<u32x4 *>(dst));
+        } else if (n + per <= N) {  // rows that start off 16-byte boundaries (N ragged): the same store at the alignment of an output
+            *reinterpret_cast<u32x4_a2 *>(dst) = u32x4_a2{pack.x, pack.y, pack.z, pack.w};
         } else {
             for (int e = 0; e < per && n + e < N; e++) {
                 if (mode == 1) reinterpret_cast<uint16_t *>(dst)[e] = (uint16_t)bf16_rne_bits(v[e]);
@@ -1179,24 +1185,29 @@ __device__ __forceinline__ void small_add_kept(const float4_t *keep, int n_tiles
     }
 }
 
-// After the last tile: y[m][16 t0 + j] for j over the workgroup's columns (consecutive threads store consecutive columns of
-// one row), scaled by the rows' powers of two; or, when a long row is cut into runs over the grid's second dimension,
-// the fp32 partial tile of this run, not yet scaled, for k_rw_reduce.
+// After the last tile: the finished tiles leave, scaled by the rows' powers of two (`rs`: that of row `lane`, requested when the
+// kernel starts: asked for here it would be a trip to memory at the kernel's end); or, when a long row is cut into runs over
+// the grid's second dimension, as the fp32 partial tile of this run, not yet scaled, for k_rw_reduce.  A thread takes a lane
+// slot: four rows of one column.
 // (mt: 16-row blocks of activations per row tile of weights; the finished tile of block b of row tile ti is slot ti * mt + b)
-__device__ __forceinline__ void small_store(const float4_t *out_tiles, int t0, int t1, int M, int Mp, int N,
-                                            const float *__restrict__ rowscale, void *__restrict__ yg, int ybf16,
-                                            float *__restrict__ partial, const int mt = 1) {
+__device__ __forceinline__ float small_row_scale(const float *__restrict__ rowscale) { return rowscale[threadIdx.x & 31]; }
+
+__device__ __forceinline__ void small_store(const float4_t *out_tiles, int t0, int t1, int M, int Mp, int N, const float rs,
+                                            void *__restrict__ yg, int ybf16, float *__restrict__ partial, const int mt = 1) {
+    __shared__ float scales[32];
+    if (threadIdx.x < 32) scales[threadIdx.x] = rs;
     __syncthreads();
-    const int cols = (t1 - t0) * 16;
-    for (int idx = (int)threadIdx.x; idx < M * cols; idx += (int)blockDim.x) {
-        const int m = idx / cols, j = idx - m * cols;
-        const int n = t0 * 16 + j;
-        if (n < N) {
-            const float sum = out_tiles[((j >> 4) * mt + (m >> 4)) * 64 + ((m & 15) >> 2) * 16 + (j & 15)][m & 3];
-            const float o = sum * rowscale[m];
-            if (partial) partial[((size_t)blockIdx.y * Mp + m) * N + n] = sum;
-            else if (ybf16) reinterpret_cast<uint16_t *>(yg)[(size_t)m * N + n] = (uint16_t)bf16_rne_bits(o);
-            else reinterpret_cast<float *>(yg)[(size_t)m * N + n] = o;
+    for (int idx = (int)threadIdx.x; idx < (t1 - t0) * mt * 64; idx += (int)blockDim.x) {
+        const int tile = mt == 1 ? idx >> 6 : idx >> 7, b = mt == 1 ? 0 : (idx >> 6) & 1, l = idx & 63;
+        const int n = (t0 + tile) * 16 + (l & 15), m = 16 * b + 4 * (l >> 4);
+        const float4_t v = out_tiles[idx], o = v * *reinterpret_cast<const float4_t *>(scales + m);
+        if (n >= N) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            if (m + r >= M) break;
+            if (partial) partial[((size_t)blockIdx.y * Mp + m + r) * N + n] = v[r];
+            else if (ybf16) reinterpret_cast<uint16_t *>(yg)[(size_t)(m + r) * N + n] = (uint16_t)bf16_rne_bits(o[r]);
+            else reinterpret_cast<float *>(yg)[(size_t)(m + r) * N + n] = o[r];
         }
     }
 }
@@ -1219,6 +1230,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
                                                                    float *__restrict__ partial) {
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64]: lane slots of the finished tiles; then the waves' stages
+    const float rs = small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1362,7 +1374,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
         issue(2 * rd + 3, ring1);
     }
     small_add_kept(keep, rounds * kSmallDepth * MT, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rowscale, yg, ybf16, partial, MT);
+    small_store(out_tiles, t0, t1, M, Mp, N, rs, yg, ybf16, partial, MT);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1390,6 +1402,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
                                                                    float *__restrict__ partial) {
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
+    const float rs = small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1499,7 +1512,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
         issue(2 * rd + 3, ring1a, ring1b);
     }
     small_add_kept(keep, rounds * kSmallDepth * MT, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rowscale, yg, ybf16, partial, MT);
+    small_store(out_tiles, t0, t1, M, Mp, N, rs, yg, ybf16, partial, MT);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1542,6 +1555,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
     constexpr int P = SmallQ6<NSB, ANY>::kRowPieces, kLoads = SmallQ6<NSB, ANY>::kLoads;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
+    const float rs = small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1667,55 +1681,55 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
         issue(2 * rd + 3, ring1);
     }
     small_add_kept(keep, rounds * kSmallDepth, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rowscale, yg, ybf16, partial);
+    small_store(out_tiles, t0, t1, M, Mp, N, rs, yg, ybf16, partial);
 }
 
-// y[m][n] = rowscale[m] * (partial[0][m][n] + partial[1][m][n] + ...), added in this order
-template <bool YBF16>
+// y[m][n] = rowscale[m] * (partial[0][m][n] + partial[1][m][n] + ...), added in this order.  A thread takes PER consecutive
+// outputs of the row-major result, whatever the row length: eight, in 16-byte accesses (rows of a length that is no multiple
+// of 8 went one output per thread: with the tile store's wide form for them 4674 x 1024 at M = 829 39.8 -> 29.9 us a call), or
+// one where the result is small and the kernel is the time of one trip to memory (7 x 1661: 1.5 us longer with eight).
+template <bool YBF16, int PER>
 __global__ __launch_bounds__(256) void k_rw_reduce(const float *__restrict__ partial, int splits, int M, int Mp, int N,
                                                     const float *__restrict__ rowscale, void *__restrict__ yg) {
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (size_t)M * N) return;
-    const int m = (int)(idx / N);
+    const size_t first = (size_t)blockIdx.x * (256 * PER), total = (size_t)M * N, idx = first + threadIdx.x * PER;
+    if (idx >= total) return;
+    // the row of the first output, and how far into it (the 64-bit division once per workgroup, in scalar registers)
+    const uint32_t m_first = (uint32_t)(first / (uint32_t)N);
+    const uint32_t at = (uint32_t)(first - (size_t)m_first * (uint32_t)N) + threadIdx.x * PER;
+    const uint32_t m = m_first + at / (uint32_t)N, col = at % (uint32_t)N;
     const size_t plane = (size_t)Mp * N;
-    float s = partial[idx];
-    for (int z = 1; z < splits; z++) s += partial[(size_t)z * plane + idx];
-    const float v = s * rowscale[m];
-    if (YBF16) {
-        uint32_t u = __builtin_bit_cast(uint32_t, v);
-        u = ((u & 0x7FFFFFFFu) > 0x7F800000u) ? ((u >> 16) | 0x40u) : ((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-        reinterpret_cast<uint16_t *>(yg)[idx] = (uint16_t)u;
+    auto one = [&](const int e) {  // output idx + e: its row may be a later one
+        float t = partial[idx + e];
+        for (int z = 1; z < splits; z++) t += partial[(size_t)z * plane + idx + e];
+        t *= rowscale[m + (col + e) / (uint32_t)N];
+        if (YBF16) reinterpret_cast<uint16_t *>(yg)[idx + e] = (uint16_t)bf16_rne_bits(t);
+        else reinterpret_cast<float *>(yg)[idx + e] = t;
+    };
+    if (PER == 1) {
+        one(0);
+    } else if (total - idx < 8 || N < 8) {
+        for (int e = 0; e < 8 && idx + e < total; e++) one(e);
     } else {
-        reinterpret_cast<float *>(yg)[idx] = v;
-    }
-}
-
-// The same over eight consecutive outputs of one row per thread (N a multiple of 8): 16-byte loads and stores.
-template <bool YBF16>
-__global__ __launch_bounds__(256) void k_rw_reduce8(const float *__restrict__ partial, int splits, int M, int Mp, int N,
-                                                     const float *__restrict__ rowscale, void *__restrict__ yg) {
-    const size_t idx = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
-    if (idx >= (size_t)M * N) return;
-    const int m = (int)(idx / N);
-    const size_t plane = (size_t)Mp * N;
-    const float4 *p = reinterpret_cast<const float4 *>(partial + idx);
-    float4 a = p[0], b = p[1];
-    for (int z = 1; z < splits; z++) {
-        const float4 *q = reinterpret_cast<const float4 *>(partial + (size_t)z * plane + idx);
-        const float4 c = q[0], d = q[1];
-        a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
-        b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
-    }
-    const float sc = rowscale[m];
-    const float v[8] = {a.x * sc, a.y * sc, a.z * sc, a.w * sc, b.x * sc, b.y * sc, b.z * sc, b.w * sc};
-    if (YBF16) {
-        *reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(yg) + idx) =
-            make_uint4(bf16_rne_bits(v[0]) | (bf16_rne_bits(v[1]) << 16), bf16_rne_bits(v[2]) | (bf16_rne_bits(v[3]) << 16),
-                       bf16_rne_bits(v[4]) | (bf16_rne_bits(v[5]) << 16), bf16_rne_bits(v[6]) | (bf16_rne_bits(v[7]) << 16));
-    } else {
-        float4 *o = reinterpret_cast<float4 *>(reinterpret_cast<float *>(yg) + idx);
-        o[0] = make_float4(v[0], v[1], v[2], v[3]);
-        o[1] = make_float4(v[4], v[5], v[6], v[7]);
+        const float s0 = rowscale[m], s1 = rowscale[m + 1 < (uint32_t)M ? m + 1 : m];  // at most one row ends among the eight
+        float4 a = reinterpret_cast<const float4 *>(partial + idx)[0], b = reinterpret_cast<const float4 *>(partial + idx)[1];
+        for (int z = 1; z < splits; z++) {
+            const float4 *q = reinterpret_cast<const float4 *>(partial + (size_t)z * plane + idx);
+            const float4 c = q[0], d = q[1];
+            a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
+            b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
+        }
+        float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] *= col + e < (uint32_t)N ? s0 : s1;
+        if (YBF16) {
+            *reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(yg) + idx) =
+                make_uint4(bf16_rne_bits(v[0]) | (bf16_rne_bits(v[1]) << 16), bf16_rne_bits(v[2]) | (bf16_rne_bits(v[3]) << 16),
+                           bf16_rne_bits(v[4]) | (bf16_rne_bits(v[5]) << 16), bf16_rne_bits(v[6]) | (bf16_rne_bits(v[7]) << 16));
+        } else {
+            float4 *o = reinterpret_cast<float4 *>(reinterpret_cast<float *>(yg) + idx);
+            o[0] = make_float4(v[0], v[1], v[2], v[3]);
+            o[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
     }
 }
 
@@ -1764,6 +1778,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
     using B = Block16<FMT>;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the kept partial tiles
+    const float rs = small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1906,7 +1921,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         issue(2 * rd + 3, ring1);
     }
     small_add_kept(keep, rounds * kSmallDepth, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rowscale, yg, ybf16, partial);
+    small_store(out_tiles, t0, t1, M, Mp, N, rs, yg, ybf16, partial);
 }
 
 }  // namespace
@@ -1958,8 +1973,8 @@ bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
 }
 
 // The tile kernel's best tile and K split for a shape, and the microseconds it is expected to take behind the pre-pass.  Fitted
-// to 1400 measured times (rms 12 %): per round of 256 workgroups a wave's super-blocks cost 1/113 us per KB of activations and
-// 1/41 us per KB of weights the workgroup takes in, plus 0.7 us per 32 x 32 tile (twice the matrix instructions for Q6_K).
+// to 1500 measured times (rms 12 %): per round of 256 workgroups a wave's super-blocks cost 1/124 us per KB of activations and
+// 1/34 us per KB of weights the workgroup takes in, plus 0.8 us per 32 x 32 tile (Q6_K has twice the matrix instructions).
 struct KwChoice {
     int mb, nr, splits;
     double us, rounds;
@@ -1967,7 +1982,7 @@ struct KwChoice {
 static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
     const double block = type == kTypeQ4K ? 144 : type == kTypeQ5K ? 176 : type == kTypeQ6K ? 210 : type == kTypeQ8_0 ? 272 : type == kTypeQ3K ? 110 : 84;
     const double items = type == kTypeQ3K || type == kTypeQ2K ? 40 : type == kTypeQ6K || type == kTypeQ8_0 ? 32 : 36;  // per row and super-block
-    const double cost = type == kTypeQ6K ? 2.0 : type == kTypeQ8_0 ? 1.5 : 1.0;
+    const double cost = type == kTypeQ6K ? 1.35 : 0.79;
     KwChoice best = {1, 1, 1, 0.0, 0.0};
     bool have = false;
     for (int mb = 1; mb <= (m <= 32 ? 1 : 2); mb++)
@@ -1975,11 +1990,11 @@ static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
             if (m > 32 && mb == 1 && nr == 2) continue;  // never the best tile
             const int64_t tiles = ((n + 32 * nr - 1) / (32 * nr)) * ((m + 32 * mb - 1) / (32 * mb));
             for (int splits = 1; splits <= 4 && splits <= spr; splits *= 2) {
-                if (splits > 1 && (tiles * splits > 288 || (m <= 32 && nr == 2))) break;  // only to fill the machine
+                if (splits > 1 && (tiles * splits > 256 || (m <= 32 && nr == 2))) break;  // only to fill the machine
                 const int64_t chunk = (spr + splits - 1) / splits, per = (chunk + 7) / 8, wgs = tiles * splits;
-                double rounds = ((double)wgs / 256.0 + (double)((wgs + 255) / 256)) / 2;
-                const double one = (double)per * 8.0 * (mb * 32 * items * 16 / 1e3 / 113.0 + nr * 32 * block / 1e3 / 41.0) + 0.7 * cost * mb * nr * per;
-                const double us = 6.0 + (1.0 + (rounds - 1.0) * 0.77) * one + (splits > 1 ? 2.2 + splits * (double)m * (double)n * 8.0 * 0.7 / 4.0e6 : 0.0);
+                const double rounds = ((double)wgs / 256.0 + (double)((wgs + 255) / 256)) / 2;
+                const double one = (double)per * 8.0 * (mb * 32 * items * 16 / 1e3 / 124.0 + nr * 32 * block / 1e3 / 34.0) + cost * mb * nr * per;
+                const double us = 5.9 + (1.0 + (rounds - 1.0) * 0.78) * one + (splits > 1 ? 2.5 + splits * (double)m * (double)n * 8.0 * 0.7 / 4.0e6 : 0.0);
                 if (!have || us < best.us) best = {mb, nr, splits, us, (double)wgs / 256.0}, have = true;
             }
         }
@@ -2034,13 +2049,14 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         waves = n * k < ((int64_t)96 << 20) || (small && spr > run && spr % run != 0 && type != kTypeQ8_0);
         waves = waves || (type == kTypeQ2K);  // (no short-batch form for two blocks; ahead at every size: 128256 x 4096 98 -> 90 us)
     } else {
-        // against the row kernels, by the times fitted to both over 1000...14336 weight rows of 1536...14336 elements and
-        // 64...256 activation rows (the chosen kernel is within 2 % of the best one on average)
-        const double half = type == kTypeQ4K ? 0.96 : type == kTypeQ5K ? 1.2 : type == kTypeQ6K ? 1.83 : type == kTypeQ8_0 ? 3.2 : type == kTypeQ3K ? 1.35 : 1.03;
-        const double rounds = (double)((base * p.splits + 255) / 256);
-        const double t_rows = rounds * 2.0 * p.chunk * half * (p.mb == 4 ? 1.33 : 1.0) +
-                              (p.splits > 1 ? 13.2 + (double)p.splits * (double)m * (double)n * 8.0 * 0.9 / 4.0e6 : 0.0);
-        waves = kw.rounds <= 3.0 && kw.us - 6.0 < t_rows;
+        // against the row kernels, by the times fitted to both over 1000...14336 weight rows of 1024...14336 elements and
+        // 64...2048 activation rows (the chosen kernel is within 2 % of the better one on average); from the third round of
+        // workgroups on (Q6_K, two matrix instructions per step: the second; Q8_0, whose row kernel is the slowest: the
+        // fifth) the row kernels, which read the activations once per 256 weight rows, are ahead
+        const double half = type == kTypeQ4K ? 1.17 : type == kTypeQ5K ? 1.47 : type == kTypeQ6K ? 1.98 : type == kTypeQ8_0 ? 2.88 : type == kTypeQ3K ? 1.52 : 1.31;
+        const double t_rows = 9.6 + (double)((base * p.splits + 255) / 256) * 2.0 * p.chunk * half * (p.mb == 4 ? 1.45 : 1.0) +
+                              (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
+        waves = kw.rounds <= (type == kTypeQ6K ? 1.9 : type == kTypeQ8_0 ? 4.0 : type == kTypeQ3K || type == kTypeQ5K ? 2.1 : 2.6) && kw.us < t_rows;
     }
     if (waves) {
         p.kernel = GemmKernel::kWaves;
@@ -2316,15 +2332,14 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     }
     // the partial tiles of a K split (of the large kernels or of the short-batch kernels' runs), added in split order
     const size_t total = (size_t)m * n;
-    if (n % 8 == 0) {
-        const dim3 grid8((unsigned)((total / 8 + 255) / 256));
-        if (ybf) hipLaunchKernelGGL(k_rw_reduce8<true>, grid8, dim3(256), 0, s, partial, p.splits, (int)m, (int)p.mp, (int)n, rowscale, y);
-        else hipLaunchKernelGGL(k_rw_reduce8<false>, grid8, dim3(256), 0, s, partial, p.splits, (int)m, (int)p.mp, (int)n, rowscale, y);
-        return hipGetLastError();
-    }
-    const dim3 rgrid((unsigned)((total + 255) / 256));
-    if (ybf) hipLaunchKernelGGL(k_rw_reduce<true>, rgrid, dim3(256), 0, s, partial, p.splits, (int)m, (int)p.mp, (int)n, rowscale, y);
-    else hipLaunchKernelGGL(k_rw_reduce<false>, rgrid, dim3(256), 0, s, partial, p.splits, (int)m, (int)p.mp, (int)n, rowscale, y);
+    const bool few = total < ((size_t)1 << 17);
+    const dim3 rgrid((unsigned)((total + (few ? 255 : 2047)) / (few ? 256 : 2048)));
+#define PMH_REDUCE(B, P) hipLaunchKernelGGL((k_rw_reduce<B, P>), rgrid, dim3(256), 0, s, partial, p.splits, (int)m, (int)p.mp, (int)n, rowscale, y)
+    if (ybf && few) PMH_REDUCE(true, 1);
+    else if (ybf) PMH_REDUCE(true, 8);
+    else if (few) PMH_REDUCE(false, 1);
+    else PMH_REDUCE(false, 8);
+#undef PMH_REDUCE
     return hipGetLastError();
 }
 

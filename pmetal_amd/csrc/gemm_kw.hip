@@ -376,19 +376,22 @@ __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__
     }
 }
 
-// grid (8, blocks of activation rows x splits of K, groups of eight tiles of weight rows), up to eight waves; wave w of split z
-// takes super-blocks [z * chunk + w * per, + per) below min(spr, (z + 1) * chunk).  The blocks of activation rows of one tile of weights are eight workgroups apart, so on one die.
+// grid (8, inner x splits of K, outer / 8), up to eight waves; wave w of split z takes super-blocks [z * chunk + w * per, + per)
+// below min(spr, (z + 1) * chunk).  Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the
+// blocks of activation rows, otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of
+// the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: BY_M_US).
 template <class F, int MB, int NR>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
-                                                             int spr, int per, int chunk, int mblocks, int tiles, int ybf16,
+                                                             int spr, int per, int chunk, int inner, int outer, int by_m, int ybf16,
                                                              float *__restrict__ partial) {
     using K = Kw<F, MB, NR>;
     extern __shared__ uint4 smem[];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = (int)(blockDim.x >> 6);
-    const int nt = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / mblocks, m0 = ((int)blockIdx.y - z * mblocks) * (32 * MB);
-    if (nt >= tiles) return;  // (the whole workgroup)
+    const int out = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / inner, in = (int)blockIdx.y - z * inner;
+    if (out >= outer) return;  // (the whole workgroup)
+    const int nt = by_m ? in : out, m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
     int sb0 = z * chunk + wave * per, cnt = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - sb0;
     const bool idle = cnt < 1;  // the last split is the shortest: a wave left without work multiplies one super-block for nothing
@@ -508,8 +511,10 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
         if (a != hipSuccess) return a;
     }
     const int tiles = (int)((n + 32 * NR - 1) / (32 * NR)), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
-    const dim3 grid(8, (unsigned)(mblocks * p.splits), (unsigned)((tiles + 7) / 8));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, per, p.chunk, mblocks, tiles, y_bf16 ? 1 : 0,
+    const bool by_m = mblocks >= 8 && (int64_t)mblocks * MB * 2 * 256 > (int64_t)tiles * NR * F::kBytes;
+    const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
+    const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, per, p.chunk, inner, outer, by_m ? 1 : 0, y_bf16 ? 1 : 0,
                        p.splits > 1 ? partial : nullptr);
     return hipGetLastError();
 }
