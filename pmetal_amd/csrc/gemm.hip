@@ -42,9 +42,11 @@ namespace {
 
 
 // ------------------------------------------------------------------------------------------------
-// Pre-pass: a workgroup takes R activation rows m < Mp (R = 1: 512 threads on one row, for few rows; R = 4: 256 threads
-// per row with the row index fastest across lanes, so that four lanes write 64 contiguous bytes of every item row).  rowscale[m] = 2^e with the row maximum * 2^-e in
-// [2^9, 2^10) (bf16 activations are then exact in f16 and block sums stay below 2^15); rows >= M are zero.
+// Pre-pass: a workgroup takes R activation rows m < Mp (R = 1: 512 threads on one row, for few rows; otherwise 1024 / R threads
+// per row with the row index fastest across lanes, so that R lanes write 16 R contiguous bytes of every item row).  Bound by
+// latency for few rows and by its scattered stores and the reads for many: the elements are read once and held (with a second read
+// for the conversion, k = 14336, bf16: M = 16 6.0 -> 4.7 us, M = 512 18.1 -> 9.8, M = 2048 30.2 -> 26.5; f32 M = 2048 43 -> 30).
+// rowscale[m] = 2^e with the row maximum * 2^-e in [2^9, 2^10) (bf16 activations are then exact in f16 and block sums stay below 2^15); rows >= M are zero.
 // One thread per operand item: chunk u = 64 elements = sub-blocks 2u, 2u+1 (u = 4 sb + 2 h + g), k-step t.
 // ORDER 0 / 1: Q4_K element orders REF / GGML (1 is also Q5_K's GGML order); ORDER 2: the Q6_K layout, ORDER 3: the
 // natural order (Q8_0), both without block sums; ORDER 4: Q5_K's REF order, whose sub-block j holds its 32 elements as
@@ -53,7 +55,13 @@ namespace {
 // t / 2 of the bytes 16 g .. 16 g + 15 of a half with the shifts s = 2 (t % 2) (first run) and 2 (t % 2) + 1 (second run), and
 // the sums are those of the four 16-element sub-blocks 4 (t % 2) + 2 (run) + g of the half: 20 items per half.
 // ------------------------------------------------------------------------------------------------
-template <bool XF32, int ORDER, int R>
+template <bool XF32>
+struct PrepRaw {  // the eight elements of an item as they lie in memory
+    uint4 a, b;   // (bf16: all in a)
+};
+
+// NI > 0: k <= 8 NI NT / R; a thread's items stay in registers between the row maximum and the conversion.  NI = 0: any k.
+template <bool XF32, int ORDER, int R, int NI>
 __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__restrict__ xg, int64_t k, int M, int Mp,
                                                                   float *__restrict__ rowscale, uint4 *__restrict__ xs) {
     constexpr int NT = R == 1 ? 512 : 1024, JN = NT / R, NWV = NT / 64;
@@ -61,46 +69,9 @@ __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__r
     const int tid = threadIdx.x, lane = tid & 63, r = tid % R, j = tid / R;
     const int m = blockIdx.x * R + r;
     const bool live = m < M;
-    __shared__ float red[NWV][R];
-    float amax = 0.0f;
-    if (live) {
-        if (XF32) {
-            const float4 *row = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(xg) + (int64_t)m * k);
-            for (int64_t i = j; i < k / 4; i += JN) {
-                const float4 v = row[i];
-                amax = __builtin_fmaxf(__builtin_fmaxf(amax, __builtin_fmaxf(__builtin_fabsf(v.x), __builtin_fabsf(v.y))),
-                                       __builtin_fmaxf(__builtin_fabsf(v.z), __builtin_fabsf(v.w)));
-            }
-        } else {
-            const uint4 *row = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(xg) + (int64_t)m * k);
-            for (int64_t i = j; i < k / 8; i += JN) {
-                const uint4 v = row[i];
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    amax = __builtin_fmaxf(amax, __builtin_fmaxf(__builtin_fabsf(bf16_to_f32(w[q] & 0xFFFFu)),
-                                                                 __builtin_fabsf(bf16_to_f32(w[q] >> 16))));
-            }
-        }
-    }
-    for (int off = 32; off >= R; off >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, off));
-    if (lane < R) red[tid >> 6][lane] = amax;
-    __syncthreads();
-    amax = red[0][r];
-#pragma unroll
-    for (int w = 1; w < NWV; w++) amax = __builtin_fmaxf(amax, red[w][r]);
-    const int eb = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFFu);  // amax in [2^(eb-127), 2^(eb-126))
-    int e = eb - 126 - 10;
-    e = e < -126 ? -126 : (e > 126 ? 126 : e);
-    if (eb == 255) e = 0;  // inf / NaN: let them through
-    const float up = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
-    if (j == 0) rowscale[m] = up;
-    const float down = live ? 1.0f / up : 0.0f;  // exact: a power of two
-
-    for (int64_t q = j; q < k / 8; q += JN) {
-        // the item's two runs of four elements (lo, hi), its half super-block and its operand group
-        int64_t lo, hi, half;
-        int t, g;
+    const int64_t items = k / 8;
+    // an item's two runs of four elements (lo, hi), its half super-block and its operand group
+    auto place = [&](const int64_t q, int64_t &lo, int64_t &hi, int64_t &half, int &t, int &g) __attribute__((always_inline)) {
         if (ORDER == 2 || ORDER == 3) {  // half = 128 elements, 16 items
             half = q >> 4;
             t = (int)(q & 15) >> 1, g = (int)q & 1;
@@ -120,19 +91,76 @@ __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__r
                               : (ORDER == 0 ? 64 * u + 32 * (t >> 2) + 4 * (t & 3) : 64 * u + 4 * t);
             hi = lo + (ORDER == 4 ? 4 : (ORDER == 0 ? 16 : 32));
         }
-        float v[8];
-        if (!live) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) v[i] = 0.0f;
-        } else if (XF32) {
+    };
+    auto fetch = [&](const int64_t q) __attribute__((always_inline)) {
+        int64_t lo, hi, half;
+        int t, g;
+        place(q, lo, hi, half, t, g);
+        PrepRaw<XF32> w;
+        if (XF32) {
             const float *row = reinterpret_cast<const float *>(xg) + (int64_t)m * k;
-            const float4 a = *reinterpret_cast<const float4 *>(row + lo), b = *reinterpret_cast<const float4 *>(row + hi);
-            v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+            w.a = *reinterpret_cast<const uint4 *>(row + lo), w.b = *reinterpret_cast<const uint4 *>(row + hi);
         } else {
             const uint16_t *row = reinterpret_cast<const uint16_t *>(xg) + (int64_t)m * k;
             const uint2 a = *reinterpret_cast<const uint2 *>(row + lo), b = *reinterpret_cast<const uint2 *>(row + hi);
-            v[0] = bf16_to_f32(a.x & 0xFFFFu), v[1] = bf16_to_f32(a.x >> 16), v[2] = bf16_to_f32(a.y & 0xFFFFu), v[3] = bf16_to_f32(a.y >> 16);
-            v[4] = bf16_to_f32(b.x & 0xFFFFu), v[5] = bf16_to_f32(b.x >> 16), v[6] = bf16_to_f32(b.y & 0xFFFFu), v[7] = bf16_to_f32(b.y >> 16);
+            w.a = make_uint4(a.x, a.y, b.x, b.y);
+        }
+        return w;
+    };
+    auto widen = [&](const PrepRaw<XF32> &w, float (&v)[8]) __attribute__((always_inline)) {
+        const uint32_t a[8] = {w.a.x, w.a.y, w.a.z, w.a.w, XF32 ? w.b.x : 0u, XF32 ? w.b.y : 0u, XF32 ? w.b.z : 0u, XF32 ? w.b.w : 0u};
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = XF32 ? __builtin_bit_cast(float, a[i]) : bf16_to_f32(i & 1 ? a[i / 2] >> 16 : a[i / 2] & 0xFFFFu);
+    };
+    auto max_with = [&](float amax, const PrepRaw<XF32> &w) __attribute__((always_inline)) {
+        float v[8];
+        widen(w, v);
+#pragma unroll
+        for (int i = 0; i < 8; i++) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[i]));
+        return amax;
+    };
+    __shared__ float red[NWV][R];
+    float amax = 0.0f;
+    constexpr int kHeld = NI > 0 ? NI : 1;
+    PrepRaw<XF32> held[kHeld];
+    if (live) {
+        if (NI > 0) {
+#pragma unroll
+            for (int i = 0; i < kHeld; i++) {
+                const int64_t q = j + i * JN;
+                held[i] = fetch(q < items ? q : items - 1);  // (past the row: its last item again, which does not change the maximum)
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kHeld; i++) amax = max_with(amax, held[i]);
+        } else {
+            for (int64_t q = j; q < items; q += JN) amax = max_with(amax, fetch(q));
+        }
+    }
+    for (int off = 32; off >= R; off >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, off));
+    if (lane < R) red[tid >> 6][lane] = amax;
+    __syncthreads();
+    amax = red[0][r];
+#pragma unroll
+    for (int w = 1; w < NWV; w++) amax = __builtin_fmaxf(amax, red[w][r]);
+    const int eb = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFFu);  // amax in [2^(eb-127), 2^(eb-126))
+    int e = eb - 126 - 10;
+    e = e < -126 ? -126 : (e > 126 ? 126 : e);
+    if (eb == 255) e = 0;  // inf / NaN: let them through
+    const float up = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+    if (j == 0) rowscale[m] = up;
+    const float down = live ? 1.0f / up : 0.0f;  // exact: a power of two
+
+    auto emit = [&](const int64_t q, const PrepRaw<XF32> &raw) __attribute__((always_inline)) {
+        int64_t lo, hi, half;
+        int t, g;
+        place(q, lo, hi, half, t, g);
+        float v[8];
+        if (live) {
+            widen(raw, v);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = 0.0f;
         }
         if (ORDER == 4) {  // eight consecutive elements: the even ones, then the odd ones
             const float e[8] = {v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]};
@@ -149,7 +177,7 @@ __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__r
         }
         const size_t base = (size_t)(half * kGroups) * Mp + m;
         xs[base + (size_t)(t * 2 + g) * Mp] = __builtin_bit_cast(uint4, h);
-        if (ORDER == 2 || ORDER == 3) continue;  // Q6_K and Q8_0 have no min term: no block sums
+        if (ORDER == 2 || ORDER == 3) return;  // Q6_K and Q8_0 have no min term: no block sums
         // sums of the two sub-blocks of the chunk over its 8 k-steps (8 lanes, R apart)
         float s0, s1;
         if (ORDER == 5) {
@@ -163,7 +191,7 @@ __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__r
                 const half8_t item = {h0, l0, h0, l0, h1, l1, h1, l1};
                 xs[base + (size_t)(16 + 2 * t + g) * Mp] = __builtin_bit_cast(uint4, item);
             }
-            continue;
+            return;
         }
         if (ORDER == 0 || ORDER == 4) {  // sub-block 2u: k-steps 0..3 (low and high nibbles), 2u+1: k-steps 4..7
             float s = slo + shi;
@@ -183,6 +211,15 @@ __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__r
             const half8_t item = {h0, l0, h0, l0, h1, l1, h1, l1};
             xs[base + (size_t)(16 + g) * Mp] = __builtin_bit_cast(uint4, item);
         }
+    };
+    if (NI > 0) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++) {
+            const int64_t q = j + i * JN;
+            if (q < items) emit(q, held[i]);  // (the eight threads of a chunk together)
+        }
+    } else {
+        for (int64_t q = j; q < items; q += JN) emit(q, live ? fetch(q) : PrepRaw<XF32>{});
     }
 }
 
@@ -2151,14 +2188,27 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     float *partial = reinterpret_cast<float *>(ws + xs_bytes + align256((size_t)p.mp * 4));
     const bool xf32 = x_dtype == kDtypeF32, q6 = type == kTypeQ6K, q8 = type == kTypeQ8_0, q5 = type == kTypeQ5K, ref = order == kOrderRef;
     const int xorder = q23 ? 5 : (q8 ? 3 : (q6 ? 2 : (ref ? (q5 ? 4 : 0) : 1)));  // the element order the pre-pass lays the activations out for
-#define PMH_PREP(F, O)                                                                                                       \
-    do {                                                                                                                     \
-        if (p.mp >= 1024)                                                                                                    \
-            hipLaunchKernelGGL((k_prep_rw<F, O, 4>), dim3((unsigned)p.mp / 4), dim3(1024), 0, s, x, k, (int)m, (int)p.mp,    \
-                               rowscale, xs);                                                                                \
-        else                                                                                                                 \
-            hipLaunchKernelGGL((k_prep_rw<F, O, 1>), dim3((unsigned)p.mp), dim3(512), 0, s, x, k, (int)m, (int)p.mp,         \
-                               rowscale, xs);                                                                                \
+    // Rows per workgroup: one for few rows (a chain of latencies: 512 threads on it), two from 384 rows on and four from 1024 on,
+    // whose threads write 32 and 64 bytes at a place instead of 16 (us of the pre-pass with one / two / four rows, bf16, k = 14336:
+    // M = 64 7.6 / 8.7 / 15.2, M = 512 15.1 / 9.8 / 14.0, M = 2048 56 / 35 / 27).  An item count beyond eight per thread is read twice.
+    const int per_wg = p.mp >= 1024 ? 4 : p.mp >= 384 ? 2 : 1;
+    const int64_t ni = (k / 8 * per_wg + (per_wg == 1 ? 511 : 1023)) / (per_wg == 1 ? 512 : 1024);
+#define PMH_PREP_N(F, O, R, NI)                                                                                              \
+    hipLaunchKernelGGL((k_prep_rw<F, O, R, NI>), dim3((unsigned)p.mp / (R)), dim3((R) == 1 ? 512 : 1024), 0, s, x, k, (int)m, \
+                       (int)p.mp, rowscale, xs)
+#define PMH_PREP_R(F, O, R)                       \
+    do {                                          \
+        if (ni <= 1) PMH_PREP_N(F, O, R, 1);      \
+        else if (ni <= 2) PMH_PREP_N(F, O, R, 2); \
+        else if (ni <= 4) PMH_PREP_N(F, O, R, 4); \
+        else if (ni <= 8) PMH_PREP_N(F, O, R, 8); \
+        else PMH_PREP_N(F, O, R, 0);              \
+    } while (0)
+#define PMH_PREP(F, O)                          \
+    do {                                        \
+        if (per_wg == 4) PMH_PREP_R(F, O, 4);   \
+        else if (per_wg == 2) PMH_PREP_R(F, O, 2); \
+        else PMH_PREP_R(F, O, 1);               \
     } while (0)
     if (reuse_prepass) {
         // the workspace still holds the converted activations of the previous call (same x, m, k and weight type)
@@ -2178,6 +2228,8 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         else PMH_PREP(false, 5);
     }
 #undef PMH_PREP
+#undef PMH_PREP_R
+#undef PMH_PREP_N
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const bool ybf = y_dtype == kDtypeBf16;

@@ -46,3 +46,21 @@ def test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k):
         assert np.max(np.abs(got - want)) <= bound * np.max(np.abs(want)), order
         got16 = gpu_qgemm(t, raw, n, k, bits, m, y_dtype=pm.DTYPE_BF16, order=order)
         assert np.max(np.abs(got16 - want)) <= (2.0 ** -8 + bound) * np.max(np.abs(want)), order
+
+
+# The pre-pass holds 1, 2, 4 or 8 items per thread, or reads a longer row twice; one, two (from 384 rows on) or four rows (from
+# 1024 on) per workgroup.  Rows of activations that end inside a workgroup, row lengths on both sides of each step.
+@pytest.mark.parametrize("m,k", [(3, 4096), (18, 4352), (17, 16384), (20, 16640), (33, 32768), (2, 33024), (385, 4096), (390, 4352), (385, 33024),
+                                 (1025, 2048), (1026, 2304), (1025, 8192), (1027, 8448), (1025, 16640)])
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 10])
+def test_prepared_activations(oracle, t, m, k):
+    n = 5
+    rng = np.random.default_rng(t + m + k)
+    raw = random_blocks(rng, t, n, k)
+    bits = oracle.f32_to_bf16_bits(rng.standard_normal(m * k).astype(np.float32)).reshape(m, k)
+    x = oracle.bf16_bits_to_f32(bits.reshape(-1)).reshape(m, k)
+    for order in (0, 1) if t in (Q4K, 13) else (0,):
+        want = reference(oracle, t, raw, n, k, x, order)
+        for given in (bits, x):  # the same values in either type: exact operands for both, the bound of the test above
+            got = gpu_qgemm(t, raw, n, k, given, m, order=order, x_dtype=pm.DTYPE_BF16 if given is bits else pm.DTYPE_F32)
+            assert np.max(np.abs(got - want)) <= (k / 16 + 16) * 2.0 ** -24 * 4 * np.max(np.abs(want)), (order, given.dtype)
