@@ -1051,11 +1051,29 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
     // ... and through the padded row count of the launch plan, which follows n: the item stride and the place of the row
     // scales behind the items change with it, so a narrow weight behind a wide one gets a pre-pass of its own
     int have = -1, have_mp = -1;
+    auto one_kind = [](const pmetal_hip_gemm_desc &a, const pmetal_hip_gemm_desc &b) {
+        return a.ggml_type == b.ggml_type && a.order == b.order && a.y_dtype == b.y_dtype;
+    };
+    auto apart = [&](const pmetal_hip_gemm_desc &a, const pmetal_hip_gemm_desc &b) {
+        const size_t es = a.y_dtype == PMETAL_HIP_DTYPE_F32 ? 4 : 2, block = pmetal_hip_type_size(a.ggml_type), per = pmetal_hip_block_size(a.ggml_type);
+        auto over = [](const void *p, size_t pn, const void *q, size_t qn) { return (uintptr_t)p < (uintptr_t)q + qn && (uintptr_t)q < (uintptr_t)p + pn; };
+        const size_t ya = (size_t)m * a.n * es, yb = (size_t)m * b.n * es;
+        return !over(a.y_dev, ya, b.y_dev, yb) && !over(a.y_dev, ya, b.w_dev, (size_t)b.n * k / per * block) &&
+               !over(b.y_dev, yb, a.w_dev, (size_t)a.n * k / per * block);
+    };
     for (size_t i = 0; i < count; i++) {
         const pmetal_hip_gemm_desc &d = descs[i];
         const int want = layout(d), want_mp = pmh::qgemm_plan(m, d.n, k, d.ggml_type).mp;
-        hipError_t e = pmh::launch_qgemm(d.ggml_type, d.w_dev, d.n, k, x, x_dtype, m, d.y_dev, d.y_dtype, d.order, ws, (hipStream_t)stream,
-                                         want == have && want_mp == have_mp);
+        // two neighbours of one kind share a launch, unless one's results lie over what the other reads or writes
+        pmh::GemmSecond second{};
+        pmh::GemmPlan plan;
+        if (i + 1 < count && one_kind(d, descs[i + 1]) && apart(d, descs[i + 1]) &&
+            pmh::qgemm_pair_plan(m, d.n, descs[i + 1].n, k, d.ggml_type, &plan)) {
+            second.w = (const uint8_t *)descs[i + 1].w_dev, second.y = descs[i + 1].y_dev, second.n = (int)descs[i + 1].n;
+            i++;
+        }
+        hipError_t e = pmh::launch_qgemm(d.ggml_type, (const uint8_t *)d.w_dev, d.n, k, x, x_dtype, m, d.y_dev, d.y_dtype, d.order, ws, (hipStream_t)stream,
+                                         want == have && want_mp == have_mp, second);
         if (e == hipErrorNotSupported) return fail(PMETAL_HIP_ERR_UNSUPPORTED_TYPE, "qgemm: configuration not supported");
         if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
         have = want, have_mp = want_mp;

@@ -486,7 +486,7 @@ __device__ __forceinline__ void rw_half(const uint4 *__restrict__ a_cur, uint4 *
 template <int ORDER, int MB, int NR, int NW, int FMT = 0>
 __global__ __launch_bounds__(64 * NW, MB * NR <= 1 && NW <= 8 ? 2 : 1) void k_qgemm_rw(
     const uint8_t *__restrict__ W, const uint4 *__restrict__ xs, const float *__restrict__ rowscale, void *__restrict__ yg,
-    float *__restrict__ partial, int M, int Mp, int N, int spr, int chunk, int mode) {
+    float *__restrict__ partial, int M, int Mp, int N, int spr, int chunk, int mode, const pmh::GemmSecond second) {
     constexpr int BM = 32 * MB, kThreads = 64 * NW, kRows = 32 * NR * NW;
     constexpr int kBlockBytes = BlockFmt<FMT>::kBytes, kQs = BlockFmt<FMT>::kQs;
     extern __shared__ uint4 smem[];
@@ -497,7 +497,9 @@ __global__ __launch_bounds__(64 * NW, MB * NR <= 1 && NW <= 8 ? 2 : 1) void k_qg
     L.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     L.col = lane & 31, L.g = lane >> 5;
-    const int n0 = blockIdx.x * kRows, m0 = blockIdx.y * BM;
+    int bx = (int)blockIdx.x;
+    take_weight(second, mode, bx, W, yg, N);
+    const int n0 = bx * kRows, m0 = blockIdx.y * BM;
     const int nw0 = n0 + 32 * NR * L.wave;  // first weight row of this wave
     const int sb0 = blockIdx.z * chunk;
     const int cnt = spr - sb0 < chunk ? spr - sb0 : chunk;
@@ -727,7 +729,7 @@ template <int FMT, int MB>
 __global__ __launch_bounds__(512, MB <= 1 ? 2 : 1) void k_qgemm_rw16(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                                       const float *__restrict__ rowscale, void *__restrict__ yg,
                                                                       float *__restrict__ partial, int M, int Mp, int N, int spr, int chunk,
-                                                                      int mode) {
+                                                                      int mode, const pmh::GemmSecond second) {
     using B = Block16<FMT>;
     constexpr int BM = 32 * MB, NW = 8, kThreads = 512, kRows = 256, kARounds = (kGroups16 * BM + kThreads - 1) / kThreads;
     extern __shared__ uint4 smem[];
@@ -735,7 +737,9 @@ __global__ __launch_bounds__(512, MB <= 1 ? 2 : 1) void k_qgemm_rw16(const uint8
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, col = lane & 31, g = lane >> 5;
-    const int n0 = blockIdx.x * kRows, m0 = blockIdx.y * BM;
+    int bx = (int)blockIdx.x;
+    take_weight(second, mode, bx, W, yg, N);
+    const int n0 = bx * kRows, m0 = blockIdx.y * BM;
     const int nw0 = n0 + 32 * wave;  // first weight row of this wave
     const int sb0 = blockIdx.z * chunk;
     const int cnt = spr - sb0 < chunk ? spr - sb0 : chunk;
@@ -933,7 +937,7 @@ template <int MB>
 __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q6(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                          const float *__restrict__ rowscale, void *__restrict__ yg,
                                                          float *__restrict__ partial, int M, int Mp, int N, int spr, int chunk,
-                                                         int mode) {
+                                                         int mode, const pmh::GemmSecond second) {
     constexpr int BM = 32 * MB, kThreads = 512, NW = 8;
     extern __shared__ uint4 smem[];
     uint4 *a0 = smem, *a1 = a0 + kQ6Groups * BM, *qbase = a1 + kQ6Groups * BM, *hb = qbase + 3 * NW * kQ6Stage;
@@ -942,7 +946,9 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q6(const uint8_t *__restric
     L.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     L.col = lane & 31, L.g = lane >> 5;
-    const int n0 = blockIdx.x * 256, m0 = blockIdx.y * BM;
+    int bx = (int)blockIdx.x;
+    take_weight(second, mode, bx, W, yg, N);
+    const int n0 = bx * 256, m0 = blockIdx.y * BM;
     const int nw0 = n0 + 32 * L.wave;
     const int sb0 = blockIdx.z * chunk;
     const int cnt = spr - sb0 < chunk ? spr - sb0 : chunk;
@@ -1098,7 +1104,7 @@ template <int MB>
 __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                          const float *__restrict__ rowscale, void *__restrict__ yg,
                                                          float *__restrict__ partial, int M, int Mp, int N, int spr, int chunk,
-                                                         int mode) {
+                                                         int mode, const pmh::GemmSecond second) {
     constexpr int BM = 32 * MB, kThreads = 512;
     extern __shared__ uint4 smem[];
     uint4 *a0 = smem, *a1 = a0 + kQ6Groups * BM;
@@ -1107,7 +1113,9 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restric
     L.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     L.col = lane & 31, L.g = lane >> 5;
-    const int n0 = blockIdx.x * 256, m0 = blockIdx.y * BM;
+    int bx = (int)blockIdx.x;
+    take_weight(second, mode, bx, W, yg, N);
+    const int n0 = bx * 256, m0 = blockIdx.y * BM;
     const int n = n0 + 32 * L.wave + L.col;
     const int sb0 = blockIdx.z * chunk;
     const int cnt = spr - sb0 < chunk ? spr - sb0 : chunk;
@@ -1264,7 +1272,12 @@ template <int ORDER, int NSB, int FMT = 0, int MT = 1>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                                    const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                    int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
-                                                                   float *__restrict__ partial) {
+                                                                   float *__restrict__ partial, const pmh::GemmSecond second) {
+    int bx = (int)blockIdx.x;
+    if (ybf16 & kHasSecond) {
+        take_weight(second, ybf16, bx, W, yg, N);
+        tiles = (N + 15) / 16;
+    }
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64]: lane slots of the finished tiles; then the waves' stages
     const float rs = small_row_scale(rowscale);
@@ -1302,7 +1315,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
                 asum[i][b] = z;
             }
         }
-    const int t0 = (int)blockIdx.x * tiles_per_wg;
+    const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;  // t1 > t0 by the launch geometry
     constexpr int kPerSb = SmallRun<NSB, FMT>::kPerSb, kBlockBytes = BlockFmt<FMT>::kBytes, kQ0 = FMT ? 3 : 1;  // kQ0: first quant piece
     const uint32_t row_bytes = (uint32_t)spr * (uint32_t)kBlockBytes;
@@ -1436,7 +1449,12 @@ template <int NSB, int MT = 1>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                                       const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                       int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
-                                                                   float *__restrict__ partial) {
+                                                                   float *__restrict__ partial, const pmh::GemmSecond second) {
+    int bx = (int)blockIdx.x;
+    if (ybf16 & kHasSecond) {
+        take_weight(second, ybf16, bx, W, yg, N);
+        tiles = (N + 15) / 16;
+    }
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
     const float rs = small_row_scale(rowscale);
@@ -1469,7 +1487,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
                 af[i][mb][b] = __builtin_bit_cast(half8_t, *item);
                 if (!sbv[i]) af[i][mb][b] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
             }
-    const int t0 = (int)blockIdx.x * tiles_per_wg;
+    const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;
     const uint32_t row_bytes = (uint32_t)spr * (uint32_t)kQ8RunBytes;
     // piece j of this lane: index lane + 64 j of the tile's 272 (the fifth exists for the first 16 lanes; the others load
@@ -1588,7 +1606,13 @@ template <int NSB, bool ANY>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                                       const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                       int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
-                                                                      uint32_t w_last, float *__restrict__ partial) {
+                                                                      uint32_t w_last, float *__restrict__ partial, const pmh::GemmSecond second) {
+    int bx = (int)blockIdx.x;
+    if (ybf16 & kHasSecond) {
+        take_weight(second, ybf16, bx, W, yg, N);
+        tiles = (N + 15) / 16;
+        w_last = (uint32_t)(((uint64_t)N * (uint64_t)spr * 210u - 1) & ~(uint64_t)15);
+    }
     constexpr int P = SmallQ6<NSB, ANY>::kRowPieces, kLoads = SmallQ6<NSB, ANY>::kLoads;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
@@ -1624,7 +1648,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
                     af[i][hh][lh][gp] = __builtin_bit_cast(half8_t, *item);
                     if (!sbv[i]) af[i][hh][lh][gp] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
                 }
-    const int t0 = (int)blockIdx.x * tiles_per_wg;
+    const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;
     const uint32_t row_bytes = (uint32_t)spr * 210u;
     uint32_t piece_row[kLoads], piece_off[kLoads];
@@ -1811,7 +1835,12 @@ template <int FMT, int NSB>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                                      const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                      int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
-                                                                     float *__restrict__ partial) {
+                                                                     float *__restrict__ partial, const pmh::GemmSecond second) {
+    int bx = (int)blockIdx.x;
+    if (ybf16 & kHasSecond) {
+        take_weight(second, ybf16, bx, W, yg, N);
+        tiles = (N + 15) / 16;
+    }
     using B = Block16<FMT>;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the kept partial tiles
@@ -1847,7 +1876,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
             asum[i][0] = z, asum[i][1] = z;
         }
     }
-    const int t0 = (int)blockIdx.x * tiles_per_wg;
+    const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;  // t1 > t0 by the launch geometry
     const uint32_t row_bytes = (uint32_t)spr * (uint32_t)B::kBytes;
     auto block_at = [&](int ti, int i) -> uint32_t {  // byte offset of super-block sbi[i] of this lane's row of tile ti (the tensor is smaller than 4 GiB)
@@ -2038,6 +2067,14 @@ static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
     return best;
 }
 
+// The same for the row kernels, whose tile and K split are the plan's.
+static double rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
+    const double half = type == kTypeQ4K ? 1.17 : type == kTypeQ5K ? 1.47 : type == kTypeQ6K ? 1.98 : type == kTypeQ8_0 ? 2.88 : type == kTypeQ3K ? 1.52 : 1.31;
+    const int64_t wgs = (n + 255) / 256 * (p.mp / (32 * p.mb)) * p.splits;
+    return 9.6 + (double)((wgs + 255) / 256) * 2.0 * p.chunk * half * (p.mb == 4 ? 1.45 : 1.0) +
+           (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
+}
+
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     GemmPlan p;
     p.kernel = GemmKernel::kRows, p.nr = 1;
@@ -2090,9 +2127,7 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         // 64...2048 activation rows (the chosen kernel is within 2 % of the better one on average); from the third round of
         // workgroups on (Q6_K, two matrix instructions per step: the second; Q8_0, whose row kernel is the slowest: the
         // fifth) the row kernels, which read the activations once per 256 weight rows, are ahead
-        const double half = type == kTypeQ4K ? 1.17 : type == kTypeQ5K ? 1.47 : type == kTypeQ6K ? 1.98 : type == kTypeQ8_0 ? 2.88 : type == kTypeQ3K ? 1.52 : 1.31;
-        const double t_rows = 9.6 + (double)((base * p.splits + 255) / 256) * 2.0 * p.chunk * half * (p.mb == 4 ? 1.45 : 1.0) +
-                              (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
+        const double t_rows = rows_us(p, m, n, type);
         waves = kw.rounds <= (type == kTypeQ6K ? 1.9 : type == kTypeQ8_0 ? 4.0 : type == kTypeQ3K || type == kTypeQ5K ? 2.1 : 2.6) && kw.us < t_rows;
     }
     if (waves) {
@@ -2118,9 +2153,40 @@ size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k) {
     return xs + align256((size_t)p.mp * 4) + part + kw_slack(p);
 }
 
+bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan) {
+    if (!qgemm_fits(type, m, n0 + n1, k)) return false;
+    const GemmPlan p = qgemm_plan(m, n0, k, type), q = qgemm_plan(m, n1, k, type);
+    // the same kernel for both and no K split: every result is then the sum, in the same order, that it is in a call of its own
+    if (p.kernel != q.kernel || p.mp != q.mp || p.splits > 1 || q.splits > 1) return false;
+    *plan = p;
+    // Short batches and wave tiles gain the second launch's start and the idle end of the first (us for two weights sharing their
+    // activations, apart -> together: Q4_K 14336 x 4096 M = 16 27.2 -> 21.7, M = 64 41.9 -> 41.0; Q6_K 4096 x 4096 M = 16 21.9 ->
+    // 13.4).  Row kernels, one workgroup per compute unit, only where a round of workgroups that neither weight fills goes
+    // (Q4_K 14336 x 4096 M = 2048 566 -> 525; with as many rounds together 9728 x 2560 M = 512 was 86 -> 93).
+    if (p.kernel == GemmKernel::kRows) {
+        if (p.mb != q.mb) return false;
+        auto rounds = [&](int64_t tiles) { return (tiles * (p.mp / (32 * p.mb)) + 255) / 256; };
+        const int64_t t0 = (n0 + 255) / 256, t1 = (n1 + 255) / 256;
+        return rounds(t0 + t1) < rounds(t0) + rounds(t1);
+    }
+    if (p.kernel == GemmKernel::kWaves) {
+        const KwChoice kw = kw_choice(m, n0 + n1, k / 256, type);
+        if (kw.splits == 1) plan->mb = kw.mb, plan->nr = kw.nr;
+    }
+    return true;
+}
+
+// Tiles of `rows` weight rows along the grid; with a second weight also where its tiles begin and the bit that says so.
+static unsigned tiles_of_both(int64_t n, int rows, GemmSecond &second, int &mode) {
+    const unsigned tiles = (unsigned)((n + rows - 1) / rows);
+    if (second.n == 0) return tiles;
+    second.first = (int)tiles, mode |= kHasSecond;
+    return tiles + (unsigned)((second.n + rows - 1) / rows);
+}
+
 template <int ORDER, int MB, int NR, int NW, int FMT = 0>
 static hipError_t launch_rw(hipStream_t s, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, float *partial,
-                            int64_t m, int64_t n, int spr, const GemmPlan &p, int mode) {
+                            int64_t m, int64_t n, int spr, const GemmPlan &p, int mode, GemmSecond second) {
     auto kern = k_qgemm_rw<ORDER, MB, NR, NW, FMT>;
     constexpr size_t lds = rw_lds_bytes<MB, NR, NW, FMT>();
     constexpr int kRows = 32 * NR * NW;
@@ -2128,41 +2194,41 @@ static hipError_t launch_rw(hipStream_t s, const uint8_t *w, const uint4 *xs, co
         hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (a != hipSuccess) return a;
     }
-    const dim3 grid((unsigned)((n + kRows - 1) / kRows), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode);
+    const dim3 grid(tiles_of_both(n, kRows, second, mode), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode, second);
     return hipGetLastError();
 }
 
 template <int FMT, int MB>
 static hipError_t launch_rw16(hipStream_t s, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, float *partial, int64_t m,
-                              int64_t n, int spr, const GemmPlan &p, int mode) {
+                              int64_t n, int spr, const GemmPlan &p, int mode, GemmSecond second) {
     auto kern = k_qgemm_rw16<FMT, MB>;
     constexpr size_t lds = rw16_lds_bytes<FMT, MB>();
     if (lds > 64 * 1024) {
         hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (a != hipSuccess) return a;
     }
-    const dim3 grid((unsigned)((n + 255) / 256), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
-    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode);
+    const dim3 grid(tiles_of_both(n, 256, second, mode), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
+    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode, second);
     return hipGetLastError();
 }
 
 template <int MB>
 static hipError_t launch_rw_q6(hipStream_t s, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, float *partial,
-                               int64_t m, int64_t n, int spr, const GemmPlan &p, int mode) {
+                               int64_t m, int64_t n, int spr, const GemmPlan &p, int mode, GemmSecond second) {
     auto kern = k_qgemm_rw_q6<MB>;
     constexpr size_t stages = (size_t)(2 * kQ6Groups * 32 * MB + 8 * (3 * kQ6Stage + 64)) * 16;
     constexpr size_t lds = stages > tile_lds_bytes<MB>() ? stages : tile_lds_bytes<MB>();
     hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (a != hipSuccess) return a;
-    const dim3 grid((unsigned)((n + 255) / 256), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
-    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode);
+    const dim3 grid(tiles_of_both(n, 256, second, mode), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
+    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode, second);
     return hipGetLastError();
 }
 
 template <int MB>
 static hipError_t launch_rw_q8(hipStream_t s, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, float *partial,
-                               int64_t m, int64_t n, int spr, const GemmPlan &p, int mode) {
+                               int64_t m, int64_t n, int spr, const GemmPlan &p, int mode, GemmSecond second) {
     auto kern = k_qgemm_rw_q8<MB>;
     constexpr size_t stages = (size_t)(2 * kQ6Groups * 32 * MB) * 16;
     constexpr size_t lds = stages > tile_lds_bytes<MB>() ? stages : tile_lds_bytes<MB>();
@@ -2170,15 +2236,19 @@ static hipError_t launch_rw_q8(hipStream_t s, const uint8_t *w, const uint4 *xs,
         hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (a != hipSuccess) return a;
     }
-    const dim3 grid((unsigned)((n + 255) / 256), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
-    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode);
+    const dim3 grid(tiles_of_both(n, 256, second, mode), (unsigned)(p.mp / (32 * MB)), (unsigned)p.splits);
+    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, w, xs, rowscale, y, partial, (int)m, (int)p.mp, (int)n, spr, p.chunk, mode, second);
     return hipGetLastError();
 }
 
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,
-                                int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s, bool reuse_prepass) {
+                                int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s, bool reuse_prepass,
+                                const GemmSecond &second_weight) {
     if (!qgemm_fits(type, m, n, k)) return hipErrorInvalidValue;
-    const GemmPlan p = qgemm_plan(m, n, k, type);
+    GemmSecond second = second_weight;
+    GemmPlan p;
+    if (second.n == 0) p = qgemm_plan(m, n, k, type);
+    else if (!qgemm_pair_plan(m, n, second.n, k, type, &p)) return hipErrorInvalidValue;
     const int spr = (int)(k / 256);
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
     uint4 *xs = reinterpret_cast<uint4 *>(ws);
@@ -2234,7 +2304,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     if (e != hipSuccess) return e;
     const bool ybf = y_dtype == kDtypeBf16;
     if (p.kernel == GemmKernel::kWaves) {
-        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, s);
+        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, second, s);
         if (e != hipSuccess || p.splits == 1) return e;
     } else if (p.kernel == GemmKernel::kSmall) {
         const int nwaves = spr < kSmallWaves ? spr : kSmallWaves;
@@ -2245,8 +2315,10 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         const int runs_of_row = p.splits;
         int64_t slots = (int64_t)compute_units_gemm() * (kSmallWaves / nwaves) / runs_of_row;
         slots = slots < 1 ? 1 : slots;
-        const int n_wg = (int)(tiles < slots ? tiles : slots);
-        int tiles_per_wg = (tiles + n_wg - 1) / n_wg;
+        const int tiles1 = (second.n + 15) / 16;  // of the second weight: a workgroup's tiles are of one weight
+        const int n_wg = (int)(tiles + tiles1 < slots ? tiles + tiles1 : slots);
+        int tiles_per_wg = (tiles + tiles1 + n_wg - 1) / n_wg;
+        if (tiles1 > 0 && (tiles + tiles_per_wg - 1) / tiles_per_wg + (tiles1 + tiles_per_wg - 1) / tiles_per_wg > n_wg) tiles_per_wg++;
         const int mt = m > kSmallMaxM ? 2 : 1;  // 16-row blocks of activations
         // the finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and the 16 KiB of the
         // reduction buffers: 64 of them keep the workgroup within 160 KiB for every type
@@ -2255,7 +2327,9 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         const int runs = runs_of_row;
         float *const part_out = runs > 1 ? partial : nullptr;
         const int nsb = run > kSmallWaves && spr > kSmallWaves ? 2 : 1;
-        const dim3 grid((unsigned)((tiles + tiles_per_wg - 1) / tiles_per_wg), (unsigned)runs), block((unsigned)(64 * nwaves));
+        second.first = (tiles + tiles_per_wg - 1) / tiles_per_wg;
+        const int ybf16 = (ybf ? 1 : 0) | (tiles1 > 0 ? kHasSecond : 0);
+        const dim3 grid((unsigned)(second.first + (tiles1 + tiles_per_wg - 1) / tiles_per_wg), (unsigned)runs), block((unsigned)(64 * nwaves));
         // (a workgroup of few tiles also keeps every wave's partial tile of each until the end)
         const size_t lds = (size_t)((tiles_per_wg + kSmallDepth - 1) / kSmallDepth * kSmallDepth) * mt * 1024 *
                            (tiles_per_wg * mt <= kSmallKeepTiles ? 1 + nwaves : 1);
@@ -2268,7 +2342,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             if (e != hipSuccess) return e;                                                                                       \
         }                                                                                                                        \
         hipLaunchKernelGGL((k_qgemm_small<O, S, F, T>), grid, block, lds4, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf ? 1 : 0, part_out);                                                                           \
+                           tiles_per_wg, ybf16, part_out, second);                                                                           \
     } while (0)
 #define PMH_SMALL_F(O, S, F)               \
     do {                                   \
@@ -2289,7 +2363,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             if (e != hipSuccess) return e;                                                                                       \
         }                                                                                                                        \
         hipLaunchKernelGGL((k_qgemm_small16<F, S>), grid, block, lds, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf ? 1 : 0, part_out);                                                                 \
+                           tiles_per_wg, ybf16, part_out, second);                                                                 \
     } while (0)
             if (type == kTypeQ2K) {
                 if (nsb == 2) PMH_SMALL16(3, 2);
@@ -2312,7 +2386,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             if (e != hipSuccess) return e;                                                                                       \
         }                                                                                                                        \
         hipLaunchKernelGGL((k_qgemm_small_q6<S, A>), grid, block, lds6, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf ? 1 : 0, w_last, part_out);                                                                   \
+                           tiles_per_wg, ybf16, w_last, part_out, second);                                                                   \
     } while (0)
             if (nsb == 2 && any) PMH_SMALL_Q6(2, true);
             else if (nsb == 2) PMH_SMALL_Q6(2, false);
@@ -2329,7 +2403,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             if (e != hipSuccess) return e;                                                                                       \
         }                                                                                                                        \
         hipLaunchKernelGGL((k_qgemm_small_q8<S, T>), grid, block, lds8, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf ? 1 : 0, part_out);                                                                           \
+                           tiles_per_wg, ybf16, part_out, second);                                                                           \
     } while (0)
             if (mt == 2) PMH_SMALL_Q8(1, 2);  // (two blocks of activations: one run of eight blocks per wave)
             else if (nsb == 2) PMH_SMALL_Q8(2, 1);
@@ -2350,24 +2424,24 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         if (e != hipSuccess || runs == 1) return e;
     } else {
     const int mode = p.splits > 1 ? 2 : (ybf ? 1 : 0);
-#define PMH_RW_CASE(O, B, R, NWV) launch_rw<O, B, R, NWV>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
+#define PMH_RW_CASE(O, B, R, NWV) launch_rw<O, B, R, NWV>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
     if (q8) {
-        e = p.mb == 1   ? launch_rw_q8<1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-            : p.mb == 2 ? launch_rw_q8<2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-                        : launch_rw_q8<4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode);
+        e = p.mb == 1   ? launch_rw_q8<1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+            : p.mb == 2 ? launch_rw_q8<2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+                        : launch_rw_q8<4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second);
     } else if (q6) {
-        e = p.mb == 1   ? launch_rw_q6<1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-            : p.mb == 2 ? launch_rw_q6<2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-                        : launch_rw_q6<4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode);
+        e = p.mb == 1   ? launch_rw_q6<1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+            : p.mb == 2 ? launch_rw_q6<2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+                        : launch_rw_q6<4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second);
     } else if (q23) {
-        e = type == kTypeQ2K ? (p.mb == 1   ? launch_rw16<3, 1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-                                : p.mb == 2 ? launch_rw16<3, 2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-                                            : launch_rw16<3, 4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode))
-                             : (p.mb == 1   ? launch_rw16<2, 1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-                                : p.mb == 2 ? launch_rw16<2, 2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
-                                            : launch_rw16<2, 4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode));
+        e = type == kTypeQ2K ? (p.mb == 1   ? launch_rw16<3, 1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+                                : p.mb == 2 ? launch_rw16<3, 2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+                                            : launch_rw16<3, 4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second))
+                             : (p.mb == 1   ? launch_rw16<2, 1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+                                : p.mb == 2 ? launch_rw16<2, 2>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
+                                            : launch_rw16<2, 4>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second));
     } else if (q5) {
-#define PMH_RW5_CASE(O, B) launch_rw<O, B, 1, 8, 1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode)
+#define PMH_RW5_CASE(O, B) launch_rw<O, B, 1, 8, 1>(s, w, xs, rowscale, y, partial, m, n, spr, p, mode, second)
         e = p.mb == 1   ? (ref ? PMH_RW5_CASE(0, 1) : PMH_RW5_CASE(1, 1))
             : p.mb == 2 ? (ref ? PMH_RW5_CASE(0, 2) : PMH_RW5_CASE(1, 2))
                         : (ref ? PMH_RW5_CASE(0, 4) : PMH_RW5_CASE(1, 4));

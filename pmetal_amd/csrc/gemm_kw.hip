@@ -384,14 +384,16 @@ template <class F, int MB, int NR>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
                                                              int spr, int per, int chunk, int inner, int outer, int by_m, int ybf16,
-                                                             float *__restrict__ partial) {
+                                                             float *__restrict__ partial, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
     extern __shared__ uint4 smem[];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = (int)(blockDim.x >> 6);
     const int out = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / inner, in = (int)blockIdx.y - z * inner;
     if (out >= outer) return;  // (the whole workgroup)
-    const int nt = by_m ? in : out, m0 = (by_m ? out : in) * (32 * MB);
+    int nt = by_m ? in : out;
+    take_weight(second, ybf16, nt, W, yg, N);
+    const int m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
     int sb0 = z * chunk + wave * per, cnt = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - sb0;
     const bool idle = cnt < 1;  // the last split is the shortest: a wave left without work multiplies one super-block for nothing
@@ -500,7 +502,7 @@ namespace pmh {
 
 template <class F, int MB, int NR>
 static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n, int spr,
-                            float *partial, hipStream_t s) {
+                            float *partial, GemmSecond second, hipStream_t s) {
     using K = Kw<F, MB, NR>;
     auto kern = k_qgemm_kw<F, MB, NR>;
     const int per = (p.chunk + kKwWaves - 1) / kKwWaves, nwaves = (p.chunk + per - 1) / per;
@@ -510,29 +512,30 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
         hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (a != hipSuccess) return a;
     }
-    const int tiles = (int)((n + 32 * NR - 1) / (32 * NR)), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
+    second.first = (int)((n + 32 * NR - 1) / (32 * NR));
+    const int tiles = second.first + (second.n + 32 * NR - 1) / (32 * NR), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
     const bool by_m = mblocks >= 8 && (int64_t)mblocks * MB * 2 * 256 > (int64_t)tiles * NR * F::kBytes;
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, per, p.chunk, inner, outer, by_m ? 1 : 0, y_bf16 ? 1 : 0,
-                       p.splits > 1 ? partial : nullptr);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, per, p.chunk, inner, outer, by_m ? 1 : 0,
+                       (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond : 0), p.splits > 1 ? partial : nullptr, second);
     return hipGetLastError();
 }
 
 template <class F>
 static hipError_t launch_kw_tile(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n,
-                                 int spr, float *partial, hipStream_t s) {
-    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
-    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
-    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
-    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, s);
+                                 int spr, float *partial, GemmSecond second, hipStream_t s) {
+    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
+    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
+    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
+    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
 }
 
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &p, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
-                           int64_t n, int spr, uint32_t order, float *partial, hipStream_t s) {
+                           int64_t n, int spr, uint32_t order, float *partial, const GemmSecond &second, hipStream_t s) {
     const uint4 *x4 = reinterpret_cast<const uint4 *>(xs);
     const bool ref = order == kOrderRef;
-    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, s); };
+    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, second, s); };
     switch (type) {
     case kTypeQ4K: return ref ? go(KwQ45<0, 0>{}) : go(KwQ45<1, 0>{});
     case kTypeQ5K: return ref ? go(KwQ45<0, 1>{}) : go(KwQ45<1, 1>{});

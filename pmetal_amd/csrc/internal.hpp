@@ -66,6 +66,13 @@ enum class GemmKernel {
     kWaves,  // gemm_kw.hip: a tile of Y per workgroup, K split between its waves
     kRows,   // gemm.hip, k_qgemm_rw*: every wave owns 32 weight rows, activations shared through LDS
 };
+// A second weight of the same type, element order and row length for the launch: its tiles lie behind the first weight's.
+struct GemmSecond {
+    const uint8_t *w;
+    void *y;
+    int n;      // weight rows; 0: no second weight
+    int first;  // its first workgroup along the grid's x dimension (kWaves: its first tile)
+};
 struct GemmPlan {
     GemmKernel kernel;
     int mb;      // 32-row activation blocks per workgroup (kRows: 1, 2 or 4; kWaves: 1 or 2)
@@ -80,15 +87,18 @@ bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k);
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type = kTypeQ4K);
 // Bytes of device workspace qgemm needs for a weight of `type` at (m, n, k); the caller provides it.
 size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k);
+// Whether two weights of one type and element order that share their activations go in one launch (launch_qgemm with `second`), and
+// the launch's plan: the padded rows and the workspace are those of either weight alone, as are the results to the bit.
+bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan);
 // reuse_prepass: the workspace still holds the converted activations of the previous launch_qgemm on this stream with the same
 // x, m, k and weight type (two weights that share their activations: the pre-pass runs once)
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,
                         int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s,
-                        bool reuse_prepass = false);
+                        bool reuse_prepass = false, const GemmSecond &second = GemmSecond{});
 
 // gemm_kw.hip (spr: super-blocks per row; partial: fp32 tiles [splits][mp][n] when plan.splits > 1, not scaled by rowscale)
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &plan, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
-                           int64_t n, int spr, uint32_t order, float *partial, hipStream_t s);
+                           int64_t n, int spr, uint32_t order, float *partial, const GemmSecond &second, hipStream_t s);
 
 // ---- q8k.hip: Q8_K activation blocks and the integer dot products over them ----
 hipError_t launch_quantize_q8k(const float *x, size_t n, uint8_t *dst, hipStream_t s);

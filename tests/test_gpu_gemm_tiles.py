@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import pmetal_amd as pm
+from pmetal_amd import _lib
 from gpu_util import Q4K, Q6K, Q8_0
 from test_gpu_gemm import gpu_qgemm, reference
 
@@ -64,3 +65,45 @@ def test_prepared_activations(oracle, t, m, k):
         for given in (bits, x):  # the same values in either type: exact operands for both, the bound of the test above
             got = gpu_qgemm(t, raw, n, k, given, m, order=order, x_dtype=pm.DTYPE_BF16 if given is bits else pm.DTYPE_F32)
             assert np.max(np.abs(got - want)) <= (k / 16 + 16) * 2.0 ** -24 * 4 * np.max(np.abs(want)), (order, given.dtype)
+
+
+# Two weights that share their activations go in one launch: every kernel that takes such a pair (short batches, the wave tiles,
+# the rows, whose rounds of workgroups neither weight fills), row counts off every tile, the seam between the two inside a
+# round; three weights of which two are neighbours of one kind; results of one in place of the other's stay calls of their own.
+@pytest.mark.parametrize("m,k,ns", [(3, 512, (17, 130)), (16, 4096, (1, 1000)), (16, 2304, (4600, 33)), (17, 1024, (31, 65)), (64, 1792, (97, 64)),
+                                    (100, 768, (300, 129)), (600, 512, (7000, 6300)), (1030, 256, (3900, 4111)), (40, 512, (70, 50, 20))])
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_pairs_match_separate_calls(oracle, t, m, k, ns):
+    rng = np.random.default_rng(t + m + k)
+    raws = [random_blocks(rng, t, n, k) for n in ns]
+    bits = oracle.f32_to_bf16_bits(rng.standard_normal(m * k).astype(np.float32)).reshape(m, k)
+    x = oracle.bf16_bits_to_f32(bits.reshape(-1)).reshape(m, k)
+    lib = _lib.load()
+    dx, dws = pm.DeviceBuffer.from_host(bits), [pm.DeviceBuffer.from_host(raw) for raw in raws]
+    for order in (0, 1) if t in (Q4K, 13) else (0,):
+        dys = [pm.DeviceBuffer(m * n * 4 + 256) for n in ns]
+        for dy in dys:
+            pm.check(lib.pmetal_hip_memset(dy.ptr, 0xFF, dy.nbytes, None))
+        descs = (_lib.GemmDesc * len(ns))(*[_lib.GemmDesc(t, pm.DTYPE_F32, order, 0, n, w.ptr, y.ptr) for n, w, y in zip(ns, dws, dys)])
+        pm.check(lib.pmetal_hip_qgemm_batch(descs, len(ns), k, dx.ptr, pm.DTYPE_BF16, m, None))
+        pm.check(lib.pmetal_hip_sync(None))
+        for n, raw, dy in zip(ns, raws, dys):
+            out = dy.to_host(np.uint8)
+            assert np.all(out[m * n * 4:] == 0xFF)
+            got, want = out[:m * n * 4].view(np.float32).reshape(m, n), reference(oracle, t, raw, n, k, x, order)
+            assert np.max(np.abs(got - want)) <= (k / 16 + 16) * 2.0 ** -24 * 4 * np.max(np.abs(want)), order
+            assert np.array_equal(got, gpu_qgemm(t, raw, n, k, bits, m, order=order)), order
+
+
+def test_results_in_one_place_are_not_paired(oracle):
+    m, n, k = 64, 300, 512
+    rng = np.random.default_rng(5)
+    raws = [random_blocks(rng, Q4K, n, k) for _ in range(2)]
+    bits = oracle.f32_to_bf16_bits(rng.standard_normal(m * k).astype(np.float32)).reshape(m, k)
+    lib = _lib.load()
+    dx, dws, dy = pm.DeviceBuffer.from_host(bits), [pm.DeviceBuffer.from_host(raw) for raw in raws], pm.DeviceBuffer(m * n * 4)
+    descs = (_lib.GemmDesc * 2)(*[_lib.GemmDesc(Q4K, pm.DTYPE_F32, 0, 0, n, w.ptr, dy.ptr) for w in dws])
+    pm.check(lib.pmetal_hip_qgemm_batch(descs, 2, k, dx.ptr, pm.DTYPE_BF16, m, None))
+    pm.check(lib.pmetal_hip_sync(None))
+    want = gpu_qgemm(Q4K, raws[1], n, k, bits, m)  # the last one's
+    assert np.array_equal(dy.to_host(np.float32).reshape(m, n), want)
