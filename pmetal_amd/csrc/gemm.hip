@@ -37,6 +37,7 @@
 // which measured slower, as did one wave per SIMD with a 128 x 64 tile), so a 128-row workgroup is bound by the
 // LDS read rate at about 60 % of the matrix peak.
 #include "gemm_common.hpp"
+#include "../../include/pmetal_hip.h"
 
 namespace {
 
@@ -2075,6 +2076,15 @@ static double rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
            (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
 }
 
+// the tile kernel requests up to six k-steps of items past the last one (32 bytes per row each): they lie in the workspace
+static size_t kw_slack(const GemmPlan &p) { return p.kernel == GemmKernel::kWaves ? (size_t)p.mp * 256 : 0; }
+
+static size_t plan_bytes(const GemmPlan &p, uint32_t type, int64_t n, int64_t k) {
+    const size_t xs = align256((size_t)(k / 256) * 2 * (type == kTypeQ3K || type == kTypeQ2K ? kGroups16 : kGroups) * p.mp * 16);
+    const size_t part = p.splits > 1 ? align256((size_t)p.splits * p.mp * n * 4) : 0;
+    return xs + align256((size_t)p.mp * 4) + part + kw_slack(p);
+}
+
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     GemmPlan p;
     p.kernel = GemmKernel::kRows, p.nr = 1;
@@ -2130,28 +2140,25 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         const double t_rows = rows_us(p, m, n, type);
         waves = kw.rounds <= (type == kTypeQ6K ? 1.9 : type == kTypeQ8_0 ? 4.0 : type == kTypeQ3K || type == kTypeQ5K ? 2.1 : 2.6) && kw.us < t_rows;
     }
-    if (waves) {
-        p.kernel = GemmKernel::kWaves;
-        p.mb = kw.mb, p.nr = kw.nr, p.splits = kw.splits, p.chunk = (int)((spr + kw.splits - 1) / kw.splits);
-        // (one padding for both block heights, so that weights of one batch share their converted activations)
-        p.mp = (int)(m <= 32 ? 32 : (m + 63) / 64 * 64);
-    } else if (small) {
+    if (small) {
         // short batches: rows longer than a run are cut into runs of 16 (or 8) super-blocks, these kernels' K split
         p.kernel = GemmKernel::kSmall;
         p.chunk = spr > run ? run : (int)spr, p.splits = (int)((spr + p.chunk - 1) / p.chunk);
     }
+    if (waves) {
+        GemmPlan t = p;
+        t.kernel = GemmKernel::kWaves;
+        t.mb = kw.mb, t.nr = kw.nr, t.splits = kw.splits, t.chunk = (int)((spr + kw.splits - 1) / kw.splits);
+        // (one padding for both block heights, so that weights of one batch share their converted activations)
+        t.mp = (int)(m <= 32 ? 32 : (m + 63) / 64 * 64);
+        // its items past the end (and now and then more splits) take more scratch: not where only the other kernel's fits the array of
+        // the entry point that allocates nothing
+        if (plan_bytes(t, type, n, k) <= PMETAL_HIP_NOALLOC_SCRATCH_BYTES || plan_bytes(p, type, n, k) > PMETAL_HIP_NOALLOC_SCRATCH_BYTES) p = t;
+    }
     return p;
 }
 
-// the tile kernel requests up to six k-steps of items past the last one (32 bytes per row each): they lie in the workspace
-static size_t kw_slack(const GemmPlan &p) { return p.kernel == GemmKernel::kWaves ? (size_t)p.mp * 256 : 0; }
-
-size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k) {
-    const GemmPlan p = qgemm_plan(m, n, k, type);
-    const size_t xs = align256((size_t)(k / 256) * 2 * (type == kTypeQ3K || type == kTypeQ2K ? kGroups16 : kGroups) * p.mp * 16);
-    const size_t part = p.splits > 1 ? align256((size_t)p.splits * p.mp * n * 4) : 0;
-    return xs + align256((size_t)p.mp * 4) + part + kw_slack(p);
-}
+size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k) { return plan_bytes(qgemm_plan(m, n, k, type), type, n, k); }
 
 bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan) {
     if (!qgemm_fits(type, m, n0 + n1, k)) return false;

@@ -64,6 +64,15 @@ def test_noalloc_equals_qgemm_two_calls_in_a_row():
         assert not np.all(a == 0xFF)
 
 
+# Shapes whose scratch fills the array to the last per cent: a kernel that takes more is not chosen for them.
+@pytest.mark.parametrize("t,m,n,k", [(8, 3281, 12, 4352), (10, 1738, 4, 7424), (11, 1027, 1, 12288), (13, 1859, 2, 7680), (14, 2539, 18, 5632)])
+def test_noalloc_takes_what_nearly_fills_its_scratch(t, m, n, k):
+    lib = _lib.load()
+    pm.init(0)
+    a, b = _both(lib, _bind(lib), t, n, k, m, seed=n + m)
+    assert np.array_equal(a, b)
+
+
 def test_noalloc_rejects_what_does_not_fit():
     lib = _lib.load()
     pm.init(0)
