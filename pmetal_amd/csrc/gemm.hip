@@ -2119,12 +2119,29 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     }
     // The tile kernel (gemm_kw.hip) needs no second pass over partial tiles and no barrier per step, but reads the activations
     // once per 32 or 64 weight rows: the better one for few activation rows and for narrow weights.
-    const KwChoice kw = kw_choice(m, n, spr, type);
+    KwChoice kw = kw_choice(m, n, spr, type);
     const int run = small_run_spr(type, m);
     const bool small = qgemm_small_applies(type, m, n, k);
     bool waves;
     if (m <= kSmallMaxM) {
-        waves = false;
+        // The short-batch kernels' workgroups walk 16 super-blocks of a row at a time however few of them there are, and add the
+        // runs of a longer row in a third launch; the tile kernel's waves share what there is.  Tile kernel against them, us at
+        // M = 12 and how many times faster over the six types:
+        //   rows of 9 to 12 super-blocks, without a K split, so that a second weight can share the launch (1504...7168 rows of
+        //     nine 1.05 to 1.33, 4096 rows of twelve 1.06 to 1.30; two weights of 4096 rows of ten together 1.07 to 1.18)
+        //   rows of 17 to 20: 1.02 to 1.54 (Q4_K 8192 x 5120 15.9 -> 13.6, Q6_K 14336 x 5120 41.4 -> 28.7)
+        //   rows of 21 to 24 and of 33 to 36, where the tiles fill half or three quarters of the machine without a K split: 5008 and
+        //     8192 rows of 24 1.07 to 1.31, 7008 rows of 36 1.04 to 1.42 (4096 rows of 24 Q6_K 0.93, 5008 of 36 Q5_K 0.90)
+        // 13 to 16, 25 to 32 and longer rows leave the short-batch kernels little idle: 14336 rows of 14, 28 and 48 0.77 to 1.10.
+        if (spr > 8 && spr <= 12) {
+            waves = n <= (spr == 9 ? 7168 : 4096);
+            if (waves) kw.splits = 1, kw.nr = 1;
+        } else if (spr > 16 && spr <= 20) {
+            waves = n <= 14336;
+        } else {
+            const double filled = spr > 20 && spr <= 24 ? 0.5 : spr > 32 && spr <= 36 && type != kTypeQ8_0 ? 0.75 : 1.0;
+            waves = kw.splits == 1 && kw.rounds > filled && kw.rounds <= 1.0;
+        }
     } else if (m <= kSmallMaxM2) {
         // 17 to 32 rows, against the short-batch kernels with two blocks of activations or, for the types without them, the
         // 32-row blocks: ahead up to four rounds of workgroups (Q4_K 4096 x 4096 12.8 -> 10.9 us, Q6_K 21.9 -> 13.4, 14336 x 4096

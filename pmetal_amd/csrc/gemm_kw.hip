@@ -379,7 +379,7 @@ __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__
 // grid (8, inner x splits of K, outer / 8), up to eight waves; wave w of split z takes super-blocks [z * chunk + w * per, + per)
 // below min(spr, (z + 1) * chunk).  Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the
 // blocks of activation rows, otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of
-// the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: BY_M_US).
+// the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
 template <class F, int MB, int NR>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,

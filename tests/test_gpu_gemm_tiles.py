@@ -49,6 +49,22 @@ def test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k):
         assert np.max(np.abs(got16 - want)) <= (2.0 ** -8 + bound) * np.max(np.abs(want)), order
 
 
+# Up to 16 activation rows: both sides of each line between this kernel and the short-batch kernels (9, 12, 13, 17, 20, 21, 24, 25,
+# 33, 36 and 37 super-blocks a row; 4096 and 7168 weight rows), one and sixteen activation rows, a weight row count off every tile
+@pytest.mark.parametrize("m,n,k", [(1, 33, 2304), (16, 1, 2304), (5, 7168, 2304), (4, 7169, 2304), (16, 70, 3072), (16, 4097, 2560), (3, 65, 3328), (2, 97, 4352),
+                                   (16, 31, 5120), (7, 4129, 5376), (16, 40, 6144), (9, 33, 6400), (16, 4100, 8448), (1, 64, 9216), (6, 30, 9472)])
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_short_batches_match_dequantize_then_matmul(oracle, t, m, n, k):
+    test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k)
+
+
+# Two weights of a batch on either side of the line share their prepared activations and take a kernel each; two on one side a launch.
+@pytest.mark.parametrize("m,k,ns", [(16, 2560, (33, 4097)), (5, 3072, (4100, 70)), (12, 2304, (97, 64)), (16, 5376, (4129, 40))])
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_short_batch_pairs_match_separate_calls(oracle, t, m, k, ns):
+    test_pairs_match_separate_calls(oracle, t, m, k, ns)
+
+
 # The pre-pass holds 1, 2, 4 or 8 items per thread, or reads a longer row twice; one, two (from 384 rows on) or four rows (from
 # 1024 on) per workgroup.  Rows of activations that end inside a workgroup, row lengths on both sides of each step.
 @pytest.mark.parametrize("m,k", [(3, 4096), (18, 4352), (17, 16384), (20, 16640), (33, 32768), (2, 33024), (385, 4096), (390, 4352), (385, 33024),
