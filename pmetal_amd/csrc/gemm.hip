@@ -2076,6 +2076,10 @@ static double rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
            (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
 }
 
+// The tile kernel's grid counts eighths of its row tiles along z, which holds 65535; tiles of 32 rows, and two ragged ends for a
+// pair.  Only Q2_K at 17 to 32 rows, which takes the tile kernel at every size, has weights this tall (the row kernels take them).
+constexpr int64_t kKwMaxRows = (int64_t)32 * 8 * 65534;
+
 // the tile kernel requests up to six k-steps of items past the last one (32 bytes per row each): they lie in the workspace
 static size_t kw_slack(const GemmPlan &p) { return p.kernel == GemmKernel::kWaves ? (size_t)p.mp * 256 : 0; }
 
@@ -2162,7 +2166,7 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         p.kernel = GemmKernel::kSmall;
         p.chunk = spr > run ? run : (int)spr, p.splits = (int)((spr + p.chunk - 1) / p.chunk);
     }
-    if (waves) {
+    if (waves && n <= kKwMaxRows) {
         GemmPlan t = p;
         t.kernel = GemmKernel::kWaves;
         t.mb = kw.mb, t.nr = kw.nr, t.splits = kw.splits, t.chunk = (int)((spr + kw.splits - 1) / kw.splits);
@@ -2194,6 +2198,7 @@ bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type
         return rounds(t0 + t1) < rounds(t0) + rounds(t1);
     }
     if (p.kernel == GemmKernel::kWaves) {
+        if (n0 + n1 > kKwMaxRows) return false;
         const KwChoice kw = kw_choice(m, n0 + n1, k / 256, type);
         if (kw.splits == 1) plan->mb = kw.mb, plan->nr = kw.nr;
     }

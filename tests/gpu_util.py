@@ -73,3 +73,36 @@ def first_mismatch(a, b, block):
     i = int(bad[0])
     return (f"{bad.size} differing bytes in {np.unique(bad // block).size} blocks; first at byte {i} "
             f"(block {i // block}, offset {i % block}): got {a[i]} want {b[i]}")
+
+
+# ---- the GEMM's launch plan, so that a test can say which kernel its shape takes ---------------------------------
+# qgemm_plan and qgemm_pair_plan (csrc/internal.hpp) are host code and need no device; the library exports them under their
+# C++ names, which carry the argument types: a change of either signature is a missing symbol here and not a wrong answer.
+SMALL, WAVES, ROWS = 0, 1, 2  # GemmKernel
+
+
+class Plan(C.Structure):
+    _fields_ = [(f, C.c_int) for f in ("kernel", "mb", "nr", "mp", "nw", "splits", "chunk")]
+
+    def __repr__(self):
+        return f"{('small', 'waves', 'rows')[self.kernel]} " + " ".join(f"{f}={getattr(self, f)}" for f, _ in self._fields_[1:])
+
+
+def gemm_plan(t, m, n, k):
+    fn = _lib.load()._ZN3pmh10qgemm_planElllj
+    fn.restype, fn.argtypes = Plan, [C.c_int64, C.c_int64, C.c_int64, C.c_uint32]
+    return fn(m, n, k, t)
+
+
+def gemm_pair_plan(t, m, n0, n1, k):
+    """The plan of two weights in one launch, or None where each goes on its own."""
+    fn = _lib.load()._ZN3pmh15qgemm_pair_planElllljPNS_8GemmPlanE
+    fn.restype, fn.argtypes = C.c_bool, [C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_uint32, C.POINTER(Plan)]
+    p = Plan()
+    return p if fn(m, n0, n1, k, t, C.byref(p)) else None
+
+
+def gemm_workspace_bytes(t, m, n, k):
+    fn = _lib.load()._ZN3pmh21qgemm_workspace_bytesEjlll
+    fn.restype, fn.argtypes = C.c_size_t, [C.c_uint32, C.c_int64, C.c_int64, C.c_int64]
+    return fn(t, m, n, k)
