@@ -1240,13 +1240,13 @@ __device__ __forceinline__ float small_row_scale(const float *__restrict__ rowsc
 
 __device__ __forceinline__ void small_store(const float4_t *out_tiles, int t0, int t1, int M, int Mp, int N, const float rs,
                                             void *__restrict__ yg, int ybf16, float *__restrict__ partial, const int mt = 1) {
-    __shared__ float scales[32];
-    if (threadIdx.x < 32) scales[threadIdx.x] = rs;
+    __shared__ float4_t scales[8];  // (of the type that is read back: only that aligns an LDS object to 16 bytes)
+    if (threadIdx.x < 32) reinterpret_cast<float *>(scales)[threadIdx.x] = rs;
     __syncthreads();
     for (int idx = (int)threadIdx.x; idx < (t1 - t0) * mt * 64; idx += (int)blockDim.x) {
         const int tile = mt == 1 ? idx >> 6 : idx >> 7, b = mt == 1 ? 0 : (idx >> 6) & 1, l = idx & 63;
         const int n = (t0 + tile) * 16 + (l & 15), m = 16 * b + 4 * (l >> 4);
-        const float4_t v = out_tiles[idx], o = v * *reinterpret_cast<const float4_t *>(scales + m);
+        const float4_t v = out_tiles[idx], o = v * scales[m / 4];
         if (n >= N) continue;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
