@@ -187,7 +187,7 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
     static __device__ __forceinline__ int slot(int p, int) { return p; }
     uint32_t qd[4], hm[4];
     half2_t sc2[4], off2[4];
-    half8_t br[2];
+    half8_t br[FMT == 3 ? 2 : 1];  // Q2_K's mins
     float d;
     template <int H>
     __device__ __forceinline__ void load(const uint4 *st, int, const int g) {
@@ -207,8 +207,8 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
             dbits = sd.w >> 16;
         }
         d = f16_bits_to_f32(dbits & 0xFFFFu);
-        // scales (and what a sub-block subtracts per unit of its activation sum) of sub-blocks 8 H + 4 sp + 2 lh + g
-        float nm[4];
+        // scales (Q2_K: and what a sub-block subtracts per unit of its activation sum) of sub-blocks 8 H + 4 sp + 2 lh + g
+        float nm[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // (Q2_K)
 #pragma unroll
         for (int sp = 0; sp < 2; sp++)
 #pragma unroll
@@ -222,17 +222,11 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
                     const uint32_t lo4 = (hdr[sp] >> (8u * (uint32_t)g + 16u * lh + 4u * H)) & 15u;
                     const uint32_t hi2 = (hdr[2] >> (8u * (uint32_t)g + 16u * lh + 2u * (2 * H + sp))) & 3u;
                     scf = (float)((int)(lo4 | (hi2 << 4)) - 32);
-                    nm[2 * sp + lh] = -(d * (4.0f * scf));
                 }
                 const _Float16 sh = (_Float16)scf, oh = (_Float16)(-1024.0f * scf);  // exact: |sc| <= 32
                 sc2[2 * sp + lh] = half2_t{sh, sh}, off2[2 * sp + lh] = half2_t{oh, oh};
             }
-#pragma unroll
-        for (int sp = 0; sp < 2; sp++) {
-            const _Float16 h0 = (_Float16)nm[2 * sp], h1 = (_Float16)nm[2 * sp + 1];
-            const _Float16 l0 = (_Float16)(nm[2 * sp] - (float)h0), l1 = (_Float16)(nm[2 * sp + 1] - (float)h1);
-            br[sp] = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
-        }
+        if constexpr (FMT == 3) br[0] = split(nm[0], nm[1]), br[1] = split(nm[2], nm[3]);
         if (FMT == 2) {
 #pragma unroll
             for (int i = 0; i < 4; i++) hm[i] >>= 4 * H;
@@ -252,7 +246,18 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
         const half2_t r3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u)), sc2[2 * sp + 1], off2[2 * sp + 1]);
         b[0] = half8_t{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
     }
-    __device__ __forceinline__ half8_t sums(int i) const { return br[i]; }
+    // the two values as f16 heads and tails
+    static __device__ __forceinline__ half8_t split(const float m0, const float m1) {
+        const _Float16 h0 = (_Float16)m0, h1 = (_Float16)m1;
+        const _Float16 l0 = (_Float16)(m0 - (float)h0), l1 = (_Float16)(m1 - (float)h1);
+        return half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
+    }
+    // (Q3_K subtracts 4 d sc: made from the scales where it is used.  Held over the half it took the 64 x 64 tile past 256 registers
+    // and one of them to scratch memory)
+    __device__ __forceinline__ half8_t sums(int i) const {
+        if constexpr (FMT == 3) return br[i];
+        else return split(-(d * (4.0f * (float)sc2[2 * i][0])), -(d * (4.0f * (float)sc2[2 * i + 1][0])));
+    }
     __device__ __forceinline__ float scale(int) const { return d; }
 };
 
