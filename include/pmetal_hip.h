@@ -203,7 +203,8 @@ int32_t pmetal_hip_qgemm(uint32_t ggml_type, const uint8_t *w_dev, int64_t n, in
  * Same arguments, kernels and results (bit for bit) as pmetal_hip_qgemm; the scratch memory
  * (converted activations, row scales, partial tiles of a K split) is a fixed array of
  * PMETAL_HIP_NOALLOC_SCRATCH_BYTES inside the library's code object, one copy per device, held until the process ends.
- * A shape that needs more (roughly: m * k * 2.25 bytes plus, for few activation rows, splits * m * n * 4) fails with
+ * A shape that needs more (roughly: m * k * 2.25 bytes -- 2 for Q6_K and Q8_0, 2.5 for Q3_K and Q2_K -- plus, where K is split,
+ * splits * m * n * 4) fails with
  * PMETAL_HIP_ERR_SHAPE_TOO_LARGE before anything is launched.  Calls no hipMalloc / hipFree and nothing else that allocates.
  * pmetal_hip_init(device) looks the array's address up; without it the first call on a device does.  All calls on one
  * device share the array: calls on one stream are ordered and may follow each other without a synchronisation; a call

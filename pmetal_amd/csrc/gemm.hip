@@ -2083,8 +2083,14 @@ constexpr int64_t kKwMaxRows = (int64_t)32 * 8 * 65534;
 // the tile kernel requests up to six k-steps of items past the last one (32 bytes per row each): they lie in the workspace
 static size_t kw_slack(const GemmPlan &p) { return p.kernel == GemmKernel::kWaves ? (size_t)p.mp * 256 : 0; }
 
+// the pre-pass's items (the types without a min term have no block sums)
+static size_t prep_bytes(uint32_t type, int64_t k, int mp) {
+    const int groups = type == kTypeQ3K || type == kTypeQ2K ? kGroups16 : type == kTypeQ6K || type == kTypeQ8_0 ? kQ6Groups : kGroups;
+    return align256((size_t)(k / 256) * 2 * groups * mp * 16);
+}
+
 static size_t plan_bytes(const GemmPlan &p, uint32_t type, int64_t n, int64_t k) {
-    const size_t xs = align256((size_t)(k / 256) * 2 * (type == kTypeQ3K || type == kTypeQ2K ? kGroups16 : kGroups) * p.mp * 16);
+    const size_t xs = prep_bytes(type, k, p.mp);
     const size_t part = p.splits > 1 ? align256((size_t)p.splits * p.mp * n * 4) : 0;
     return xs + align256((size_t)p.mp * 4) + part + kw_slack(p);
 }
@@ -2282,7 +2288,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
     uint4 *xs = reinterpret_cast<uint4 *>(ws);
     const bool q23 = type == kTypeQ3K || type == kTypeQ2K;
-    const size_t xs_bytes = align256((size_t)spr * 2 * (q23 ? kGroups16 : kGroups) * p.mp * 16);
+    const size_t xs_bytes = prep_bytes(type, k, p.mp);
     float *rowscale = reinterpret_cast<float *>(ws + xs_bytes);
     float *partial = reinterpret_cast<float *>(ws + xs_bytes + align256((size_t)p.mp * 4));
     const bool xf32 = x_dtype == kDtypeF32, q6 = type == kTypeQ6K, q8 = type == kTypeQ8_0, q5 = type == kTypeQ5K, ref = order == kOrderRef;

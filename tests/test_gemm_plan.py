@@ -1,7 +1,7 @@
 """The GEMM's launch plan (host code, no device needed): what it names can be launched."""
 import pytest
 
-from gpu_util import Q4K, Q6K, Q8_0, WAVES, gemm_pair_plan, gemm_plan
+from gpu_util import Q4K, Q6K, Q8_0, WAVES, gemm_pair_plan, gemm_plan, gemm_workspace_bytes
 
 Q5K, Q3K, Q2K = 13, 11, 10
 TYPES = [Q4K, Q6K, Q8_0, Q5K, Q3K, Q2K]
@@ -27,3 +27,17 @@ def test_tall_weights_stay_within_the_grid(t):
             p = gemm_pair_plan(t, m, n0, n1, 256)
             if p is not None and p.kernel == WAVES:
                 assert (-(-n0 // (32 * p.nr)) - (-n1 // (32 * p.nr)) + 7) // 8 <= GRID_YZ, (m, n0, n1, p)
+
+
+# What the kernels keep there: the pre-pass's items (16 bytes per row, operand group and half super-block: 16 groups, and one or
+# two per half for sums of sub-blocks of 32 or 16 elements where the type has mins), the row scales, the partial tiles of a K
+# split, and what the tile kernel requests past the last item.
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("m,n,k", [(5, 700, 256), (16, 4096, 4096), (24, 1000, 14336), (64, 4096, 2304), (300, 96, 5120), (512, 14336, 4096),
+                                   (1800, 64, 7168), (2048, 1024, 4096)])
+def test_workspace_holds_what_is_written(t, m, n, k):
+    p = gemm_plan(t, m, n, k)
+    groups = {Q6K: 16, Q8_0: 16, Q3K: 20, Q2K: 20}.get(t, 18)
+    up = lambda v: -(-v // 256) * 256
+    need = up(k // 256 * 2 * groups * p.mp * 16) + up(4 * p.mp) + (up(4 * p.splits * p.mp * n) if p.splits > 1 else 0)
+    assert gemm_workspace_bytes(t, m, n, k) == need + (256 * p.mp if p.kernel == WAVES else 0)

@@ -65,7 +65,8 @@ def test_noalloc_equals_qgemm_two_calls_in_a_row():
 
 
 # Shapes whose scratch fills the array to the last per cent: a kernel that takes more is not chosen for them.
-@pytest.mark.parametrize("t,m,n,k", [(8, 3281, 12, 4352), (10, 1738, 4, 7424), (11, 1027, 1, 12288), (13, 1859, 2, 7680), (14, 2539, 18, 5632)])
+@pytest.mark.parametrize("t,m,n,k", [(8, 3281, 12, 4352), (10, 1738, 4, 7424), (11, 1027, 1, 12288), (13, 1859, 2, 7680), (14, 2539, 18, 5632),
+                                     (8, 3777, 18, 4352), (14, 3201, 12, 5120), (8, 4929, 3, 3328), (14, 1921, 500, 4352)])
 def test_noalloc_takes_what_nearly_fills_its_scratch(t, m, n, k):
     lib = _lib.load()
     pm.init(0)
