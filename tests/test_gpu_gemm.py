@@ -514,14 +514,17 @@ def test_qgemm_batch_wide_and_narrow_weights_share_x(oracle, t, m):
                                  # rows of more than 16 super-blocks: runs of 16, partial tiles added in a second kernel
                                  (500, 14336), (130, 6144), (77, 11008), (64, 32768),
                                  # rows of 11, 1, 3, 20 and 13 super-blocks: Q6_K rows then start at any even address, the last
-                                 # wave with work owns one super-block where the others own two, a second run holds four
+                                 # waves own one super-block where the others own two (13)
                                  (333, 2816), (1001, 256), (250, 768), (123, 5120), (47, 3328),
-                                 # rows of 72 and 136 super-blocks: more runs than the fused kernels take (Q8_0 with two blocks of
-                                 # activations: eight runs of 8; the others: eight runs of 16), so the large kernel with its own K split
+                                 # rows of 72 and 136 super-blocks; 136 are more runs than the fused kernels take (eight of 16): the
+                                 # row kernels with a K split of their own at up to 16 activation rows
                                  (40, 18432), (24, 34816)])
 def test_qgemm_short_batches(oracle, t, m, n, k):
-    """At most 16 activation rows (Q4_K, Q5_K, Q8_0 and Q2_K: at most 32, two 16-row blocks per weight operand): the fused kernels that read the weights once (rows of any number of super-blocks, in runs of 16).  Random block bytes (every scale, min and quant pattern), row counts that are no multiple of the 16-row
-    tiles, one full tile, more tiles than workgroups take in one round; bf16 and f32 activations, f32 and bf16 outputs;
+    """Few activation rows.  Up to 16: the fused kernels that read the weights once (rows of up to 16 super-blocks whole, longer ones in
+    runs of 16), or, for the rows of 11 and of 20 super-blocks, the tile kernel; 17 to 32: the tile kernel (the weights are too small
+    here for the fused kernels' two-block form, which the tall weights of test_gpu_gemm_tiles.py take).  Random block bytes (every
+    scale, min and quant pattern), row counts that are no multiple of the 16-row tiles, one full tile, more tiles than workgroups take
+    in one round; bf16 and f32 activations, f32 and bf16 outputs;
     unit activations that pick single weights out of the matrix."""
     rng = np.random.default_rng(1000 * t + 31 * m + n + k)
     block = {Q4K: 144, Q6K: 210, Q8_0: 34, 13: 176, 11: 110, 10: 84}[t]

@@ -4,7 +4,7 @@ import pytest
 
 import pmetal_amd as pm
 from pmetal_amd import _lib
-from gpu_util import Q4K, Q6K, Q8_0
+from gpu_util import Q4K, Q6K, Q8_0, ROWS, SMALL, WAVES, gemm_pair_plan, gemm_plan
 from test_gpu_gemm import gpu_qgemm, reference
 
 pytestmark = pytest.mark.gpu
@@ -27,9 +27,9 @@ def random_blocks(rng, t, n, k):
     return raw.reshape(-1)
 
 
-# (m, n, k): one weight row, one super-block; edges of the 32- and 64-row blocks of both sides; rows of 7, 8, 9 and 17
-# super-blocks (waves of equal and of different length); a narrow weight with long rows (K split over workgroups, the last
-# split shorter than the others); enough tiles for more than one round of workgroups
+# (m, n, k): one weight row, one super-block; row counts around 32 and 64 on both sides (all in 32 x 32 tiles: test_each_tile has the
+# others); rows of 7, 8, 9 and 17 super-blocks (waves of equal and of different length); a narrow weight with long rows (K split over
+# workgroups, the last split shorter than the others); (200, 4100, 768): the row kernels for all types but Q8_0
 @pytest.mark.parametrize("m,n,k", [(17, 1, 256), (32, 31, 1792), (33, 33, 2048), (64, 64, 2304), (65, 65, 4352), (63, 97, 512),
                                    (48, 40, 18688), (29, 70, 33024), (130, 1000, 1024), (200, 4100, 768)])
 @pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
@@ -83,9 +83,9 @@ def test_prepared_activations(oracle, t, m, k):
             assert np.max(np.abs(got - want)) <= (k / 16 + 16) * 2.0 ** -24 * 4 * np.max(np.abs(want)), (order, given.dtype)
 
 
-# Two weights that share their activations go in one launch: every kernel that takes such a pair (short batches, the wave tiles,
-# the rows, whose rounds of workgroups neither weight fills), row counts off every tile, the seam between the two inside a
-# round; three weights of which two are neighbours of one kind; results of one in place of the other's stay calls of their own.
+# Two weights that share their activations, against a call each: short batches and wave tiles, which go in one launch, row counts off
+# every tile, the seam between the two inside a round; row kernels, which at these sizes do not share a launch (test_pairs_in_one_launch
+# has sizes that do); three weights of which two are neighbours of one kind.
 @pytest.mark.parametrize("m,k,ns", [(3, 512, (17, 130)), (16, 4096, (1, 1000)), (16, 2304, (4600, 33)), (17, 1024, (31, 65)), (64, 1792, (97, 64)),
                                     (100, 768, (300, 129)), (600, 512, (7000, 6300)), (1030, 256, (3900, 4111)), (40, 512, (70, 50, 20))])
 @pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
@@ -123,3 +123,116 @@ def test_results_in_one_place_are_not_paired(oracle):
     pm.check(lib.pmetal_hip_sync(None))
     want = gpu_qgemm(Q4K, raws[1], n, k, bits, m)  # the last one's
     assert np.array_equal(dy.to_host(np.float32).reshape(m, n), want)
+
+
+# ---- every kernel that the plan names, at shapes for which it is asserted to name it -------------------------------
+TYPES = [Q4K, Q6K, Q8_0, 13, 11, 10]
+
+
+def orders(t):
+    return (0, 1) if t in (Q4K, 13) else (0,)
+
+
+def bf16_rows(oracle, rng, m, k):
+    bits = oracle.f32_to_bf16_bits(rng.standard_normal(m * k).astype(np.float32)).reshape(m, k)
+    return bits, oracle.bf16_bits_to_f32(bits.reshape(-1)).reshape(m, k)
+
+
+def bound(k):  # as above: at most k / 16 + 16 additions in f32 on partial sums within four times the largest result
+    return (k / 16 + 16) * 2.0 ** -24 * 4
+
+
+# The four tiles of the tile kernel: 32 or 64 activation rows by 32 or 64 weight rows.  Rows just past a tile on either side, rows of
+# 2, 3, 7 and 9 super-blocks (2, 3, 7 and 5 waves; 9: the last wave has one where the others have two); 700 activation rows: the dies
+# share out the activations and not the weights, over more than one tile of these.
+@pytest.mark.parametrize("mb,nr,m,n,k", [(1, 1, 33, 4000, 512), (1, 1, 600, 100, 512), (1, 1, 600, 130, 2304),
+                                         (1, 2, 17, 12289, 512), (1, 2, 32, 10049, 1792), (1, 2, 17, 12289, 2304),
+                                         (2, 1, 33, 8129, 768), (2, 1, 161, 2561, 512), (2, 1, 300, 1473, 1792), (2, 1, 700, 705, 512),
+                                         (2, 2, 33, 8257, 2304), (2, 2, 97, 4097, 1792), (2, 2, 700, 1000, 1024)])
+@pytest.mark.parametrize("t", TYPES)
+def test_each_tile(oracle, t, mb, nr, m, n, k):
+    p = gemm_plan(t, m, n, k)
+    assert (p.kernel, p.mb, p.nr, p.splits) == (WAVES, mb, nr, 1), p
+    test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k)
+
+
+# ... and with K split over workgroups, which the plan does for long rows; the last split is shorter than the others (69, 73 and 17
+# super-blocks in four, 73 in two)
+@pytest.mark.parametrize("t,mb,nr,splits,m,n,k", [(Q4K, 2, 1, 4, 161, 321, 18688), (Q6K, 2, 1, 4, 33, 1025, 4352), (Q8_0, 2, 1, 4, 33, 1025, 4352),
+                                                  (13, 2, 1, 4, 33, 1025, 4352), (Q6K, 2, 2, 2, 97, 2561, 18688), (Q8_0, 2, 2, 4, 33, 2049, 18688),
+                                                  (13, 2, 2, 4, 193, 577, 18688), (11, 2, 2, 4, 63, 2561, 18688), (10, 2, 2, 4, 33, 2561, 18688),
+                                                  (Q4K, 2, 2, 4, 513, 321, 18688), (Q4K, 2, 1, 2, 700, 321, 18688)])
+def test_each_tile_with_a_k_split(oracle, t, mb, nr, splits, m, n, k):
+    p = gemm_plan(t, m, n, k)
+    assert (p.kernel, p.mb, p.nr, p.splits) == (WAVES, mb, nr, splits), p
+    test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k)
+
+
+# Weights so tall that the plan keeps the short-batch kernels with two blocks of activations (Q4_K, Q5_K, Q8_0) and the row kernels with
+# 32 and with 64 activation rows; a sample of rows at both ends and in the middle against the oracle.  Rows of 1, 2, 9 and 16 super-blocks
+# and, in runs with partial tiles, of 32 and (Q8_0) 9 and 16; 136: longer than the short-batch kernels take.  The first two: rows of 20 and
+# 17 super-blocks where the tile kernel ends, whose second run of the short-batch kernels leaves waves without a super-block.
+TWO_BLOCKS = {Q4K: SMALL, 13: SMALL, Q8_0: SMALL, Q6K: ROWS, 11: ROWS, 10: WAVES}
+ALL_ROWS, ALL_SMALL = dict.fromkeys(TYPES, ROWS), dict.fromkeys(TYPES, SMALL)
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [(9, 14401, 5120, ALL_SMALL), (16, 14401, 4352, ALL_SMALL), (17, 24577, 4096, TWO_BLOCKS), (32, 24577, 4096, TWO_BLOCKS), (17, 12289, 8192, TWO_BLOCKS), (32, 12289, 8192, TWO_BLOCKS),
+                                          (29, 50001, 2304, TWO_BLOCKS), (24, 400001, 256, TWO_BLOCKS), (25, 200001, 512, TWO_BLOCKS), (24, 3100, 34816, {**ALL_ROWS, 10: WAVES}),
+                                          (33, 70001, 512, ALL_ROWS), (64, 40001, 512, ALL_ROWS), (192, 40001, 256, ALL_ROWS), (33, 60001, 2304, ALL_ROWS)])
+@pytest.mark.parametrize("t", TYPES)
+def test_tall_weights(oracle, t, m, n, k, kernel):
+    p = gemm_plan(t, m, n, k)
+    assert p.kernel == kernel[t] and (p.kernel != ROWS or p.mb == (1 if m <= 32 else 2)), p
+    rng = np.random.default_rng(t + m + n + k)
+    raw = random_blocks(rng, t, n, k)
+    bits, x = bf16_rows(oracle, rng, m, k)
+    rows = np.r_[0:300, n // 2 - 100:n // 2 + 100, n - 300:n]
+    sample = raw.reshape(n, -1)[rows].reshape(-1)
+    for order in orders(t):
+        want = reference(oracle, t, sample, len(rows), k, x, order)
+        got = gpu_qgemm(t, raw, n, k, bits, m, order=order)
+        assert np.all(np.isfinite(got))
+        assert np.max(np.abs(got[:, rows] - want)) <= bound(k) * np.max(np.abs(want)), order
+        got16 = gpu_qgemm(t, raw, n, k, bits, m, y_dtype=pm.DTYPE_BF16, order=order)
+        assert np.max(np.abs(got16[:, rows] - want)) <= (2.0 ** -8 + bound(k)) * np.max(np.abs(want)), order
+
+
+# Two weights in one launch, for each kernel that takes them: the plan is asked that it is one launch.  Row kernels with 128, 64 and 32
+# activation rows, short batches with two blocks of activations, tiles whose plan for the pair is a larger tile than each weight's own.
+@pytest.mark.parametrize("m,k,ns,kernel", [(300, 512, (8200, 8201), ALL_ROWS), (200, 512, (9000, 9401), ALL_ROWS), (1030, 512, (8200, 8301), ALL_ROWS),
+                                           (40, 256, (76801, 76900), ALL_ROWS), (24, 256, (400001, 400100), TWO_BLOCKS), (24, 4096, (24577, 24600), {Q4K: SMALL, 13: SMALL, 10: WAVES}),
+                                           (20, 512, (4100, 4201), dict.fromkeys(TYPES, WAVES)), (64, 512, (4100, 4201), dict.fromkeys(TYPES, WAVES))])
+@pytest.mark.parametrize("t", TYPES)
+def test_pairs_in_one_launch(oracle, t, m, k, ns, kernel):
+    if t not in kernel:
+        assert gemm_pair_plan(t, m, *ns, k) is None  # (a K split: each on its own)
+        return
+    p, alone = gemm_pair_plan(t, m, *ns, k), gemm_plan(t, m, ns[0], k)
+    assert p is not None and p.kernel == kernel[t], p
+    if kernel[t] == WAVES and m == 64:
+        assert (p.mb, p.nr) != (alone.mb, alone.nr), (p, alone)
+    rng = np.random.default_rng(t + m + k)
+    raws = [random_blocks(rng, t, n, k) for n in ns]
+    bits, x = bf16_rows(oracle, rng, m, k)
+    lib = _lib.load()
+    dx, dws = pm.DeviceBuffer.from_host(bits), [pm.DeviceBuffer.from_host(raw) for raw in raws]
+    for order in orders(t):
+        for y_dtype, size in ((pm.DTYPE_F32, 4), (pm.DTYPE_BF16, 2)):
+            dys = [pm.DeviceBuffer(m * n * size + 256) for n in ns]
+            alone = [pm.DeviceBuffer(m * n * size) for n in ns]
+            for dy in dys:
+                pm.check(lib.pmetal_hip_memset(dy.ptr, 0xFF, dy.nbytes, None))
+            descs = (_lib.GemmDesc * 2)(*[_lib.GemmDesc(t, y_dtype, order, 0, n, w.ptr, y.ptr) for n, w, y in zip(ns, dws, dys)])
+            pm.check(lib.pmetal_hip_qgemm_batch(descs, 2, k, dx.ptr, pm.DTYPE_BF16, m, None))
+            for n, w, y in zip(ns, dws, alone):
+                pm.check(lib.pmetal_hip_qgemm(t, w.ptr, n, k, dx.ptr, pm.DTYPE_BF16, m, y.ptr, y_dtype, order, None))
+            pm.check(lib.pmetal_hip_sync(None))
+            for n, raw, dy, one in zip(ns, raws, dys, alone):
+                out = dy.to_host(np.uint8)
+                assert np.all(out[m * n * size:] == 0xFF)
+                assert np.array_equal(out[:m * n * size], one.to_host(np.uint8)), (order, y_dtype)
+                if y_dtype == pm.DTYPE_F32:
+                    rows = np.r_[0:200, n - 200:n]
+                    want = reference(oracle, t, raw.reshape(n, -1)[rows].reshape(-1), len(rows), k, x, order)
+                    got = out[:m * n * 4].view(np.float32).reshape(m, n)[:, rows]
+                    assert np.max(np.abs(got - want)) <= bound(k) * np.max(np.abs(want)), order
