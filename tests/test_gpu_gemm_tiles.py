@@ -236,3 +236,43 @@ def test_pairs_in_one_launch(oracle, t, m, k, ns, kernel):
                     want = reference(oracle, t, raw.reshape(n, -1)[rows].reshape(-1), len(rows), k, x, order)
                     got = out[:m * n * 4].view(np.float32).reshape(m, n)[:, rows]
                     assert np.max(np.abs(got - want)) <= bound(k) * np.max(np.abs(want)), order
+
+
+# Two weights that the plan would put in one launch, but one's results lie over what the other reads or writes.  In one launch the order
+# of the workgroups makes each of these wrong for certain: the launch takes three rounds of workgroups, its nine blocks of 128
+# activation rows one after the other, both weights in each.  (a) The second weight's first blocks of results lie over the last blocks
+# of the first one's.  (b) The first one's results lie over the second one's blocks, (c) the other way round: the first 72 rows of
+# results replace a weight that eight more blocks of rows read.
+@pytest.mark.parametrize("over", ["results", "second weight", "first weight"])
+def test_results_over_the_neighbour_are_not_paired(oracle, over):
+    t, m, n, k = Q4K, 1030, 8200, 512
+    p = gemm_pair_plan(t, m, n, n, k)
+    assert p is not None and p.kernel == ROWS and p.mb == 4, p
+    rng = np.random.default_rng(11)
+    raws = [random_blocks(rng, t, n, k) for _ in range(2)]
+    bits, _ = bf16_rows(oracle, rng, m, k)
+    lib = _lib.load()
+    dx = pm.DeviceBuffer.from_host(bits)
+    y_bytes = m * n * 4
+
+    def outputs(batch):
+        buf = pm.DeviceBuffer(2 * y_bytes)
+        pm.check(lib.pmetal_hip_memset(buf.ptr, 0, buf.nbytes, None))
+        dws = [pm.DeviceBuffer.from_host(raw) for raw in raws]
+        ys, ws = [buf.ptr, buf.ptr + y_bytes], [w.ptr for w in dws]
+        if over == "results":
+            ys[1] = buf.ptr + 900 * n * 4
+        else:
+            at = 1 if over == "second weight" else 0
+            ws[at] = ys[1 - at]
+            pm.check(lib.pmetal_hip_h2d(ws[at], raws[at].ctypes.data, raws[at].size))
+        if batch:
+            descs = (_lib.GemmDesc * 2)(*[_lib.GemmDesc(t, pm.DTYPE_F32, 0, 0, n, w, y) for w, y in zip(ws, ys)])
+            pm.check(lib.pmetal_hip_qgemm_batch(descs, 2, k, dx.ptr, pm.DTYPE_BF16, m, None))
+        else:
+            for w, y in zip(ws, ys):
+                pm.check(lib.pmetal_hip_qgemm(t, w, n, k, dx.ptr, pm.DTYPE_BF16, m, y, pm.DTYPE_F32, 0, None))
+        pm.check(lib.pmetal_hip_sync(None))
+        return buf.to_host(np.uint8)
+
+    assert np.array_equal(outputs(True), outputs(False))
