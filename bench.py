@@ -420,6 +420,20 @@ def cpu_baseline_calibrate(budget_elems=1 << 20):
             "sample": f"{reps} x calibrate_tensor over {budget_elems} elements, six candidates, {dt:.1f} s"}
 
 
+def _gemm_kernel(_lib, t, m, n, k):
+    """The kernels that a call of this shape launches, as the library's launch plan names them."""
+    p = _lib.gemm_plan(t, m, n, k)
+    if p.kernel == _lib.GEMM_SMALL:
+        name = {Q4K: "k_qgemm_small", 13: "k_qgemm_small<FMT = 1>", Q6K: "k_qgemm_small_q6", Q8_0: "k_qgemm_small_q8",
+                11: "k_qgemm_small16<Q3_K>", 10: "k_qgemm_small16<Q2_K>"}[t]
+    elif p.kernel == _lib.GEMM_WAVES:
+        name = {Q4K: "k_qgemm_kw<KwQ45", 13: "k_qgemm_kw<KwQ45<FMT = 1>", Q6K: "k_qgemm_kw<KwQ6", Q8_0: "k_qgemm_kw<KwQ8", 11: "k_qgemm_kw<KwQ23<Q3_K>",
+                10: "k_qgemm_kw<KwQ23<Q2_K>"}[t] + f", {p.mb}, {p.nr}>"
+    else:
+        name = {Q4K: "k_qgemm_rw", 13: "k_qgemm_rw<FMT = 1>", Q6K: "k_qgemm_rw_q6", Q8_0: "k_qgemm_rw_q8", 11: "k_qgemm_rw16<Q3_K>", 10: "k_qgemm_rw16<Q2_K>"}[t]
+    return name + " (+ k_prep_rw" + (f", k_rw_reduce over {p.splits} K splits)" if p.splits > 1 else ")")
+
+
 def bench_gemm(args, m, n, k, t=Q4K):
     pm, _lib, lib = load()
     timer = Timer(pm, lib)
@@ -524,11 +538,7 @@ def bench_gemm(args, m, n, k, t=Q4K):
         "value": tflops, "ms_per_step": wall_ms / args.steps, "event_ms_per_step": ev_ms / args.steps,
         "roofline": {"bound": "mfma", "achieved": round(tflops, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / BF16_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": ({Q4K: "k_qgemm_small", 13: "k_qgemm_small<FMT = 1>", Q6K: "k_qgemm_small_q6", Q8_0: "k_qgemm_small_q8",
-                                 11: "k_qgemm_small16<Q3_K>", 10: "k_qgemm_small16<Q2_K>"}[t] + " (+ k_prep_rw)"
-                                if m <= 16 else
-                                {Q4K: "k_qgemm_rw", 13: "k_qgemm_rw<FMT = 1>", Q6K: "k_qgemm_rw_q6", Q8_0: "k_qgemm_rw_q8", 11: "k_qgemm_rw16<Q3_K>", 10: "k_qgemm_rw16<Q2_K>"}[t]
-                                + " (+ k_prep_rw, k_rw_reduce when K is split)"),
+                     "kernel": _gemm_kernel(_lib, t, m, n, k),
                      "flops_per_launch": flops, "us_per_launch": round(us, 3)},
         "extra": {"calls_per_step": copies, "submission": submission, "eager_us_per_call": round(eager_us, 3),
                   "replayed_us_per_call": None if replay_us is None else round(replay_us, 3), "weights": f"{copies} tensor(s) in turn" + (" (from HBM)" if copies > 1 else " (one tensor: stays in the last-level cache)"),

@@ -100,3 +100,22 @@ def load() -> C.CDLL:
             fn.restype, fn.argtypes = restype, argtypes
         _lib = lib
     return _lib
+
+
+# ---- which kernel a GEMM takes (for the benchmark's record and for tests) --------------------------------------------
+GEMM_SMALL, GEMM_WAVES, GEMM_ROWS = 0, 1, 2  # GemmKernel in csrc/internal.hpp
+
+
+class GemmPlan(C.Structure):
+    _fields_ = [(f, C.c_int) for f in ("kernel", "mb", "nr", "mp", "nw", "splits", "chunk")]
+
+    def __repr__(self):
+        return f"{('small', 'waves', 'rows')[self.kernel]} " + " ".join(f"{f}={getattr(self, f)}" for f, _ in self._fields_[1:])
+
+
+def gemm_plan(ggml_type: int, m: int, n: int, k: int) -> GemmPlan:
+    """The launch plan (``qgemm_plan`` in csrc/internal.hpp: host code, needs no device).  It is not part of the C ABI and goes by its
+    C++ name, which carries the argument types: a change of its signature is a missing symbol here and not a wrong answer."""
+    fn = load()._ZN3pmh10qgemm_planElllj
+    fn.restype, fn.argtypes = GemmPlan, [C.c_int64, C.c_int64, C.c_int64, _u32]
+    return fn(m, n, k, ggml_type)

@@ -76,22 +76,9 @@ def first_mismatch(a, b, block):
 
 
 # ---- the GEMM's launch plan, so that a test can say which kernel its shape takes ---------------------------------
-# qgemm_plan and qgemm_pair_plan (csrc/internal.hpp) are host code and need no device; the library exports them under their
-# C++ names, which carry the argument types: a change of either signature is a missing symbol here and not a wrong answer.
-SMALL, WAVES, ROWS = 0, 1, 2  # GemmKernel
-
-
-class Plan(C.Structure):
-    _fields_ = [(f, C.c_int) for f in ("kernel", "mb", "nr", "mp", "nw", "splits", "chunk")]
-
-    def __repr__(self):
-        return f"{('small', 'waves', 'rows')[self.kernel]} " + " ".join(f"{f}={getattr(self, f)}" for f, _ in self._fields_[1:])
-
-
-def gemm_plan(t, m, n, k):
-    fn = _lib.load()._ZN3pmh10qgemm_planElllj
-    fn.restype, fn.argtypes = Plan, [C.c_int64, C.c_int64, C.c_int64, C.c_uint32]
-    return fn(m, n, k, t)
+# (qgemm_pair_plan and qgemm_workspace_bytes by their C++ names, as _lib.gemm_plan finds qgemm_plan)
+Plan, gemm_plan = _lib.GemmPlan, _lib.gemm_plan
+SMALL, WAVES, ROWS = _lib.GEMM_SMALL, _lib.GEMM_WAVES, _lib.GEMM_ROWS
 
 
 def gemm_pair_plan(t, m, n0, n1, k):
