@@ -2060,7 +2060,8 @@ static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
                 if (splits > 1 && (tiles * splits > 256 || (m <= 32 && nr == 2))) break;  // only to fill the machine
                 const int64_t chunk = (spr + splits - 1) / splits, per = (chunk + 7) / 8, wgs = tiles * splits;
                 const double rounds = ((double)wgs / 256.0 + (double)((wgs + 255) / 256)) / 2;
-                const double one = (double)per * 8.0 * (mb * 32 * items * 16 / 1e3 / 124.0 + nr * 32 * block / 1e3 / 34.0) + cost * mb * nr * per;
+                const double nwaves = m <= kSmallMaxM2 && spr < 8 ? (double)spr : 8.0;  // (a short row's workgroup has a wave per super-block)
+                const double one = (double)per * nwaves * (mb * 32 * items * 16 / 1e3 / 124.0 + nr * 32 * block / 1e3 / 34.0) + cost * mb * nr * per;
                 const double us = 5.9 + (1.0 + (rounds - 1.0) * 0.78) * one + (splits > 1 ? 2.5 + splits * (double)m * (double)n * 8.0 * 0.7 / 4.0e6 : 0.0);
                 if (!have || us < best.us) best = {mb, nr, splits, us, (double)wgs / 256.0}, have = true;
             }
@@ -2074,6 +2075,30 @@ static double rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
     const int64_t wgs = (n + 255) / 256 * (p.mp / (32 * p.mb)) * p.splits;
     return 9.6 + (double)((wgs + 255) / 256) * 2.0 * p.chunk * half * (p.mb == 4 ? 1.45 : 1.0) +
            (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
+}
+
+// 17 to 32 activation rows, Q4_K, Q5_K and Q8_0: microseconds of a whole call with the tile kernel and with the short-batch kernel's
+// two blocks of activations, fitted to 4900 drawn shapes of 200 to 60000 weight rows of 1 to 130 super-blocks that were timed with
+// both (rms 9 and 9 %).  Both are staircases: the tile kernel's in the workgroups of the busiest compute unit, each as long as its share of
+// a row, none faster than the weights come from memory (the 4-norm of the two times); the short-batch kernel's in the row
+// tiles of a workgroup, taken in pairs, with a step where it no longer keeps all partial tiles to the end.
+static double two_blocks_tile_us(const KwChoice &kw, int64_t m, int64_t n, int64_t spr, uint32_t type) {
+    const double block = type == kTypeQ4K ? 144 : type == kTypeQ5K ? 176 : 272, work = type == kTypeQ4K ? 0.47 : type == kTypeQ5K ? 0.96 : 0.85;
+    const int64_t chunk = (spr + kw.splits - 1) / kw.splits, per = (chunk + 7) / 8, wgs = (n + 32 * kw.nr - 1) / (32 * kw.nr) * kw.splits;
+    const double one = 0.3 * kw.nr + (double)per * (0.79 + kw.nr * work) + 0.155 * kw.nr * (double)chunk;
+    const double us = (1.0 + (kw.nr == 1 ? 0.65 : 1.0) * (double)((wgs + 255) / 256 - 1)) * one, mem = (double)n * (double)spr * block * 4.1e-7;
+    return 5.1 + __builtin_sqrt(__builtin_sqrt(us * us * us * us + mem * mem * mem * mem)) +
+           (kw.splits > 1 ? 2.5 + 3.7e-6 * kw.splits * (double)m * (double)n : 0.0);
+}
+static double two_blocks_small_us(int64_t m, int64_t n, int64_t spr, uint32_t type) {
+    const int64_t run = small_run_spr(type, m), runs = (spr + run - 1) / run, tiles = (n + 15) / 16;
+    const int64_t per_cu = kSmallWaves / (spr < kSmallWaves ? spr : kSmallWaves), room = 256 * per_cu / runs, slots = room < 1 ? 1 : room;
+    const int64_t wgs = tiles < slots ? tiles : slots, want = (tiles + wgs - 1) / wgs, t = want < 32 ? want : 32;
+    const int64_t rounds = ((tiles + t - 1) / t * runs + 256 * per_cu - 1) / (256 * per_cu);
+    const bool pair = run > kSmallWaves && spr > kSmallWaves, q4 = type == kTypeQ4K, q8 = type == kTypeQ8_0;  // (two super-blocks a wave)
+    const double first = pair ? (q4 ? 4.0 : 4.7) : 0.0, next = pair ? (q4 ? 4.8 : 5.9) : (q4 ? 3.2 : 3.7);
+    return 8.0 + (double)rounds * (first + next * (double)((t + 1) / 2 - 1) + (2 * t > kSmallKeepTiles ? 1.6 : 0.0)) +
+           (runs > 1 ? (q8 ? 2.0 : 0.6) + (q8 ? 0.63 : 1.16) * (double)runs + 6e-7 * (double)(runs * m) * (double)n : 0.0);
 }
 
 // The tile kernel's grid counts eighths of its row tiles along z, which holds 65535; tiles of 32 rows, and two ragged ends for a
@@ -2136,13 +2161,21 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     if (m <= kSmallMaxM) {
         // The short-batch kernels' workgroups walk 16 super-blocks of a row at a time however few of them there are, and add the
         // runs of a longer row in a third launch; the tile kernel's waves share what there is.  Tile kernel against them, us at
-        // M = 12 and how many times faster over the six types:
-        //   rows of 9 to 12 super-blocks, without a K split, so that a second weight can share the launch (1504...7168 rows of
-        //     nine 1.05 to 1.33, 4096 rows of twelve 1.06 to 1.30; two weights of 4096 rows of ten together 1.07 to 1.18)
-        //   rows of 17 to 20: 1.02 to 1.54 (Q4_K 8192 x 5120 15.9 -> 13.6, Q6_K 14336 x 5120 41.4 -> 28.7)
+        // M = 12 and how many times faster:
+        //   rows of 9 to 12 super-blocks, without a K split, so that a second weight can share the launch: ahead for every type up to
+        //     7168 rows of nine and 4096 of twelve (1.05 to 1.33; two weights of 4096 rows of ten together 1.07 to 1.18).  Above, the
+        //     types part: 12288 rows of nine Q3_K 16.1 -> 12.9, Q5_K 15.8 -> 15.2, 9216 rows Q8_0 15.7 -> 16.3; 8192 rows of twelve
+        //     Q6_K 16.7 -> 14.5, Q8_0 12.8 -> 13.6; 12288 rows Q4_K 14.6 -> 16.6
+        //   rows of 17 to 20: up to 14336 rows (Q4_K 8192 x 5120 15.9 -> 13.6, Q6_K 14336 x 5120 41.4 -> 28.7).  Above, Q4_K, Q5_K and
+        //     Q8_0 are behind (27648 x 5120 34.3 -> 38.8, 41.9 -> 47.0, 47.4 -> 51.5), Q3_K and Q2_K at 20480 rows (34.2 -> 40.5, 30.7
+        //     -> 34.5) and not at 27648 (43.3 -> 42.1, 38.4 -> 35.4); Q6_K alone stays ahead (75.4 -> 58.4)
         //   rows of 21 to 24 and of 33 to 36, where the tiles fill half or three quarters of the machine without a K split: 5008 and
-        //     8192 rows of 24 1.07 to 1.31, 7008 rows of 36 1.04 to 1.42 (4096 rows of 24 Q6_K 0.93, 5008 of 36 Q5_K 0.90)
+        //     8192 rows of 24 1.07 to 1.31, 7008 rows of 36 1.04 to 1.42 (one Q5_K weight is behind there, 25.0 -> 27.0; two of 6208 x 8448 44.3 -> 38.0)
         // 13 to 16, 25 to 32 and longer rows leave the short-batch kernels little idle: 14336 rows of 14, 28 and 48 0.77 to 1.10.
+        // Weights of 8193 to 12288 rows are one row of tiles too many for a round of 32-row tiles and fill less than three quarters
+        // of one of 64-row tiles: a single one is behind for Q5_K and Q8_0 (10818 x 5120 23.3 -> 25.2, 25.2 -> 26.8) and, with rows of 24, for
+        // Q4_K and Q6_K (1.06, 1.14 times as long).  They stay here for the launch that two of a batch share: Q8_0 8957 x 4352 43.5 -> 35.6
+        // for two, Q6_K 9465 x 5632 56.6 -> 45.5.
         if (spr > 8 && spr <= 12) {
             waves = n <= (spr == 9 ? 7168 : 4096);
             if (waves) kw.splits = 1, kw.nr = 1;
@@ -2154,11 +2187,19 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         }
     } else if (m <= kSmallMaxM2) {
         // 17 to 32 rows, against the short-batch kernels with two blocks of activations or, for the types without them, the
-        // 32-row blocks: ahead up to four rounds of workgroups (Q4_K 4096 x 4096 12.8 -> 10.9 us, Q6_K 21.9 -> 13.4, 14336 x 4096
-        // 29.2 -> 26.1; behind at 128256 x 4096: Q4_K 87 -> 103, Q6_K 141 -> 154) and where a row is not whole runs (32000 x 5120:
-        // Q4_K 50.8 -> 40.5)
+        // 32-row blocks: below 96 Mi elements (Q4_K 4096 x 4096 12.8 -> 10.9 us, Q6_K 21.9 -> 13.4, 14336 x 4096 29.2 -> 26.1; behind at
+        // 128256 x 4096: Q4_K 87 -> 103, Q6_K 141 -> 154) and where a row is not whole runs (32000 x 5120: Q4_K 50.8 -> 40.5)
         waves = n * k < ((int64_t)96 << 20) || (small && spr > run && spr % run != 0 && type != kTypeQ8_0);
         waves = waves || (type == kTypeQ2K);  // (no short-batch form for two blocks; ahead at every size: 128256 x 4096 98 -> 90 us)
+        // Not where the short-batch kernel's two blocks are expected to be clearly ahead: long rows, and rounds of workgroups that end soon
+        // after they began (Q5_K 17096 x 19712 135.3 -> 83.7 us, 16796 x 22016 150.3 -> 98.8, 4355 x 26112 63.4 -> 44.9, Q4_K 17542 x
+        // 14848 79.5 -> 59.4, Q8_0 37321 x 2048 35.8 -> 26.7).  By how much follows from the fits' errors and from the launch that two
+        // weights of a batch share, which the short-batch kernel's runs cannot (two of Q8_0 6772 x 8192 39.8 us, in runs 50.5): closely
+        // for the long rows of Q4_K and Q5_K, on which two weights gain nothing.
+        if (small && spr > 2) {
+            const double margin = spr > 32 && type != kTypeQ8_0 ? 1.05 : spr > run ? 1.25 : 1.2;
+            waves = waves && two_blocks_tile_us(kw, m, n, spr, type) < margin * two_blocks_small_us(m, n, spr, type);
+        }
     } else {
         // against the row kernels, by the times fitted to both over 1000...14336 weight rows of 1024...14336 elements and
         // 64...2048 activation rows (the chosen kernel is within 2 % of the better one on average); from the third round of

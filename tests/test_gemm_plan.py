@@ -1,7 +1,7 @@
 """The GEMM's launch plan (host code, no device needed): what it names can be launched."""
 import pytest
 
-from gpu_util import Q4K, Q6K, Q8_0, WAVES, gemm_pair_plan, gemm_plan, gemm_workspace_bytes
+from gpu_util import Q4K, Q6K, Q8_0, SMALL, WAVES, gemm_pair_plan, gemm_plan, gemm_workspace_bytes
 
 Q5K, Q3K, Q2K = 13, 11, 10
 TYPES = [Q4K, Q6K, Q8_0, Q5K, Q3K, Q2K]
@@ -41,3 +41,28 @@ def test_workspace_holds_what_is_written(t, m, n, k):
     up = lambda v: -(-v // 256) * 256
     need = up(k // 256 * 2 * groups * p.mp * 16) + up(4 * p.mp) + (up(4 * p.splits * p.mp * n) if p.splits > 1 else 0)
     assert gemm_workspace_bytes(t, m, n, k) == need + (256 * p.mp if p.kernel == WAVES else 0)
+
+
+# Few activation rows: the kernel that measured faster (us with the short-batch kernel, with the tile kernel), clear cases of either.
+@pytest.mark.parametrize("t,m,n,k,kernel", [
+    (Q5K, 19, 17096, 19712, SMALL),  # 84, 135: long rows in three rounds of tiles
+    (Q5K, 30, 4355, 26112, SMALL),   # 45, 63: long rows that half fill one round
+    (Q4K, 26, 16541, 18944, SMALL),  # 71, 100
+    (Q4K, 19, 17542, 14848, SMALL),  # 59, 80
+    (Q8_0, 19, 37321, 2048, SMALL),  # 27, 36
+    (Q4K, 24, 4096, 4096, WAVES),    # 12.8, 10.9
+    (Q4K, 17, 8192, 5120, WAVES),    # 18, 13
+    (Q5K, 20, 4096, 3072, WAVES),    # 13, 10
+    (Q8_0, 32, 6144, 3072, WAVES),   # 18, 13
+    (Q8_0, 20, 1024, 20480, WAVES),  # 40, 23
+    (Q4K, 12, 8192, 5120, WAVES),    # 15.9, 13.6
+    (Q5K, 12, 14336, 4352, WAVES)])  # 24, 22
+def test_few_rows_take_the_faster_kernel(t, m, n, k, kernel):
+    assert gemm_plan(t, m, n, k).kernel == kernel, gemm_plan(t, m, n, k)
+
+
+# A row of one or two super-blocks has as many waves: tiles of 64 weight rows for them only where 32 would be several rounds.
+@pytest.mark.parametrize("t,m,n,k", [(Q8_0, 20, 10275, 256), (Q2K, 21, 9389, 256), (Q5K, 28, 9202, 256), (Q2K, 22, 18800, 512)])
+def test_short_rows_take_the_small_tile(t, m, n, k):
+    p = gemm_plan(t, m, n, k)
+    assert (p.kernel, p.nr) == (WAVES, 1), p  # (8.5 us, 11 with 64 rows)

@@ -143,10 +143,10 @@ def bound(k):  # as above: at most k / 16 + 16 additions in f32 on partial sums 
 
 
 # The four tiles of the tile kernel: 32 or 64 activation rows by 32 or 64 weight rows.  Rows just past a tile on either side, rows of
-# 2, 3, 7 and 9 super-blocks (2, 3, 7 and 5 waves; 9: the last wave has one where the others have two); 700 activation rows: the dies
+# 2, 3, 7, 9 and 10 super-blocks (2, 3, 7 and 5 waves; 9: the last wave has one where the others have two); 700 activation rows: the dies
 # share out the activations and not the weights, over more than one tile of these.
 @pytest.mark.parametrize("mb,nr,m,n,k", [(1, 1, 33, 4000, 512), (1, 1, 600, 100, 512), (1, 1, 600, 130, 2304),
-                                         (1, 2, 17, 12289, 512), (1, 2, 32, 10049, 1792), (1, 2, 17, 12289, 2304),
+                                         (1, 2, 17, 12289, 2304), (1, 2, 32, 10049, 2560), (1, 2, 17, 10049, 4352),
                                          (2, 1, 33, 8129, 768), (2, 1, 161, 2561, 512), (2, 1, 300, 1473, 1792), (2, 1, 700, 705, 512),
                                          (2, 2, 33, 8257, 2304), (2, 2, 97, 4097, 1792), (2, 2, 700, 1000, 1024)])
 @pytest.mark.parametrize("t", TYPES)
