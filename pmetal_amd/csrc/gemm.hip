@@ -1187,7 +1187,7 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restric
 constexpr int kSmallWaves = 8;  // waves per workgroup (fewer when a row has fewer super-blocks); 16 waves of one super-block each run alike
 constexpr int kSmallDepth = 2;  // row tiles in flight per wave (four are slower: 16.5 against 12.7 us at 14336 x 4096)
 constexpr int kSmallMaxM = 16, kSmallMaxSpr = 16;
-constexpr int kSmallMaxM2 = 32;  // Q4_K and Q5_K: two 16-row blocks of activations per weight operand
+constexpr int kSmallMaxM2 = 32;  // Q4_K, Q5_K and Q8_0: two 16-row blocks of activations per weight operand
 
 // The two steps the short-batch kernels share.  A row tile's 16 x 16 partial tiles, one per wave: every wave leaves its
 // own in LDS, and after one barrier the first wave adds them in wave order and keeps the sum as finished tile `ti` (the
@@ -2039,8 +2039,9 @@ bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
     return (type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ6K || type == kTypeQ8_0 || type == kTypeQ3K || type == kTypeQ2K) && m >= 1 && m <= (int64_t)1 << 22 && n >= 1 && k >= 256 && k % 256 == 0 && k <= (int64_t)1 << 22 && n <= 0x7FFFFF00;
 }
 
-// The tile kernel's best tile and K split for a shape, and the microseconds it is expected to take behind the pre-pass.  Fitted
-// to 1500 measured times (rms 12 %): per round of 256 workgroups a wave's super-blocks cost 1/124 us per KB of activations and
+// The tile kernel's best tile and K split for a shape, and the microseconds it is expected to take behind the pre-pass, the gap in front
+// of its launch (2.7 us) included.  Fitted to times of 1500 shapes (rms 12 %; 14 % over 150 others, drawn from 2 to 700 activation
+// rows and timed by kernel trace): per round of 256 workgroups a wave's super-blocks cost 1/124 us per KB of activations and
 // 1/34 us per KB of weights the workgroup takes in, plus 0.8 us per 32 x 32 tile (Q6_K has twice the matrix instructions).
 struct KwChoice {
     int mb, nr, splits;

@@ -16,8 +16,14 @@
 //     unit is never longer than that for its first fragments.
 //   * The operands of k-step s + 1 are made between the matrix instructions of step s.
 //
-// What bounds it: a compute unit takes in cold data at about 50 bytes per clock behind a fixed 3800 clocks (a plain
-// read of data that another kernel wrote), and a tile needs (32 MB * 2.25 + 32 NR * bytes per weight) * K of it.
+// What bounds it: no one unit.  The time goes in whole rounds of 256 workgroups, each as long as its share of the row: 7 us, launch and
+// pre-pass included, and per round and eight super-blocks of a row 2.9 (Q2_K), 3.5 (Q4_K, Q3_K), 4.6 (Q5_K), 4.9 us (Q8_0, Q6_K) with 32 x
+// 32 tiles (up to 32 activation rows, rows of 32 super-blocks and more); 0.6 to 0.8 of that where fewer than 64 workgroups run.  Inside, by
+// counters (share of the waves' time that they issue / are ready and cannot issue / wait for memory, LDS or each other; share of the
+// time that the matrix cores work):
+//   Q4_K, two of 14336 x 4096, M = 64 (64 x 64, 448 workgroups)       34.0 us  28 / 50 / 22 %, matrix cores 25 %
+//   Q8_0, 4999 x 3584, M = 203 (64 x 32, 628 workgroups)              28.8 us  37 / 29 / 34 %, 17 % (LDS bank conflicts 15 %: rows of 144 bytes)
+//   Q6_K, 4096 x 14336, M = 27 (32 x 32, two splits, 256 workgroups)  21.7 us  33 / 36 / 32 %, 17 %
 #include "gemm_common.hpp"
 
 namespace {
