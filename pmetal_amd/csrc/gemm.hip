@@ -2338,6 +2338,8 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     // Rows per workgroup: one for few rows (a chain of latencies: 512 threads on it), two from 384 rows on and four from 1024 on,
     // whose threads write 32 and 64 bytes at a place instead of 16 (us of the pre-pass with one / two / four rows, bf16, k = 14336:
     // M = 64 7.6 / 8.7 / 15.2, M = 512 15.1 / 9.8 / 14.0, M = 2048 56 / 35 / 27).  An item count beyond eight per thread is read twice.
+    // Threads hold 1, 2, 3, 4, 6 or 8 items, the least that is enough: what a row does not fill is its last item again (bf16, k = 10240,
+    // 2.5 or 5 items a thread held as 4 or 8: M = 2048 27.0 -> 19.5 us, k = 5120, M = 1500 14.2 -> 12.6; read twice 22.5, 12.7).
     const int per_wg = p.mp >= 1024 ? 4 : p.mp >= 384 ? 2 : 1;
     const int64_t ni = (k / 8 * per_wg + (per_wg == 1 ? 511 : 1023)) / (per_wg == 1 ? 512 : 1024);
 #define PMH_PREP_N(F, O, R, NI)                                                                                              \
@@ -2347,7 +2349,9 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     do {                                          \
         if (ni <= 1) PMH_PREP_N(F, O, R, 1);      \
         else if (ni <= 2) PMH_PREP_N(F, O, R, 2); \
+        else if (ni <= 3) PMH_PREP_N(F, O, R, 3); \
         else if (ni <= 4) PMH_PREP_N(F, O, R, 4); \
+        else if (ni <= 6) PMH_PREP_N(F, O, R, 6); \
         else if (ni <= 8) PMH_PREP_N(F, O, R, 8); \
         else PMH_PREP_N(F, O, R, 0);              \
     } while (0)

@@ -65,10 +65,12 @@ def test_short_batch_pairs_match_separate_calls(oracle, t, m, k, ns):
     test_pairs_match_separate_calls(oracle, t, m, k, ns)
 
 
-# The pre-pass holds 1, 2, 4 or 8 items per thread, or reads a longer row twice; one, two (from 384 rows on) or four rows (from
+# The pre-pass holds 1, 2, 3, 4, 6 or 8 items per thread, or reads a longer row twice; one, two (from 384 rows on) or four rows (from
 # 1024 on) per workgroup.  Rows of activations that end inside a workgroup, row lengths on both sides of each step.
 @pytest.mark.parametrize("m,k", [(3, 4096), (18, 4352), (17, 16384), (20, 16640), (33, 32768), (2, 33024), (385, 4096), (390, 4352), (385, 33024),
-                                 (1025, 2048), (1026, 2304), (1025, 8192), (1027, 8448), (1025, 16640)])
+                                 (1025, 2048), (1026, 2304), (1025, 8192), (1027, 8448), (1025, 16640),
+                                 (18, 8448), (3, 12288), (17, 12544), (33, 24576), (2, 24832), (385, 12288), (390, 12544), (385, 24576),
+                                 (1026, 4352), (1025, 6144), (1025, 6400), (1025, 12288), (1027, 12544)])
 @pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 10])
 def test_prepared_activations(oracle, t, m, k):
     n = 5
