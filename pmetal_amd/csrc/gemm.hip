@@ -2192,7 +2192,7 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         // 32-row blocks: below 96 Mi elements (Q4_K 4096 x 4096 12.8 -> 10.9 us, Q6_K 21.9 -> 13.4, 14336 x 4096 29.2 -> 26.1; behind at
         // 128256 x 4096: Q4_K 87 -> 103, Q6_K 141 -> 154) and where a row is not whole runs (32000 x 5120: Q4_K 50.8 -> 40.5)
         waves = n * k < ((int64_t)96 << 20) || (small && spr > run && spr % run != 0 && type != kTypeQ8_0);
-        waves = waves || (type == kTypeQ2K);  // (no short-batch form for two blocks; ahead at every size: 128256 x 4096 98 -> 90 us)
+        waves = waves || (type == kTypeQ2K);  // (no short-batch form for two blocks; ahead at most sizes: 128256 x 4096 98 -> 90 us; 0.85 over 765 drawn shapes)
         // Not where the short-batch kernel's two blocks are expected to be clearly ahead: long rows, and rounds of workgroups that end soon
         // after they began (Q5_K 17096 x 19712 135.3 -> 83.7 us, 16796 x 22016 150.3 -> 98.8, 4355 x 26112 63.4 -> 44.9, Q4_K 17542 x
         // 14848 79.5 -> 59.4, Q8_0 37321 x 2048 35.8 -> 26.7).  By how much follows from the fits' errors and from the launch that two
@@ -2204,7 +2204,8 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         }
     } else {
         // against the row kernels, by the times fitted to both over 1000...14336 weight rows of 1024...14336 elements and
-        // 64...2048 activation rows (the chosen kernel is within 2 % of the better one on average); from the third round of
+        // 64...2048 activation rows (within 2 % of the better one there on average; over 1600 shapes drawn
+        // up to 60000 rows of 130 super-blocks within 3 %, one in ten more than a tenth from it); from the third round of
         // workgroups on (Q6_K, two matrix instructions per step: the second; Q8_0, whose row kernel is the slowest: the
         // fifth) the row kernels, which read the activations once per 256 weight rows, are ahead
         const double t_rows = rows_us(p, m, n, type);
