@@ -145,10 +145,11 @@ int32_t pmetal_hip_quantize(uint32_t ggml_type, const float *src_host, size_t n,
 int32_t pmetal_hip_quantize_dev(uint32_t ggml_type, const float *src_dev, size_t n, uint8_t *dst_dev,
                                 size_t dst_len, void *stream);
 /* The tensor loop of a model (run_quantization, crates/pmetal/src/commands/quantize.rs:1378-1428: one quantize call
- * per tensor) in one call: the bytes of one pmetal_hip_quantize_dev per descriptor.  The tensors are independent, so the
- * library spreads them over `stream` and a second stream of its own (per calling thread, default priority): one kernel's
- * last workgroups overlap the next kernel's first (a batch of one k-quant tensor of 2^24 elements or more is cut in two for
- * the same reason).  Asynchronous like the single call: the batch starts behind what
+ * per tensor) in one call: the bytes of one pmetal_hip_quantize_dev per descriptor.  The tensors are independent: those
+ * of one of the types Q4_K, Q5_K and Q6_K share launches, up to 64 in each, and launches are spread over `stream` and a
+ * second stream of the library's own (per calling thread, default priority), so that one kernel's last workgroups overlap
+ * the next kernel's first (a batch of one Q2_K or Q3_K tensor of 2^24 elements or more is cut in two for the same reason).
+ * Asynchronous like the single call: the batch starts behind what
  * `stream` holds, and work given to `stream` afterwards runs behind every tensor of the batch.  All descriptors are checked
  * before anything is launched.  A batch issued while `stream` is being recorded runs on `stream` alone.               */
 typedef struct pmetal_hip_quantize_desc {

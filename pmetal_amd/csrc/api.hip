@@ -558,18 +558,19 @@ int32_t pmetal_hip_quantize_dev(uint32_t t, const float *src, size_t n, uint8_t 
     hipError_t e;
     if (legacy32_type(t)) e = pmh::launch_quantize_legacy32(t, src, n, dst, s);
     else if (t == PMETAL_GGML_TYPE_Q8_0) e = pmh::launch_quantize_q8_0(src, n, dst, s);
-    else if (t == PMETAL_GGML_TYPE_Q4K) e = pmh::launch_quantize_q4k(src, n, dst, s);
-    else if (t == PMETAL_GGML_TYPE_Q5K) e = pmh::launch_quantize_q5k(src, n, dst, s);
     else if (t == PMETAL_GGML_TYPE_Q8K) e = pmh::launch_quantize_q8k(src, n, dst, s);
     else if (t == PMETAL_GGML_TYPE_Q2K) e = pmh::launch_quantize_q2k(src, n, dst, s);
     else if (t == PMETAL_GGML_TYPE_Q3K) e = pmh::launch_quantize_q3k(src, n, dst, s);
-    else e = pmh::launch_quantize_q6k(src, n, dst, s);
+    else {
+        const pmh::TileTensor one = {src, dst, n};
+        e = pmh::launch_quantize_tiles(t, &one, 1, s);
+    }
     if (e != hipSuccess) return hip_fail(e, "quantize kernel launch");
     return ok();
 }
 
 // ---- several tensors in one call ----
-// A second stream of the library, per calling thread, that takes every other tensor of a batch: a quantizer kernel's last
+// A second stream of the library, per calling thread, that takes every other launch of a batch: a quantizer kernel's last
 // workgroups and the next kernel's first then overlap instead of leaving the machine half empty between the launches.
 struct SideStream {
     int device = -1;
@@ -611,7 +612,9 @@ int32_t side_stream(hipStream_t s, SideStream **out) {
 
 int32_t pmetal_hip_quantize_batch_dev(const pmetal_hip_quantize_desc *descs, size_t count, void *stream) {
     if (count && !descs) return fail(PMETAL_HIP_ERR_INVALID_ARG, "NULL descriptor array");
-    size_t work = 0, only = 0;  // tensors with elements; the last of them
+    // tensors with elements by how they are launched: those of a searching type together, the others (the last of them: `only`) one by one
+    size_t in_tiles[3] = {0, 0, 0}, alone = 0, only = 0;
+    auto kind = [](uint32_t t) { return t == PMETAL_GGML_TYPE_Q4K ? 0 : t == PMETAL_GGML_TYPE_Q5K ? 1 : 2; };
     for (size_t i = 0; i < count; i++) {  // every descriptor is checked before anything is launched
         const pmetal_hip_quantize_desc &d = descs[i];
         if (!codec_type(d.ggml_type))
@@ -623,29 +626,49 @@ int32_t pmetal_hip_quantize_batch_dev(const pmetal_hip_quantize_desc *descs, siz
         if (!d.src_dev || !d.dst_dev) return fail(PMETAL_HIP_ERR_INVALID_ARG, "NULL pointer (tensor %zu)", i);
         if (!aligned16(d.src_dev) || !aligned16(d.dst_dev))
             return fail(PMETAL_HIP_ERR_INVALID_ARG, "device pointers must be 16-byte aligned (tensor %zu)", i);
-        work++, only = i;
+        if (pmh::quantizes_in_tiles(d.ggml_type)) in_tiles[kind(d.ggml_type)]++;
+        else alone++, only = i;
     }
-    if (work == 0) return ok();
+    size_t launches = alone;
+    for (size_t c : in_tiles) launches += (c + pmh::kMaxTileTensors - 1) / pmh::kMaxTileTensors;
+    if (launches == 0) return ok();
     if (int32_t rc = require_device()) return rc;
     hipStream_t s = (hipStream_t)stream;
-    // a single large tensor of a k-quant type is cut in two for the same reason (its super-blocks are independent; Q4_K at
-    // 14336 x 4096: 122 -> 114 us, Q6_K 171 -> 149)
+    // a single large tensor of Q2_K or Q3_K is cut in two (its super-blocks are independent), so that its halves overlap
     constexpr size_t kSplitMin = (size_t)1 << 24;
-    const bool split = work == 1 && descs[only].n >= kSplitMin && pmetal_hip_block_size(descs[only].ggml_type) == 256;
+    const bool split = launches == 1 && alone == 1 && descs[only].n >= kSplitMin && pmetal_hip_block_size(descs[only].ggml_type) == 256;
     SideStream *side = nullptr;
-    if (work >= 2 || split)
+    if (launches >= 2 || split)
         if (int32_t rc = side_stream(s, &side)) return rc;
     if (side) {
         HIP_TRY(hipEventRecord(side->fork, s));
         HIP_TRY(hipStreamWaitEvent(side->s, side->fork, 0));
     }
-    // The tensors take turns between the two streams.  (Giving each to the stream with less work so far keeps the streams in
-    // step, so that their kernels end together and the overlap is lost: 15.6 against 15.0 ms for a Llama-3-8B-shaped model.)
+    // The launches take turns between the two streams: one's first workgroups start where the other's last ones end.
     int32_t rc = PMETAL_HIP_OK;
     bool to_side = false;
+    auto turn = [&]() {
+        hipStream_t t = to_side ? side->s : s;
+        to_side = side && !to_side;
+        return t;
+    };
+    for (uint32_t t : {(uint32_t)PMETAL_GGML_TYPE_Q4K, (uint32_t)PMETAL_GGML_TYPE_Q5K, (uint32_t)PMETAL_GGML_TYPE_Q6K}) {
+        pmh::TileTensor group[pmh::kMaxTileTensors];
+        int held = 0;
+        size_t left = in_tiles[kind(t)];
+        for (size_t i = 0; i < count && left > 0 && rc == PMETAL_HIP_OK; i++) {
+            const pmetal_hip_quantize_desc &d = descs[i];
+            if (d.n == 0 || d.ggml_type != t) continue;
+            group[held++] = {d.src_dev, d.dst_dev, d.n};
+            if (--left > 0 && held < pmh::kMaxTileTensors) continue;
+            const hipError_t e = pmh::launch_quantize_tiles(t, group, held, turn());
+            if (e != hipSuccess) rc = hip_fail(e, "quantize kernel launch");
+            held = 0;
+        }
+    }
     for (size_t i = 0; i < count && rc == PMETAL_HIP_OK; i++) {
         const pmetal_hip_quantize_desc &d = descs[i];
-        if (d.n == 0) continue;
+        if (d.n == 0 || pmh::quantizes_in_tiles(d.ggml_type)) continue;
         if (split && side) {
             const size_t head = (d.n / 2 + 2047) / 2048 * 2048, head_bytes = pmetal_hip_tensor_size(d.ggml_type, head);
             rc = pmetal_hip_quantize_dev(d.ggml_type, d.src_dev, head, d.dst_dev, head_bytes, stream);
@@ -653,8 +676,7 @@ int32_t pmetal_hip_quantize_batch_dev(const pmetal_hip_quantize_desc *descs, siz
                 rc = pmetal_hip_quantize_dev(d.ggml_type, d.src_dev + head, d.n - head, d.dst_dev + head_bytes, d.dst_len - head_bytes, side->s);
             continue;
         }
-        rc = pmetal_hip_quantize_dev(d.ggml_type, d.src_dev, d.n, d.dst_dev, d.dst_len, to_side ? (void *)side->s : stream);
-        to_side = side && !to_side;
+        rc = pmetal_hip_quantize_dev(d.ggml_type, d.src_dev, d.n, d.dst_dev, d.dst_len, (void *)turn());
     }
     if (side) {  // the caller's stream continues behind both, also after a failed launch
         const hipError_t e1 = hipEventRecord(side->join, side->s);

@@ -2025,16 +2025,6 @@ static bool qgemm_small_applies(uint32_t type, int64_t m, int64_t n, int64_t k) 
     return false;
 }
 
-static int compute_units_gemm() {
-    static const int n = [] {
-        int dev = 0, cu = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return 256;
-        if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) return 256;
-        return cu;
-    }();
-    return n;
-}
-
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
     // byte offsets inside a workgroup's rows and item offsets inside the activation copy are 32-bit
     return (type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ6K || type == kTypeQ8_0 || type == kTypeQ3K || type == kTypeQ2K) && m >= 1 && m <= (int64_t)1 << 22 && n >= 1 && k >= 256 && k % 256 == 0 && k <= (int64_t)1 << 22 && n <= 0x7FFFFF00;
@@ -2396,7 +2386,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         // operands in registers (one tile per workgroup and four times the workgroups: 35 against 27 us at M = 16, 4096 x 14336)
         const int run = small_run_spr(type, m);
         const int runs_of_row = p.splits;
-        int64_t slots = (int64_t)compute_units_gemm() * (kSmallWaves / nwaves) / runs_of_row;
+        int64_t slots = (int64_t)compute_units() * (kSmallWaves / nwaves) / runs_of_row;
         slots = slots < 1 ? 1 : slots;
         const int tiles1 = (second.n + 15) / 16;  // of the second weight: a workgroup's tiles are of one weight
         const int n_wg = (int)(tiles + tiles1 < slots ? tiles + tiles1 : slots);

@@ -76,16 +76,7 @@ inline int pow2_divisor(int64_t v, int cap) {
     return t;
 }
 
-// compute units of the current device (256 on MI355X); falls back to 256 if the query fails
-inline int compute_units() {
-    static const int n = [] {
-        int dev = 0, cu = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return 256;
-        if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) return 256;
-        return cu;
-    }();
-    return n;
-}
+using pmh::compute_units;
 
 }  // namespace gemv
 

@@ -879,7 +879,7 @@ static hipError_t launch_kernel_rows(const uint8_t *const *w, const int64_t *n, 
     if ((uint64_t)n_max * (uint64_t)spr * 144u >= (1ull << 32)) return hipErrorNotSupported;
     // Two workgroups per compute unit; a launch of several matrices that would leave a wave more tasks than the ring holds
     // takes four per compute unit instead (two rounds, and the end of one workgroup overlaps the start of the next).
-    const int64_t cus = gemv::compute_units();
+    const int64_t cus = compute_units();
     const int64_t max_rows_per_wg = (int64_t)kRowsWaves * (kDepth / ks);
     int64_t want = 2 * cus;
     if (count > 1 && (total + want - 1) / want > max_rows_per_wg) want = 4 * cus;
@@ -943,7 +943,7 @@ static hipError_t launch_kernel_a(const uint8_t *w0, int64_t n0, float *y0, cons
     const size_t lds_x = slots * 16 * (xf32 ? 6 : 5) + slots * 16;
     if (lds_x > gemv::kMaxLds) return hipErrorNotSupported;
     // Workgroups own contiguous chunks of rows, one per compute unit (x is staged once per workgroup).
-    const int64_t n = n0 + n1, want = gemv::compute_units();
+    const int64_t n = n0 + n1, want = compute_units();
     int64_t n_wg = n < want ? n : want;
     const int64_t rows_per_wg = (n + n_wg - 1) / n_wg;
     const int64_t wg0 = (n0 + rows_per_wg - 1) / rows_per_wg, wg1 = (n1 + rows_per_wg - 1) / rows_per_wg;

@@ -11,15 +11,32 @@ constexpr uint32_t kTypeQ8_0 = 8, kTypeQ2K = 10, kTypeQ3K = 11, kTypeQ4K = 12, k
 constexpr uint32_t kOrderRef = 0, kOrderGgml = 1;
 constexpr uint32_t kDtypeF32 = 0, kDtypeBf16 = 1;
 
+// compute units of the current device (256 on MI355X); falls back to 256 if the query fails
+inline int compute_units() {
+    static const int n = [] {
+        int dev = 0, cu = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return 256;
+        if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) return 256;
+        return cu;
+    }();
+    return n;
+}
+
 // ---- codec.hip: bit-exact quantize / dequantize (compiled without fp contraction) ----
 hipError_t launch_quantize_q8_0(const float *x, size_t n, uint8_t *dst, hipStream_t s);
 hipError_t launch_quantize_legacy32(uint32_t type, const float *x, size_t n, uint8_t *dst, hipStream_t s);
 hipError_t launch_dequantize_legacy32(uint32_t type, const uint8_t *src, size_t n, float *dst, hipStream_t s);
-hipError_t launch_quantize_q4k(const float *x, size_t n, uint8_t *dst, hipStream_t s);
-hipError_t launch_quantize_q5k(const float *x, size_t n, uint8_t *dst, hipStream_t s);
+// Q4_K, Q5_K and Q6_K: up to kMaxTileTensors tensors of one type in one launch
+struct TileTensor {
+    const float *x;
+    uint8_t *dst;
+    size_t n;  // elements
+};
+constexpr int kMaxTileTensors = 64;
+inline bool quantizes_in_tiles(uint32_t type) { return type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ6K; }
+hipError_t launch_quantize_tiles(uint32_t type, const TileTensor *tensors, int count, hipStream_t s);
 hipError_t launch_quantize_q2k(const float *x, size_t n, uint8_t *dst, hipStream_t s);
 hipError_t launch_quantize_q3k(const float *x, size_t n, uint8_t *dst, hipStream_t s);
-hipError_t launch_quantize_q6k(const float *x, size_t n, uint8_t *dst, hipStream_t s);
 hipError_t launch_dequantize_q8_0(const uint8_t *src, size_t n, float *dst, hipStream_t s);
 hipError_t launch_dequantize_q4k(const uint8_t *src, size_t n, float *dst, uint32_t order, hipStream_t s);
 hipError_t launch_dequantize_q5k(const uint8_t *src, size_t n, float *dst, uint32_t order, hipStream_t s);

@@ -54,6 +54,50 @@ def test_quantize_edge_cases_bit_exact(oracle, t):
         assert np.array_equal(got, want), f"{name}: {first_mismatch(got, want, BLOCK[t])}"
 
 
+@pytest.mark.parametrize("t", [Q4K, 13, Q6K])
+def test_quantize_batch_of_many_tensors_of_one_type(oracle, t):
+    """More tensors than one launch takes, of sizes at the edges of its tiles (4 and 8 super-blocks) and of a workgroup's
+    share, some empty, some with a partial super-block, between tensors of other types; whole tensors of values that
+    leave the fast searches (tiny, huge, NaN, equal extremes of both signs) beside ordinary ones."""
+    from pmetal_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(11)
+    odd = list(edge_inputs(256).values())
+    parts = [(t, weights(700 + i, 256 * n + r)) for i, (n, r) in enumerate([(1, 0), (3, 0), (4, 0), (5, 1), (7, 255), (8, 0), (9, 0), (16, 3), (17, 0)] * 5)]
+    parts += [(t, x) for x in odd] + [(Q8_0, weights(800, 1000)), (t, weights(801, 0)), (t, weights(802, 256 * 4097)), (10, weights(803, 2048))]
+    parts += [(t, np.tile(np.array([1, -1], np.float32) * np.float32(0.25 + i), 640)) for i in range(4)]
+    parts = [parts[i] for i in rng.permutation(len(parts))]
+    assert sum(p[0] == t for p in parts) > 64
+    src = [pm.DeviceBuffer.from_host(x) if x.size else pm.DeviceBuffer(16) for _, x in parts]
+    sizes = [lib.pmetal_hip_tensor_size(q, x.size) for q, x in parts]
+    dst = [pm.DeviceBuffer(max(b, 16)) for b in sizes]
+    for d, b in zip(dst, sizes):
+        pm.check(lib.pmetal_hip_memset(d.ptr, 0xA5, max(b, 16), None))
+    descs = (_lib.QuantizeDesc * len(parts))(*[_lib.QuantizeDesc(q, 0, s.ptr, x.size, d.ptr, b) for (q, x), s, d, b in zip(parts, src, dst, sizes)])
+    pm.check(lib.pmetal_hip_quantize_batch_dev(descs, len(parts), None))
+    pm.check(lib.pmetal_hip_sync(None))
+    for i, (q, x) in enumerate(parts):
+        got = dst[i].to_host(np.uint8, sizes[i])
+        assert np.array_equal(got, oracle.quantize(q, x)), (i, q, x.size)
+
+
+def test_quantize_q6k_corner_cases_inside_a_large_tensor(oracle):
+    """As for Q4_K below, with runs whose largest magnitude occurs with both signs."""
+    rng = np.random.default_rng(12)
+    parts, i = [], 0
+    cases = list(edge_inputs(256).values())
+    while sum(c.size for c in parts) < (8192 + 3) * 256 + 9:
+        c = cases[i % len(cases)] if i % 4 == 0 else weights(900 + i, int(rng.integers(1, 40)) * 512)
+        if i % 5 == 3:
+            c = (rng.integers(-3, 4, int(rng.integers(1, 64)) * 16) * np.float32(0.125)).astype(np.float32)
+        parts.append(c)
+        i += 1
+    x = np.concatenate(parts)[:(8192 + 3) * 256 + 9].astype(np.float32)
+    got, want = gpu_quantize_dev(Q6K, x), oracle.quantize(Q6K, x)
+    assert np.array_equal(got, want), first_mismatch(got, want, BLOCK[Q6K])
+
+
 def test_quantize_q4k_corner_cases_inside_a_large_tensor(oracle):
     """The corner cases above, Gaussian data with outliers and runs of constants, laid end to end to 32768 + 5
     super-blocks and a ragged tail: sub-blocks that need one, two or all five passes of the search side by side in one

@@ -109,3 +109,76 @@ def test_a_reciprocal_one_ulp_off_rounds_like_the_division_outside_the_wider_mar
         sure = np.abs(np.abs(q - fast.astype(np.float32)) - np.float32(0.5)) >= np.float32(2e-5)
         assert sure.mean() > 0.1
         assert np.array_equal(fast[sure], exact[sure])
+
+
+# ---- division by f32 arithmetic alone (codec.hip rcp_rn, div_rn) ----
+def fma32(a, b, c):
+    """Correctly rounded f32 a * b + c: the product is exact in f64, the sum is rounded to odd there and then to f32."""
+    p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)
+    s = p + c
+    bb = s - p
+    err = (p - (s - bb)) + (c - bb)
+    even = (s.view(np.int64) & 1) == 0
+    toward = np.where(err > 0, np.inf, -np.inf)
+    return np.where((err != 0) & even, np.nextafter(s, toward), s).astype(np.float32)
+
+
+def rcp_ulp(b):
+    one = np.ones_like(b)
+    y = (np.uint32(0x7EF36000) - b.view(np.uint32)).view(np.float32)
+    for _ in range(2):
+        e = fma32(-b, y, one)
+        y = fma32(y, fma32(e, e, e), y)
+    return y
+
+
+def rcp_rn(b):
+    y = rcp_ulp(b)
+    return fma32(y, fma32(-b, y, np.ones_like(b)), y)
+
+
+def div_rn(a, b):
+    y = rcp_rn(b)
+    q = (a * y).astype(np.float32)
+    for _ in range(2):
+        q = fma32(fma32(-b, q, a), y, q)
+    return q
+
+
+def test_reciprocal_without_the_hardware_one_is_the_ieee_quotient_for_every_significand():
+    for first in range(0, 1 << 23, 1 << 21):
+        b = (np.arange(first, first + (1 << 21), dtype=np.uint32) | np.uint32(0x3F800000)).view(np.float32)
+        assert np.array_equal(rcp_rn(b), np.float32(1) / b)
+        assert np.max(np.abs(rcp_ulp(b).astype(np.float64) * b - 1)) <= 1.0001 * 2.0**-24  # before the last step (at the worst, half an ulp's rounding)
+    # the exponent only scales it, the sign is carried along
+    rng = np.random.default_rng(4)
+    b = (np.exp2(rng.uniform(-80, 80, 500_000)) * rng.choice([-1, 1], 500_000)).astype(np.float32)
+    assert np.array_equal(rcp_rn(b), np.float32(1) / b)
+
+
+def test_division_without_the_hardware_reciprocal_is_the_ieee_quotient():
+    rng = np.random.default_rng(5)
+    n = 1_000_000
+    a, b = ((np.exp2(rng.uniform(-40, 40, n)) * rng.choice([-1, 1], n)).astype(np.float32) for _ in range(2))
+    assert np.array_equal(div_rn(a, b), a / b)
+    # quotients next to a midpoint of two floats: (2^24 + odd) / 2 times a divisor, and both of its neighbours
+    b = rng.integers(1 << 23, 1 << 24, n).astype(np.float32)
+    a = (b.astype(np.float64) * (rng.integers(1 << 23, 1 << 24, n) + 0.5)).astype(np.float32)
+    for x in (a, np.nextafter(a, np.float32(np.inf)), np.nextafter(a, np.float32(0))):
+        assert np.array_equal(div_rn(x, b), x / b)
+    for c in (63.0, 31.0, 15.0, 32.0, 128.0):  # the constants the quantizers divide by, and divide
+        k = np.full(n, c, np.float32)
+        assert np.array_equal(div_rn(b, k), b / k) and np.array_equal(div_rn(k, b), k / b)
+
+
+def test_bytes_of_the_product_shifted_both_ways_agree_only_away_from_the_boundaries():
+    """Requantization: product plus and minus the margin, rounded to nearest even; equal bytes are the quotient's integer."""
+    rng = np.random.default_rng(6)
+    for lo, hi, plus, minus in ((0, 15, 8e-6, -8e-6), (0, 31, 8e-6, -8e-6), (-32, 31, 32.000008, 31.999992)):
+        num, den = _quotients_near_boundaries(rng, 3_000_000, lo - 1, hi + 1)
+        exact = nearest_int_clamped((num / den).astype(np.float32), lo, hi)
+        q = np.clip((num * rcp_ulp(den)).astype(np.float32), np.float32(lo), np.float32(hi))
+        above, below = (np.clip(np.rint((q + np.float32(d)).astype(np.float32)), 0, 255).astype(np.int32) for d in (plus, minus))
+        sure = above == below
+        assert sure.mean() > 0.2 and (~sure).mean() > 0.2
+        assert np.array_equal(above[sure], exact[sure] - min(lo, 0))
