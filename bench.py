@@ -431,7 +431,9 @@ def _gemm_kernel(_lib, t, m, n, k):
                 10: "k_qgemm_kw<KwQ23<Q2_K>"}[t] + f", {p.mb}, {p.nr}>"
     else:
         name = {Q4K: "k_qgemm_rw", 13: "k_qgemm_rw<FMT = 1>", Q6K: "k_qgemm_rw_q6", Q8_0: "k_qgemm_rw_q8", 11: "k_qgemm_rw16<Q3_K>", 10: "k_qgemm_rw16<Q2_K>"}[t]
-    return name + " (+ k_prep_rw" + (f", k_rw_reduce over {p.splits} K splits)" if p.splits > 1 else ")")
+    # (up to 16 rows of bf16 activations the short-batch kernels convert them themselves)
+    around = ([] if p.kernel == _lib.GEMM_SMALL and m <= 16 else ["k_prep_rw"]) + ([f"k_rw_reduce over {p.splits} K splits"] if p.splits > 1 else [])
+    return name + (f" (+ {', '.join(around)})" if around else "")
 
 
 def bench_gemm(args, m, n, k, t=Q4K):

@@ -1085,7 +1085,8 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
     };
     for (size_t i = 0; i < count; i++) {
         const pmetal_hip_gemm_desc &d = descs[i];
-        const int want = layout(d), want_mp = pmh::qgemm_plan(m, d.n, k, d.ggml_type).mp;
+        const pmh::GemmPlan one = pmh::qgemm_plan(m, d.n, k, d.ggml_type);
+        const int want = layout(d), want_mp = one.mp;
         // two neighbours of one kind share a launch, unless one's results lie over what the other reads or writes
         pmh::GemmSecond second{};
         pmh::GemmPlan plan;
@@ -1098,7 +1099,8 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
                                          want == have && want_mp == have_mp, second);
         if (e == hipErrorNotSupported) return fail(PMETAL_HIP_ERR_UNSUPPORTED_TYPE, "qgemm: configuration not supported");
         if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
-        have = want, have_mp = want_mp;
+        // (a second weight's plan has the same kernel; a K split's partial tiles may lie over items of another layout)
+        have = pmh::qgemm_converts_itself(one, d.ggml_type, m, k, x_dtype) ? -1 : want, have_mp = want_mp;
     }
     return ok();
 }

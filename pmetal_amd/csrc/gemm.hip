@@ -1259,6 +1259,148 @@ __device__ __forceinline__ void small_store(const float4_t *out_tiles, int t0, i
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// At most 16 activation rows: every wave converts the activations it multiplies.  A pre-pass for so few rows is 16 workgroups and a
+// chain of latencies (3 to 4 us of 15) in front of a kernel whose waves then wait for their first weights; here the
+// conversion runs while those are on their way.  A wave's super-block of the 16 rows comes in whole-wave 16-byte loads, goes through the
+// wave's own LDS (piece p of row r at piece p ^ r: neither the writes nor the reads collide), and a lane takes its eight items:
+// two runs of four elements each, of row lane % 16, where the pre-pass's order of the same number puts them.  The power of two that
+// takes a row into [2^9, 2^10) is that of the wave's part of it and not of the whole row: its inverse multiplies the wave's tiles,
+// exactly, before they are added, so nothing is rounded that a pre-pass would not round.
+// Measured (us a call, 14336 x 4096, M = 16, bf16, from memory, with the pre-pass -> so): see the launcher.
+// ------------------------------------------------------------------------------------------------
+constexpr int kSmallXItems = 512;  // 16-byte items of LDS for a super-block of 16 rows in bf16; f32: twice as many
+template <bool XF32, int ORDER, int NSB>
+struct SmallX {
+    static constexpr int kPieces = XF32 ? 64 : 32, kLoads = 16 * kPieces / 64;  // per row and super-block; per lane
+    u32x4 piece[NSB][kLoads];
+    // Past the last row, and of a super-block past the end of the row (valid false), the buffer returns zeros.
+    __device__ __forceinline__ void request(const int i, const __amdgpu_buffer_rsrc_t r, const uint32_t row_bytes, const int sb, const bool valid, const int lane) {
+        uint32_t base = valid ? (uint32_t)sb * (16u * kPieces) : 0x7F000000u;
+        asm("" : "+s"(base));  // (opaque: a choice the compiler sees becomes a branch around each load, with a wait for it)
+        base += 16u * ((uint32_t)lane % kPieces) + (XF32 ? 0u : ((uint32_t)lane >> 5) * row_bytes);
+#pragma unroll
+        for (int j = 0; j < kLoads; j++)
+            piece[i][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, base + (XF32 ? j : 2 * j) * row_bytes, 0, 0));
+    }
+    // first element of the two runs of item t of k-group kg
+    static __device__ __forceinline__ void runs(const int t, const int kg, int &lo, int &hi) {
+        if (ORDER == 2) lo = 128 * (t >> 2) + 32 * (t & 1) + 16 * ((t >> 1) & 1) + 4 * kg, hi = lo + 64;  // t = 4 hh + 2 lh + gp
+        else if (ORDER == 3) lo = 32 * t + 8 * kg, hi = lo + 4;
+        else if (ORDER == 5) lo = 128 * (kg >> 1) + 64 * (t & 1) + 16 * (kg & 1) + 4 * (t >> 1), hi = lo + 32;
+        else if (ORDER == 4) lo = 64 * kg + 8 * t, hi = lo + 4;
+        else if (ORDER == 0) lo = 64 * kg + 32 * (t >> 2) + 4 * (t & 3), hi = lo + 16;
+        else lo = 64 * kg + 4 * t, hi = lo + 32;
+    }
+    // af: the items; up: 2^e of the rows 4 kg .. 4 kg + 3 (the rows of the lane's part of a product tile).  (In instructions that two
+    // waves of a SIMD can issue at a time: packed ones and v_fma_mix would end that)
+    __device__ __forceinline__ void convert(u32x4 *stage, const int lane, half8_t *const (&af)[NSB], float4_t &up) const {
+        const int nl = lane & 15, kg = lane >> 4;
+        const u32x4 *mine = stage + nl * kPieces;
+        uint32_t raw[NSB][8][XF32 ? 8 : 4];
+        float most[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // the largest magnitudes of the row (a NaN does not count)
+#pragma unroll
+        for (int i = 0; i < NSB; i++) {
+#pragma unroll
+            for (int j = 0; j < kLoads; j++) {
+                const int row = XF32 ? j : 2 * j + (lane >> 5), p = lane % kPieces;
+                stage[row * kPieces + (p ^ row)] = piece[i][j];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                int lo, hi;
+                runs(t, kg, lo, hi);
+                uint32_t (&w)[XF32 ? 8 : 4] = raw[i][t];
+                if (XF32) {
+                    const u32x4 a = mine[(lo >> 2) ^ nl], b = mine[(hi >> 2) ^ nl];
+#pragma unroll
+                    for (int c = 0; c < 4; c++) w[c] = a[c], w[XF32 ? 4 + c : 0] = b[c];
+                } else if (hi == lo + 4) {
+                    const u32x4 a = mine[(lo >> 3) ^ nl];
+#pragma unroll
+                    for (int c = 0; c < 4; c++) w[c] = a[c];
+                } else {
+                    const uint2 a = reinterpret_cast<const uint2 *>(mine + ((lo >> 3) ^ nl))[(lo >> 2) & 1], b = reinterpret_cast<const uint2 *>(mine + ((hi >> 3) ^ nl))[(hi >> 2) & 1];
+                    w[0] = a.x, w[1] = a.y, w[2] = b.x, w[3] = b.y;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)  // (bf16: the low half's bits do not change the exponent of the high one)
+                    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most[c]) : "v"(raw[i][t][c]), "v"(XF32 ? raw[i][t][XF32 ? 4 + c : 0] : raw[i][t][c] << 16));
+        }
+        float amax = __builtin_fmaxf(__builtin_fmaxf(most[0], most[1]), __builtin_fmaxf(most[2], most[3]));
+        amax = __builtin_fmaxf(amax, __shfl_xor(amax, 16));
+        amax = __builtin_fmaxf(amax, __shfl_xor(amax, 32));
+        const int eb = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFFu);  // it lies in [2^(eb-127), 2^(eb-126))
+        int e = eb - 126 - 10;
+        e = e < -126 ? -126 : (e > 126 ? 126 : e);
+        if (eb == 255) e = 0;  // inf: let them through
+        const float down = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23), mine_up = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+#pragma unroll
+        for (int q = 0; q < 4; q++) up[q] = __shfl(mine_up, 4 * kg + q);  // (lane r holds row r)
+#pragma unroll
+        for (int i = 0; i < NSB; i++)
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                float v[8];
+#pragma unroll
+                for (int c = 0; c < 8; c++)
+                    v[c] = down * __builtin_bit_cast(float, XF32 ? raw[i][t][XF32 ? c : 0] : c & 1 ? raw[i][t][c / 2] & 0xFFFF0000u : raw[i][t][c / 2] << 16);
+                half8_t h;
+#pragma unroll
+                for (int c = 0; c < 8; c++) {  // (ORDER 4: eight consecutive elements, the even ones first)
+                    float a = v[ORDER == 4 ? 2 * (c & 3) + (c >> 2) : c];
+                    asm("" : "+v"(a));  // (the product and its rounding apart, not one v_fma_mix.  The conversion itself is not written as asm:
+                                        // what reads its result has to wait, which the compiler sees to for instructions it knows)
+                    h[c] = (_Float16)a;
+                }
+                af[i][t] = h;
+            }
+    }
+};
+
+// The sums of the sub-blocks over the converted activations, as head + tail items (H0, L0, H0, L0, H1, L1, H1, L1) like the pre-pass's: ORDER 5
+// two of them (k-steps of one parity: their first runs are one sub-block, their second runs another), the others one (its sub-blocks
+// 2 kg and 2 kg + 1).  A product with a matrix of zeros and ones adds them up over lanes that hold parts of them; it leaves
+// the sum of column c for row 4 kg + r in lane (c, kg), and LDS takes it to the lane of its row.
+template <int ORDER>
+__device__ __forceinline__ void small_sums(const half8_t (&af)[8], float *stage, const int lane, half8_t (&sums)[ORDER == 5 ? 2 : 1]) {
+    const int nl = lane & 15, kg = lane >> 4;
+    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int lo = ORDER == 5 ? 4 * kg + 2 * (t & 1) : ORDER == 1 ? 2 * kg : 2 * kg + (t >> 2), hi = ORDER == 5 || ORDER == 1 ? lo + 1 : lo;
+        const _Float16 a = (_Float16)(nl == lo ? 1.0f : 0.0f), b = (_Float16)(nl == hi ? 1.0f : 0.0f);
+        const half8_t ones = {a, a, a, a, b, b, b, b};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], ones, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) stage[(4 * kg + r) * 17 + nl] = acc[r];
+    constexpr int kSums = ORDER == 5 ? 2 : 1;
+#pragma unroll
+    for (int i = 0; i < kSums; i++) {
+        const float s0 = stage[nl * 17 + 2 * kSums * kg + 2 * i], s1 = stage[nl * 17 + 2 * kSums * kg + 2 * i + 1];
+        const _Float16 h0 = (_Float16)s0, h1 = (_Float16)s1;
+        const _Float16 l0 = (_Float16)(s0 - (float)h0), l1 = (_Float16)(s1 - (float)h1);
+        sums[i] = half8_t{h0, l0, h0, l0, h1, l1, h1, l1};
+    }
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t small_x_buffer(const void *x, const int M, const uint32_t row_bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(x), 0, M * (int)row_bytes, 0x00027000);
+}
+// Before a wave's LDS takes another use that other waves share: its own reads have returned, and everyone is here.  (Requests for
+// weights stay in flight; __syncthreads() would wait for them.)
+__device__ __forceinline__ void barrier_lds() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 template <int NSB, int FMT = 0>
 struct SmallRun {
     static constexpr int kPerSb = BlockFmt<FMT>::kBytes / 16;  // 16-byte pieces of a super-block: 9 (Q4_K) or 11 (Q5_K)
@@ -1270,8 +1412,10 @@ struct SmallRun {
 // FMT 1: Q5_K -- eleven pieces per super-block (header, two of qh, eight of quants); a lane takes the qh bytes of its two
 // sub-blocks out of its stage as well and ors the fifth bits into the quant dwords as in the large kernel.
 // MT: 16-row blocks of activations (1: at most 16 rows, 2: at most 32); a weight operand then feeds MT matrix instructions.
-template <int ORDER, int NSB, int FMT = 0, int MT = 1>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
+// XT: what xg is: 0 the pre-pass's items (MT = 2: twice the rows to convert would not hide behind the first weights), 1 and 2 the
+// activations themselves in bf16 and in f32.
+template <int ORDER, int NSB, int FMT, int MT, int XT>
+__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t *__restrict__ W, const void *__restrict__ xg,
                                                                    const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                    int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
                                                                    float *__restrict__ partial, const pmh::GemmSecond second) {
@@ -1282,7 +1426,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
     }
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64]: lane slots of the finished tiles; then the waves' stages
-    const float rs = small_row_scale(rowscale);
+    const float rs = XT ? 1.0f : small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1302,21 +1446,33 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
     }
     // activation operands of this wave's super-blocks: item (2 sb + kg / 2, group 2 t + kg % 2) of rows nl (and 16 + nl), and the sums item
     half8_t af[NSB][MT][8], asum[NSB][MT];
+    constexpr int kXOrder = ORDER == 1 ? 1 : FMT ? 4 : 0;
+    SmallX<XT == 2, kXOrder, NSB> X;
+    float4_t up;
+    const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
+    const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
+    if constexpr (XT != 0) {
 #pragma unroll
-    for (int i = 0; i < NSB; i++)
+        for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sbi[i], sbv[i], lane);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        const uint4 *xs = reinterpret_cast<const uint4 *>(xg);
 #pragma unroll
-        for (int b = 0; b < MT; b++) {
-            const uint4 *base = xs + (size_t)((2 * sbi[i] + (kg >> 1)) * kGroups) * Mp + 16 * b + nl;
+        for (int i = 0; i < NSB; i++)
 #pragma unroll
-            for (int t = 0; t < 8; t++) af[i][b][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (kg & 1)) * Mp]);
-            asum[i][b] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (kg & 1)) * Mp]);
-            if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
-                const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+            for (int b = 0; b < MT; b++) {
+                const uint4 *base = xs + (size_t)((2 * sbi[i] + (kg >> 1)) * kGroups) * Mp + 16 * b + nl;
 #pragma unroll
-                for (int t = 0; t < 8; t++) af[i][b][t] = z;
-                asum[i][b] = z;
+                for (int t = 0; t < 8; t++) af[i][b][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (kg & 1)) * Mp]);
+                asum[i][b] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (kg & 1)) * Mp]);
+                if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
+                    const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+                    for (int t = 0; t < 8; t++) af[i][b][t] = z;
+                    asum[i][b] = z;
+                }
             }
-        }
+    }
     const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;  // t1 > t0 by the launch geometry
     constexpr int kPerSb = SmallRun<NSB, FMT>::kPerSb, kBlockBytes = BlockFmt<FMT>::kBytes, kQ0 = FMT ? 3 : 1;  // kQ0: first quant piece
@@ -1410,13 +1566,30 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
                 for (int r = 0; r < 4; r++) acc[b][r] = __builtin_fmaf(dd, part[b][r], acc[b][r]);
             }
         }
+        if (XT) acc[0] *= up;
 #pragma unroll
         for (int b = 0; b < MT; b++) small_add_waves(red, keep, ti * MT + b, wave, nwaves, lane, acc[b], out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRun<NSB, FMT> ring0, ring1;
     issue(0, ring0);
-    issue(1, ring1);
+    if (XT != 2 || NSB == 1) issue(1, ring1);
+    if constexpr (XT != 0) {  // while the first weights are on their way
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
+        half8_t *to[NSB];
+#pragma unroll
+        for (int i = 0; i < NSB; i++) to[i] = af[i][0];
+        X.convert(x_stage, lane, to, up);
+#pragma unroll
+        for (int i = 0; i < NSB; i++) {
+            half8_t sums[1];
+            small_sums<kXOrder>(af[i][0], reinterpret_cast<float *>(x_stage), lane, sums);
+            asum[i][0] = sums[0];
+        }
+        barrier_lds();
+        if (XT == 2 && NSB == 2) issue(1, ring1);  // (in f32 two super-blocks' activations leave no registers for it before)
+    }
     // Whole rounds of two tiles, with nothing conditional around the loads, so that the outstanding loads are counted
     // exactly at every wait; the tiles past the workgroup's last one are computed on repeated data and dropped.
     for (int rd = 0; rd < rounds; rd++) {
@@ -1447,8 +1620,8 @@ struct SmallRunQ8 {
     u32x4 piece[5];  // (a vector type: copies of it are loads and stores that stay in registers)
 };
 
-template <int NSB, int MT = 1>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
+template <int NSB, int MT, int XT>  // (XT as above)
+__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8_t *__restrict__ W, const void *__restrict__ xg,
                                                                       const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                       int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
                                                                    float *__restrict__ partial, const pmh::GemmSecond second) {
@@ -1459,7 +1632,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
     }
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
-    const float rs = small_row_scale(rowscale);
+    const float rs = XT ? 1.0f : small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1479,16 +1652,27 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
     // activation operands: block b of run sb holds elements 256 sb + 32 b ..; the item of its k-group kg is item
     // 4 (b % 4) + kg of half 2 sb + b / 4 (the pre-pass writes 16 items of eight consecutive elements per 128)
     half8_t af[NSB][MT][8];  // (MT 16-row blocks of activations: rows nl, 16 + nl)
+    SmallX<XT == 2, 3, NSB> X;
+    float4_t up;
+    const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
+    const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
+    if constexpr (XT != 0) {
 #pragma unroll
-    for (int i = 0; i < NSB; i++)
+        for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sbi[i], sbv[i], lane);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        const uint4 *xs = reinterpret_cast<const uint4 *>(xg);
 #pragma unroll
-        for (int mb = 0; mb < MT; mb++)
+        for (int i = 0; i < NSB; i++)
 #pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const uint4 *item = xs + (size_t)((2 * sbi[i] + (b >> 2)) * kQ6Groups + 4 * (b & 3) + kg) * Mp + 16 * mb + nl;
-                af[i][mb][b] = __builtin_bit_cast(half8_t, *item);
-                if (!sbv[i]) af[i][mb][b] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-            }
+            for (int mb = 0; mb < MT; mb++)
+#pragma unroll
+                for (int b = 0; b < 8; b++) {
+                    const uint4 *item = xs + (size_t)((2 * sbi[i] + (b >> 2)) * kQ6Groups + 4 * (b & 3) + kg) * Mp + 16 * mb + nl;
+                    af[i][mb][b] = __builtin_bit_cast(half8_t, *item);
+                    if (!sbv[i]) af[i][mb][b] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+                }
+    }
     const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;
     const uint32_t row_bytes = (uint32_t)spr * (uint32_t)kQ8RunBytes;
@@ -1555,13 +1739,24 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
                 }
             }
         }
+        if (XT) acc[0] *= up;
 #pragma unroll
         for (int mb = 0; mb < MT; mb++) small_add_waves(red, keep, ti * MT + mb, wave, nwaves, lane, acc[mb], out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRunQ8 ring0a, ring0b, ring1a, ring1b;  // (the b halves are unused with one run per wave)
     issue(0, ring0a, ring0b);
-    issue(1, ring1a, ring1b);
+    if (XT != 2 || NSB == 1) issue(1, ring1a, ring1b);
+    if constexpr (XT != 0) {  // while the first weights are on their way
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
+        half8_t *to[NSB];
+#pragma unroll
+        for (int i = 0; i < NSB; i++) to[i] = af[i][0];
+        X.convert(x_stage, lane, to, up);
+        barrier_lds();
+        if (XT == 2 && NSB == 2) issue(1, ring1a, ring1b);  // (in f32 two super-blocks' activations leave no registers for it before)
+    }
     for (int rd = 0; rd < rounds; rd++) {
         consume(2 * rd, ring0a, ring0b);
         issue(2 * rd + 2, ring0a, ring0b);
@@ -1604,9 +1799,8 @@ struct SmallRunQ6 {
 // ANY: rows of any number of super-blocks.  A row then starts at any even address, so where a wave's super-blocks lie in
 // their first piece, and whether their fields sit two bytes off a dword boundary, differs from row to row (per lane); the
 // last wave with work may own one super-block where the others own two.
-template <int NSB, bool ANY>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
-                                                                      const float *__restrict__ rowscale, void *__restrict__ yg, int M,
+template <int NSB, bool ANY, bool XF32>
+__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8_t *__restrict__ W, const void *__restrict__ xg, void *__restrict__ yg, int M,
                                                                       int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
                                                                       uint32_t w_last, float *__restrict__ partial, const pmh::GemmSecond second) {
     int bx = (int)blockIdx.x;
@@ -1618,7 +1812,6 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
     constexpr int P = SmallQ6<NSB, ANY>::kRowPieces, kLoads = SmallQ6<NSB, ANY>::kLoads;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
-    const float rs = small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1636,20 +1829,15 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
     for (int i = 0; i < NSB; i++) sbv[i] = sb_here + i < spr;
     const int sb0 = sbv[0] ? sb_here : 0;
     const uint32_t run_start = 210u * (uint32_t)sb0, delta = run_start & 15u;
-    // activation operands: item (t = 4 lh + kg, gp) of half 2 sb + hh; index [hh][lh][gp]
-    half8_t af[NSB][2][2][2];
+    // activation operands: item (t = 4 lh + kg, gp) of half 2 sb + hh; index 4 hh + 2 lh + gp
+    half8_t af[NSB][8];
+    SmallX<XF32, 2, NSB> X;
+    float4_t up;
+    const uint32_t x_row = (uint32_t)spr * (XF32 ? 1024u : 512u);
+    const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
 #pragma unroll
-    for (int i = 0; i < NSB; i++)
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++)
-#pragma unroll
-            for (int lh = 0; lh < 2; lh++)
-#pragma unroll
-                for (int gp = 0; gp < 2; gp++) {
-                    const uint4 *item = xs + (size_t)((2 * (sbv[i] ? sb0 + i : 0) + hh) * kQ6Groups + 2 * (4 * lh + kg) + gp) * Mp + nl;
-                    af[i][hh][lh][gp] = __builtin_bit_cast(half8_t, *item);
-                    if (!sbv[i]) af[i][hh][lh][gp] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-                }
+    for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sb0 + i, sbv[i], lane);
+    __builtin_amdgcn_sched_barrier(0);
     const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;
     const uint32_t row_bytes = (uint32_t)spr * 210u;
@@ -1711,7 +1899,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
 #pragma unroll
                     for (int gp = 0; gp < 2; gp++) {
                         const uint32_t ql = field(16 * hh + 8 * gp + 4 * lh + kg);
-                        const half8_t a8 = af[i][hh][lh][gp];
+                        const half8_t a8 = af[i][4 * hh + 2 * lh + gp];
 #pragma unroll
                         for (int up = 0; up < 2; up++) {  // group g = gp + 2 up: the low, then the high nibbles
                             const int g = gp + 2 * up;
@@ -1731,12 +1919,21 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
                     }
                 }
         }
+        acc *= up;
         small_add_waves(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRunQ6<NSB> ring0, ring1;
     issue(0, ring0);
-    issue(1, ring1);
+    if (!XF32 || NSB == 1) issue(1, ring1);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XF32 ? 2 : 1) * kSmallXItems);  // while the first weights are on their way
+    half8_t *to[NSB];
+#pragma unroll
+    for (int i = 0; i < NSB; i++) to[i] = af[i];
+    X.convert(x_stage, lane, to, up);
+    barrier_lds();
+    if (XF32 && NSB == 2) issue(1, ring1);  // (in f32 two super-blocks' activations leave no registers for it before)
     for (int rd = 0; rd < rounds; rd++) {
         consume(2 * rd, ring0);
         issue(2 * rd + 2, ring0);
@@ -1744,10 +1941,15 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
         issue(2 * rd + 3, ring1);
     }
     small_add_kept(keep, rounds * kSmallDepth, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rs, yg, ybf16, partial);
+    small_store(out_tiles, t0, t1, M, Mp, N, 1.0f, yg, ybf16, partial);
 }
 
-// y[m][n] = rowscale[m] * (partial[0][m][n] + partial[1][m][n] + ...), added in this order.  A thread takes PER consecutive
+__global__ __launch_bounds__(256) void k_copy16(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t items) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < items) dst[i] = src[i];
+}
+
+// y[m][n] = rowscale[m] * (partial[0][m][n] + partial[1][m][n] + ...), added in this order (rowscale NULL: the tiles are scaled already).  A thread takes PER consecutive
 // outputs of the row-major result, whatever the row length: eight, in 16-byte accesses (rows of a length that is no multiple
 // of 8 went one output per thread: with the tile store's wide form for them 4674 x 1024 at M = 829 39.8 -> 29.9 us a call), or
 // one where the result is small and the kernel is the time of one trip to memory (7 x 1661: 1.5 us longer with eight).
@@ -1764,7 +1966,7 @@ __global__ __launch_bounds__(256) void k_rw_reduce(const float *__restrict__ par
     auto one = [&](const int e) {  // output idx + e: its row may be a later one
         float t = partial[idx + e];
         for (int z = 1; z < splits; z++) t += partial[(size_t)z * plane + idx + e];
-        t *= rowscale[m + (col + e) / (uint32_t)N];
+        if (rowscale) t *= rowscale[m + (col + e) / (uint32_t)N];
         if (YBF16) reinterpret_cast<uint16_t *>(yg)[idx + e] = (uint16_t)bf16_rne_bits(t);
         else reinterpret_cast<float *>(yg)[idx + e] = t;
     };
@@ -1773,7 +1975,7 @@ __global__ __launch_bounds__(256) void k_rw_reduce(const float *__restrict__ par
     } else if (total - idx < 8 || N < 8) {
         for (int e = 0; e < 8 && idx + e < total; e++) one(e);
     } else {
-        const float s0 = rowscale[m], s1 = rowscale[m + 1 < (uint32_t)M ? m + 1 : m];  // at most one row ends among the eight
+        const float s0 = rowscale ? rowscale[m] : 1.0f, s1 = rowscale ? rowscale[m + 1 < (uint32_t)M ? m + 1 : m] : 1.0f;  // at most one row ends among the eight
         float4 a = reinterpret_cast<const float4 *>(partial + idx)[0], b = reinterpret_cast<const float4 *>(partial + idx)[1];
         for (int z = 1; z < splits; z++) {
             const float4 *q = reinterpret_cast<const float4 *>(partial + (size_t)z * plane + idx);
@@ -1833,8 +2035,8 @@ struct SmallRun16 {  // what a lane holds of a row tile
     u32x4 sc[NSB];         // Q3_K: scales and d; Q2_K: x, y = scale bytes 8 h .., z = d | dmin << 16
 };
 
-template <int FMT, int NSB>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
+template <int FMT, int NSB, int XT>  // (XT as above)
+__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_t *__restrict__ W, const void *__restrict__ xg,
                                                                      const float *__restrict__ rowscale, void *__restrict__ yg, int M,
                                                                      int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
                                                                      float *__restrict__ partial, const pmh::GemmSecond second) {
@@ -1846,7 +2048,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
     using B = Block16<FMT>;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the kept partial tiles
-    const float rs = small_row_scale(rowscale);
+    const float rs = XT ? 1.0f : small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -1864,18 +2066,29 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         sbi[i] = sbv[i] ? sbi[i] : 0;
     }
     half8_t af[NSB][8], asum[NSB][2];
+    SmallX<XT == 2, 5, NSB> X;
+    float4_t up;
+    const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
+    const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
+    if constexpr (XT != 0) {
 #pragma unroll
-    for (int i = 0; i < NSB; i++) {
-        const uint4 *base = xs + (size_t)((2 * sbi[i] + (int)h) * kGroups16) * Mp + nl;
+        for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sbi[i], sbv[i], lane);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        const uint4 *xs = reinterpret_cast<const uint4 *>(xg);
 #pragma unroll
-        for (int t = 0; t < 8; t++) af[i][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (int)g) * Mp]);
-        asum[i][0] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (int)g) * Mp]);
-        asum[i][1] = __builtin_bit_cast(half8_t, base[(size_t)(18 + (int)g) * Mp]);
-        if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
-            const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int i = 0; i < NSB; i++) {
+            const uint4 *base = xs + (size_t)((2 * sbi[i] + (int)h) * kGroups16) * Mp + nl;
 #pragma unroll
-            for (int t = 0; t < 8; t++) af[i][t] = z;
-            asum[i][0] = z, asum[i][1] = z;
+            for (int t = 0; t < 8; t++) af[i][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (int)g) * Mp]);
+            asum[i][0] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (int)g) * Mp]);
+            asum[i][1] = __builtin_bit_cast(half8_t, base[(size_t)(18 + (int)g) * Mp]);
+            if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
+                const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+                for (int t = 0; t < 8; t++) af[i][t] = z;
+                asum[i][0] = z, asum[i][1] = z;
+            }
         }
     }
     const int t0 = bx * tiles_per_wg;
@@ -1976,12 +2189,25 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(d, part[r], acc[r]);
         }
+        if (XT) acc *= up;
         small_add_waves(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRun16<FMT, NSB> ring0, ring1;
     issue(0, ring0);
-    issue(1, ring1);
+    if (XT != 2 || NSB == 1) issue(1, ring1);
+    if constexpr (XT != 0) {  // while the first weights are on their way
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
+        half8_t *to[NSB];
+#pragma unroll
+        for (int i = 0; i < NSB; i++) to[i] = af[i];
+        X.convert(x_stage, lane, to, up);
+#pragma unroll
+        for (int i = 0; i < NSB; i++) small_sums<5>(af[i], reinterpret_cast<float *>(x_stage), lane, asum[i]);
+        barrier_lds();
+        if (XT == 2 && NSB == 2) issue(1, ring1);  // (in f32 two super-blocks' activations leave no registers for it before)
+    }
     for (int rd = 0; rd < rounds; rd++) {  // whole rounds of two tiles, nothing conditional around the loads
         consume(2 * rd, ring0);
         issue(2 * rd + 2, ring0);
@@ -2023,6 +2249,14 @@ static bool qgemm_small_applies(uint32_t type, int64_t m, int64_t n, int64_t k) 
     if (type == kTypeQ3K) return (uint64_t)n * (uint64_t)spr * 110u < (1ull << 32);
     if (type == kTypeQ2K) return (uint64_t)n * (uint64_t)spr * 84u < (1ull << 32);
     return false;
+}
+
+// Not for f32 activations of Q8_0 and Q3_K rows of more than eight super-blocks: a wave converts two of them, 128 registers of f32, and its second
+// row tile has to be asked for behind them (us a call, M = 16, 14336 x 4096 with a pre-pass / without: Q8_0 18.4 / 19.3; Q3_K, M = 4, 1024 x 4096
+// 11.9 / 12.2, M = 9, 4096 x 3328 11.9 / 12.4; Q4_K 14.9 / 14.5, 9.7 / 9.5, 10.6 / 10.2).
+bool qgemm_converts_itself(const GemmPlan &p, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype) {
+    if (p.kernel != GemmKernel::kSmall || m > kSmallMaxM) return false;
+    return x_dtype != kDtypeF32 || k <= kSmallWaves * 256 || (type != kTypeQ8_0 && type != kTypeQ3K);
 }
 
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
@@ -2353,7 +2587,20 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         else if (per_wg == 2) PMH_PREP_R(F, O, 2); \
         else PMH_PREP_R(F, O, 1);               \
     } while (0)
-    if (reuse_prepass) {
+    const bool own = qgemm_converts_itself(p, type, m, k, x_dtype);
+    if (own) {
+        // Every wave converts what it multiplies.  Results over the activations would race with other workgroups' reads of them.
+        const uintptr_t xb = reinterpret_cast<uintptr_t>(x), xe = xb + (size_t)m * k * (xf32 ? 4 : 2);
+        auto over_x = [&](const void *out, int64_t rows) {
+            const uintptr_t b = reinterpret_cast<uintptr_t>(out);
+            return b < xe && xb < b + (size_t)m * rows * (y_dtype == kDtypeF32 ? 4 : 2);
+        };
+        if (over_x(y, n) || (second.n > 0 && over_x(second.y, second.n))) {  // (16 f32 rows are what 32 rows of items take)
+            const size_t items = (xe - xb) / 16;
+            hipLaunchKernelGGL(k_copy16, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, reinterpret_cast<const uint4 *>(x), xs, items);
+            x = xs;
+        }
+    } else if (reuse_prepass) {
         // the workspace still holds the converted activations of the previous call (same x, m, k and weight type)
     } else if (xf32) {
         if (xorder == 0) PMH_PREP(true, 0);
@@ -2393,6 +2640,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         int tiles_per_wg = (tiles + tiles1 + n_wg - 1) / n_wg;
         if (tiles1 > 0 && (tiles + tiles_per_wg - 1) / tiles_per_wg + (tiles1 + tiles_per_wg - 1) / tiles_per_wg > n_wg) tiles_per_wg++;
         const int mt = m > kSmallMaxM ? 2 : 1;  // 16-row blocks of activations
+        const size_t x_lds = !own ? 0 : (size_t)nwaves * (xf32 ? 2 : 1) * kSmallXItems * 16;  // the activations pass through before the tiles do
         // the finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and the 16 KiB of the
         // reduction buffers: 64 of them keep the workgroup within 160 KiB for every type
         tiles_per_wg = tiles_per_wg < 64 / mt ? tiles_per_wg : 64 / mt;
@@ -2406,94 +2654,59 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         // (a workgroup of few tiles also keeps every wave's partial tile of each until the end)
         const size_t lds = (size_t)((tiles_per_wg + kSmallDepth - 1) / kSmallDepth * kSmallDepth) * mt * 1024 *
                            (tiles_per_wg * mt <= kSmallKeepTiles ? 1 + nwaves : 1);
-#define PMH_SMALL_FM(O, S, F, T)                                                                                                 \
-    do {                                                                                                                         \
-        const size_t lds4 = lds + (size_t)nwaves * SmallRun<S, F>::kPieces * 16; /* the waves' stages behind the finished tiles */ \
-        if (lds4 > 48 * 1024) {                                                                                                   \
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_qgemm_small<O, S, F, T>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                    (int)lds4);                                                                                   \
-            if (e != hipSuccess) return e;                                                                                       \
-        }                                                                                                                        \
-        hipLaunchKernelGGL((k_qgemm_small<O, S, F, T>), grid, block, lds4, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf16, part_out, second);                                                                           \
-    } while (0)
-#define PMH_SMALL_F(O, S, F)               \
-    do {                                   \
-        if (mt == 2) PMH_SMALL_FM(O, S, F, 2); \
-        else PMH_SMALL_FM(O, S, F, 1);         \
-    } while (0)
-#define PMH_SMALL(O, S)         \
-    do {                        \
-        if (q5) PMH_SMALL_F(O, S, 1); \
-        else PMH_SMALL_F(O, S, 0);    \
-    } while (0)
+        // (LDS beyond the launch default has to be asked for)
+        auto go = [&](auto kern, size_t bytes, auto... args) {
+            bytes = bytes > x_lds ? bytes : x_lds;
+            if (bytes > 48 * 1024) {
+                const hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+                if (a != hipSuccess) return a;
+            }
+            hipLaunchKernelGGL(kern, grid, block, bytes, s, args...);
+            return hipGetLastError();
+        };
+        const void *const xa = own ? x : (const void *)xs;
+        const size_t waves = (size_t)nwaves;
         if (q23) {
-#define PMH_SMALL16(F, S)                                                                                                     \
-    do {                                                                                                                         \
-        if (lds > 48 * 1024) {                                                                                                   \
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_qgemm_small16<F, S>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                    (int)lds);                                                                                   \
-            if (e != hipSuccess) return e;                                                                                       \
-        }                                                                                                                        \
-        hipLaunchKernelGGL((k_qgemm_small16<F, S>), grid, block, lds, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf16, part_out, second);                                                                 \
-    } while (0)
+#define PMH_SMALL16(F, S, X) go(k_qgemm_small16<F, S, X>, lds, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
             if (type == kTypeQ2K) {
-                if (nsb == 2) PMH_SMALL16(3, 2);
-                else PMH_SMALL16(3, 1);
+                if (nsb == 2) e = xf32 ? PMH_SMALL16(3, 2, 2) : PMH_SMALL16(3, 2, 1);
+                else e = xf32 ? PMH_SMALL16(3, 1, 2) : PMH_SMALL16(3, 1, 1);
             } else {
-                if (nsb == 2) PMH_SMALL16(2, 2);
-                else PMH_SMALL16(2, 1);
+                if (nsb == 2) e = own ? PMH_SMALL16(2, 2, 1) : PMH_SMALL16(2, 2, 0);
+                else e = xf32 ? PMH_SMALL16(2, 1, 2) : PMH_SMALL16(2, 1, 1);
             }
 #undef PMH_SMALL16
         } else if (q6) {
             const bool any = spr % 8 != 0;  // rows that do not start on 16-byte boundaries
-            const size_t stage = (size_t)(nsb == 2 ? SmallQ6<2, true>::kStageDwords : SmallQ6<1>::kStageDwords) * 4;
-            const size_t lds6 = lds + (size_t)nwaves * stage;  // the waves' stages behind the finished tiles
+            // the waves' stages behind the finished tiles
+            const size_t lds6 = lds + waves * (size_t)(nsb == 2 ? SmallQ6<2, true>::kStageDwords : SmallQ6<1>::kStageDwords) * 4;
             const uint32_t w_last = (uint32_t)(((uint64_t)n * (uint64_t)spr * 210u - 1) & ~(uint64_t)15);
-#define PMH_SMALL_Q6(S, A)                                                                                                        \
-    do {                                                                                                                         \
-        if (lds6 > 48 * 1024) {                                                                                                  \
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_qgemm_small_q6<S, A>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                    (int)lds6);                                                                                  \
-            if (e != hipSuccess) return e;                                                                                       \
-        }                                                                                                                        \
-        hipLaunchKernelGGL((k_qgemm_small_q6<S, A>), grid, block, lds6, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf16, w_last, part_out, second);                                                                   \
-    } while (0)
-            if (nsb == 2 && any) PMH_SMALL_Q6(2, true);
-            else if (nsb == 2) PMH_SMALL_Q6(2, false);
-            else if (any) PMH_SMALL_Q6(1, true);
-            else PMH_SMALL_Q6(1, false);
+#define PMH_SMALL_Q6(S, A)                                                                                                                             \
+    (xf32 ? go(k_qgemm_small_q6<S, A, true>, lds6, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second)    \
+          : go(k_qgemm_small_q6<S, A, false>, lds6, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second))
+            e = nsb == 2 ? (any ? PMH_SMALL_Q6(2, true) : PMH_SMALL_Q6(2, false)) : (any ? PMH_SMALL_Q6(1, true) : PMH_SMALL_Q6(1, false));
 #undef PMH_SMALL_Q6
         } else if (q8) {
-            const size_t lds8 = lds + (size_t)nwaves * nsb * kQ8TileRunPieces * 16;  // the waves' stages behind the finished tiles
-#define PMH_SMALL_Q8(S, T)                                                                                                       \
-    do {                                                                                                                         \
-        if (lds8 > 48 * 1024) {                                                                                                  \
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_qgemm_small_q8<S, T>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                    (int)lds8);                                                                                  \
-            if (e != hipSuccess) return e;                                                                                       \
-        }                                                                                                                        \
-        hipLaunchKernelGGL((k_qgemm_small_q8<S, T>), grid, block, lds8, s, w, xs, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, \
-                           tiles_per_wg, ybf16, part_out, second);                                                                           \
-    } while (0)
-            if (mt == 2) PMH_SMALL_Q8(1, 2);  // (two blocks of activations: one run of eight blocks per wave)
-            else if (nsb == 2) PMH_SMALL_Q8(2, 1);
-            else PMH_SMALL_Q8(1, 1);
+            const size_t lds8 = lds + waves * nsb * kQ8TileRunPieces * 16;
+#define PMH_SMALL_Q8(S, T, X) go(k_qgemm_small_q8<S, T, X>, lds8, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
+            if (mt == 2) e = PMH_SMALL_Q8(1, 2, 0);  // (two blocks of activations: one run of eight blocks per wave)
+            else if (nsb == 2) e = own ? PMH_SMALL_Q8(2, 1, 1) : PMH_SMALL_Q8(2, 1, 0);
+            else e = xf32 ? PMH_SMALL_Q8(1, 1, 2) : PMH_SMALL_Q8(1, 1, 1);
 #undef PMH_SMALL_Q8
-        } else if (spr > kSmallWaves) {
-            static_assert(2 * kSmallWaves >= kSmallMaxSpr, "two super-blocks per wave must cover the longest row");
-            if (ref) PMH_SMALL(0, 2);
-            else PMH_SMALL(1, 2);
         } else {
-            if (ref) PMH_SMALL(0, 1);
-            else PMH_SMALL(1, 1);
-        }
+            static_assert(2 * kSmallWaves >= kSmallMaxSpr, "two super-blocks per wave must cover the longest row");
+#define PMH_SMALL_X(O, S, F, T, X)                                                                                                                       \
+    go(k_qgemm_small<O, S, F, T, X>, lds + waves * SmallRun<S, F>::kPieces * 16, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, \
+       ybf16, part_out, second)
+#define PMH_SMALL_F(O, S, F) (mt == 2 ? PMH_SMALL_X(O, S, F, 2, 0) : xf32 ? PMH_SMALL_X(O, S, F, 1, 2) : PMH_SMALL_X(O, S, F, 1, 1))
+#define PMH_SMALL(O, S) (q5 ? PMH_SMALL_F(O, S, 1) : PMH_SMALL_F(O, S, 0))
+            if (spr > kSmallWaves) e = ref ? PMH_SMALL(0, 2) : PMH_SMALL(1, 2);
+            else e = ref ? PMH_SMALL(0, 1) : PMH_SMALL(1, 1);
 #undef PMH_SMALL
 #undef PMH_SMALL_F
-#undef PMH_SMALL_FM
-        e = hipGetLastError();
+#undef PMH_SMALL_X
+        }
+        if (own) rowscale = nullptr;  // the tiles leave scaled
         if (e != hipSuccess || runs == 1) return e;
     } else {
     const int mode = p.splits > 1 ? 2 : (ybf ? 1 : 0);

@@ -107,6 +107,8 @@ size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k);
 // Whether two weights of one type and element order that share their activations go in one launch (launch_qgemm with `second`), and
 // the launch's plan: the padded rows and the workspace are those of either weight alone, as are the results to the bit.
 bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan);
+// Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.
+bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype);
 // reuse_prepass: the workspace still holds the converted activations of the previous launch_qgemm on this stream with the same
 // x, m, k and weight type (two weights that share their activations: the pre-pass runs once)
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,

@@ -278,3 +278,69 @@ def test_results_over_the_neighbour_are_not_paired(oracle, over):
         return buf.to_host(np.uint8)
 
     assert np.array_equal(outputs(True), outputs(False))
+
+
+# Up to 16 rows the short-batch kernels' waves convert the activations they multiply, one or two super-blocks of each row with a scale of
+# their own.  Magnitudes that change from super-block to super-block, rows of zeros and of denormals, sizes below and above two
+# super-blocks a wave, whole and partial last runs, 1 to 16 rows, both activation types and orders.
+@pytest.mark.parametrize("m,n,k", [(1, 40, 256), (16, 33, 768), (5, 50, 2048), (15, 20, 3328), (16, 70, 4096), (9, 130, 7168), (2, 35, 11008)])
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_short_batches_convert_rows_of_any_scale(oracle, t, m, n, k):
+    rng = np.random.default_rng(31 * t + m + k)
+    raw = random_blocks(rng, t, n, k)
+    x = rng.standard_normal((m, k // 256, 256)) * np.exp2(rng.integers(-30, 30, (m, k // 256, 1)))
+    x[rng.random((m, k // 256)) < 0.1] = 0.0
+    x = x.reshape(m, k).astype(np.float32)
+    if m > 4:
+        x[1], x[3] = 0.0, x[3] * np.float32(1e-38)
+    bits = oracle.f32_to_bf16_bits(x.reshape(-1)).reshape(m, k)
+    xb = oracle.bf16_bits_to_f32(bits.reshape(-1)).reshape(m, k)
+    for order in (0, 1) if t in (Q4K, 13) else (0,):
+        w = np.abs(oracle.dequantize(t, raw, [n, k], order=order).reshape(n, k).astype(np.float64))
+        # against the sum of the products' magnitudes: f32 sums of integer tiles up to four times it (the min terms), and, for f32
+        # activations, their rounding to eleven bits; below the smallest normal f16, 2^-14 of 2^9, a step of 2^-25
+        for values, dtype, rounding in ((bits, pm.DTYPE_BF16, 0.0), (x, pm.DTYPE_F32, 2.0 ** -12)):
+            xv = xb if dtype == pm.DTYPE_BF16 else x
+            got = gpu_qgemm(t, raw, n, k, values, m, order=order, x_dtype=dtype)
+            want = reference(oracle, t, raw, n, k, xv, order)
+            size = np.abs(xv.astype(np.float64)) @ w.T
+            assert np.all(np.abs(got - want) <= ((k / 16 + 16) * 2.0 ** -24 * 4 + 2 * rounding) * size + k * 2.0 ** -149), (order, dtype)
+
+
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_short_batches_write_over_their_activations(oracle, t):
+    rng = np.random.default_rng(t)
+    lib = _lib.load()
+    for m, n, k, dtype, size in ((16, 2048, 2048, pm.DTYPE_F32, 4), (7, 4096, 2048, pm.DTYPE_BF16, 2), (16, 500, 7168, pm.DTYPE_F32, 4)):
+        raw = random_blocks(rng, t, n, k)
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        values = x if dtype == pm.DTYPE_F32 else oracle.f32_to_bf16_bits(x.reshape(-1)).reshape(m, k)
+        want = gpu_qgemm(t, raw, n, k, values, m, x_dtype=dtype)
+        dw, both = pm.DeviceBuffer.from_host(raw), pm.DeviceBuffer(max(m * k * size, m * n * 4) + 512)
+        for at in (0, 256):  # results from the activations' start, and from a little behind it
+            pm.check(lib.pmetal_hip_h2d(both.ptr, np.ascontiguousarray(values).ctypes.data, m * k * size))
+            pm.check(lib.pmetal_hip_qgemm(t, dw.ptr, n, k, both.ptr, dtype, m, both.ptr + at, pm.DTYPE_F32, 0, None))
+            pm.check(lib.pmetal_hip_sync(None))
+            got = both.to_host(np.uint8)[at:at + m * n * 4].view(np.float32).reshape(m, n)
+            assert np.array_equal(got, want), (m, n, k, at)
+
+
+@pytest.mark.parametrize("x_dtype", [pm.DTYPE_BF16, pm.DTYPE_F32])
+def test_batches_of_kernels_with_and_without_a_pre_pass(oracle, x_dtype):
+    """Weights of one call whose plans differ in who converts the activations, and in where the workspace keeps what."""
+    rng = np.random.default_rng(3)
+    lib = _lib.load()
+    for m, k, specs in ((12, 2304, [(Q4K, 300), (Q4K, 9000), (Q4K, 400), (Q8_0, 9000), (Q4K, 300)]),
+                        (12, 14336, [(Q6K, 300), (Q4K, 300), (Q6K, 400), (11, 300), (Q4K, 500)]),
+                        (9, 5120, [(Q4K, 300), (Q6K, 14400), (Q4K, 300), (Q8_0, 300), (Q6K, 14400), (Q8_0, 300)])):
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        dx = pm.DeviceBuffer.from_host(x if x_dtype == pm.DTYPE_F32 else oracle.f32_to_bf16_bits(x.reshape(-1)).reshape(m, k))
+        ws = [pm.DeviceBuffer.from_host(random_blocks(rng, t, n, k)) for t, n in specs]
+        ys, ones = ([pm.DeviceBuffer(m * n * 4) for _, n in specs] for _ in range(2))
+        descs = (_lib.GemmDesc * len(specs))(*[_lib.GemmDesc(t, pm.DTYPE_F32, 0, 0, n, w.ptr, y.ptr) for (t, n), w, y in zip(specs, ws, ys)])
+        pm.check(lib.pmetal_hip_qgemm_batch(descs, len(specs), k, dx.ptr, x_dtype, m, None))
+        for (t, n), w, y in zip(specs, ws, ones):
+            pm.check(lib.pmetal_hip_qgemm(t, w.ptr, n, k, dx.ptr, x_dtype, m, y.ptr, pm.DTYPE_F32, 0, None))
+        pm.check(lib.pmetal_hip_sync(None))
+        for i, (a, b) in enumerate(zip(ys, ones)):
+            assert np.array_equal(a.to_host(np.uint8), b.to_host(np.uint8)), (m, k, i)
