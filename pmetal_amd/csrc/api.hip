@@ -965,8 +965,8 @@ static int32_t qgemm_over_reblocked(uint32_t t, const uint8_t *wa, int64_t n, in
     if (parts == 1) {
         e = pmh::launch_qgemm(PMETAL_GGML_TYPE_Q6K, wa, n, k, x, x_dtype, m, y, y_dtype, 0, scratch, s);
     } else {  // the second product reuses the first one's converted activations
-        e = pmh::launch_qgemm(PMETAL_GGML_TYPE_Q6K, wa, n, k, x, x_dtype, m, ya, PMETAL_HIP_DTYPE_F32, 0, scratch, s);
-        if (e == hipSuccess) e = pmh::launch_qgemm(PMETAL_GGML_TYPE_Q6K, wb, n, k, x, x_dtype, m, yb, PMETAL_HIP_DTYPE_F32, 0, scratch, s, true);
+        e = pmh::launch_qgemm(PMETAL_GGML_TYPE_Q6K, wa, n, k, x, x_dtype, m, ya, PMETAL_HIP_DTYPE_F32, 0, scratch, s, false, {}, true);
+        if (e == hipSuccess) e = pmh::launch_qgemm(PMETAL_GGML_TYPE_Q6K, wb, n, k, x, x_dtype, m, yb, PMETAL_HIP_DTYPE_F32, 0, scratch, s, true, {}, true);
         if (e == hipSuccess) e = pmh::launch_add_store(ya, yb, y_elems, y, !y_f32, s);
     }
     if (e == hipErrorNotSupported) return fail(PMETAL_HIP_ERR_UNSUPPORTED_TYPE, "qgemm: configuration not supported");
@@ -1083,24 +1083,33 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
         return !over(a.y_dev, ya, b.y_dev, yb) && !over(a.y_dev, ya, b.w_dev, (size_t)b.n * k / per * block) &&
                !over(b.y_dev, yb, a.w_dev, (size_t)a.n * k / per * block);
     };
+    // two neighbours of one kind share a launch, unless one's results lie over what the other reads or writes
+    auto pair_at = [&](size_t i) {
+        pmh::GemmPlan plan;
+        return i + 1 < count && one_kind(descs[i], descs[i + 1]) && apart(descs[i], descs[i + 1]) &&
+               pmh::qgemm_pair_plan(m, descs[i].n, descs[i + 1].n, k, descs[i].ggml_type, &plan);
+    };
+    // what a launch's converted activations look like: their layout, per row or (at most 16 rows) per pair of super-blocks
+    auto form = [&](const pmetal_hip_gemm_desc &d, const pmh::GemmPlan &p) { return layout(d) + (pmh::qgemm_small_rows(p, m) ? 6 : 0); };
+    int launches[12] = {};  // of each form
+    for (size_t i = 0; i < count; i += pair_at(i) ? 2 : 1) launches[form(descs[i], pmh::qgemm_plan(m, descs[i].n, k, descs[i].ggml_type))]++;
     for (size_t i = 0; i < count; i++) {
         const pmetal_hip_gemm_desc &d = descs[i];
         const pmh::GemmPlan one = pmh::qgemm_plan(m, d.n, k, d.ggml_type);
-        const int want = layout(d), want_mp = one.mp;
-        // two neighbours of one kind share a launch, unless one's results lie over what the other reads or writes
+        const int want = form(d, one), want_mp = one.mp;
+        const bool shared = launches[want] > 1;
         pmh::GemmSecond second{};
-        pmh::GemmPlan plan;
-        if (i + 1 < count && one_kind(d, descs[i + 1]) && apart(d, descs[i + 1]) &&
-            pmh::qgemm_pair_plan(m, d.n, descs[i + 1].n, k, d.ggml_type, &plan)) {
+        if (pair_at(i)) {
             second.w = (const uint8_t *)descs[i + 1].w_dev, second.y = descs[i + 1].y_dev, second.n = (int)descs[i + 1].n;
             i++;
         }
         hipError_t e = pmh::launch_qgemm(d.ggml_type, (const uint8_t *)d.w_dev, d.n, k, x, x_dtype, m, d.y_dev, d.y_dtype, d.order, ws, (hipStream_t)stream,
-                                         want == have && want_mp == have_mp, second);
+                                         want == have && want_mp == have_mp, second, shared);
         if (e == hipErrorNotSupported) return fail(PMETAL_HIP_ERR_UNSUPPORTED_TYPE, "qgemm: configuration not supported");
         if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
         // (a second weight's plan has the same kernel; a K split's partial tiles may lie over items of another layout)
-        have = pmh::qgemm_converts_itself(one, d.ggml_type, m, k, x_dtype) ? -1 : want, have_mp = want_mp;
+        const bool two_q3k = d.ggml_type == PMETAL_GGML_TYPE_Q3K && second.n > 0;
+        have = pmh::qgemm_converts_itself(one, d.ggml_type, m, k, x_dtype, shared || two_q3k) ? -1 : want, have_mp = want_mp;
     }
     return ok();
 }

@@ -1163,13 +1163,13 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_rw_q8(const uint8_t *__restric
 
 // ------------------------------------------------------------------------------------------------
 // Q4_K with at most 16 activation rows (a decode batch, a speculative window) and rows of at most 16 super-blocks: the
-// weights are read once, at the pace of the GEMV, and nothing but the pre-pass runs before or after this kernel.
+// weights are read once, at the pace of the GEMV, and (rows of at most eight super-blocks, see SmallX) no other kernel runs.
 //   * v_mfma_f32_16x16x32_f16: 16 activation rows x 16 weight rows x 32 k.  Lane (r = lane % 16, kg = lane / 16) holds
 //     the eight k of k-group kg for activation row r (first operand) resp. weight row r (second operand); the output
 //     tile has column lane % 16 (weight row) and rows 4 (lane / 16) + 0..3 (activation rows).
 //   * A wave owns one or two super-block columns of W (wave w: super-blocks w and w + 8) and walks the row tiles of its
 //     workgroup.  Its activation operands for those super-blocks -- per super-block eight items (k-step t, k-group kg)
-//     and the item of sub-block sums, exactly the items the pre-pass writes -- are loaded once and stay in registers.
+//     and the item of sub-block sums, as a pre-pass arranges them -- are converted or loaded once and stay in registers.
 //   * Per row tile the wave copies its one or two super-blocks of the 16 rows (144 or 288 contiguous bytes per row)
 //     through registers into its own piece of LDS with whole-wave 16-byte loads, a row tile ahead (every load
 //     unconditional, so the outstanding loads are counted exactly); a lane then takes the 16-byte header of its weight
@@ -1267,7 +1267,9 @@ __device__ __forceinline__ void small_store(const float4_t *out_tiles, int t0, i
 // two runs of four elements each, of row lane % 16, where the pre-pass's order of the same number puts them.  The power of two that
 // takes a row into [2^9, 2^10) is that of the wave's part of it and not of the whole row: its inverse multiplies the wave's tiles,
 // exactly, before they are added, so nothing is rounded that a pre-pass would not round.
-// Measured (us a call, 14336 x 4096, M = 16, bf16, from memory, with the pre-pass -> so): see the launcher.
+// Measured (us a call, M = 16, from memory, with a pre-pass in front -> so): bf16 14336 x 4096 Q4_K 14.9 -> 13.3, Q5_K 16.5 -> 15.9,
+// Q6_K 18.3 -> 17.6, Q8_0 18.9 -> 18.4, Q2_K 14.5 -> 13.3; f32 14336 x 4096 Q4_K 14.7 -> 14.2; 4096 x 14336 18.8 -> 16.1.  1.13 times as
+// fast over 42 shapes of 1 to 16 rows.
 // ------------------------------------------------------------------------------------------------
 constexpr int kSmallXItems = 512;  // 16-byte items of LDS for a super-block of 16 rows in bf16; f32: twice as many
 template <bool XF32, int ORDER, int NSB>
@@ -1295,6 +1297,11 @@ struct SmallX {
     // af: the items; up: 2^e of the rows 4 kg .. 4 kg + 3 (the rows of the lane's part of a product tile).  (In instructions that two
     // waves of a SIMD can issue at a time: packed ones and v_fma_mix would end that)
     __device__ __forceinline__ void convert(u32x4 *stage, const int lane, half8_t *const (&af)[NSB], float4_t &up) const {
+        convert(stage, lane, af, up, [](float most) { return most; });
+    }
+    // join: the largest magnitude of the row over what other waves hold of it, too
+    template <class Join>
+    __device__ __forceinline__ void convert(u32x4 *stage, const int lane, half8_t *const (&af)[NSB], float4_t &up, const Join &join) const {
         const int nl = lane & 15, kg = lane >> 4;
         const u32x4 *mine = stage + nl * kPieces;
         uint32_t raw[NSB][8][XF32 ? 8 : 4];
@@ -1333,7 +1340,7 @@ struct SmallX {
         }
         float amax = __builtin_fmaxf(__builtin_fmaxf(most[0], most[1]), __builtin_fmaxf(most[2], most[3]));
         amax = __builtin_fmaxf(amax, __shfl_xor(amax, 16));
-        amax = __builtin_fmaxf(amax, __shfl_xor(amax, 32));
+        amax = join(__builtin_fmaxf(amax, __shfl_xor(amax, 32)));
         const int eb = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFFu);  // it lies in [2^(eb-127), 2^(eb-126))
         int e = eb - 126 - 10;
         e = e < -126 ? -126 : (e > 126 ? 126 : e);
@@ -1401,6 +1408,58 @@ __device__ __forceinline__ void barrier_lds() {
     asm volatile("" ::: "memory");
 }
 
+// Where several launches multiply the same activations by rows of more than eight super-blocks, a workgroup per pair of them converts
+// them ahead, by the same code (the results do not depend on who converts): per pair the items, the sums' items and the scales, an
+// item per lane and 64 items, 1 KiB, at a time.
+template <int ORDER>
+constexpr int kPairItems = 2 * (8 + (ORDER == 2 || ORDER == 3 ? 0 : ORDER == 5 ? 2 : 1)) + 1;
+template <bool XF32, int ORDER>
+__global__ __launch_bounds__(128) void k_prep_pairs(const void *__restrict__ x, int M, int spr, uint4 *__restrict__ out) {  // a wave per super-block
+    __shared__ u32x4 stages[2][(XF32 ? 2 : 1) * kSmallXItems];
+    __shared__ float most[2][16];
+    constexpr int kSums = ORDER == 2 || ORDER == 3 ? 0 : ORDER == 5 ? 2 : 1;
+    const int lane = threadIdx.x & 63, i = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), sb = 2 * (int)blockIdx.x + i;
+    const uint32_t x_row = (uint32_t)spr * (XF32 ? 1024u : 512u);
+    const __amdgpu_buffer_rsrc_t xr = small_x_buffer(x, M, x_row);
+    SmallX<XF32, ORDER, 1> X;
+    X.request(0, xr, x_row, sb, sb < spr, lane);
+    half8_t af[8];
+    half8_t *const to[1] = {af};
+    float4_t up;
+    X.convert(stages[i], lane, to, up, [&](float v) {
+        if (lane < 16) most[i][lane] = v;
+        __syncthreads();
+        return __builtin_fmaxf(most[0][lane & 15], most[1][lane & 15]);
+    });
+    uint4 *mine = out + (size_t)blockIdx.x * (64 * kPairItems<ORDER>) + lane;
+#pragma unroll
+    for (int t = 0; t < 8; t++) mine[64 * (8 * i + t)] = __builtin_bit_cast(uint4, af[t]);
+    if (i == 0) mine[64 * (kPairItems<ORDER> - 1)] = __builtin_bit_cast(uint4, up);
+    if constexpr (kSums > 0) {
+        half8_t sums[kSums];
+        small_sums<ORDER>(af, reinterpret_cast<float *>(stages[i]), lane, sums);
+#pragma unroll
+        for (int c = 0; c < kSums; c++) mine[64 * (16 + kSums * i + c)] = __builtin_bit_cast(uint4, sums[c]);
+    }
+}
+// A wave's pair, or zeros where the row has ended (valid false).  item: of super-block i number t (from 8 on: its sums)
+template <int ORDER>
+struct SmallPair {
+    const uint4 *at;
+    uint32_t keep;
+    __device__ __forceinline__ SmallPair(const void *ws, const int sb, const bool valid, const int lane)
+        : at(reinterpret_cast<const uint4 *>(ws) + (size_t)(sb >> 1) * (64 * kPairItems<ORDER>) + lane), keep(valid ? 0xFFFFFFFFu : 0u) {}
+    __device__ __forceinline__ u32x4 get(const int n) const {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(at + 64 * n);
+        return v & u32x4{keep, keep, keep, keep};
+    }
+    __device__ __forceinline__ half8_t item(const int i, const int t) const {
+        constexpr int kSums = (kPairItems<ORDER> - 17) / 2;
+        return __builtin_bit_cast(half8_t, get(t < 8 ? 8 * i + t : 16 + kSums * i + t - 8));
+    }
+    __device__ __forceinline__ float4_t up() const { return __builtin_bit_cast(float4_t, get(kPairItems<ORDER> - 1)); }
+};
+
 template <int NSB, int FMT = 0>
 struct SmallRun {
     static constexpr int kPerSb = BlockFmt<FMT>::kBytes / 16;  // 16-byte pieces of a super-block: 9 (Q4_K) or 11 (Q5_K)
@@ -1413,7 +1472,7 @@ struct SmallRun {
 // sub-blocks out of its stage as well and ors the fifth bits into the quant dwords as in the large kernel.
 // MT: 16-row blocks of activations (1: at most 16 rows, 2: at most 32); a weight operand then feeds MT matrix instructions.
 // XT: what xg is: 0 the pre-pass's items (MT = 2: twice the rows to convert would not hide behind the first weights), 1 and 2 the
-// activations themselves in bf16 and in f32.
+// activations themselves in bf16 and in f32, 3 the pairs of super-blocks that k_prep_pairs has converted (NSB = 2).
 template <int ORDER, int NSB, int FMT, int MT, int XT>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t *__restrict__ W, const void *__restrict__ xg,
                                                                    const float *__restrict__ rowscale, void *__restrict__ yg, int M,
@@ -1447,14 +1506,24 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
     // activation operands of this wave's super-blocks: item (2 sb + kg / 2, group 2 t + kg % 2) of rows nl (and 16 + nl), and the sums item
     half8_t af[NSB][MT][8], asum[NSB][MT];
     constexpr int kXOrder = ORDER == 1 ? 1 : FMT ? 4 : 0;
+    constexpr bool kOwn = XT == 1 || XT == 2;
     SmallX<XT == 2, kXOrder, NSB> X;
     float4_t up;
     const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
     const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
-    if constexpr (XT != 0) {
+    if constexpr (kOwn) {
 #pragma unroll
         for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sbi[i], sbv[i], lane);
         __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (XT == 3) {
+        const SmallPair<kXOrder> pair(xg, sbi[0], sbv[0], lane);
+#pragma unroll
+        for (int i = 0; i < NSB; i++) {
+#pragma unroll
+            for (int t = 0; t < 8; t++) af[i][0][t] = pair.item(i, t);
+            asum[i][0] = pair.item(i, 8);
+        }
+        up = pair.up();
     } else {
         const uint4 *xs = reinterpret_cast<const uint4 *>(xg);
 #pragma unroll
@@ -1574,7 +1643,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
     SmallRun<NSB, FMT> ring0, ring1;
     issue(0, ring0);
     if (XT != 2 || NSB == 1) issue(1, ring1);
-    if constexpr (XT != 0) {  // while the first weights are on their way
+    if constexpr (kOwn) {  // while the first weights are on their way
         __builtin_amdgcn_sched_barrier(0);
         u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
         half8_t *to[NSB];
@@ -1652,14 +1721,22 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
     // activation operands: block b of run sb holds elements 256 sb + 32 b ..; the item of its k-group kg is item
     // 4 (b % 4) + kg of half 2 sb + b / 4 (the pre-pass writes 16 items of eight consecutive elements per 128)
     half8_t af[NSB][MT][8];  // (MT 16-row blocks of activations: rows nl, 16 + nl)
+    constexpr bool kOwn = XT == 1 || XT == 2;
     SmallX<XT == 2, 3, NSB> X;
     float4_t up;
     const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
     const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
-    if constexpr (XT != 0) {
+    if constexpr (kOwn) {
 #pragma unroll
         for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sbi[i], sbv[i], lane);
         __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (XT == 3) {
+        const SmallPair<3> pair(xg, sbi[0], sbv[0], lane);
+#pragma unroll
+        for (int i = 0; i < NSB; i++)
+#pragma unroll
+            for (int b = 0; b < 8; b++) af[i][0][b] = pair.item(i, b);
+        up = pair.up();
     } else {
         const uint4 *xs = reinterpret_cast<const uint4 *>(xg);
 #pragma unroll
@@ -1747,7 +1824,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
     SmallRunQ8 ring0a, ring0b, ring1a, ring1b;  // (the b halves are unused with one run per wave)
     issue(0, ring0a, ring0b);
     if (XT != 2 || NSB == 1) issue(1, ring1a, ring1b);
-    if constexpr (XT != 0) {  // while the first weights are on their way
+    if constexpr (kOwn) {  // while the first weights are on their way
         __builtin_amdgcn_sched_barrier(0);
         u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
         half8_t *to[NSB];
@@ -1799,8 +1876,9 @@ struct SmallRunQ6 {
 // ANY: rows of any number of super-blocks.  A row then starts at any even address, so where a wave's super-blocks lie in
 // their first piece, and whether their fields sit two bytes off a dword boundary, differs from row to row (per lane); the
 // last wave with work may own one super-block where the others own two.
-template <int NSB, bool ANY, bool XF32>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8_t *__restrict__ W, const void *__restrict__ xg, void *__restrict__ yg, int M,
+template <int NSB, bool ANY, int XT>  // (XT as above)
+__global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8_t *__restrict__ W, const void *__restrict__ xg,
+                                                                      void *__restrict__ yg, int M,
                                                                       int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
                                                                       uint32_t w_last, float *__restrict__ partial, const pmh::GemmSecond second) {
     int bx = (int)blockIdx.x;
@@ -1831,13 +1909,23 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
     const uint32_t run_start = 210u * (uint32_t)sb0, delta = run_start & 15u;
     // activation operands: item (t = 4 lh + kg, gp) of half 2 sb + hh; index 4 hh + 2 lh + gp
     half8_t af[NSB][8];
-    SmallX<XF32, 2, NSB> X;
+    constexpr bool kOwn = XT == 1 || XT == 2;
+    SmallX<XT == 2, 2, NSB> X;
     float4_t up;
-    const uint32_t x_row = (uint32_t)spr * (XF32 ? 1024u : 512u);
+    const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
     const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
+    if constexpr (kOwn) {
 #pragma unroll
-    for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sb0 + i, sbv[i], lane);
-    __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sb0 + i, sbv[i], lane);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        const SmallPair<2> pair(xg, sb0, sbv[0], lane);
+#pragma unroll
+        for (int i = 0; i < NSB; i++)
+#pragma unroll
+            for (int t = 0; t < 8; t++) af[i][t] = pair.item(i, t);
+        up = pair.up();
+    }
     const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;
     const uint32_t row_bytes = (uint32_t)spr * 210u;
@@ -1925,15 +2013,17 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRunQ6<NSB> ring0, ring1;
     issue(0, ring0);
-    if (!XF32 || NSB == 1) issue(1, ring1);
-    __builtin_amdgcn_sched_barrier(0);
-    u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XF32 ? 2 : 1) * kSmallXItems);  // while the first weights are on their way
-    half8_t *to[NSB];
+    if (XT != 2 || NSB == 1) issue(1, ring1);
+    if constexpr (kOwn) {  // while the first weights are on their way
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
+        half8_t *to[NSB];
 #pragma unroll
-    for (int i = 0; i < NSB; i++) to[i] = af[i];
-    X.convert(x_stage, lane, to, up);
-    barrier_lds();
-    if (XF32 && NSB == 2) issue(1, ring1);  // (in f32 two super-blocks' activations leave no registers for it before)
+        for (int i = 0; i < NSB; i++) to[i] = af[i];
+        X.convert(x_stage, lane, to, up);
+        barrier_lds();
+        if (XT == 2 && NSB == 2) issue(1, ring1);  // (in f32 two super-blocks' activations leave no registers for it before)
+    }
     for (int rd = 0; rd < rounds; rd++) {
         consume(2 * rd, ring0);
         issue(2 * rd + 2, ring0);
@@ -2037,7 +2127,7 @@ struct SmallRun16 {  // what a lane holds of a row tile
 
 template <int FMT, int NSB, int XT>  // (XT as above)
 __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_t *__restrict__ W, const void *__restrict__ xg,
-                                                                     const float *__restrict__ rowscale, void *__restrict__ yg, int M,
+                                                                     void *__restrict__ yg, int M,
                                                                      int Mp, int N, int spr, int tiles, int tiles_per_wg, int ybf16,
                                                                      float *__restrict__ partial, const pmh::GemmSecond second) {
     int bx = (int)blockIdx.x;
@@ -2048,7 +2138,6 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
     using B = Block16<FMT>;
     __shared__ float4_t red[2][kSmallWaves][64];
     extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the kept partial tiles
-    const float rs = XT ? 1.0f : small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -2066,30 +2155,24 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         sbi[i] = sbv[i] ? sbi[i] : 0;
     }
     half8_t af[NSB][8], asum[NSB][2];
+    constexpr bool kOwn = XT == 1 || XT == 2;
     SmallX<XT == 2, 5, NSB> X;
     float4_t up;
     const uint32_t x_row = (uint32_t)spr * (XT == 2 ? 1024u : 512u);
     const __amdgpu_buffer_rsrc_t xr = small_x_buffer(xg, M, x_row);
-    if constexpr (XT != 0) {
+    if constexpr (kOwn) {
 #pragma unroll
         for (int i = 0; i < NSB; i++) X.request(i, xr, x_row, sbi[i], sbv[i], lane);
         __builtin_amdgcn_sched_barrier(0);
     } else {
-        const uint4 *xs = reinterpret_cast<const uint4 *>(xg);
+        const SmallPair<5> pair(xg, sbi[0], sbv[0], lane);
 #pragma unroll
         for (int i = 0; i < NSB; i++) {
-            const uint4 *base = xs + (size_t)((2 * sbi[i] + (int)h) * kGroups16) * Mp + nl;
 #pragma unroll
-            for (int t = 0; t < 8; t++) af[i][t] = __builtin_bit_cast(half8_t, base[(size_t)(2 * t + (int)g) * Mp]);
-            asum[i][0] = __builtin_bit_cast(half8_t, base[(size_t)(16 + (int)g) * Mp]);
-            asum[i][1] = __builtin_bit_cast(half8_t, base[(size_t)(18 + (int)g) * Mp]);
-            if (!sbv[i]) {  // a super-block past the end of the row multiplies zeros (no branch in the streaming loop)
-                const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-                for (int t = 0; t < 8; t++) af[i][t] = z;
-                asum[i][0] = z, asum[i][1] = z;
-            }
+            for (int t = 0; t < 8; t++) af[i][t] = pair.item(i, t);
+            asum[i][0] = pair.item(i, 8), asum[i][1] = pair.item(i, 9);
         }
+        up = pair.up();
     }
     const int t0 = bx * tiles_per_wg;
     const int t1 = t0 + tiles_per_wg < tiles ? t0 + tiles_per_wg : tiles;  // t1 > t0 by the launch geometry
@@ -2189,14 +2272,14 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(d, part[r], acc[r]);
         }
-        if (XT) acc *= up;
+        acc *= up;
         small_add_waves(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRun16<FMT, NSB> ring0, ring1;
     issue(0, ring0);
     if (XT != 2 || NSB == 1) issue(1, ring1);
-    if constexpr (XT != 0) {  // while the first weights are on their way
+    if constexpr (kOwn) {  // while the first weights are on their way
         __builtin_amdgcn_sched_barrier(0);
         u32x4 *x_stage = reinterpret_cast<u32x4 *>(dyn) + wave * ((XT == 2 ? 2 : 1) * kSmallXItems);
         half8_t *to[NSB];
@@ -2215,7 +2298,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         issue(2 * rd + 3, ring1);
     }
     small_add_kept(keep, rounds * kSmallDepth, wave, nwaves, lane, out_tiles);
-    small_store(out_tiles, t0, t1, M, Mp, N, rs, yg, ybf16, partial);
+    small_store(out_tiles, t0, t1, M, Mp, N, 1.0f, yg, ybf16, partial);
 }
 
 }  // namespace
@@ -2251,12 +2334,18 @@ static bool qgemm_small_applies(uint32_t type, int64_t m, int64_t n, int64_t k) 
     return false;
 }
 
-// Not for f32 activations of Q8_0 and Q3_K rows of more than eight super-blocks: a wave converts two of them, 128 registers of f32, and its second
-// row tile has to be asked for behind them (us a call, M = 16, 14336 x 4096 with a pre-pass / without: Q8_0 18.4 / 19.3; Q3_K, M = 4, 1024 x 4096
-// 11.9 / 12.2, M = 9, 4096 x 3328 11.9 / 12.4; Q4_K 14.9 / 14.5, 9.7 / 9.5, 10.6 / 10.2).
-bool qgemm_converts_itself(const GemmPlan &p, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype) {
-    if (p.kernel != GemmKernel::kSmall || m > kSmallMaxM) return false;
-    return x_dtype != kDtypeF32 || k <= kSmallWaves * 256 || (type != kTypeQ8_0 && type != kTypeQ3K);
+// (Who converts does not change a bit of the result: k_prep_pairs does as the waves do.)
+// Up to eight super-blocks a row a wave converts one, which its first weights hide.  Of longer rows it converts two, which costs 1 to 3 us of
+// the pre-pass's 4: not where several launches share one pre-pass (us for three bf16 weights of 4096, 1024 and 1024 x 4096, M = 16, two launches,
+// with one / without: Q4_K 17.1 / 18.3, Q3_K 21.3 / 24.3; of 2048 x 2048 12.6 / 12.4), and not f32 activations of Q8_0 and Q3_K, 128 registers of
+// them, behind which the second row tile has to be asked for (M = 16, 14336 x 4096: Q8_0 18.4 / 19.3; Q3_K, M = 4, 1024 x 4096 11.9 / 12.2, M = 9,
+// 4096 x 3328 11.9 / 12.4; Q4_K 14.9 / 14.5, 9.7 / 9.5, 10.6 / 10.2) or two Q3_K weights in one launch (14336 x 4096, M = 16, 24.6 / 25.1: their sums
+// of sixteen elements take the longest to make).
+bool qgemm_small_rows(const GemmPlan &p, int64_t m) { return p.kernel == GemmKernel::kSmall && m <= kSmallMaxM; }
+bool qgemm_converts_itself(const GemmPlan &p, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype, bool shared) {
+    if (!qgemm_small_rows(p, m)) return false;
+    if (k <= kSmallWaves * 256) return true;
+    return !shared && (x_dtype != kDtypeF32 || (type != kTypeQ8_0 && type != kTypeQ3K));
 }
 
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
@@ -2546,7 +2635,7 @@ static hipError_t launch_rw_q8(hipStream_t s, const uint8_t *w, const uint4 *xs,
 
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,
                                 int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s, bool reuse_prepass,
-                                const GemmSecond &second_weight) {
+                                const GemmSecond &second_weight, bool shared) {
     if (!qgemm_fits(type, m, n, k)) return hipErrorInvalidValue;
     GemmSecond second = second_weight;
     GemmPlan p;
@@ -2587,7 +2676,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         else if (per_wg == 2) PMH_PREP_R(F, O, 2); \
         else PMH_PREP_R(F, O, 1);               \
     } while (0)
-    const bool own = qgemm_converts_itself(p, type, m, k, x_dtype);
+    const bool own = qgemm_converts_itself(p, type, m, k, x_dtype, shared || (type == kTypeQ3K && second.n > 0));
     if (own) {
         // Every wave converts what it multiplies.  Results over the activations would race with other workgroups' reads of them.
         const uintptr_t xb = reinterpret_cast<uintptr_t>(x), xe = xb + (size_t)m * k * (xf32 ? 4 : 2);
@@ -2602,6 +2691,21 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         }
     } else if (reuse_prepass) {
         // the workspace still holds the converted activations of the previous call (same x, m, k and weight type)
+    } else if (qgemm_small_rows(p, m)) {
+#define PMH_PAIRS(F, O) hipLaunchKernelGGL((k_prep_pairs<F, O>), dim3((unsigned)((spr + 1) / 2)), dim3(128), 0, s, x, (int)m, spr, xs)
+#define PMH_PAIRS_X(O)               \
+    do {                             \
+        if (xf32) PMH_PAIRS(true, O); \
+        else PMH_PAIRS(false, O);    \
+    } while (0)
+        if (xorder == 0) PMH_PAIRS_X(0);
+        else if (xorder == 1) PMH_PAIRS_X(1);
+        else if (xorder == 2) PMH_PAIRS_X(2);
+        else if (xorder == 3) PMH_PAIRS_X(3);
+        else if (xorder == 4) PMH_PAIRS_X(4);
+        else PMH_PAIRS_X(5);
+#undef PMH_PAIRS_X
+#undef PMH_PAIRS
     } else if (xf32) {
         if (xorder == 0) PMH_PREP(true, 0);
         else if (xorder == 1) PMH_PREP(true, 1);
@@ -2667,12 +2771,12 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         const void *const xa = own ? x : (const void *)xs;
         const size_t waves = (size_t)nwaves;
         if (q23) {
-#define PMH_SMALL16(F, S, X) go(k_qgemm_small16<F, S, X>, lds, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
+#define PMH_SMALL16(F, S, X) go(k_qgemm_small16<F, S, X>, lds, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
             if (type == kTypeQ2K) {
-                if (nsb == 2) e = xf32 ? PMH_SMALL16(3, 2, 2) : PMH_SMALL16(3, 2, 1);
+                if (nsb == 2) e = !own ? PMH_SMALL16(3, 2, 3) : xf32 ? PMH_SMALL16(3, 2, 2) : PMH_SMALL16(3, 2, 1);
                 else e = xf32 ? PMH_SMALL16(3, 1, 2) : PMH_SMALL16(3, 1, 1);
             } else {
-                if (nsb == 2) e = own ? PMH_SMALL16(2, 2, 1) : PMH_SMALL16(2, 2, 0);
+                if (nsb == 2) e = own ? PMH_SMALL16(2, 2, 1) : PMH_SMALL16(2, 2, 3);
                 else e = xf32 ? PMH_SMALL16(2, 1, 2) : PMH_SMALL16(2, 1, 1);
             }
 #undef PMH_SMALL16
@@ -2681,16 +2785,17 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             // the waves' stages behind the finished tiles
             const size_t lds6 = lds + waves * (size_t)(nsb == 2 ? SmallQ6<2, true>::kStageDwords : SmallQ6<1>::kStageDwords) * 4;
             const uint32_t w_last = (uint32_t)(((uint64_t)n * (uint64_t)spr * 210u - 1) & ~(uint64_t)15);
-#define PMH_SMALL_Q6(S, A)                                                                                                                             \
-    (xf32 ? go(k_qgemm_small_q6<S, A, true>, lds6, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second)    \
-          : go(k_qgemm_small_q6<S, A, false>, lds6, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second))
-            e = nsb == 2 ? (any ? PMH_SMALL_Q6(2, true) : PMH_SMALL_Q6(2, false)) : (any ? PMH_SMALL_Q6(1, true) : PMH_SMALL_Q6(1, false));
+#define PMH_SMALL_Q6(S, A, X) go(k_qgemm_small_q6<S, A, X>, lds6, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second)
+            if (nsb == 2 && any) e = !own ? PMH_SMALL_Q6(2, true, 3) : xf32 ? PMH_SMALL_Q6(2, true, 2) : PMH_SMALL_Q6(2, true, 1);
+            else if (nsb == 2) e = !own ? PMH_SMALL_Q6(2, false, 3) : xf32 ? PMH_SMALL_Q6(2, false, 2) : PMH_SMALL_Q6(2, false, 1);
+            else if (any) e = xf32 ? PMH_SMALL_Q6(1, true, 2) : PMH_SMALL_Q6(1, true, 1);
+            else e = xf32 ? PMH_SMALL_Q6(1, false, 2) : PMH_SMALL_Q6(1, false, 1);
 #undef PMH_SMALL_Q6
         } else if (q8) {
             const size_t lds8 = lds + waves * nsb * kQ8TileRunPieces * 16;
 #define PMH_SMALL_Q8(S, T, X) go(k_qgemm_small_q8<S, T, X>, lds8, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
             if (mt == 2) e = PMH_SMALL_Q8(1, 2, 0);  // (two blocks of activations: one run of eight blocks per wave)
-            else if (nsb == 2) e = own ? PMH_SMALL_Q8(2, 1, 1) : PMH_SMALL_Q8(2, 1, 0);
+            else if (nsb == 2) e = own ? PMH_SMALL_Q8(2, 1, 1) : PMH_SMALL_Q8(2, 1, 3);
             else e = xf32 ? PMH_SMALL_Q8(1, 1, 2) : PMH_SMALL_Q8(1, 1, 1);
 #undef PMH_SMALL_Q8
         } else {
@@ -2699,14 +2804,14 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     go(k_qgemm_small<O, S, F, T, X>, lds + waves * SmallRun<S, F>::kPieces * 16, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, \
        ybf16, part_out, second)
 #define PMH_SMALL_F(O, S, F) (mt == 2 ? PMH_SMALL_X(O, S, F, 2, 0) : xf32 ? PMH_SMALL_X(O, S, F, 1, 2) : PMH_SMALL_X(O, S, F, 1, 1))
-#define PMH_SMALL(O, S) (q5 ? PMH_SMALL_F(O, S, 1) : PMH_SMALL_F(O, S, 0))
-            if (spr > kSmallWaves) e = ref ? PMH_SMALL(0, 2) : PMH_SMALL(1, 2);
-            else e = ref ? PMH_SMALL(0, 1) : PMH_SMALL(1, 1);
-#undef PMH_SMALL
+#define PMH_SMALL_2(O, F) (mt == 1 && !own ? PMH_SMALL_X(O, 2, F, 1, 3) : PMH_SMALL_F(O, 2, F))
+            if (spr > kSmallWaves) e = ref ? (q5 ? PMH_SMALL_2(0, 1) : PMH_SMALL_2(0, 0)) : (q5 ? PMH_SMALL_2(1, 1) : PMH_SMALL_2(1, 0));
+            else e = ref ? (q5 ? PMH_SMALL_F(0, 1, 1) : PMH_SMALL_F(0, 1, 0)) : (q5 ? PMH_SMALL_F(1, 1, 1) : PMH_SMALL_F(1, 1, 0));
+#undef PMH_SMALL_2
 #undef PMH_SMALL_F
 #undef PMH_SMALL_X
         }
-        if (own) rowscale = nullptr;  // the tiles leave scaled
+        if (mt == 1) rowscale = nullptr;  // the tiles leave scaled
         if (e != hipSuccess || runs == 1) return e;
     } else {
     const int mode = p.splits > 1 ? 2 : (ybf ? 1 : 0);

@@ -107,13 +107,16 @@ size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k);
 // Whether two weights of one type and element order that share their activations go in one launch (launch_qgemm with `second`), and
 // the launch's plan: the padded rows and the workspace are those of either weight alone, as are the results to the bit.
 bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan);
-// Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.
-bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype);
+// Whether the plan's kernel takes at most 16 rows, converted per pair of super-blocks and not per row: no other kernel can use those.
+bool qgemm_small_rows(const GemmPlan &plan, int64_t m);
+// Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.  shared: another
+// launch could use the converted ones.
+bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype, bool shared);
 // reuse_prepass: the workspace still holds the converted activations of the previous launch_qgemm on this stream with the same
 // x, m, k and weight type (two weights that share their activations: the pre-pass runs once)
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,
                         int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s,
-                        bool reuse_prepass = false, const GemmSecond &second = GemmSecond{});
+                        bool reuse_prepass = false, const GemmSecond &second = GemmSecond{}, bool shared = false);
 
 // gemm_kw.hip (spr: super-blocks per row; partial: fp32 tiles [splits][mp][n] when plan.splits > 1, not scaled by rowscale)
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &plan, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
