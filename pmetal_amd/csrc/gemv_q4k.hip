@@ -469,7 +469,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_qgemv_q4k_rows(const void *
     if (Q6LAST && bx >= wg_b3) {
         // Q6LAST: the fourth member is a small Q6_K matrix over the same activations (an attention v projection beside
         // q and k); its workgroups run the small-matrix Q6_K kernel's body, one team per wave
-        q6k_small_body<64, XF32>(w3, xg, y3, n3, spr, bx - wg_b3, (int)gridDim.x - wg_b3, kRowsWaves, smem);
+        q6k_member_body<64, XF32>(w3, xg, y3, n3, spr, bx - wg_b3, (int)gridDim.x - wg_b3, kRowsWaves, smem);
         return;
     }
     const int g = MULTI ? (bx >= wg_b1 ? 1 : 0) + (bx >= wg_b2 ? 1 : 0) + (bx >= wg_b3 ? 1 : 0) : 0;
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg,
     const int bx = (int)blockIdx.x;
     if (Q6LAST && bx >= wg_b3) {  // workgroup-uniform
         extern __shared__ uint4 smem6[];
-        q6k_small_body<T, XF32>(w3, xg, y3, n3, spr, bx - wg_b3, (int)gridDim.x - wg_b3, q6_teams, smem6);
+        q6k_member_body<T, XF32>(w3, xg, y3, n3, spr, bx - wg_b3, (int)gridDim.x - wg_b3, q6_teams, smem6);
         return;
     }
     const int g = (bx >= wg_b1 ? 1 : 0) + (bx >= wg_b2 ? 1 : 0) + (bx >= wg_b3 ? 1 : 0);
@@ -773,8 +773,7 @@ hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *
     grp.w[3] = w6, grp.y[3] = y6, grp.n[3] = (int)n6;
     const dim3 grid((unsigned)(begin + wgs6));
     const int teams_per_wave = 64 / T;
-    const int64_t rows6 = (n6 + wgs6 - 1) / wgs6;                 // rows of a Q6_K workgroup: two per team at a time
-    int64_t q6_teams = (rows6 + 1) / 2;
+    const int64_t rows6 = (n6 + wgs6 - 1) / wgs6;  // rows of a Q6_K workgroup: one per team, or two at a time where that is not enough
     int best_waves = 16;
     int64_t best_cost = INT64_MAX;
     for (int waves = 16; waves >= 1; waves--) {  // as in launch_group_general
@@ -783,7 +782,8 @@ hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *
         if (per_team < best_cost) best_cost = per_team, best_waves = waves;
     }
     const int64_t teams_avail = (int64_t)best_waves * teams_per_wave;
-    q6_teams = q6_teams < 1 ? 1 : (q6_teams > teams_avail ? teams_avail : q6_teams);
+    int64_t q6_teams = rows6 <= teams_avail ? rows6 : (rows6 + 1) / 2;
+    q6_teams = q6_teams > teams_avail ? teams_avail : q6_teams;
     const int per_team = (int)((rows_per_wg + teams_avail - 1) / teams_avail);
     const dim3 block((unsigned)best_waves * 64);
     if (order == pmh::kOrderRef)
@@ -883,11 +883,11 @@ static hipError_t launch_kernel_rows(const uint8_t *const *w, const int64_t *n, 
     const int64_t max_rows_per_wg = (int64_t)kRowsWaves * (kDepth / ks);
     int64_t want = 2 * cus;
     if (count > 1 && (total + want - 1) / want > max_rows_per_wg) want = 4 * cus;
-    // the Q6_K member: a team (one wave) walks two rows at a time, so one workgroup per 16 rows, at most half of all
+    // the Q6_K member: a team (one wave) for every row, so a workgroup per 8 rows; at most half of all (the teams then walk two rows at a time)
     int64_t wgs6 = 0;
     if (n6 > 0) {
         if ((uint64_t)n6 * (uint64_t)spr * 210u >= (1ull << 31)) return hipErrorNotSupported;
-        wgs6 = (n6 + 2 * kRowsWaves - 1) / (2 * kRowsWaves);
+        wgs6 = (n6 + kRowsWaves - 1) / kRowsWaves;
         wgs6 = wgs6 > want / 2 ? want / 2 : wgs6;
         want -= wgs6;
     }

@@ -28,13 +28,17 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
                                            false);
 }
 
-// Split an f32 into three bf16 terms hi + mid + lo; 3 x 8 significant bits hold all 24 bits of the
-// f32, so the sum is exact (barring underflow of the low terms).
-__device__ __forceinline__ void split3(float f, uint32_t &h, uint32_t &m, uint32_t &l) {
-    h = bf16_rne(f);
-    const float r1 = f - bf16_to_f32(h);
-    m = bf16_rne(r1);
-    l = bf16_rne(r1 - bf16_to_f32(m));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t bf16_pair(const f32x2_t v) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t)); }
+
+// Split two f32 into three bf16 terms hi + mid + lo each; 3 x 8 significant bits hold all 24 bits of an
+// f32, so the sums are exact (barring underflow of the low terms).
+__device__ __forceinline__ void split3(const f32x2_t f, uint32_t &h, uint32_t &m, uint32_t &l) {
+    h = bf16_pair(f);
+    const f32x2_t r1 = {f[0] - bf16_to_f32(h & 0xFFFFu), f[1] - bf16_to_f32(h >> 16)};
+    m = bf16_pair(r1);
+    l = bf16_pair(f32x2_t{r1[0] - bf16_to_f32(m & 0xFFFFu), r1[1] - bf16_to_f32(m >> 16)});
 }
 
 // Load NE (8 or 16) consecutive activations starting at element `e` as PLANES planes of NE/2 packed
@@ -49,15 +53,10 @@ __device__ __forceinline__ float load_x(const void *xg, size_t e, uint32_t (&pl)
         for (int q = 0; q < NE / 4; q++) {
             const float4 v = p[q];
             const float f[4] = {v.x, v.y, v.z, v.w};
-            uint32_t h[4], m[4], l[4];
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                split3(f[c], h[c], m[c], l[c]);
-                sum += f[c];
-            }
-            pl[0][2 * q] = h[0] | (h[1] << 16), pl[0][2 * q + 1] = h[2] | (h[3] << 16);
-            pl[1][2 * q] = m[0] | (m[1] << 16), pl[1][2 * q + 1] = m[2] | (m[3] << 16);
-            pl[2][2 * q] = l[0] | (l[1] << 16), pl[2][2 * q + 1] = l[2] | (l[3] << 16);
+            for (int c = 0; c < 4; c++) sum += f[c];
+#pragma unroll
+            for (int c = 0; c < 2; c++) split3(f32x2_t{f[2 * c], f[2 * c + 1]}, pl[0][2 * q + c], pl[1][2 * q + c], pl[2][2 * q + c]);
         }
     } else {
         const uint4 *p = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(xg) + e);
@@ -90,6 +89,26 @@ __device__ __forceinline__ void even_odd_pairs(uint32_t p0, uint32_t p1, uint32_
 template <int PLANES, bool XF32>
 __device__ __forceinline__ void stage_x_q6k(const void *xg, int spr, uint4 *xl, float4 *xs) {
     const int slots = spr * 8;
+    // Short rows in a workgroup of enough waves: a wave for each of the four groups of 64 slots, so that the conversion takes a quarter as long
+    // (us, 4096 x 2048 4.07 -> 3.92, f32 5.14 -> 4.59; 8192 x 1024 f32 5.10 -> 4.51).  Not where a wave would have a second one to wait for (1024 x 11008
+    // 7.1 -> 7.6), nor with most of its lanes idle (14000 x 768 5.0 -> 5.5).
+    const int parts = 4 * ((slots + 63) >> 6), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (slots >= 32 && parts * 64 <= (int)blockDim.x) {
+        const int g = wave & 3, slot = (wave >> 2) * 64 + (int)(threadIdx.x & 63);
+        if (wave < parts && slot < slots) {
+            uint32_t pl[3][4];
+            const float sum = load_x<XF32, 8>(xg, (size_t)(slot >> 3) * 256 + 128 * ((slot & 7) >> 2) + 8 * (slot & 3) + 32 * g, pl);
+#pragma unroll
+            for (int p = 0; p < PLANES; p++) {
+                uint4 v;
+                even_odd_pairs(pl[p][0], pl[p][1], v.x, v.y);
+                even_odd_pairs(pl[p][2], pl[p][3], v.z, v.w);
+                xl[(p * 4 + g) * slots + slot] = v;
+            }
+            reinterpret_cast<float *>(xs + slot)[g] = sum;
+        }
+        return;
+    }
     for (int slot = threadIdx.x; slot < slots; slot += blockDim.x) {
         const int s = slot >> 3, t = slot & 7;
         const int base = 128 * (t >> 2) + 8 * (t & 3);
@@ -164,6 +183,7 @@ __device__ __forceinline__ float q6k_lane(const Q6Raw &raw, const int t, const u
     return d * total;
 }
 
+// Matrices with more rows than a launch of other kinds has teams, and tall ones with rows of five super-blocks (see the launcher).
 // A team of T lanes walks two rows at a time; the two lanes' shares of the next task (the next chunk of the
 // row pair, or the first chunk of the next pair) are requested before the current one is multiplied, and the
 // first request goes out before x is converted.
@@ -223,5 +243,59 @@ __device__ __forceinline__ void q6k_small_body(const uint8_t *__restrict__ W, co
     }
 }
 
+// A team for every row (team >= n_rows: none): it asks for the first D chunks of its row before x is converted, and for chunk it + D where
+// chunk it has been used.  Any number of super-blocks a row: the lanes of the last chunk that lie past its end repeat its last super-block
+// and count for nothing.
+// What bounds it: latency.  A matrix of this size is one task of a few hundred instructions a wave, between the launch and the sum over a team; so every
+// wave of the machine takes a short row's whole work at once, and all of a row's requests go out together.  (Two rows a team, one chunk
+// ahead, had half the waves for twice the time, and multiplied a second row for nothing where there was none.  A loop over further rows behind
+// the same ring was 0.1 to 0.4 us slower at every size.)
+template <int T, bool XF32, int D>
+__device__ __forceinline__ void q6k_row_body(const uint8_t *__restrict__ W, const void *__restrict__ xg, float *__restrict__ y, int n_rows,
+                                             int spr, int team, uint4 *smem) {
+    constexpr int PLANES = XF32 ? 3 : 1;
+    constexpr int SEG = T / 8;
+    const int slots = spr * 8;
+    uint4 *xl = smem;
+    float4 *xs = reinterpret_cast<float4 *>(xl + PLANES * 4 * slots);
+    const int lt = threadIdx.x & (T - 1), t = lt & 7;
+    const int iters = (spr + SEG - 1) / SEG;
+    const uint8_t *row = W + (size_t)(team < n_rows ? team : n_rows - 1) * ((size_t)spr * 210);
+    auto block_of = [&](int it) { return min(it * SEG + (lt >> 3), spr - 1); };
+    Q6Raw c[D];
+#pragma unroll
+    for (int i = 0; i < D; i++) c[i] = q6k_load(row + (uint32_t)block_of(i) * 210u, t);
+    stage_x_q6k<PLANES, XF32>(xg, spr, xl, xs);
+    __syncthreads();
+    float acc = 0.0f;
+    for (int first = 0; first < iters; first += D) {
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            const int it = first + i;
+            if (it < iters) {
+                const int slot = block_of(it) * 8 + t;
+                const float v = q6k_lane<PLANES>(c[i], t, xl, slots, slot, xs[slot]);
+                acc += it * SEG + (lt >> 3) < spr ? v : 0.0f;
+                if (it + D < iters) c[i] = q6k_load(row + (uint32_t)block_of(it + D) * 210u, t);
+            }
+        }
+    }
+    acc = team_sum_last<T>(acc);
+    if (lt == T - 1 && team < n_rows) y[team] = acc;
+}
+
+// The workgroups of a launch that belong to a Q6_K matrix: a team for every row where there are enough, two rows a team at a time otherwise.
+template <int T, bool XF32>
+__device__ __forceinline__ void q6k_member_body(const uint8_t *__restrict__ W, const void *__restrict__ xg, float *__restrict__ y,
+                                                int n_rows, int spr, int block, int n_blocks, int teams_per_wg, uint4 *smem) {
+    if (!(XF32 && T == 8) && n_rows <= n_blocks * teams_per_wg) {  // (f32 x beside the Q4_K digits of eight-lane teams: a spill)
+        const int mine = (int)threadIdx.x / T, team = mine < teams_per_wg ? block * teams_per_wg + mine : n_rows;
+        // (a chunk ahead for f32: the digits of two kinds of x leave no registers for more)
+        if (XF32 || spr <= T / 8) q6k_row_body<T, XF32, 1>(W, xg, y, n_rows, spr, team, smem);
+        else q6k_row_body<T, XF32, 3>(W, xg, y, n_rows, spr, team, smem);
+    } else {
+        q6k_small_body<T, XF32>(W, xg, y, n_rows, spr, block, n_blocks, teams_per_wg, smem);
+    }
+}
 
 }  // namespace

@@ -47,6 +47,23 @@ def test_qgemv_matches_dequantize_then_matmul(oracle, t, n, k, x_dtype):
         assert elem <= TOL and norm <= TOL
 
 
+# A team of 1 to 64 lanes per row of Q6_K (k / 256 groups of eight lanes) or Q8_0 (k / 32 lanes): rows that no team takes whole, one, two, three and
+# more chunks, row counts around the teams of a workgroup, workgroups of 64, 128 and 256 threads, and (24577 x 1280) two rows a team.
+ROW_CASES = [(Q6K, 1, 1280), (Q6K, 255, 2304), (Q6K, 1025, 3584), (Q6K, 2049, 3072), (Q6K, 1700, 4352), (Q6K, 4097, 1280), (Q6K, 8191, 1280),
+             (Q6K, 13999, 768), (Q6K, 24577, 1280), (Q6K, 300, 11008), (Q6K, 33, 14336), (Q6K, 3073, 512),
+             (Q8_0, 1, 32), (Q8_0, 300, 32), (Q8_0, 1000, 64), (Q8_0, 77, 128), (Q8_0, 4099, 160), (Q8_0, 515, 224), (Q8_0, 9, 288),
+             (Q8_0, 8191, 1280), (Q8_0, 1025, 2080), (Q8_0, 2047, 3584), (Q8_0, 300, 11008), (Q8_0, 13999, 768)]
+
+
+@pytest.mark.parametrize("t,n,k", ROW_CASES)
+@pytest.mark.parametrize("x_dtype", [pm.DTYPE_BF16, pm.DTYPE_F32])
+def test_qgemv_rows_that_no_team_takes_whole(oracle, t, n, k, x_dtype):
+    wq = oracle.quantize(t, weights(n * 31 + k, n * k, outliers=1e-3))
+    x_dev, x_ref = activations(oracle, k, k, x_dtype)
+    elem, norm = rel_errors(gpu_qgemv(t, wq, n, k, x_dev, x_dtype, 0), oracle.qmatvec(t, wq, n, k, x_ref))
+    assert elem <= TOL and norm <= TOL
+
+
 # Shapes of 12 MiB and more take the large-matrix kernels.  Rows of one or two chunks (k = 2048, 4096) with at most
 # eight tasks per wave go to the kernel whose waves own whole rows (6001 x 4096, 12001 x 2048, 32767 x 2048: ragged row
 # counts, so the last workgroup and its waves are short); more rows than that (20000 x 4096, 40001 x 2048) and every
