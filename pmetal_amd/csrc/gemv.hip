@@ -152,25 +152,19 @@ hipError_t launch(Kern kern, unsigned grid, size_t lds, hipStream_t s, const uin
     return hipGetLastError();
 }
 
-// Lanes of a team that takes one row of `lanes` lanes' work, and threads of a workgroup.  Fitted to 40 shapes of Q6_K of 256 to 14000 rows
-// of 3 to 43 super-blocks, each with teams of 8, 16, 32 and 64 lanes: a wave costs 20 for each of its chunks, lanes past the row's end
-// included, and 5, on each of its SIMD's turns, and a chunk 15 of latency (us, 8 / 16 / 32 / 64 lanes: 1024 x 3584 9.1 / 6.0 / 4.2 / 3.6,
-// 4096 x 3584 9.6 / 7.3 / 6.9 / 6.7, 8192 x 768 4.0 / 4.4 / 3.9 / 5.6, 14000 x 768 5.0 / 6.2 / 5.6 / 7.8).
+// Lanes of a team that takes one row of `lanes` lanes' work, by team_cost, and threads of a workgroup.
 struct RowTeams {
     int team;
     unsigned threads;
 };
 RowTeams row_teams(int64_t n_rows, uint32_t lanes, size_t slots) {
-    // (32-bit: the divisions would be a tenth of a microsecond of host time a call otherwise)
     const uint32_t cus = (uint32_t)compute_units(), n = n_rows < (1 << 24) ? (uint32_t)n_rows : 1u << 24;
     RowTeams t{0, 256};
     uint32_t best = 0, whole = 0;
     for (uint32_t log = 6; log >= 3; log--) {
-        const uint32_t team = 1u << log, chunks = (lanes + team - 1) >> log;
-        const uint32_t turns = (((n + (64 >> log) - 1) >> (6 - log)) + 4 * cus - 1) / (4 * cus);
-        const uint32_t cost = turns * (20 * chunks + 5) + 15 * chunks, fits = (lanes & (team - 1)) == 0;
+        const uint32_t cost = pmh::gemv::team_cost(n, lanes, log), fits = (lanes & ((1u << log) - 1)) == 0;
         // (as long either way: the one that the row fills)
-        if (t.team == 0 || cost < best || (cost == best && fits > whole)) t.team = (int)team, best = cost, whole = fits;
+        if (t.team == 0 || cost < best || (cost == best && fits > whole)) t.team = 1 << log, best = cost, whole = fits;
     }
     // Smaller workgroups where they spread the waves more evenly and one of them converts x in one go (us, 3072 x 1536: 192 workgroups of
     // 256 threads 3.9 us, 768 of 64 3.7; 2048 x 1280 4.8, 3.9).

@@ -78,6 +78,16 @@ inline int pow2_divisor(int64_t v, int cap) {
 
 using pmh::compute_units;
 
+// What a matrix of n rows of `lanes` lanes' work costs in teams of 2^log lanes: a wave costs 20 for each of its chunks of a row, lanes past the
+// row's end included, and 5, on each of its SIMD's turns, and a chunk 15 of latency.  Fitted to 40 shapes of Q6_K of 256 to 14000 rows of 3 to 43
+// super-blocks with teams of 8, 16, 32 and 64 lanes (us: 1024 x 3584 9.1 / 6.0 / 4.2 / 3.6, 4096 x 3584 9.6 / 7.3 / 6.9 / 6.7, 8192 x 768
+// 4.0 / 4.4 / 3.9 / 5.6, 14000 x 768 5.0 / 6.2 / 5.6 / 7.8).  (32-bit: the divisions would be a tenth of a microsecond of host time a call otherwise.)
+inline uint32_t team_cost(int64_t n_rows, uint32_t lanes, uint32_t log) {
+    const uint32_t simds = 4 * (uint32_t)compute_units(), n = n_rows < (1 << 24) ? (uint32_t)n_rows : 1u << 24;
+    const uint32_t chunks = (lanes + (1u << log) - 1) >> log, turns = (((n + (64 >> log) - 1) >> (6 - log)) + simds - 1) / simds;
+    return turns * (20 * chunks + 5) + 15 * chunks;
+}
+
 }  // namespace gemv
 
 }  // namespace pmh

@@ -565,7 +565,8 @@ struct GemvGroup {
 // -amdgpu-kernarg-preload-count=16), so the first weight request does not wait for an argument fetch.
 // Q6LAST: the fourth member is a Q6_K matrix (the v projection of a layer whose q and k are Q4_K): the workgroups from
 // wg_b3 on run the small-matrix Q6_K GEMV over it, with q6_teams teams of T lanes each taking rows.
-template <int ORDER, bool XF32, int T, bool Q6LAST>
+// RAGGED: T lanes do not take a row whole; those of its last chunk that lie past its end repeat its last super-block and count for nothing.
+template <int ORDER, bool XF32, int T, bool Q6LAST, bool RAGGED = false>
 __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg, const uint8_t *__restrict__ w0,
                                                      const uint8_t *__restrict__ w1, const uint8_t *__restrict__ w2,
                                                      const uint8_t *__restrict__ w3, int wg_b1, int wg_b2, int wg_b3,
@@ -595,7 +596,7 @@ __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg,
     const int lane = threadIdx.x & 63;
     const int lt = lane & (T - 1);
     const int j = lane & 7;
-    const int iters = spr / SEG;  // tasks per row
+    const int iters = RAGGED ? (spr + SEG - 1) / SEG : spr / SEG;  // tasks per row
     constexpr int kTeamsPerWave = 64 / T;
     // with full-wave teams everything about a team is wave-uniform: keep it in scalar registers
     auto uni = [](int v) { return T == 64 ? __builtin_amdgcn_readfirstlane(v) : v; };
@@ -610,8 +611,16 @@ __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg,
     const int n_nominal = per_team * iters;               // workgroup-uniform upper bound
 
     // A team's tasks are one linear stream: task t of the team starts STRIDE * t bytes after its first.
-    const uint8_t *ph = W + (size_t)(n_tasks > 0 ? r0 : 0) * spr * 144 + (size_t)(lt >> 3) * 144;
+    // (RAGGED: ph is the row of the next request, task lit of it)
+    const uint8_t *ph = W + (size_t)(n_tasks > 0 ? r0 : 0) * spr * 144 + (RAGGED ? 0 : (size_t)(lt >> 3) * 144);
     const uint8_t *pq = ph + 16 + 16 * j;
+    int lit = 0;
+    auto block_of = [&](int i) { return min(i * SEG + (lt >> 3), spr - 1); };
+    auto request = [&](uint4 &h, uint4 &q) {
+        const uint8_t *blk = ph + (uint32_t)block_of(lit) * 144u;
+        h = *reinterpret_cast<const uint4 *>(blk), q = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * j);
+        if (++lit == iters) lit = 0, ph += (size_t)spr * 144;
+    };
 
     // kRing tasks are in flight per team.  They are requested before x is converted, so the memory system
     // streams while the staging runs, and each buffer is refilled as soon as it has been consumed.
@@ -621,8 +630,12 @@ __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg,
 #pragma unroll
     for (int i = 0; i < kRing; i++) {
         if (i < n_tasks) {
-            bh[i] = *reinterpret_cast<const uint4 *>(ph + i * STRIDE);
-            bq[i] = *reinterpret_cast<const uint4 *>(pq + i * STRIDE);
+            if constexpr (RAGGED) {
+                request(bh[i], bq[i]);
+            } else {
+                bh[i] = *reinterpret_cast<const uint4 *>(ph + i * STRIDE);
+                bq[i] = *reinterpret_cast<const uint4 *>(pq + i * STRIDE);
+            }
         }
     }
     stage_x_finish<ORDER, NDIG, XF32>(xg, slots, nthreads, x_lo, x_hi, xd, xm, slots);
@@ -639,15 +652,20 @@ __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg,
             if (first + i < n_nominal) {
                 const bool valid = first + i < n_tasks;
                 if (valid) {
-                    const int slot = it * T + lt;
+                    const int slot = RAGGED ? block_of(it) * 8 + j : it * T + lt;
                     uint4 xdig[NDIG];
 #pragma unroll
                     for (int k = 0; k < NDIG; k++) xdig[k] = xd[k * slots + slot];
-                    acc += lane_dot<ORDER, NDIG>(bh[i], bq[i], s0, s1, xdig, xm[slot]);
+                    const float v = lane_dot<ORDER, NDIG>(bh[i], bq[i], s0, s1, xdig, xm[slot]);
+                    acc += !RAGGED || it * SEG + (lt >> 3) < spr ? v : 0.0f;
                 }
                 if (first + i + kRing < n_tasks) {  // refill this buffer with the task kRing ahead
-                    bh[i] = *reinterpret_cast<const uint4 *>(ph + (size_t)(i + kRing) * STRIDE);
-                    bq[i] = *reinterpret_cast<const uint4 *>(pq + (size_t)(i + kRing) * STRIDE);
+                    if constexpr (RAGGED) {
+                        request(bh[i], bq[i]);
+                    } else {
+                        bh[i] = *reinterpret_cast<const uint4 *>(ph + (size_t)(i + kRing) * STRIDE);
+                        bq[i] = *reinterpret_cast<const uint4 *>(pq + (size_t)(i + kRing) * STRIDE);
+                    }
                 }
                 if (++it == iters) {
                     const float total = team_sum_last<T>(acc);
@@ -658,8 +676,7 @@ __global__ __launch_bounds__(1024) void k_qgemv_q4k(const void *__restrict__ xg,
                 }
             }
         }
-        ph += kRing * STRIDE;
-        pq += kRing * STRIDE;
+        if (!RAGGED) ph += kRing * STRIDE, pq += kRing * STRIDE;
     }
 }
 
@@ -722,6 +739,13 @@ hipError_t launch_general(int T, dim3 grid, dim3 block, size_t lds, hipStream_t 
         case 16: return go(k_qgemv_q4k<ORDER, XF32, 16, true>);
         case 32: return go(k_qgemv_q4k<ORDER, XF32, 32, true>);
         default: return go(k_qgemv_q4k<ORDER, XF32, 64, true>);
+        }
+    }
+    if (spr % (T / 8) != 0) {
+        switch (T) {
+        case 16: return go(k_qgemv_q4k<ORDER, XF32, 16, false, true>);
+        case 32: return go(k_qgemv_q4k<ORDER, XF32, 32, false, true>);
+        default: return go(k_qgemv_q4k<ORDER, XF32, 64, false, true>);
         }
     }
     switch (T) {
@@ -798,12 +822,18 @@ hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *
 hipError_t launch_group_general(const uint8_t *const *w, const int64_t *n, float *const *y, int count, int64_t k,
                                 const void *x, bool xf32, uint32_t order, hipStream_t s) {
     const int spr = (int)(k / 256);
-    const int T = 8 * pow2_divisor(spr, 8);
     const size_t slots = (size_t)spr * 8;
     const size_t lds_x = slots * 16 * (xf32 ? 6 : 5) + slots * 16;
     if (lds_x > kMaxLds) return hipErrorInvalidValue;
     int64_t total = 0;
     for (int i = 0; i < count; i++) total += n[i];
+    // The widest team that takes a row whole, or a wider one whose last chunk of a row is short where that is less work in a line (us, such a
+    // team / the cheapest: 1024 x 1280 3.6 / 2.9, 4096 x 2304 5.7 / 4.4, 2048 x 3584 4.7 / 3.8, 1024 x 4352 9.9 / 3.7, 1024 x 11008 25.6 / 5.2;
+    // 14000 x 768, where it is not, 4.2 / 4.5).
+    int log_t = 3 + (spr % 2 == 0) + (spr % 4 == 0) + (spr % 8 == 0);
+    for (int log = 6, whole = log_t; log > whole; log--)
+        if (team_cost(total, (uint32_t)slots, log) < team_cost(total, (uint32_t)slots, log_t)) log_t = log;
+    const int T = 1 << log_t;
     const int64_t want = compute_units();
     int64_t n_wg = total < want ? total : want;
     int64_t rows_per_wg = (total + n_wg - 1) / n_wg;
