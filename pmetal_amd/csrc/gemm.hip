@@ -1267,9 +1267,9 @@ __device__ __forceinline__ void small_store(const float4_t *out_tiles, int t0, i
 // two runs of four elements each, of row lane % 16, where the pre-pass's order of the same number puts them.  The power of two that
 // takes a row into [2^9, 2^10) is that of the wave's part of it and not of the whole row: its inverse multiplies the wave's tiles,
 // exactly, before they are added, so nothing is rounded that a pre-pass would not round.
-// Measured (us a call, M = 16, from memory, with a pre-pass in front -> so): bf16 14336 x 4096 Q4_K 14.9 -> 13.3, Q5_K 16.5 -> 15.9,
-// Q6_K 18.3 -> 17.6, Q8_0 18.9 -> 18.4, Q2_K 14.5 -> 13.3; f32 14336 x 4096 Q4_K 14.7 -> 14.2; 4096 x 14336 18.8 -> 16.1.  1.13 times as
-// fast over 42 shapes of 1 to 16 rows.
+// Measured (us a call, weights from memory, with a pre-pass in front -> so): 14336 x 4096, M = 10, bf16 Q4_K 14.5 -> 12.8, Q5_K 16.1 -> 15.3, Q6_K
+// 18.0 -> 17.3, Q8_0 18.3 -> 18.1, Q3_K 17.9 -> 17.5, Q2_K 14.2 -> 12.9; M = 16, f32 Q4_K 14.7 -> 14.2; 4096 x 14336, M = 12, f32 Q4_K 18.8 -> 16.1,
+// Q6_K 22.4 -> 19.7.  1.13 times as fast over 42 shapes of 1 to 16 rows.
 // ------------------------------------------------------------------------------------------------
 constexpr int kSmallXItems = 512;  // 16-byte items of LDS for a super-block of 16 rows in bf16; f32: twice as many
 template <bool XF32, int ORDER, int NSB>

@@ -733,6 +733,13 @@ hipError_t launch_general(int T, dim3 grid, dim3 block, size_t lds, hipStream_t 
                                grp.wg_begin[2], grp.wg_begin[3], spr, rows_per_wg, per_team, grp.n[0], grp.n[1], grp.n[2],
                                grp.n[3], grp.y[0], grp.y[1], grp.y[2], grp.y[3], (int)block.x, q6_teams);
     };
+    if (q6_teams > 0 && spr % (T / 8) != 0) {
+        switch (T) {
+        case 16: return go(k_qgemv_q4k<ORDER, XF32, 16, true, true>);
+        case 32: return go(k_qgemv_q4k<ORDER, XF32, 32, true, true>);
+        default: return go(k_qgemv_q4k<ORDER, XF32, 64, true, true>);
+        }
+    }
     if (q6_teams > 0) {
         switch (T) {
         case 8: return go(k_qgemv_q4k<ORDER, XF32, 8, true>);
@@ -756,12 +763,23 @@ hipError_t launch_general(int T, dim3 grid, dim3 block, size_t lds, hipStream_t 
     }
 }
 
+// log2 of the lanes of kernel B's teams: the widest team that takes a row whole, or a wider one whose last chunk of a row is short where that is less work
+// in a line (us, such a team / the cheapest: 1024 x 1280 3.6 / 2.9, 4096 x 2304 5.7 / 4.4, 2048 x 3584 4.7 / 3.8, 1024 x 4352 9.9 / 3.7, 1024 x 11008
+// 25.6 / 5.2; 14000 x 768, where it is not, 4.2 / 4.5).
+int whole_team(int spr) { return 3 + (spr % 2 == 0) + (spr % 4 == 0) + (spr % 8 == 0); }
+int cheapest_team(int64_t rows, int spr) {
+    const int whole = whole_team(spr);
+    int best = whole;
+    for (int log = 6; log > whole; log--)
+        if (team_cost(rows, 8u * (uint32_t)spr, log) < team_cost(rows, 8u * (uint32_t)spr, best)) best = log;
+    return best;
+}
+
 // One to three small Q4_K matrices and one small Q6_K matrix that share k and x in one launch of kernel B: the workgroups
 // are divided between the two kinds by their bytes.
 hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *const *y, int count, const uint8_t *w6, int64_t n6,
                               float *y6, int64_t k, const void *x, bool xf32, uint32_t order, hipStream_t s) {
     const int spr = (int)(k / 256);
-    const int T = 8 * pow2_divisor(spr, 8);
     const size_t slots = (size_t)spr * 8;
     const size_t lds4 = slots * 16 * (xf32 ? 6 : 5) + slots * 16, lds6 = slots * 64 * (xf32 ? 3 : 1) + slots * 16;
     const size_t lds = lds4 > lds6 ? lds4 : lds6;
@@ -796,16 +814,20 @@ hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *
     grp.wg_begin[3] = begin;  // the Q6_K member starts here
     grp.w[3] = w6, grp.y[3] = y6, grp.n[3] = (int)n6;
     const dim3 grid((unsigned)(begin + wgs6));
-    const int teams_per_wave = 64 / T;
     const int64_t rows6 = (n6 + wgs6 - 1) / wgs6;  // rows of a Q6_K workgroup: one per team, or two at a time where that is not enough
-    int best_waves = 16;
-    int64_t best_cost = INT64_MAX;
-    for (int waves = 16; waves >= 1; waves--) {  // as in launch_group_general
-        const int64_t teams = (int64_t)waves * teams_per_wave;
-        const int64_t per_team = (rows_per_wg + teams - 1) / teams;
-        if (per_team < best_cost) best_cost = per_team, best_waves = waves;
+    int best_waves = 16, log_t = cheapest_team(total + n6, spr);
+    int64_t teams_avail;
+    for (;; log_t = whole_team(spr)) {
+        int64_t best_cost = INT64_MAX;
+        for (int waves = 16; waves >= 1; waves--) {  // as in launch_group_general
+            const int64_t teams = (int64_t)waves * (64 >> log_t);
+            const int64_t per_team = (rows_per_wg + teams - 1) / teams;
+            if (per_team < best_cost) best_cost = per_team, best_waves = waves;
+        }
+        teams_avail = (int64_t)best_waves * (64 >> log_t);
+        if (rows6 <= teams_avail || log_t == whole_team(spr)) break;  // (two rows of Q6_K at a time only where the teams take a row whole)
     }
-    const int64_t teams_avail = (int64_t)best_waves * teams_per_wave;
+    const int T = 1 << log_t;
     int64_t q6_teams = rows6 <= teams_avail ? rows6 : (rows6 + 1) / 2;
     q6_teams = q6_teams > teams_avail ? teams_avail : q6_teams;
     const int per_team = (int)((rows_per_wg + teams_avail - 1) / teams_avail);
@@ -827,13 +849,7 @@ hipError_t launch_group_general(const uint8_t *const *w, const int64_t *n, float
     if (lds_x > kMaxLds) return hipErrorInvalidValue;
     int64_t total = 0;
     for (int i = 0; i < count; i++) total += n[i];
-    // The widest team that takes a row whole, or a wider one whose last chunk of a row is short where that is less work in a line (us, such a
-    // team / the cheapest: 1024 x 1280 3.6 / 2.9, 4096 x 2304 5.7 / 4.4, 2048 x 3584 4.7 / 3.8, 1024 x 4352 9.9 / 3.7, 1024 x 11008 25.6 / 5.2;
-    // 14000 x 768, where it is not, 4.2 / 4.5).
-    int log_t = 3 + (spr % 2 == 0) + (spr % 4 == 0) + (spr % 8 == 0);
-    for (int log = 6, whole = log_t; log > whole; log--)
-        if (team_cost(total, (uint32_t)slots, log) < team_cost(total, (uint32_t)slots, log_t)) log_t = log;
-    const int T = 1 << log_t;
+    const int T = 1 << cheapest_team(total, spr);
     const int64_t want = compute_units();
     int64_t n_wg = total < want ? total : want;
     int64_t rows_per_wg = (total + n_wg - 1) / n_wg;

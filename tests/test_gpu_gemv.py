@@ -330,8 +330,8 @@ def test_qgemv_batch_groups_that_are_large_as_a_whole(oracle, order, k, x_dtype)
         assert np.abs(got - single).max() <= 2e-6 * np.abs(single).max()
 
 
-@pytest.mark.parametrize("k,x_dtype", [(1024, pm.DTYPE_BF16), (2048, pm.DTYPE_F32), (768, pm.DTYPE_BF16)])
-@pytest.mark.parametrize("rows", [[2048, 1024, 1024], [517, 300], [1024, 1000, 37, 96], [2048, 1024, 1024, 1024]])
+@pytest.mark.parametrize("k,x_dtype", [(1024, pm.DTYPE_BF16), (2048, pm.DTYPE_F32), (768, pm.DTYPE_BF16), (3584, pm.DTYPE_BF16), (1280, pm.DTYPE_F32)])
+@pytest.mark.parametrize("rows", [[2048, 1024, 1024], [517, 300], [1024, 1000, 37, 96], [2048, 1024, 1024, 1024], [300, 9001]])
 @pytest.mark.parametrize("order", [0, 1])
 def test_qgemv_batch_takes_a_q6k_projection_into_a_q4k_group(oracle, order, rows, k, x_dtype):
     """q and k in Q4_K followed by v in Q6_K over the same x (a Q4_K_M layer): one launch.  The last of `rows` is the
