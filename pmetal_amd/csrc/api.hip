@@ -1091,8 +1091,9 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
     };
     // what a launch's converted activations look like: their layout, per row or (at most 16 rows) per pair of super-blocks
     auto form = [&](const pmetal_hip_gemm_desc &d, const pmh::GemmPlan &p) { return layout(d) + (pmh::qgemm_small_rows(p, m) ? 6 : 0); };
+    // (counted only where kernels convert themselves, at most 16 rows: a plan is host time)
     int launches[12] = {};  // of each form
-    for (size_t i = 0; i < count; i += pair_at(i) ? 2 : 1) launches[form(descs[i], pmh::qgemm_plan(m, descs[i].n, k, descs[i].ggml_type))]++;
+    for (size_t i = 0; m <= 16 && i < count; i += pair_at(i) ? 2 : 1) launches[form(descs[i], pmh::qgemm_plan(m, descs[i].n, k, descs[i].ggml_type))]++;
     for (size_t i = 0; i < count; i++) {
         const pmetal_hip_gemm_desc &d = descs[i];
         const pmh::GemmPlan one = pmh::qgemm_plan(m, d.n, k, d.ggml_type);
