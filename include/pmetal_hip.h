@@ -227,8 +227,10 @@ int32_t pmetal_hip_qlinear(uint32_t ggml_type, const uint8_t *w_dev, int64_t n, 
 /* Several weights against the same [m, k] activations (the gate / up or q / k / v projections of a prefill: what a layer's
  * consecutive LayerWeight::matmul_from calls on one input amount to, weights.rs:66-84): the same results as one
  * pmetal_hip_qgemm per weight, bit for bit, with the activations converted once per element order instead of once per
- * weight.  The weights may differ in type, n, output type and element order (Q4_K and Q5_K weights in the GGML order share
- * one conversion, Q3_K and Q2_K weights another).                                                                       */
+ * weight (up to 16 rows, where that is as fast, by every launch for itself).  The weights may differ in type, n, output type
+ * and element order (Q4_K and Q5_K weights in the GGML order share one conversion, Q3_K and Q2_K weights another).
+ * Results may lie over the activations: weights that follow one another and would share one conversion are all multiplied
+ * by the activations as they were before the first of them, a later one by what is there then.                         */
 typedef struct pmetal_hip_gemm_desc {
     uint32_t ggml_type;
     uint32_t y_dtype;

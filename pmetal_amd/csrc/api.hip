@@ -1060,8 +1060,6 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
         need = b > need ? b : need;
     }
     if (count == 0) return ok();
-    void *ws = nullptr;
-    if (int32_t rc = workspace(need, (hipStream_t)stream, &ws)) return rc;
     // the converted activations depend on the weight type and element order only through the order they are laid out in
     auto layout = [](const pmetal_hip_gemm_desc &d) {
         if (d.ggml_type == PMETAL_GGML_TYPE_Q8_0) return 3;
@@ -1094,11 +1092,44 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
     // (counted only where kernels convert themselves, at most 16 rows: a plan is host time)
     int launches[12] = {};  // of each form
     for (size_t i = 0; m <= 16 && i < count; i += pair_at(i) ? 2 : 1) launches[form(descs[i], pmh::qgemm_plan(m, descs[i].n, k, descs[i].ggml_type))]++;
+    // Results over the activations: weights that follow one another in one layout are all multiplied by the activations as they were
+    // before the first of them.  A pre-pass that they share sees to that; where a launch converts for itself whatever others do, or
+    // launches of one layout need two forms of them, the activations are set aside first.  Where every launch converts for itself
+    // nothing else uses the workspace, so that what a recording finds there is enough.
+    const size_t x_bytes = (size_t)m * k * (x_dtype == PMETAL_HIP_DTYPE_F32 ? 4 : 2);
+    auto over_x = [&](const pmetal_hip_gemm_desc &d) {
+        const uintptr_t y = (uintptr_t)d.y_dev, xb = (uintptr_t)x;
+        return y < xb + x_bytes && xb < y + (size_t)m * d.n * (d.y_dtype == PMETAL_HIP_DTYPE_F32 ? 4 : 2);
+    };
+    bool over = false, aside = false;
+    for (size_t i = 0; m <= 16 && i < count; i++) over = over || over_x(descs[i]);
+    size_t aside_at = 0;
+    if (over) {
+        bool own = false, all_own = true, two_forms = false;
+        int before = -1, before_form = -1;
+        for (size_t i = 0; i < count; i++) {
+            const pmh::GemmPlan p = pmh::qgemm_plan(m, descs[i].n, k, descs[i].ggml_type);
+            const bool o = pmh::qgemm_converts_itself(p, descs[i].ggml_type, m, k, x_dtype, true);
+            own = own || o, all_own = all_own && o;
+            two_forms = two_forms || (layout(descs[i]) == before && form(descs[i], p) != before_form);
+            before = layout(descs[i]), before_form = form(descs[i], p);
+        }
+        aside = own || two_forms;
+        if (aside && !all_own) aside_at = up16(need), need = aside_at + x_bytes;
+    }
+    void *ws = nullptr;
+    if (int32_t rc = workspace(need, (hipStream_t)stream, &ws)) return rc;
+    const void *const given = x;
     for (size_t i = 0; i < count; i++) {
         const pmetal_hip_gemm_desc &d = descs[i];
         const pmh::GemmPlan one = pmh::qgemm_plan(m, d.n, k, d.ggml_type);
         const int want = form(d, one), want_mp = one.mp;
-        const bool shared = launches[want] > 1;
+        const bool shared = over || launches[want] > 1;
+        if (aside && (i == 0 || layout(descs[i - 1]) != layout(d))) {
+            x = (const uint8_t *)ws + aside_at;
+            const hipError_t e = pmh::launch_copy_x(given, x_bytes, (uint8_t *)ws + aside_at, (hipStream_t)stream);
+            if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
+        }
         pmh::GemmSecond second{};
         if (pair_at(i)) {
             second.w = (const uint8_t *)descs[i + 1].w_dev, second.y = descs[i + 1].y_dev, second.n = (int)descs[i + 1].n;

@@ -2633,6 +2633,12 @@ static hipError_t launch_rw_q8(hipStream_t s, const uint8_t *w, const uint4 *xs,
     return hipGetLastError();
 }
 
+hipError_t launch_copy_x(const void *x, size_t bytes, void *to, hipStream_t s) {
+    const size_t items = bytes / 16;  // (whole super-blocks)
+    hipLaunchKernelGGL(k_copy16, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, reinterpret_cast<const uint4 *>(x), reinterpret_cast<uint4 *>(to), items);
+    return hipGetLastError();
+}
+
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,
                                 int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s, bool reuse_prepass,
                                 const GemmSecond &second_weight, bool shared) {
@@ -2685,8 +2691,8 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             return b < xe && xb < b + (size_t)m * rows * (y_dtype == kDtypeF32 ? 4 : 2);
         };
         if (over_x(y, n) || (second.n > 0 && over_x(second.y, second.n))) {  // (16 f32 rows are what 32 rows of items take)
-            const size_t items = (xe - xb) / 16;
-            hipLaunchKernelGGL(k_copy16, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, reinterpret_cast<const uint4 *>(x), xs, items);
+            const hipError_t e = launch_copy_x(x, xe - xb, xs, s);
+            if (e != hipSuccess) return e;
             x = xs;
         }
     } else if (reuse_prepass) {

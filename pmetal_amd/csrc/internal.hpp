@@ -112,6 +112,8 @@ bool qgemm_small_rows(const GemmPlan &plan, int64_t m);
 // Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.  shared: another
 // launch could use the converted ones.
 bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype, bool shared);
+// `bytes` of activations, a multiple of 16, to where results that lie over them do not reach
+hipError_t launch_copy_x(const void *x, size_t bytes, void *to, hipStream_t s);
 // reuse_prepass: the workspace still holds the converted activations of the previous launch_qgemm on this stream with the same
 // x, m, k and weight type (two weights that share their activations: the pre-pass runs once)
 hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype,

@@ -345,3 +345,36 @@ def test_batches_of_kernels_with_and_without_a_pre_pass(oracle, x_dtype):
         pm.check(lib.pmetal_hip_sync(None))
         for i, (a, b) in enumerate(zip(ys, ones)):
             assert np.array_equal(a.to_host(np.uint8), b.to_host(np.uint8)), (m, k, i)
+
+
+# A batch whose first results lie over its activations: weights that follow one another in one layout are all multiplied by the activations
+# as they were before the first of them, whoever converts them (rows of at most eight super-blocks: every launch; longer: one
+# launch for all of a form, or two forms of one layout), the next layout by what is there then.  Bit for bit as calls of their own over copies.
+@pytest.mark.parametrize("m,k,specs", [(16, 2048, [(Q4K, 300), (Q4K, 500), (Q4K, 70)]), (5, 512, [(Q8_0, 33), (Q8_0, 33), (Q8_0, 100), (Q8_0, 4)]),
+                                       (9, 1280, [(Q6K, 200), (Q6K, 40), (11, 50), (10, 60), (Q6K, 70)]), (16, 4096, [(Q4K, 300), (Q4K, 500), (Q4K, 70), (13, 90)]),
+                                       (7, 3840, [(11, 40), (11, 50), (10, 60)]), (12, 2304, [(Q4K, 300), (Q4K, 9000), (Q4K, 400), (Q8_0, 9000), (Q8_0, 300)]),
+                                       (3, 5120, [(Q6K, 14400), (Q6K, 300), (Q6K, 14500)]), (20, 1024, [(Q4K, 300), (Q4K, 500), (Q4K, 70)])])
+@pytest.mark.parametrize("dtype,size", [(pm.DTYPE_F32, 4), (pm.DTYPE_BF16, 2)])
+def test_batches_write_over_their_activations(oracle, m, k, specs, dtype, size):
+    rng = np.random.default_rng(m + k)
+    lib = _lib.load()
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    values = np.ascontiguousarray(x if dtype == pm.DTYPE_F32 else oracle.f32_to_bf16_bits(x.reshape(-1)))
+    ws = [pm.DeviceBuffer.from_host(random_blocks(rng, t, n, k)) for t, n in specs]
+    layouts = [10 if t == 11 else t for t, _ in specs]  # (in the order of the reference Q4_K and Q5_K have layouts of their own)
+    x_bytes = m * k * size
+    for at in (0, 256):
+        both = [pm.DeviceBuffer(max(x_bytes, at + m * specs[0][1] * size)) for _ in range(2)]
+        for b in both:
+            pm.check(lib.pmetal_hip_h2d(b.ptr, values.ctypes.data, x_bytes))
+        outs = [[pm.DeviceBuffer(m * n * size) for _, n in specs[1:]] for _ in range(2)]
+        descs = [_lib.GemmDesc(t, dtype, 0, 0, n, w.ptr, both[0].ptr + at if i == 0 else outs[0][i - 1].ptr) for i, ((t, n), w) in enumerate(zip(specs, ws))]
+        pm.check(lib.pmetal_hip_qgemm_batch((_lib.GemmDesc * len(specs))(*descs), len(specs), k, both[0].ptr, dtype, m, None))
+        for i, ((t, n), w) in enumerate(zip(specs, ws)):
+            if i == 0 or layouts[i] != layouts[i - 1]:
+                pm.check(lib.pmetal_hip_sync(None))
+                given = pm.DeviceBuffer.from_host(both[1].to_host(np.uint8)[:x_bytes])
+            pm.check(lib.pmetal_hip_qgemm(t, w.ptr, n, k, given.ptr, dtype, m, both[1].ptr + at if i == 0 else outs[1][i - 1].ptr, dtype, 0, None))
+        pm.check(lib.pmetal_hip_sync(None))
+        for i, (a, b) in enumerate(zip([both[0]] + outs[0], [both[1]] + outs[1])):
+            assert np.array_equal(a.to_host(np.uint8), b.to_host(np.uint8)), (at, i)
