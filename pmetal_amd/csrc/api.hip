@@ -961,7 +961,16 @@ static int32_t qgemm_over_reblocked(uint32_t t, const uint8_t *wa, int64_t n, in
     const bool y_f32 = y_dtype == PMETAL_HIP_DTYPE_F32;
     const uint8_t *wb = wa + reblocked_part_bytes(n, k);
     float *yb = (float *)(scratch + gemm_bytes), *ya = y_f32 ? (float *)y : (float *)((uint8_t *)yb + y_bytes);
-    hipError_t e;
+    hipError_t e = hipSuccess;
+    if (parts == 2 && y_f32 && pmh::qgemm_converts_itself(pmh::qgemm_plan(m, n, k, PMETAL_GGML_TYPE_Q6K), PMETAL_GGML_TYPE_Q6K, m, k, x_dtype, true)) {
+        // both products convert x for themselves: a first one that lies over it must not be what the second one reads
+        const size_t x_bytes = (size_t)m * k * (x_dtype == PMETAL_HIP_DTYPE_F32 ? 4 : 2);
+        if ((uintptr_t)y < (uintptr_t)x + x_bytes && (uintptr_t)x < (uintptr_t)y + y_elems * 4) {
+            e = pmh::launch_copy_x(x, x_bytes, scratch, s);  // (these launches leave the scratch for converted activations alone)
+            x = scratch;
+        }
+    }
+    if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
     if (parts == 1) {
         e = pmh::launch_qgemm(PMETAL_GGML_TYPE_Q6K, wa, n, k, x, x_dtype, m, y, y_dtype, 0, scratch, s);
     } else {  // the second product reuses the first one's converted activations

@@ -378,3 +378,24 @@ def test_batches_write_over_their_activations(oracle, m, k, specs, dtype, size):
         pm.check(lib.pmetal_hip_sync(None))
         for i, (a, b) in enumerate(zip([both[0]] + outs[0], [both[1]] + outs[1])):
             assert np.array_equal(a.to_host(np.uint8), b.to_host(np.uint8)), (at, i)
+
+
+# A re-blocked weight of two parts multiplies twice; its f32 results over the activations are those that lie apart from them.
+@pytest.mark.parametrize("m,n,k", [(16, 2048, 2048), (3, 40, 256), (7, 500, 1280), (16, 600, 2304), (9, 300, 4096), (20, 300, 1024)])
+@pytest.mark.parametrize("t", [13, 11, 10])
+@pytest.mark.parametrize("dtype,size", [(pm.DTYPE_F32, 4), (pm.DTYPE_BF16, 2)])
+def test_reblocked_weights_write_over_their_activations(oracle, t, m, n, k, dtype, size):
+    rng = np.random.default_rng(t + m + k)
+    lib = _lib.load()
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    values = np.ascontiguousarray(x if dtype == pm.DTYPE_F32 else oracle.f32_to_bf16_bits(x.reshape(-1)))
+    dw, parts = pm.DeviceBuffer.from_host(random_blocks(rng, t, n, k)), lib.pmetal_hip_reblock_size(t, n, k)
+    dr, dx, dy = pm.DeviceBuffer(parts), pm.DeviceBuffer.from_host(values), pm.DeviceBuffer(m * n * 4)
+    pm.check(lib.pmetal_hip_reblock_dev(t, dw.ptr, n, k, 0, dr.ptr, parts, None))
+    pm.check(lib.pmetal_hip_qgemm_reblocked(t, dr.ptr, parts, n, k, dx.ptr, dtype, m, dy.ptr, pm.DTYPE_F32, None))
+    both = pm.DeviceBuffer(max(m * k * size, m * n * 4) + 256)
+    for at in (0, 256):
+        pm.check(lib.pmetal_hip_h2d(both.ptr, values.ctypes.data, m * k * size))
+        pm.check(lib.pmetal_hip_qgemm_reblocked(t, dr.ptr, parts, n, k, both.ptr, dtype, m, both.ptr + at, pm.DTYPE_F32, None))
+        pm.check(lib.pmetal_hip_sync(None))
+        assert np.array_equal(both.to_host(np.uint8)[at:at + m * n * 4], dy.to_host(np.uint8)), at
