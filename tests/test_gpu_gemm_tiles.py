@@ -399,3 +399,31 @@ def test_reblocked_weights_write_over_their_activations(oracle, t, m, n, k, dtyp
         pm.check(lib.pmetal_hip_qgemm_reblocked(t, dr.ptr, parts, n, k, both.ptr, dtype, m, both.ptr + at, pm.DTYPE_F32, None))
         pm.check(lib.pmetal_hip_sync(None))
         assert np.array_equal(both.to_host(np.uint8)[at:at + m * n * 4], dy.to_host(np.uint8)), at
+
+
+# An infinity among ordinary activations of up to 16 rows: the results of its row are infinite, with the sign of its weight (a weight of 0:
+# NaN), and the others as ever.  It shares a word with an element far larger than the others, in the upper half of it or in the lower:
+# that one may not be overlooked for the row's largest magnitude, or it would overflow to the other infinity.  (Types without a
+# min term: the sums that those multiply are NaN.)
+@pytest.mark.parametrize("k", [256, 2048, 3328])
+@pytest.mark.parametrize("t", [Q8_0, Q6K])
+@pytest.mark.parametrize("dtype", [pm.DTYPE_BF16, pm.DTYPE_F32])
+def test_short_batches_with_infinities(oracle, t, k, dtype):
+    m, n = 16, 24
+    assert gemm_plan(t, m, n, k).kernel == SMALL
+    rng = np.random.default_rng(t + k)
+    raw = random_blocks(rng, t, n, k)
+    x = (rng.standard_normal((m, k)) * 1e-3).astype(np.float32)
+    for r in range(15):  # (the last row has none)
+        at = 2 * rng.integers(k // 2)
+        x[r, at + r % 2], x[r, at + 1 - r % 2] = -3e4 * (-1.0) ** (r // 2), np.inf * (-1.0) ** (r // 2)
+    bits = oracle.f32_to_bf16_bits(x.reshape(-1)).reshape(m, k)
+    x = oracle.bf16_bits_to_f32(bits.reshape(-1)).reshape(m, k)
+    got = gpu_qgemm(t, raw, n, k, bits if dtype == pm.DTYPE_BF16 else x, m, x_dtype=dtype)
+    w = oracle.dequantize(t, raw, [n, k]).reshape(n, k).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.T
+    assert np.isfinite(want[15]).all() and np.isinf(want[:15]).sum() > 100
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    assert np.max(np.abs(got[15] - want[15])) <= bound(k) * np.max(np.abs(want[15]))
