@@ -1194,22 +1194,26 @@ constexpr int kSmallMaxM2 = 32;  // Q4_K, Q5_K and Q8_0: two 16-row blocks of ac
 // next tile writes the other buffer; the one after that comes behind the next barrier).
 //
 // A workgroup with few tiles (at most kSmallKeepTiles) keeps every wave's partial tile of every row tile instead
-// (`keep`, [tile][wave][lane]) and adds them after the last one, in the same wave order: its waves then meet at one
+// ([tile][wave][lane]) and adds them after the last one, in the same wave order: its waves then meet at one
 // barrier, not at one per tile.
+// `red`, `keep`, behind the finished tiles: two buffers of a partial tile per wave, or those.  (All of it in dynamic LDS and as long as the
+// workgroup's waves need: with the buffers of eight waves beside what activations pass through before the first tile, fewer workgroups of
+// rows of one to four super-blocks fit a compute unit than the launch counts on, and the last ones of a round waited for the others:
+// f32, three Q4_K weights of 24737 x 256, M = 9, 20.0 -> 13.3 us; Q6_K 33017 and 8456 x 1024, M = 6, 22.0 -> 16.9.)
 constexpr int kSmallKeepTiles = 8;
-__device__ __forceinline__ void small_add_waves(float4_t (&red)[2][kSmallWaves][64], float4_t *keep, int ti, int wave, int nwaves,
-                                                int lane, const float4_t acc, float4_t *out_tiles) {
+__device__ __forceinline__ void small_add_waves(float4_t *red, float4_t *keep, int ti, int wave, int nwaves, int lane, const float4_t acc,
+                                                float4_t *out_tiles) {
     if (keep) {  // workgroup-uniform
         keep[(ti * nwaves + wave) * 64 + lane] = acc;
         return;
     }
-    const int buf = ti & 1;
-    red[buf][wave][lane] = acc;
+    const int buf = (ti & 1) * nwaves;
+    red[(buf + wave) * 64 + lane] = acc;
     __syncthreads();
     if (wave == 0) {
-        float4_t v = red[buf][0][lane];
+        float4_t v = red[buf * 64 + lane];
         for (int q = 1; q < nwaves; q++) {
-            const float4_t u = red[buf][q][lane];
+            const float4_t u = red[(buf + q) * 64 + lane];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] += u[r];
         }
@@ -1488,8 +1492,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
         take_weight(second, ybf16, bx, W, yg, N);
         tiles = (N + 15) / 16;
     }
-    __shared__ float4_t red[2][kSmallWaves][64];
-    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64]: lane slots of the finished tiles; then the waves' stages
+    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64]: lane slots of the finished tiles; the waves' partial tiles; then the waves' stages
     const float rs = XT ? 1.0f : small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1498,8 +1501,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
     const uint32_t low = kg < 2 ? 0xFFFFFFFFu : 0u;
     const int rounds = (tiles_per_wg + kSmallDepth - 1) / kSmallDepth;
     float4_t *out_tiles = dyn;
-    float4_t *keep = tiles_per_wg * MT <= kSmallKeepTiles ? dyn + rounds * kSmallDepth * MT * 64 : nullptr;
-    u32x4 *stage = reinterpret_cast<u32x4 *>(dyn + rounds * kSmallDepth * MT * 64 * (keep ? 1 + nwaves : 1)) + wave * SmallRun<NSB, FMT>::kPieces;
+    float4_t *red = dyn + rounds * kSmallDepth * MT * 64, *keep = tiles_per_wg * MT <= kSmallKeepTiles ? red : nullptr;
+    u32x4 *stage = reinterpret_cast<u32x4 *>(dyn + (rounds * kSmallDepth * MT * (keep ? 1 + nwaves : 1) + (keep ? 0 : 2 * nwaves)) * 64) + wave * SmallRun<NSB, FMT>::kPieces;
     int sbi[NSB];
     bool sbv[NSB];  // wave-uniform
 #pragma unroll
@@ -1704,8 +1707,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
         take_weight(second, ybf16, bx, W, yg, N);
         tiles = (N + 15) / 16;
     }
-    __shared__ float4_t red[2][kSmallWaves][64];
-    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
+    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], the waves' partial tiles, then the waves' stages
     const float rs = XT ? 1.0f : small_row_scale(rowscale);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1713,8 +1715,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
     const int nl = lane & 15, kg = lane >> 4;
     const int rounds = (tiles_per_wg + kSmallDepth - 1) / kSmallDepth;
     float4_t *out_tiles = dyn;
-    float4_t *keep = tiles_per_wg * MT <= kSmallKeepTiles ? dyn + rounds * kSmallDepth * MT * 64 : nullptr;
-    u32x4 *stage = reinterpret_cast<u32x4 *>(dyn + rounds * kSmallDepth * MT * 64 * (keep ? 1 + nwaves : 1)) + wave * (NSB * kQ8TileRunPieces);
+    float4_t *red = dyn + rounds * kSmallDepth * MT * 64, *keep = tiles_per_wg * MT <= kSmallKeepTiles ? red : nullptr;
+    u32x4 *stage = reinterpret_cast<u32x4 *>(dyn + (rounds * kSmallDepth * MT * (keep ? 1 + nwaves : 1) + (keep ? 0 : 2 * nwaves)) * 64) + wave * (NSB * kQ8TileRunPieces);
     int sbi[NSB];
     bool sbv[NSB];  // wave-uniform
 #pragma unroll
@@ -1893,16 +1895,15 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
         w_last = (uint32_t)(((uint64_t)N * (uint64_t)spr * 210u - 1) & ~(uint64_t)15);
     }
     constexpr int P = SmallQ6<NSB, ANY>::kRowPieces, kLoads = SmallQ6<NSB, ANY>::kLoads;
-    __shared__ float4_t red[2][kSmallWaves][64];
-    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' stages
+    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], the waves' partial tiles, then the waves' stages
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
     const int nl = lane & 15, kg = lane >> 4;
     const int rounds = (tiles_per_wg + kSmallDepth - 1) / kSmallDepth;
     float4_t *out_tiles = dyn;
-    float4_t *keep = tiles_per_wg <= kSmallKeepTiles ? dyn + rounds * kSmallDepth * 64 : nullptr;
-    uint32_t *stage = reinterpret_cast<uint32_t *>(dyn + rounds * kSmallDepth * 64 * (keep ? 1 + nwaves : 1)) + wave * SmallQ6<NSB, ANY>::kStageDwords;
+    float4_t *red = dyn + rounds * kSmallDepth * 64, *keep = tiles_per_wg <= kSmallKeepTiles ? red : nullptr;
+    uint32_t *stage = reinterpret_cast<uint32_t *>(dyn + (rounds * kSmallDepth * (keep ? 1 + nwaves : 1) + (keep ? 0 : 2 * nwaves)) * 64) + wave * SmallQ6<NSB, ANY>::kStageDwords;
     // this wave's super-blocks sb0 .. sb0 + NSB - 1 (rows are whole multiples of eight super-blocks, so the NSB of a wave
     // exist together or not at all; a wave past the end of a long row's last run works on the row's first super-blocks
     // with zero activations and zero scales)
@@ -2141,8 +2142,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
         tiles = (N + 15) / 16;
     }
     using B = Block16<FMT>;
-    __shared__ float4_t red[2][kSmallWaves][64];
-    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the kept partial tiles
+    extern __shared__ float4_t dyn[];  // out_tiles [tiles_per_wg rounded up to whole rounds][64], then the waves' partial tiles
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = (int)(blockDim.x >> 6);
@@ -2150,7 +2150,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
     const uint32_t h = (uint32_t)(kg >> 1), g = (uint32_t)(kg & 1);
     const int rounds = (tiles_per_wg + kSmallDepth - 1) / kSmallDepth;
     float4_t *out_tiles = dyn;
-    float4_t *keep = tiles_per_wg <= kSmallKeepTiles ? dyn + rounds * kSmallDepth * 64 : nullptr;
+    float4_t *red = dyn + rounds * kSmallDepth * 64, *keep = tiles_per_wg <= kSmallKeepTiles ? red : nullptr;
     int sbi[NSB];
     bool sbv[NSB];  // wave-uniform
 #pragma unroll
@@ -2638,6 +2638,22 @@ static hipError_t launch_rw_q8(hipStream_t s, const uint8_t *w, const uint4 *xs,
     return hipGetLastError();
 }
 
+// LDS of a short-batch workgroup: the finished tiles, a partial tile per wave (of each of few tiles until the end, or two in turn) and the
+// waves' stages; before the first tile the activations that the waves convert pass through the same.
+size_t qgemm_small_lds(uint32_t type, int64_t m, int64_t k, int tiles_per_wg, bool own, bool xf32) {
+    const int spr = (int)(k / 256), nwaves = spr < kSmallWaves ? spr : kSmallWaves, mt = m > kSmallMaxM ? 2 : 1;
+    const bool two = small_run_spr(type, m) > kSmallWaves && spr > kSmallWaves;  // super-blocks a wave
+    const int tiles = (tiles_per_wg + kSmallDepth - 1) / kSmallDepth * kSmallDepth * mt;
+    size_t stage = 0;  // (Q3_K and Q2_K: none)
+    if (type == kTypeQ4K) stage = 16 * (two ? SmallRun<2, 0>::kPieces : SmallRun<1, 0>::kPieces);
+    else if (type == kTypeQ5K) stage = 16 * (two ? SmallRun<2, 1>::kPieces : SmallRun<1, 1>::kPieces);
+    else if (type == kTypeQ6K) stage = 4 * (two ? SmallQ6<2, true>::kStageDwords : SmallQ6<1>::kStageDwords);
+    else if (type == kTypeQ8_0) stage = 16 * (two ? 2 : 1) * kQ8TileRunPieces;
+    const size_t work = (size_t)(tiles + (tiles_per_wg * mt <= kSmallKeepTiles ? tiles : 2) * nwaves) * 1024 + nwaves * stage;
+    const size_t x_lds = own ? (size_t)nwaves * (xf32 ? 2 : 1) * kSmallXItems * 16 : 0;
+    return work > x_lds ? work : x_lds;
+}
+
 hipError_t launch_copy_x(const void *x, size_t bytes, void *to, hipStream_t s) {
     const size_t items = bytes / 16;  // (whole super-blocks)
     hipLaunchKernelGGL(k_copy16, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, reinterpret_cast<const uint4 *>(x), reinterpret_cast<uint4 *>(to), items);
@@ -2755,8 +2771,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         int tiles_per_wg = (tiles + tiles1 + n_wg - 1) / n_wg;
         if (tiles1 > 0 && (tiles + tiles_per_wg - 1) / tiles_per_wg + (tiles1 + tiles_per_wg - 1) / tiles_per_wg > n_wg) tiles_per_wg++;
         const int mt = m > kSmallMaxM ? 2 : 1;  // 16-row blocks of activations
-        const size_t x_lds = !own ? 0 : (size_t)nwaves * (xf32 ? 2 : 1) * kSmallXItems * 16;  // the activations pass through before the tiles do
-        // the finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and the 16 KiB of the
+        // the finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and at most 16 KiB of the
         // reduction buffers: 64 of them keep the workgroup within 160 KiB for every type
         tiles_per_wg = tiles_per_wg < 64 / mt ? tiles_per_wg : 64 / mt;
         // a long row: p.splits runs, one workgroup row of the grid each, partial tiles for k_rw_reduce
@@ -2766,12 +2781,9 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         second.first = (tiles + tiles_per_wg - 1) / tiles_per_wg;
         const int ybf16 = (ybf ? 1 : 0) | (tiles1 > 0 ? kHasSecond : 0);
         const dim3 grid((unsigned)(second.first + (tiles1 + tiles_per_wg - 1) / tiles_per_wg), (unsigned)runs), block((unsigned)(64 * nwaves));
-        // (a workgroup of few tiles also keeps every wave's partial tile of each until the end)
-        const size_t lds = (size_t)((tiles_per_wg + kSmallDepth - 1) / kSmallDepth * kSmallDepth) * mt * 1024 *
-                           (tiles_per_wg * mt <= kSmallKeepTiles ? 1 + nwaves : 1);
+        const size_t bytes = qgemm_small_lds(type, m, k, tiles_per_wg, own, xf32);
         // (LDS beyond the launch default has to be asked for)
-        auto go = [&](auto kern, size_t bytes, auto... args) {
-            bytes = bytes > x_lds ? bytes : x_lds;
+        auto go = [&](auto kern, auto... args) {
             if (bytes > 48 * 1024) {
                 const hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
                 if (a != hipSuccess) return a;
@@ -2780,9 +2792,8 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
             return hipGetLastError();
         };
         const void *const xa = own ? x : (const void *)xs;
-        const size_t waves = (size_t)nwaves;
         if (q23) {
-#define PMH_SMALL16(F, S, X) go(k_qgemm_small16<F, S, X>, lds, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
+#define PMH_SMALL16(F, S, X) go(k_qgemm_small16<F, S, X>, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
             if (type == kTypeQ2K) {
                 if (nsb == 2) e = !own ? PMH_SMALL16(3, 2, 3) : xf32 ? PMH_SMALL16(3, 2, 2) : PMH_SMALL16(3, 2, 1);
                 else e = xf32 ? PMH_SMALL16(3, 1, 2) : PMH_SMALL16(3, 1, 1);
@@ -2793,27 +2804,22 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
 #undef PMH_SMALL16
         } else if (q6) {
             const bool any = spr % 8 != 0;  // rows that do not start on 16-byte boundaries
-            // the waves' stages behind the finished tiles
-            const size_t lds6 = lds + waves * (size_t)(nsb == 2 ? SmallQ6<2, true>::kStageDwords : SmallQ6<1>::kStageDwords) * 4;
             const uint32_t w_last = (uint32_t)(((uint64_t)n * (uint64_t)spr * 210u - 1) & ~(uint64_t)15);
-#define PMH_SMALL_Q6(S, A, X) go(k_qgemm_small_q6<S, A, X>, lds6, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second)
+#define PMH_SMALL_Q6(S, A, X) go(k_qgemm_small_q6<S, A, X>, w, xa, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, w_last, part_out, second)
             if (nsb == 2 && any) e = !own ? PMH_SMALL_Q6(2, true, 3) : xf32 ? PMH_SMALL_Q6(2, true, 2) : PMH_SMALL_Q6(2, true, 1);
             else if (nsb == 2) e = !own ? PMH_SMALL_Q6(2, false, 3) : xf32 ? PMH_SMALL_Q6(2, false, 2) : PMH_SMALL_Q6(2, false, 1);
             else if (any) e = xf32 ? PMH_SMALL_Q6(1, true, 2) : PMH_SMALL_Q6(1, true, 1);
             else e = xf32 ? PMH_SMALL_Q6(1, false, 2) : PMH_SMALL_Q6(1, false, 1);
 #undef PMH_SMALL_Q6
         } else if (q8) {
-            const size_t lds8 = lds + waves * nsb * kQ8TileRunPieces * 16;
-#define PMH_SMALL_Q8(S, T, X) go(k_qgemm_small_q8<S, T, X>, lds8, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
+#define PMH_SMALL_Q8(S, T, X) go(k_qgemm_small_q8<S, T, X>, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
             if (mt == 2) e = PMH_SMALL_Q8(1, 2, 0);  // (two blocks of activations: one run of eight blocks per wave)
             else if (nsb == 2) e = own ? PMH_SMALL_Q8(2, 1, 1) : PMH_SMALL_Q8(2, 1, 3);
             else e = xf32 ? PMH_SMALL_Q8(1, 1, 2) : PMH_SMALL_Q8(1, 1, 1);
 #undef PMH_SMALL_Q8
         } else {
             static_assert(2 * kSmallWaves >= kSmallMaxSpr, "two super-blocks per wave must cover the longest row");
-#define PMH_SMALL_X(O, S, F, T, X)                                                                                                                       \
-    go(k_qgemm_small<O, S, F, T, X>, lds + waves * SmallRun<S, F>::kPieces * 16, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, \
-       ybf16, part_out, second)
+#define PMH_SMALL_X(O, S, F, T, X) go(k_qgemm_small<O, S, F, T, X>, w, xa, rowscale, y, (int)m, (int)p.mp, (int)n, spr, tiles, tiles_per_wg, ybf16, part_out, second)
 #define PMH_SMALL_F(O, S, F) (mt == 2 ? PMH_SMALL_X(O, S, F, 2, 0) : xf32 ? PMH_SMALL_X(O, S, F, 1, 2) : PMH_SMALL_X(O, S, F, 1, 1))
 #define PMH_SMALL_2(O, F) (mt == 1 && !own ? PMH_SMALL_X(O, 2, F, 1, 3) : PMH_SMALL_F(O, 2, F))
             if (spr > kSmallWaves) e = ref ? (q5 ? PMH_SMALL_2(0, 1) : PMH_SMALL_2(0, 0)) : (q5 ? PMH_SMALL_2(1, 1) : PMH_SMALL_2(1, 0));

@@ -112,6 +112,8 @@ bool qgemm_small_rows(const GemmPlan &plan, int64_t m);
 // Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.  shared: another
 // launch could use the converted ones.
 bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype, bool shared);
+// LDS bytes of a workgroup of the short-batch kernels (own: it converts the activations for itself), beside the 128 it always has.
+size_t qgemm_small_lds(uint32_t type, int64_t m, int64_t k, int tiles_per_wg, bool own, bool xf32);
 // `bytes` of activations, a multiple of 16, to where results that lie over them do not reach
 hipError_t launch_copy_x(const void *x, size_t bytes, void *to, hipStream_t s);
 // reuse_prepass: the workspace still holds the converted activations of the previous launch_qgemm on this stream with the same

@@ -93,3 +93,9 @@ def gemm_workspace_bytes(t, m, n, k):
     fn = _lib.load()._ZN3pmh21qgemm_workspace_bytesEjlll
     fn.restype, fn.argtypes = C.c_size_t, [C.c_uint32, C.c_int64, C.c_int64, C.c_int64]
     return fn(t, m, n, k)
+
+
+def gemm_small_lds(t, m, k, tiles_per_wg, own, xf32):
+    fn = _lib.load()._ZN3pmh15qgemm_small_ldsEjllibb
+    fn.restype, fn.argtypes = C.c_size_t, [C.c_uint32, C.c_int64, C.c_int64, C.c_int, C.c_bool, C.c_bool]
+    return fn(t, m, k, tiles_per_wg, own, xf32)

@@ -1,7 +1,7 @@
 """The GEMM's launch plan (host code, no device needed): what it names can be launched."""
 import pytest
 
-from gpu_util import Q4K, Q6K, Q8_0, SMALL, WAVES, gemm_pair_plan, gemm_plan, gemm_workspace_bytes
+from gpu_util import Q4K, Q6K, Q8_0, SMALL, WAVES, gemm_pair_plan, gemm_plan, gemm_small_lds, gemm_workspace_bytes
 
 Q5K, Q3K, Q2K = 13, 11, 10
 TYPES = [Q4K, Q6K, Q8_0, Q5K, Q3K, Q2K]
@@ -66,3 +66,17 @@ def test_few_rows_take_the_faster_kernel(t, m, n, k, kernel):
 def test_short_rows_take_the_small_tile(t, m, n, k):
     p = gemm_plan(t, m, n, k)
     assert (p.kernel, p.nr) == (WAVES, 1), p  # (8.5 us, 11 with 64 rows)
+
+
+# A launch of rows of one to four super-blocks counts on 8, 4 or 2 workgroups a compute unit (160 KiB of LDS, 128 bytes a workgroup of which are
+# the row scales'), up to sixteen row tiles each (four of one super-block): all of them fit, whoever converts the activations.
+@pytest.mark.parametrize("xf32", [False, True])
+@pytest.mark.parametrize("t", TYPES)
+def test_short_batch_workgroups_fit_together(t, xf32):
+    for spr in range(1, 5):
+        for tiles in (1, 2, 4, 8, 9, 16)[:6 if spr > 1 else 3]:
+            assert (gemm_small_lds(t, 16, 256 * spr, tiles, True, xf32) + 128) * (8 // spr) <= 160 * 1024, (spr, tiles)
+    for tiles in (1, 8, 9, 64):
+        for m, k, own in ((16, 2048, True), (16, 4096, True), (16, 4096, False), (32, 2048, False), (32, 4096, False)):
+            if m == 16 or (t in (Q4K, Q5K, Q8_0) and tiles < 64):
+                assert gemm_small_lds(t, m, k, tiles, own, xf32) + 128 <= 160 * 1024, (m, k, own, tiles)
