@@ -962,7 +962,7 @@ static int32_t qgemm_over_reblocked(uint32_t t, const uint8_t *wa, int64_t n, in
     const uint8_t *wb = wa + reblocked_part_bytes(n, k);
     float *yb = (float *)(scratch + gemm_bytes), *ya = y_f32 ? (float *)y : (float *)((uint8_t *)yb + y_bytes);
     hipError_t e = hipSuccess;
-    if (parts == 2 && y_f32 && pmh::qgemm_converts_itself(pmh::qgemm_plan(m, n, k, PMETAL_GGML_TYPE_Q6K), PMETAL_GGML_TYPE_Q6K, m, k, x_dtype, true)) {
+    if (parts == 2 && y_f32 && pmh::qgemm_converts_itself(pmh::qgemm_plan(m, n, k, PMETAL_GGML_TYPE_Q6K), PMETAL_GGML_TYPE_Q6K, m, n, 0, k, x_dtype, true)) {
         // both products convert x for themselves: a first one that lies over it must not be what the second one reads
         const size_t x_bytes = (size_t)m * k * (x_dtype == PMETAL_HIP_DTYPE_F32 ? 4 : 2);
         if ((uintptr_t)y < (uintptr_t)x + x_bytes && (uintptr_t)x < (uintptr_t)y + y_elems * 4) {
@@ -1118,7 +1118,7 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
         int before = -1, before_form = -1;
         for (size_t i = 0; i < count; i++) {
             const pmh::GemmPlan p = pmh::qgemm_plan(m, descs[i].n, k, descs[i].ggml_type);
-            const bool o = pmh::qgemm_converts_itself(p, descs[i].ggml_type, m, k, x_dtype, true);
+            const bool o = pmh::qgemm_converts_itself(p, descs[i].ggml_type, m, descs[i].n, 0, k, x_dtype, true);
             own = own || o, all_own = all_own && o;
             two_forms = two_forms || (layout(descs[i]) == before && form(descs[i], p) != before_form);
             before = layout(descs[i]), before_form = form(descs[i], p);
@@ -1149,8 +1149,7 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
         if (e == hipErrorNotSupported) return fail(PMETAL_HIP_ERR_UNSUPPORTED_TYPE, "qgemm: configuration not supported");
         if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
         // (a second weight's plan has the same kernel; a K split's partial tiles may lie over items of another layout)
-        const bool two_q3k = d.ggml_type == PMETAL_GGML_TYPE_Q3K && second.n > 0;
-        have = pmh::qgemm_converts_itself(one, d.ggml_type, m, k, x_dtype, shared || two_q3k) ? -1 : want, have_mp = want_mp;
+        have = pmh::qgemm_converts_itself(one, d.ggml_type, m, d.n, second.n, k, x_dtype, shared) ? -1 : want, have_mp = want_mp;
     }
     return ok();
 }

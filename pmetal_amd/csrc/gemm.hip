@@ -1199,7 +1199,7 @@ constexpr int kSmallMaxM2 = 32;  // Q4_K, Q5_K and Q8_0: two 16-row blocks of ac
 // `red`, `keep`, behind the finished tiles: two buffers of a partial tile per wave, or those.  (All of it in dynamic LDS and as long as the
 // workgroup's waves need: with the buffers of eight waves beside what activations pass through before the first tile, fewer workgroups of
 // rows of one to four super-blocks fit a compute unit than the launch counts on, and the last ones of a round waited for the others:
-// f32, three Q4_K weights of 24737 x 256, M = 9, 20.0 -> 13.3 us; Q6_K 33017 and 8456 x 1024, M = 6, 22.0 -> 16.9.)
+// f32, three Q4_K weights of 24737 x 256, M = 9, 20.0 -> 14.3 us; Q6_K 33017 and 8456 x 1024, M = 6, 22.2 -> 16.1.)
 constexpr int kSmallKeepTiles = 8;
 __device__ __forceinline__ void small_add_waves(float4_t *red, float4_t *keep, int ti, int wave, int nwaves, int lane, const float4_t acc,
                                                 float4_t *out_tiles) {
@@ -2339,18 +2339,38 @@ static bool qgemm_small_applies(uint32_t type, int64_t m, int64_t n, int64_t k) 
     return false;
 }
 
+// Row tiles of a short-batch workgroup: one workgroup per compute unit (of fewer waves: as many as have eight together) over all runs of a
+// long row, each of which then walks several row tiles with its activation operands in registers (one tile per workgroup and four times the
+// workgroups: 35 against 27 us at M = 16, 4096 x 14336).  second_n: rows of the launch's second weight; a workgroup's tiles are of one weight.
+// The finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and at most 16 KiB of the
+// reduction buffers: 64 of them keep the workgroup within 160 KiB for every type.
+static int small_tiles_per_wg(const GemmPlan &p, int64_t m, int64_t n, int64_t second_n, int64_t k) {
+    const int spr = (int)(k / 256), nwaves = spr < kSmallWaves ? spr : kSmallWaves, most = m > kSmallMaxM ? 32 : 64;
+    int64_t slots = (int64_t)compute_units() * (kSmallWaves / nwaves) / p.splits;
+    slots = slots < 1 ? 1 : slots;
+    const int tiles = (int)((n + 15) / 16), tiles1 = (int)((second_n + 15) / 16);
+    const int n_wg = (int)(tiles + tiles1 < slots ? tiles + tiles1 : slots);
+    int per = (tiles + tiles1 + n_wg - 1) / n_wg;
+    if (tiles1 > 0 && (tiles + per - 1) / per + (tiles1 + per - 1) / per > n_wg) per++;
+    return per < most ? per : most;
+}
+
 // (Who converts does not change a bit of the result: k_prep_pairs does as the waves do.)
 // Up to eight super-blocks a row a wave converts one, which its first weights hide.  Of longer rows it converts two, which costs 1 to 3 us of
 // the pre-pass's 4: not where several launches share one pre-pass (us for three bf16 weights of 4096, 1024 and 1024 x 4096, M = 16, two launches,
 // with one / without: Q4_K 17.1 / 18.3, Q3_K 21.3 / 24.3; of 2048 x 2048 12.6 / 12.4), and not f32 activations of Q8_0 and Q3_K, 128 registers of
 // them, behind which the second row tile has to be asked for (M = 16, 14336 x 4096: Q8_0 18.4 / 19.3; Q3_K, M = 4, 1024 x 4096 11.9 / 12.2, M = 9,
 // 4096 x 3328 11.9 / 12.4; Q4_K 14.9 / 14.5, 9.7 / 9.5, 10.6 / 10.2) or two Q3_K weights in one launch (14336 x 4096, M = 16, 24.6 / 25.1: their sums
-// of sixteen elements take the longest to make).
+// of sixteen elements take the longest to make).  Nor of Q3_K and Q8_0 where a workgroup walks so many row tiles that its waves meet at each: the
+// kernels that convert take longer over a tile (bf16, a pre-pass / without: Q3_K 16908 x 5120 36.2 / 38.6, 47394 x 2304 36.5 / 40.5, 28582 x
+// 10496 68.6 / 75.1, Q8_0 36966 x 5376 66.0 / 67.1; with five tiles Q3_K 18833 x 4096 23.1 / 22.9, with ten Q4_K, Q5_K and Q6_K within 1 %).
 bool qgemm_small_rows(const GemmPlan &p, int64_t m) { return p.kernel == GemmKernel::kSmall && m <= kSmallMaxM; }
-bool qgemm_converts_itself(const GemmPlan &p, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype, bool shared) {
+bool qgemm_converts_itself(const GemmPlan &p, uint32_t type, int64_t m, int64_t n, int64_t second_n, int64_t k, uint32_t x_dtype, bool shared) {
     if (!qgemm_small_rows(p, m)) return false;
     if (k <= kSmallWaves * 256) return true;
-    return !shared && (x_dtype != kDtypeF32 || (type != kTypeQ8_0 && type != kTypeQ3K));
+    if (shared) return false;
+    if (type == kTypeQ3K && second_n > 0) return false;
+    return (type != kTypeQ8_0 && type != kTypeQ3K) || (x_dtype != kDtypeF32 && small_tiles_per_wg(p, m, n, second_n, k) <= kSmallKeepTiles);
 }
 
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
@@ -2703,7 +2723,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         else if (per_wg == 2) PMH_PREP_R(F, O, 2); \
         else PMH_PREP_R(F, O, 1);               \
     } while (0)
-    const bool own = qgemm_converts_itself(p, type, m, k, x_dtype, shared || (type == kTypeQ3K && second.n > 0));
+    const bool own = qgemm_converts_itself(p, type, m, n, second.n, k, x_dtype, shared);
     if (own) {
         // Every wave converts what it multiplies.  Results over the activations would race with other workgroups' reads of them.
         const uintptr_t xb = reinterpret_cast<uintptr_t>(x), xe = xb + (size_t)m * k * (xf32 ? 4 : 2);
@@ -2760,22 +2780,12 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     } else if (p.kernel == GemmKernel::kSmall) {
         const int nwaves = spr < kSmallWaves ? spr : kSmallWaves;
         const int tiles = (int)((n + 15) / 16);
-        // one workgroup per compute unit over all runs of a long row: each then walks several row tiles with its activation
-        // operands in registers (one tile per workgroup and four times the workgroups: 35 against 27 us at M = 16, 4096 x 14336)
         const int run = small_run_spr(type, m);
-        const int runs_of_row = p.splits;
-        int64_t slots = (int64_t)compute_units() * (kSmallWaves / nwaves) / runs_of_row;
-        slots = slots < 1 ? 1 : slots;
-        const int tiles1 = (second.n + 15) / 16;  // of the second weight: a workgroup's tiles are of one weight
-        const int n_wg = (int)(tiles + tiles1 < slots ? tiles + tiles1 : slots);
-        int tiles_per_wg = (tiles + tiles1 + n_wg - 1) / n_wg;
-        if (tiles1 > 0 && (tiles + tiles_per_wg - 1) / tiles_per_wg + (tiles1 + tiles_per_wg - 1) / tiles_per_wg > n_wg) tiles_per_wg++;
+        const int tiles1 = (second.n + 15) / 16;  // of the second weight
+        const int tiles_per_wg = small_tiles_per_wg(p, m, n, second.n, k);
         const int mt = m > kSmallMaxM ? 2 : 1;  // 16-row blocks of activations
-        // the finished tiles wait in LDS, 1 KiB each, beside the waves' stages (at most 70 KiB, Q8_0) and at most 16 KiB of the
-        // reduction buffers: 64 of them keep the workgroup within 160 KiB for every type
-        tiles_per_wg = tiles_per_wg < 64 / mt ? tiles_per_wg : 64 / mt;
         // a long row: p.splits runs, one workgroup row of the grid each, partial tiles for k_rw_reduce
-        const int runs = runs_of_row;
+        const int runs = p.splits;
         float *const part_out = runs > 1 ? partial : nullptr;
         const int nsb = run > kSmallWaves && spr > kSmallWaves ? 2 : 1;
         second.first = (tiles + tiles_per_wg - 1) / tiles_per_wg;

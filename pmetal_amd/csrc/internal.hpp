@@ -109,9 +109,9 @@ size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k);
 bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan);
 // Whether the plan's kernel takes at most 16 rows, converted per pair of super-blocks and not per row: no other kernel can use those.
 bool qgemm_small_rows(const GemmPlan &plan, int64_t m);
-// Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.  shared: another
-// launch could use the converted ones.
-bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t k, uint32_t x_dtype, bool shared);
+// Whether the plan's kernel reads the activations as they are: a launch with it leaves no converted ones for the next.
+// second_n: rows of the launch's second weight (0: none).  shared: another launch could use the converted ones.
+bool qgemm_converts_itself(const GemmPlan &plan, uint32_t type, int64_t m, int64_t n, int64_t second_n, int64_t k, uint32_t x_dtype, bool shared);
 // LDS bytes of a workgroup of the short-batch kernels (own: it converts the activations for itself), beside the 128 it always has.
 size_t qgemm_small_lds(uint32_t type, int64_t m, int64_t k, int tiles_per_wg, bool own, bool xf32);
 // `bytes` of activations, a multiple of 16, to where results that lie over them do not reach

@@ -99,3 +99,10 @@ def gemm_small_lds(t, m, k, tiles_per_wg, own, xf32):
     fn = _lib.load()._ZN3pmh15qgemm_small_ldsEjllibb
     fn.restype, fn.argtypes = C.c_size_t, [C.c_uint32, C.c_int64, C.c_int64, C.c_int, C.c_bool, C.c_bool]
     return fn(t, m, k, tiles_per_wg, own, xf32)
+
+
+def gemm_converts_itself(t, m, n, k, x_dtype, second_n=0, shared=False):
+    """Whether a launch's waves convert the activations they multiply."""
+    fn = _lib.load()._ZN3pmh21qgemm_converts_itselfERKNS_8GemmPlanEjlllljb
+    fn.restype, fn.argtypes = C.c_bool, [C.POINTER(Plan), C.c_uint32, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_uint32, C.c_bool]
+    return fn(C.byref(gemm_plan(t, m, n, k)), t, m, n, second_n, k, x_dtype, shared)

@@ -1,7 +1,7 @@
 """The GEMM's launch plan (host code, no device needed): what it names can be launched."""
 import pytest
 
-from gpu_util import Q4K, Q6K, Q8_0, SMALL, WAVES, gemm_pair_plan, gemm_plan, gemm_small_lds, gemm_workspace_bytes
+from gpu_util import Q4K, Q6K, Q8_0, SMALL, WAVES, gemm_converts_itself, gemm_pair_plan, gemm_plan, gemm_small_lds, gemm_workspace_bytes
 
 Q5K, Q3K, Q2K = 13, 11, 10
 TYPES = [Q4K, Q6K, Q8_0, Q5K, Q3K, Q2K]
@@ -80,3 +80,21 @@ def test_short_batch_workgroups_fit_together(t, xf32):
         for m, k, own in ((16, 2048, True), (16, 4096, True), (16, 4096, False), (32, 2048, False), (32, 4096, False)):
             if m == 16 or (t in (Q4K, Q5K, Q8_0) and tiles < 64):
                 assert gemm_small_lds(t, m, k, tiles, own, xf32) + 128 <= 160 * 1024, (m, k, own, tiles)
+
+
+# Who converts bf16 activations of a row of more than eight super-blocks, single weights (us by a pre-pass, by the waves themselves).
+@pytest.mark.parametrize("t,m,n,k,own", [
+    (Q3K, 4, 16908, 5120, False),    # 36.2, 38.6
+    (Q3K, 12, 47394, 2304, False),   # 36.5, 40.5
+    (Q3K, 16, 28582, 10496, False),  # 68.6, 75.1
+    (Q8_0, 6, 36966, 5376, False),   # 66.0, 67.1
+    (Q3K, 10, 18833, 4096, True),    # 23.1, 22.9
+    (Q3K, 6, 946, 14592, True),      # 16.2, 15.4
+    (Q4K, 5, 14336, 4096, True),
+    (Q6K, 10, 18136, 5888, True),    # 43.3, 42.9
+    (Q2K, 9, 17631, 8192, True)])    # 35.6, 30.1
+def test_who_converts(t, m, n, k, own):
+    assert gemm_plan(t, m, n, k).kernel == SMALL
+    assert gemm_converts_itself(t, m, n, k, 1) == own
+    assert not gemm_converts_itself(t, m, n, k, 1, shared=True)
+    assert gemm_converts_itself(t, m, n, 2048, 1, shared=True)
