@@ -1148,8 +1148,10 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
                                          want == have && want_mp == have_mp, second, shared);
         if (e == hipErrorNotSupported) return fail(PMETAL_HIP_ERR_UNSUPPORTED_TYPE, "qgemm: configuration not supported");
         if (e != hipSuccess) return hip_fail(e, "qgemm kernel launch");
-        // (a second weight's plan has the same kernel; a K split's partial tiles may lie over items of another layout)
-        have = pmh::qgemm_converts_itself(one, d.ggml_type, m, d.n, second.n, k, x_dtype, shared) ? -1 : want, have_mp = want_mp;
+        // (a second weight's plan has the same kernel.)  A launch that converts for itself leaves what the workspace holds to the next one, except where
+        // the partial tiles of its K split may lie over items of another layout.
+        if (!pmh::qgemm_converts_itself(one, d.ggml_type, m, d.n, second.n, k, x_dtype, shared)) have = want, have_mp = want_mp;
+        else if (one.splits > 1 && have % 6 != layout(d)) have = -1;
     }
     return ok();
 }

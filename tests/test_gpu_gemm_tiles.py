@@ -333,6 +333,9 @@ def test_batches_of_kernels_with_and_without_a_pre_pass(oracle, x_dtype):
     for m, k, specs in ((12, 2304, [(Q4K, 300), (Q4K, 9000), (Q4K, 400), (Q8_0, 9000), (Q4K, 300)]),
                         (12, 14336, [(Q6K, 300), (Q4K, 300), (Q6K, 400), (11, 300), (Q4K, 500)]),
                         (9, 5120, [(Q4K, 300), (Q6K, 14400), (Q4K, 300), (Q8_0, 300), (Q6K, 14400), (Q8_0, 300)]),
+                        # launches that convert for themselves between others of one layout; the partial tiles of the first one's K split
+                        # lie over the last converted activations, those of the second one behind them
+                        (9, 5120, [(Q4K, 300), (Q6K, 14500), (Q4K, 300), (Q4K, 14500), (Q4K, 400)]),
                         (7, 3840, [(t, 272) for t in (Q4K, Q6K, Q8_0, 10, 11, 13)] * 2)):  # a pre-pass per pair of super-blocks, the last half a pair
         x = rng.standard_normal((m, k)).astype(np.float32)
         dx = pm.DeviceBuffer.from_host(x if x_dtype == pm.DTYPE_F32 else oracle.f32_to_bf16_bits(x.reshape(-1)).reshape(m, k))
