@@ -285,14 +285,14 @@ __device__ __forceinline__ void q6k_row_body(const uint8_t *__restrict__ W, cons
 }
 
 // The workgroups of a launch that belong to a Q6_K matrix: a team for every row where there are enough, two rows a team at a time otherwise.
+// A chunk is requested ahead of x, not more: x comes back behind them (us with one / two / three, bf16: 488, 780, 838 and Q6_K 376 x 4096 5.0 / 5.7 / 6.7,
+// 2793 and 436 x 2560 5.6 / 6.4 / 7.0; with the second one requested behind x, 5.1 and more).
 template <int T, bool XF32>
 __device__ __forceinline__ void q6k_member_body(const uint8_t *__restrict__ W, const void *__restrict__ xg, float *__restrict__ y,
                                                 int n_rows, int spr, int block, int n_blocks, int teams_per_wg, uint4 *smem) {
     if (!(XF32 && T == 8) && n_rows <= n_blocks * teams_per_wg) {  // (f32 x beside the Q4_K digits of eight-lane teams: a spill)
         const int mine = (int)threadIdx.x / T, team = mine < teams_per_wg ? block * teams_per_wg + mine : n_rows;
-        // (a chunk ahead for f32: the digits of two kinds of x leave no registers for more)
-        if (XF32 || spr <= T / 8) q6k_row_body<T, XF32, 1>(W, xg, y, n_rows, spr, team, smem);
-        else q6k_row_body<T, XF32, 3>(W, xg, y, n_rows, spr, team, smem);
+        q6k_row_body<T, XF32, 1>(W, xg, y, n_rows, spr, team, smem);
     } else {
         q6k_small_body<T, XF32>(W, xg, y, n_rows, spr, block, n_blocks, teams_per_wg, smem);
     }
