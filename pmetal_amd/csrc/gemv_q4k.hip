@@ -742,7 +742,9 @@ hipError_t launch_general(int T, dim3 grid, dim3 block, size_t lds, hipStream_t 
     }
     if (q6_teams > 0) {
         switch (T) {
-        case 8: return go(k_qgemv_q4k<ORDER, XF32, 8, true>);
+        case 8:
+            if constexpr (XF32) return hipErrorNotSupported;  // (launch_group_mixed takes wider teams)
+            else return go(k_qgemv_q4k<ORDER, XF32, 8, true>);
         case 16: return go(k_qgemv_q4k<ORDER, XF32, 16, true>);
         case 32: return go(k_qgemv_q4k<ORDER, XF32, 32, true>);
         default: return go(k_qgemv_q4k<ORDER, XF32, 64, true>);
@@ -763,17 +765,23 @@ hipError_t launch_general(int T, dim3 grid, dim3 block, size_t lds, hipStream_t 
     }
 }
 
-// log2 of the lanes of kernel B's teams: the widest team that takes a row whole, or a wider one whose last chunk of a row is short where that is less work
-// in a line (us, such a team / the cheapest: 1024 x 1280 3.6 / 2.9, 4096 x 2304 5.7 / 4.4, 2048 x 3584 4.7 / 3.8, 1024 x 4352 9.9 / 3.7, 1024 x 11008
-// 25.6 / 5.2; 14000 x 768, where it is not, 4.2 / 4.5).
-int whole_team(int spr) { return 3 + (spr % 2 == 0) + (spr % 4 == 0) + (spr % 8 == 0); }
-int cheapest_team(int64_t rows, int spr) {
-    const int whole = whole_team(spr);
-    int best = whole;
-    for (int log = 6; log > whole; log--)
-        if (team_cost(rows, 8u * (uint32_t)spr, log) < team_cost(rows, 8u * (uint32_t)spr, best)) best = log;
-    return best;
+// Kernel B with teams of 2^log lanes over `rows` rows a workgroup: the rows of a team, and what the busiest compute unit costs: a team's tasks (its
+// rows' chunks), once for each of a SIMD's waves and once for the latency, and 2 for each chunk, each row and where T lanes do not take a
+// row whole.  Fitted to 677 drawn groups of one to four matrices of 200 to 16000 rows of 1 to 48 super-blocks, bf16 and f32, each timed with
+// every team: 1.003 of the best one's time, 1.08 at the most (us with 8 / 16 / 32 / 64 lanes: 4111 and 5597 x 4608 - / 13.2 / 12.4 / 12.2, 5486
+// and 4793 x 4352 17.1 / 13.2 / 12.4 / 12.8, 864, 1996 and 1446 x 1792 4.7 / 4.3 / 3.9 / 3.8, 3582, 5803 and 6473 x 1792 6.8 / 6.9 / 7.1 / 7.2).
+constexpr int kTeamWaves = 16;
+struct TeamsB {
+    int per_team;
+    uint32_t chunks, cost;
+};
+TeamsB teams_b(int64_t rows, int spr, int log) {
+    const uint32_t r = rows < (1 << 24) ? (uint32_t)rows : 1u << 24, lanes = 8u * (uint32_t)spr, in_wave = 64u >> log;
+    const uint32_t per = (r + kTeamWaves * in_wave - 1) / (kTeamWaves * in_wave), chunks = (lanes + (1u << log) - 1) >> log, waves = (r + in_wave - 1) / in_wave;
+    const uint32_t on_simd = waves < kTeamWaves ? (waves + 3) / 4 : kTeamWaves / 4, ragged = (lanes & ((1u << log) - 1)) != 0;
+    return {(int)per, chunks, per * chunks * (on_simd + 1) + 2 * (chunks + per + ragged)};
 }
+int whole_team(int spr) { return 3 + (spr % 2 == 0) + (spr % 4 == 0) + (spr % 8 == 0); }  // log2 of the widest team that takes a row whole
 
 // One to three small Q4_K matrices and one small Q6_K matrix that share k and x in one launch of kernel B: the workgroups
 // are divided between the two kinds by their bytes.
@@ -814,24 +822,30 @@ hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *
     grp.wg_begin[3] = begin;  // the Q6_K member starts here
     grp.w[3] = w6, grp.y[3] = y6, grp.n[3] = (int)n6;
     const dim3 grid((unsigned)(begin + wgs6));
-    const int64_t rows6 = (n6 + wgs6 - 1) / wgs6;  // rows of a Q6_K workgroup: one per team, or two at a time where that is not enough
-    int best_waves = 16, log_t = cheapest_team(total + n6, spr);
-    int64_t teams_avail;
-    for (;; log_t = whole_team(spr)) {
-        int64_t best_cost = INT64_MAX;
-        for (int waves = 16; waves >= 1; waves--) {  // as in launch_group_general
-            const int64_t teams = (int64_t)waves * (64 >> log_t);
-            const int64_t per_team = (rows_per_wg + teams - 1) / teams;
-            if (per_team < best_cost) best_cost = per_team, best_waves = waves;
-        }
-        teams_avail = (int64_t)best_waves * (64 >> log_t);
-        if (rows6 <= teams_avail || log_t == whole_team(spr)) break;  // (two rows of Q6_K at a time only where the teams take a row whole)
+    // The team: as above, with 12 for each chunk of the Q6_K matrix, whose teams take a row each (fitted to 228 drawn groups timed with every
+    // team: 1.0012 of the best one's time; us with 16 / 32 / 64 lanes, bf16: 166 and 711, Q6_K 2676, x 1536 - / 5.6 / -; 1721, 521, 497, 1759 x 2560 8.0 /
+    // 6.2 / 5.6; 2442, 2368, 2965 x 1536 f32 7.2 / 6.1 / 7.2), or two rows at a time: where there are not enough of them, only for teams that
+    // take a row whole; and over rows of three chunks of a wave and more, where the second row's requests hide the first one's
+    // (301 and 300 x 10240 7.7 -> 6.3, 311, 186 and 106 x 6144 5.8 -> 5.1, with two chunks 488, 780, 838 and 376 x 4096 5.0 and 5.1).  f32: no
+    // teams of eight lanes (their x beside the digits of Q4_K's spills registers).
+    const int64_t rows6 = (n6 + wgs6 - 1) / wgs6;  // of a Q6_K workgroup
+    const int whole = whole_team(spr);
+    int log_t = 0, per_team = 0;
+    uint32_t best = 0;
+    for (int log = 6; log >= (whole == 3 && xf32 ? 4 : whole); log--) {
+        const bool enough = rows6 <= (int64_t)kTeamWaves * (64 >> log);
+        if (!enough && log != whole) continue;
+        const TeamsB t = teams_b(rows_per_wg, spr, log);
+        const uint32_t cost = t.cost + 12 * t.chunks * (enough ? 1 : 2);
+        if (log_t == 0 || cost < best) log_t = log, best = cost, per_team = t.per_team;
     }
+    if (log_t == 0) return hipErrorNotSupported;
     const int T = 1 << log_t;
-    int64_t q6_teams = rows6 <= teams_avail ? rows6 : (rows6 + 1) / 2;
-    q6_teams = q6_teams > teams_avail ? teams_avail : q6_teams;
-    const int per_team = (int)((rows_per_wg + teams_avail - 1) / teams_avail);
-    const dim3 block((unsigned)best_waves * 64);
+    const int64_t teams = (int64_t)kTeamWaves * (64 >> log_t);
+    const bool two_rows = rows6 > teams || (!xf32 && whole == 6 && spr >= 24);
+    int64_t q6_teams = two_rows ? (rows6 + 1) / 2 : rows6;
+    q6_teams = q6_teams > teams ? teams : q6_teams;
+    const dim3 block(64 * kTeamWaves);
     if (order == pmh::kOrderRef)
         return xf32 ? launch_general<0, true>(T, grid, block, lds, s, grp, x, spr, (int)rows_per_wg, per_team, (int)q6_teams)
                     : launch_general<0, false>(T, grid, block, lds, s, grp, x, spr, (int)rows_per_wg, per_team, (int)q6_teams);
@@ -839,8 +853,7 @@ hipError_t launch_group_mixed(const uint8_t *const *w, const int64_t *n, float *
                 : launch_general<1, false>(T, grid, block, lds, s, grp, x, spr, (int)rows_per_wg, per_team, (int)q6_teams);
 }
 
-// Kernel B over a group of matrices: up to 16 waves; the wave count is the largest that keeps the busiest
-// team's row count minimal.
+// Kernel B over a group of matrices, with 16 waves a workgroup.
 hipError_t launch_group_general(const uint8_t *const *w, const int64_t *n, float *const *y, int count, int64_t k,
                                 const void *x, bool xf32, uint32_t order, hipStream_t s) {
     const int spr = (int)(k / 256);
@@ -849,7 +862,6 @@ hipError_t launch_group_general(const uint8_t *const *w, const int64_t *n, float
     if (lds_x > kMaxLds) return hipErrorInvalidValue;
     int64_t total = 0;
     for (int i = 0; i < count; i++) total += n[i];
-    const int T = 1 << cheapest_team(total, spr);
     const int64_t want = compute_units();
     int64_t n_wg = total < want ? total : want;
     int64_t rows_per_wg = (total + n_wg - 1) / n_wg;
@@ -874,16 +886,14 @@ hipError_t launch_group_general(const uint8_t *const *w, const int64_t *n, float
     }
     grp.wg_begin[pmh::kMaxGemvGroup] = begin;
     const dim3 grid((unsigned)begin);
-    const int teams_per_wave = 64 / T;
-    int best_waves = 16;
-    int64_t best_cost = INT64_MAX;
-    for (int waves = 16; waves >= 1; waves--) {  // ties go to more waves: more bytes in flight
-        const int64_t teams = (int64_t)waves * teams_per_wave;
-        const int64_t per_team = (rows_per_wg + teams - 1) / teams;
-        if (per_team < best_cost) best_cost = per_team, best_waves = waves;
+    int log_t = whole_team(spr);
+    TeamsB best = teams_b(rows_per_wg, spr, log_t);
+    for (int log = 6; log > whole_team(spr); log--) {
+        const TeamsB t = teams_b(rows_per_wg, spr, log);
+        if (t.cost < best.cost) log_t = log, best = t;
     }
-    const int per_team = (int)((rows_per_wg + (int64_t)best_waves * teams_per_wave - 1) / ((int64_t)best_waves * teams_per_wave));
-    const dim3 block((unsigned)best_waves * 64);
+    const int T = 1 << log_t, per_team = best.per_team;
+    const dim3 block(64 * kTeamWaves);
     if (order == pmh::kOrderRef)
         return xf32 ? launch_general<0, true>(T, grid, block, lds_x, s, grp, x, spr, (int)rows_per_wg, per_team)
                     : launch_general<0, false>(T, grid, block, lds_x, s, grp, x, spr, (int)rows_per_wg, per_team);

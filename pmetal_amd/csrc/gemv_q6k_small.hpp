@@ -290,7 +290,7 @@ __device__ __forceinline__ void q6k_row_body(const uint8_t *__restrict__ W, cons
 template <int T, bool XF32>
 __device__ __forceinline__ void q6k_member_body(const uint8_t *__restrict__ W, const void *__restrict__ xg, float *__restrict__ y,
                                                 int n_rows, int spr, int block, int n_blocks, int teams_per_wg, uint4 *smem) {
-    if (!(XF32 && T == 8) && n_rows <= n_blocks * teams_per_wg) {  // (f32 x beside the Q4_K digits of eight-lane teams: a spill)
+    if (n_rows <= n_blocks * teams_per_wg) {
         const int mine = (int)threadIdx.x / T, team = mine < teams_per_wg ? block * teams_per_wg + mine : n_rows;
         q6k_row_body<T, XF32, 1>(W, xg, y, n_rows, spr, team, smem);
     } else {

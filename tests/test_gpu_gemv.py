@@ -351,6 +351,17 @@ def test_qgemv_batch_takes_a_q6k_projection_into_a_large_q4k_group(oracle, order
     mixed_group_case(oracle, order, rows, k, x_dtype)
 
 
+# The team of a mixed launch: rows of 3 and 5 chunks of a wave (bf16: Q6_K two rows at a time), odd numbers of super-blocks with teams that a row does
+# not fill, and more Q6_K rows than a launch with f32 activations has such teams for (the two kinds then go one after the other).
+@pytest.mark.parametrize("rows,k,x_dtype", [([311, 186, 106], 6144, pm.DTYPE_BF16), ([301, 300], 10240, pm.DTYPE_BF16), ([301, 300], 6144, pm.DTYPE_F32),
+                                            ([166, 711, 2676], 1536, pm.DTYPE_BF16), ([522, 467, 718, 3695], 1280, pm.DTYPE_BF16),
+                                            ([1281, 1279], 1280, pm.DTYPE_F32), ([700, 4001], 768, pm.DTYPE_F32), ([1000, 20001], 256, pm.DTYPE_F32),
+                                            ([1000, 20001], 256, pm.DTYPE_BF16), ([5001, 64], 256, pm.DTYPE_F32)])
+@pytest.mark.parametrize("order", [0, 1])
+def test_qgemv_batch_teams_of_a_mixed_group(oracle, order, rows, k, x_dtype):
+    mixed_group_case(oracle, order, rows, k, x_dtype)
+
+
 def mixed_group_case(oracle, order, rows, k, x_dtype):
     from pmetal_amd import _lib
     lib = _lib.load()
