@@ -238,8 +238,10 @@ hipError_t launch_qgemv(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         const size_t lds = slots * 64 * planes + slots * 16;
         // Rows of five super-blocks, which no team but one of eight lanes takes whole, of a tall matrix: two rows a team at a time, x
         // converted by fewer workgroups (us, two rows / a row a team: 24000 x 1280 9.9 / 9.7, 32000 x 1280 10.3 / 11.7, 128256 x 1280 32.0 / 32.9
-        // with 16 rows per team from 65536 rows on).  Any other shape is faster with a team a row.
-        if (spr == 5 && n > 24576) {
+        // with 16 rows per team from 65536 rows on).  So are tall matrices of one or two super-blocks a row with f32 x, which is the most to convert:
+        // 11733 x 512 6.1 / 4.0, 16826 6.5 / 6.7, 26787 6.9 / 7.9, 45517 10.2 / 9.9, 57437 10.5 / 14.7; 42519 x 256 6.4 / 6.5, 60965 6.8 / 8.1,
+        // 76091 10.1 / 9.6, 115881 10.5 / 12.6.  Any other shape is faster with a team a row (three super-blocks, f32, 39488 x 768 12.8 / 10.9).
+        if ((spr == 5 && n > 24576) || (xf32 && ((spr == 2 && n >= 16384) || (spr == 1 && n >= 49152)))) {
             const unsigned grid = grid_for_rows(n, 32, n >= 65536 ? 16 : rows_per_team());
             return xf32 ? launch(k_qgemv_q6k<true>, grid, lds, s, w, x, y, (int)n, spr) : launch(k_qgemv_q6k<false>, grid, lds, s, w, x, y, (int)n, spr);
         }

@@ -48,10 +48,11 @@ def test_qgemv_matches_dequantize_then_matmul(oracle, t, n, k, x_dtype):
 
 
 # A team of 1 to 64 lanes per row of Q4_K or Q6_K (k / 256 groups of eight lanes) or Q8_0 (k / 32 lanes): rows that no team takes whole, one, two, three and
-# more chunks, row counts around the teams of a workgroup, workgroups of 64, 128 and 256 threads, and (24577 x 1280) two rows a team.
+# more chunks, row counts around the teams of a workgroup, workgroups of 64, 128 and 256 threads, and (24577 x 1280; f32 also 16385 x 512,
+# 49153 x 256) two rows a team.
 ROW_CASES = [(Q6K, 1, 1280), (Q6K, 255, 2304), (Q6K, 1025, 3584), (Q6K, 2049, 3072), (Q6K, 1700, 4352), (Q6K, 4097, 1280), (Q6K, 8191, 1280),
              (Q4K, 1, 1280), (Q4K, 2047, 768), (Q4K, 255, 2304), (Q4K, 8193, 2304), (Q4K, 1025, 3584), (Q4K, 4097, 4352), (Q4K, 300, 11008), (Q4K, 8191, 1280),
-             (Q6K, 13999, 768), (Q6K, 24577, 1280), (Q6K, 300, 11008), (Q6K, 33, 14336), (Q6K, 3073, 512),
+             (Q6K, 13999, 768), (Q6K, 24577, 1280), (Q6K, 300, 11008), (Q6K, 33, 14336), (Q6K, 3073, 512), (Q6K, 16383, 512), (Q6K, 16385, 512), (Q6K, 49153, 256),
              (Q8_0, 1, 32), (Q8_0, 300, 32), (Q8_0, 1000, 64), (Q8_0, 77, 128), (Q8_0, 4099, 160), (Q8_0, 515, 224), (Q8_0, 9, 288),
              (Q8_0, 8191, 1280), (Q8_0, 1025, 2080), (Q8_0, 2047, 3584), (Q8_0, 300, 11008), (Q8_0, 13999, 768)]
 
