@@ -296,7 +296,7 @@ void par_copy(void *dst, const void *src, size_t bytes) {
         memcpy(dst, src, bytes);
         return;
     }
-    const size_t piece = (bytes / kCopyThreads + 4095) & ~(size_t)4095;
+    const size_t piece = ((bytes + kCopyThreads - 1) / kCopyThreads + 4095) & ~(size_t)4095;  // (all of them together at least `bytes`)
     std::thread helpers[kCopyThreads - 1];
     for (int i = 1; i < kCopyThreads; i++) {
         const size_t off = piece * (size_t)i, len = off < bytes ? (bytes - off < piece ? bytes - off : piece) : 0;

@@ -1,8 +1,11 @@
 """GPU parity: quantize / dequantize through the C ABI must equal the CPU oracle bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import pmetal_amd as pm
+from pmetal_amd import _lib
 from gpu_util import Q4K, Q6K, Q8_0, first_mismatch, gpu_dequantize_dev, gpu_quantize_dev, weights
 
 pytestmark = pytest.mark.gpu
@@ -275,6 +278,25 @@ def test_quantize_random_bit_exact(oracle, t, n, outl):
 def test_quantize_host_pointer_entry_point(oracle, t):
     x = weights(7 + t, 256 * 40 + (13 if t == Q8_0 else 0))
     assert np.array_equal(pm.quantize(x, t), oracle.quantize(t, x))
+
+
+@pytest.mark.parametrize("t,n", [(Q8_0, 4750880), (Q6K, 12548352)])
+def test_host_pointer_entry_points_copy_the_last_bytes(t, n):
+    """The last staging chunk's blocks are two bytes more than a multiple of 16 KiB, which the copy threads share out."""
+    lib = _lib.load()
+    chunk = min(max((n // 4 + 8191) // 8192 * 8192, 256 << 10), 4 << 20)
+    last = lib.pmetal_hip_tensor_size(t, n - 3 * chunk)
+    assert last >= 1 << 20 and last % 16384 == 2
+    x = weights(t, n)
+    want = gpu_quantize_dev(t, x)
+    got = np.full(want.size + 16, 0xA5, np.uint8)
+    pm.check(lib.pmetal_hip_quantize(t, x.ctypes.data, n, got.ctypes.data, want.size))
+    assert np.array_equal(got[:want.size], want) and np.all(got[want.size:] == 0xA5)
+    bad = got[:want.size].copy()
+    back, ref = np.empty(n, np.float32), gpu_dequantize_dev(t, want, n)
+    shape = (C.c_int32 * 1)(n)
+    pm.check(lib.pmetal_hip_dequantize(t, bad.ctypes.data, bad.size, shape, 1, back.ctypes.data, n, 0))
+    assert np.array_equal(back.view(np.uint32), ref.view(np.uint32))
 
 
 @pytest.mark.parametrize("n", [11_000_000 + 123, 20_000_000 + 7, 1_500_000 + 31, 262_144])
