@@ -15,9 +15,9 @@
 #include <map>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
+#include "host_copy.hpp"
 #include "internal.hpp"
 
 namespace {
@@ -257,7 +257,7 @@ int32_t scratch_of_current_device(NoAllocScratch **out) {
 constexpr size_t kPipeElems = (size_t)4 << 20;  // 16 MiB of f32; a multiple of every block size
 constexpr size_t kPipeQBytes = kPipeElems / 256 * 292;  // the largest encoded chunk (Q8_K)
 constexpr size_t kPipeGrain = 8192, kPipeMinElems = (size_t)256 << 10;  // chunks are multiples of the grain, at least 1 MiB of f32
-constexpr int kPipeSlots = 3, kCopyThreads = 4;  // measured: 26 / 38 / 41 / 41 GB/s with 1 / 2 / 4 / 8 copy threads
+constexpr int kPipeSlots = 3;
 
 struct PipeSlot {
     float *h_f32 = nullptr, *d_f32 = nullptr;
@@ -289,23 +289,6 @@ int32_t host_pipe(HostPipe **out) {  // caller holds g_pipe_mutex
     }
     *out = &p;
     return PMETAL_HIP_OK;
-}
-
-void par_copy(void *dst, const void *src, size_t bytes) {
-    if (bytes < ((size_t)1 << 20)) {
-        memcpy(dst, src, bytes);
-        return;
-    }
-    const size_t piece = ((bytes + kCopyThreads - 1) / kCopyThreads + 4095) & ~(size_t)4095;  // (all of them together at least `bytes`)
-    std::thread helpers[kCopyThreads - 1];
-    for (int i = 1; i < kCopyThreads; i++) {
-        const size_t off = piece * (size_t)i, len = off < bytes ? (bytes - off < piece ? bytes - off : piece) : 0;
-        helpers[i - 1] = std::thread([=] {
-            if (len) memcpy((uint8_t *)dst + off, (const uint8_t *)src + off, len);
-        });
-    }
-    memcpy(dst, src, piece < bytes ? piece : bytes);
-    for (std::thread &h : helpers) h.join();
 }
 
 // quantize == true: f32 at `plain` -> blocks at `packed`; false: the other way (n elements, element order `order`).
@@ -774,20 +757,20 @@ int32_t codec_pipelined(bool quantize, uint32_t t, float *plain, uint8_t *packed
     auto retire = [&](size_t i) -> int32_t {  // chunk i's result: staging buffer -> caller's memory
         PipeSlot &sl = p->slot[i % kPipeSlots];
         HIP_TRY(hipEventSynchronize(sl.done));
-        if (quantize) par_copy(packed + i * q_chunk, sl.h_q, pmetal_hip_tensor_size(t, elems_of(i)));
-        else par_copy(plain + i * chunk, sl.h_f32, elems_of(i) * sizeof(float));
+        if (quantize) pmh::par_copy(packed + i * q_chunk, sl.h_q, pmetal_hip_tensor_size(t, elems_of(i)));
+        else pmh::par_copy(plain + i * chunk, sl.h_f32, elems_of(i) * sizeof(float));
         return PMETAL_HIP_OK;
     };
     auto submit = [&](size_t i) -> int32_t {
         PipeSlot &sl = p->slot[i % kPipeSlots];
         const size_t elems = elems_of(i), qb = pmetal_hip_tensor_size(t, elems);
         if (quantize) {
-            par_copy(sl.h_f32, plain + i * chunk, elems * sizeof(float));
+            pmh::par_copy(sl.h_f32, plain + i * chunk, elems * sizeof(float));
             HIP_TRY(hipMemcpyAsync(sl.d_f32, sl.h_f32, elems * sizeof(float), hipMemcpyHostToDevice, sl.st));
             if (int32_t r = pmetal_hip_quantize_dev(t, sl.d_f32, elems, sl.d_q, qb, sl.st)) return r;
             HIP_TRY(hipMemcpyAsync(sl.h_q, sl.d_q, qb, hipMemcpyDeviceToHost, sl.st));
         } else {
-            par_copy(sl.h_q, packed + i * q_chunk, qb);
+            pmh::par_copy(sl.h_q, packed + i * q_chunk, qb);
             HIP_TRY(hipMemcpyAsync(sl.d_q, sl.h_q, qb, hipMemcpyHostToDevice, sl.st));
             if (int32_t r = pmetal_hip_dequantize_dev(t, sl.d_q, qb, sl.d_f32, elems, order, sl.st)) return r;
             HIP_TRY(hipMemcpyAsync(sl.h_f32, sl.d_f32, elems * sizeof(float), hipMemcpyDeviceToHost, sl.st));

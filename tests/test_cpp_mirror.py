@@ -29,3 +29,13 @@ def test_cpp_mirror_host_only(tmp_path):
 def test_cpp_mirror_on_gpu(tmp_path):
     r = subprocess.run([_build(tmp_path)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_host_copy_without_threads(tmp_path):
+    """A thread that cannot be made is no exception out of a C entry point: the calling thread copies its share."""
+    exe = str(tmp_path / "test_host_copy")
+    # (libstdc++ linked in, so that its call of pthread_create is the one that is wrapped)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", os.path.join(ROOT, "tests", "cpp", "test_host_copy.cpp"), "-o", exe,
+                    "-static-libstdc++", "-pthread", "-Wl,--wrap=pthread_create"], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
