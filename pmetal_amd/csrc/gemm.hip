@@ -1201,6 +1201,10 @@ constexpr int kSmallMaxM2 = 32;  // Q4_K, Q5_K and Q8_0: two 16-row blocks of ac
 // rows of one to four super-blocks fit a compute unit than the launch counts on, and the last ones of a round waited for the others:
 // f32, three Q4_K weights of 24737 x 256, M = 9, 20.0 -> 14.3 us; Q6_K 33017 and 8456 x 1024, M = 6, 22.2 -> 16.1.)
 constexpr int kSmallKeepTiles = 8;
+// UNROLL: of the sum over the waves of one tile after the other.  Written out eight times it moves the rest of the kernel about: weights from
+// memory, M = 16, 14336 x 4096, us with 8 / 1: Q4_K 13.26 / 12.99, 60000 x 2048, M = 8, 21.24 / 21.16, Q3_K 17.67 / 17.61, Q2_K 13.43 / 13.35, but Q6_K 18.24 / 18.54, and 9000 x 3584,
+// M = 7, 19.3 / 21.4.
+template <int UNROLL>
 __device__ __forceinline__ void small_add_waves(float4_t *red, float4_t *keep, int ti, int wave, int nwaves, int lane, const float4_t acc,
                                                 float4_t *out_tiles) {
     if (keep) {  // workgroup-uniform
@@ -1212,6 +1216,7 @@ __device__ __forceinline__ void small_add_waves(float4_t *red, float4_t *keep, i
     __syncthreads();
     if (wave == 0) {
         float4_t v = red[buf * 64 + lane];
+#pragma unroll UNROLL
         for (int q = 1; q < nwaves; q++) {
             const float4_t u = red[(buf + q) * 64 + lane];
 #pragma unroll
@@ -1645,7 +1650,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small(const uint8_t 
         }
         if (XT) acc[0] *= up;
 #pragma unroll
-        for (int b = 0; b < MT; b++) small_add_waves(red, keep, ti * MT + b, wave, nwaves, lane, acc[b], out_tiles);
+        for (int b = 0; b < MT; b++) small_add_waves<1>(red, keep, ti * MT + b, wave, nwaves, lane, acc[b], out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRun<NSB, FMT> ring0, ring1;
@@ -1825,7 +1830,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q8(const uint8
         }
         if (XT) acc[0] *= up;
 #pragma unroll
-        for (int mb = 0; mb < MT; mb++) small_add_waves(red, keep, ti * MT + mb, wave, nwaves, lane, acc[mb], out_tiles);
+        for (int mb = 0; mb < MT; mb++) small_add_waves<1>(red, keep, ti * MT + mb, wave, nwaves, lane, acc[mb], out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRunQ8 ring0a, ring0b, ring1a, ring1b;  // (the b halves are unused with one run per wave)
@@ -2014,7 +2019,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small_q6(const uint8
                 }
         }
         acc *= up;
-        small_add_waves(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
+        small_add_waves<8>(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRunQ6<NSB> ring0, ring1;
@@ -2278,7 +2283,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_qgemm_small16(const uint8_
             for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(d, part[r], acc[r]);
         }
         acc *= up;
-        small_add_waves(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
+        small_add_waves<1>(red, keep, ti, wave, nwaves, lane, acc, out_tiles);
     };
     static_assert(kSmallDepth == 2, "the ring is written out as two tiles");
     SmallRun16<FMT, NSB> ring0, ring1;
