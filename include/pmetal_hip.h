@@ -151,7 +151,9 @@ int32_t pmetal_hip_quantize_dev(uint32_t ggml_type, const float *src_dev, size_t
  * the next kernel's first (a batch of one Q2_K or Q3_K tensor of 2^24 elements or more is cut in two for the same reason).
  * Asynchronous like the single call: the batch starts behind what
  * `stream` holds, and work given to `stream` afterwards runs behind every tensor of the batch.  All descriptors are checked
- * before anything is launched.  A batch issued while `stream` is being recorded runs on `stream` alone.               */
+ * before anything is launched.  A batch issued while `stream` is being recorded runs on `stream` alone.
+ * A Q4_K, Q5_K or Q6_K launch, of a batch or of a single call, is one large workgroup on every compute unit, with most of its LDS,
+ * until the launch's tensors are done: work on other streams waits for it meanwhile.                                   */
 typedef struct pmetal_hip_quantize_desc {
     uint32_t ggml_type;
     uint32_t reserved;

@@ -1141,8 +1141,8 @@ int32_t pmetal_hip_qgemm_batch(const pmetal_hip_gemm_desc *descs, size_t count, 
 
 // pmetal_hip_qgemm for callers that cannot allocate: the scratch is the fixed `scratch` array of the current device.
 // Calls no hipMalloc / hipFree and nothing else that allocates.  Every call on a device uses the same array, so calls that
-// overlap on one device race; nothing in it has to start at zero (the pre-pass writes every activation item and row scale
-// the main kernel reads, padding rows included, and a K split writes every partial tile before the reduction reads it).
+// overlap on one device race; nothing in it has to start at zero (a pre-pass, where there is one, writes every activation item and
+// row scale that the main kernel reads, padding rows included, and a K split writes every partial tile before the reduction reads it).
 int32_t pmetal_hip_qgemm_noalloc(uint32_t t, const uint8_t *w, int64_t n, int64_t k, const void *x, uint32_t x_dtype, int64_t m,
                                  void *y, uint32_t y_dtype, uint32_t order, void *stream) {
     if (int32_t rc = check_gemm(t, w, n, k, x, x_dtype, y, order)) return rc;
@@ -1202,14 +1202,16 @@ int32_t pmetal_hip_qlinear(uint32_t t, const uint8_t *w, int64_t n, int64_t k, c
         return fail(PMETAL_HIP_ERR_INVALID_SHAPE, "qlinear: a Q8_0 row of k=%lld (not a multiple of 256) runs through the GEMV, whose output is f32 only",
                     (long long)k);
     const bool q4k_pair = t == PMETAL_GGML_TYPE_Q4K && m == 2;
-    // Two rows of Q5_K, Q3_K or Q2_K through the short-batch GEMM beat two GEMVs (Q5_K: 17.3 against 23.1 us at 14336 x 4096,
-    // 11.6 against 12.9 at 6144 x 4096; Q2_K 14.6 against 19.2, Q3_K 17.1 against 22) except on a small weight, where the
-    // GEMM's two launches cost more than they save (Q5_K: 10.7 against 7.5 us at 1024 x 4096).
+    // Two rows of Q5_K, Q3_K or Q2_K through the short-batch GEMM beat two GEMVs (us of a recording, different weights in turn, GEMM / GEMVs: 14336 x
+    // 4096 Q5_K 16.4 / 23.8, Q3_K 17.5 / 21.6, Q2_K 13.2 / 18.3; 6144 x 4096 11.5 / 13.3, 12.8 / 13.3, 9.8 / 11.9) except on a small weight of long
+    // rows, where each takes as long as its chain of latencies (2048 x 4096 10.1 / 8.8, 12.0 / 8.7, 9.7 / 7.9; 1024 x 4096 10.0 / 7.7, 11.9 / 7.1, 9.6 /
+    // 6.8).  The line takes small weights of short rows to the GEMVs as well, which lose there (1024 x 1024 4.6 / 6.4, 4.9 / 5.8, 4.3 / 5.7).
     const bool row_loop_type = gemv_only_type(t) && m <= kRowLoopMax && n * k <= (int64_t(1) << 23);
     if ((q8_ragged || q4k_pair || row_loop_type) && y_dtype == PMETAL_HIP_DTYPE_F32 && m > 1 && n > 0 && k > 0 && x && y) {
         // The fused GEMM walks k in steps of 256, and a Q8_0 row may be any multiple of 32: one fused GEMV per activation row
-        // then, back to back on the stream.  Two Q4_K rows are two GEMVs: 13.7 against 16.1 us at 14336 x 4096
-        // (three rows: 19.6 against 16.4).
+        // then, back to back on the stream.  Two Q4_K rows are two GEMVs: 8.5 us against 9.6 at 4096 x
+        // 4096, and little longer where they are behind (13.8 against 13.5 at 14336 x 4096, 5.7 against 4.4 at 1024 x 1024); three rows are not (19.8 against
+        // 13.3 at 14336 x 4096).
         const size_t x_row = (size_t)k * (x_dtype == PMETAL_HIP_DTYPE_F32 ? 4 : 2);
         for (int64_t r = 0; r < m; r++) {
             const int32_t rc = pmetal_hip_qgemv(t, w, n, k, (const uint8_t *)x + (size_t)r * x_row, x_dtype,

@@ -778,7 +778,8 @@ struct TileCopy {
 
 // A workgroup has up to 16 waves, all that a compute unit holds at 128 registers, and its tiles, every gridDim.x-th, go to whichever
 // wave asks next: the older waves of a SIMD are served first, so that with equal shares some ended when others had half of theirs left
-// (Q4_K 14336 x 4096 114 -> 123 us, before the division above).  Workgroups of 8 and 4 waves: 91 and 98 us instead of 85.
+// (Q4_K 14336 x 4096 114 -> 123 us, before the division above).  16 / 8 / 4 waves, as many in all, on one machine (a warmer one than above): Q4_K
+// 107 / 112 / 113 us, Q5_K 102 / 109 / 110, Q6_K 157 / 166 / 175.
 constexpr int kTileWaves = 16;
 // The tensors of a launch, their tiles numbered through.  (A launch of its own for each left the vector units idle while its first tiles
 // came, 33 MB for the whole machine, and while its last ones were searched by few waves: the four layers' tensors 1433 -> 1317 us.)

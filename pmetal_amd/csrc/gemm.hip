@@ -1240,11 +1240,10 @@ __device__ __forceinline__ void small_add_kept(const float4_t *keep, int n_tiles
     }
 }
 
-// After the last tile: the finished tiles leave, scaled by the rows' powers of two (`rs`: that of row `lane`, requested when the
-// kernel starts: asked for here it would be a trip to memory at the kernel's end; put into LDS ahead of the loop instead of held, one
-// spilled register less in k_qgemm_small_q6<2, true>, Q6_K 14336 x 4096 at M = 16 went from 18.9 to 19.7 us); or, when a long row is cut into runs over
-// the grid's second dimension, as the fp32 partial tile of this run, not yet scaled, for k_rw_reduce.  A thread takes a lane
-// slot: four rows of one column.
+// After the last tile: the finished tiles leave; or, when a long row is cut into runs over the grid's second dimension, as the fp32
+// partial tile of this run for k_rw_reduce.  Of at most 16 rows every wave has scaled its tiles (`rs` is 1, k_rw_reduce is given no scales).
+// Of two blocks of rows they are scaled by the rows' powers of two, here or by k_rw_reduce (`rs`: that of row `lane`, requested when the
+// kernel starts: asked for here it would be a trip to memory at the kernel's end).  A thread takes a lane slot: four rows of one column.
 // (mt: 16-row blocks of activations per row tile of weights; the finished tile of block b of row tile ti is slot ti * mt + b)
 __device__ __forceinline__ float small_row_scale(const float *__restrict__ rowscale) { return rowscale[threadIdx.x & 31]; }
 
@@ -2505,8 +2504,8 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     bool waves;
     if (m <= kSmallMaxM) {
         // The short-batch kernels' workgroups walk 16 super-blocks of a row at a time however few of them there are, and add the
-        // runs of a longer row in a third launch; the tile kernel's waves share what there is.  Tile kernel against them, us at
-        // M = 12 and how many times faster:
+        // runs of a longer row in a launch behind; the tile kernel's waves share what there is.  Tile kernel against them, us at
+        // M = 12 and how many times faster (both behind a pre-pass, 1 to 3 us of which a short-batch launch of its own no longer takes):
         //   rows of 9 to 12 super-blocks, without a K split, so that a second weight can share the launch: ahead for every type up to
         //     7168 rows of nine and 4096 of twelve (1.05 to 1.33; two weights of 4096 rows of ten together 1.07 to 1.18).  Above, the
         //     types part: 12288 rows of nine Q3_K 16.1 -> 12.9, Q5_K 15.8 -> 15.2, 9216 rows Q8_0 15.7 -> 16.3; 8192 rows of twelve
