@@ -818,7 +818,7 @@ constexpr size_t rw16_lds_bytes() {
 // Q6_K (crates/pmetal-gguf/src/k_quants.rs:474-496: 210-byte super-blocks: ql[128] low nibbles, qh[64] top two
 // bits, 16 int8 scales, f16 d; value d * sc * (q - 32)).  Same structure as the Q4_K kernel, with these differences:
 //   * sc * (q - 32) can reach 4096 and is not always exact in f16, so it is split where the storage splits it,
-//     q - 32 = 16 (hi2 - 2) + nib, into two exact tiles  B1 = (16 sc) (hi2 - 2)  and  B2 = sc * nib  that multiply
+//     q - 32 = 16 (hi2 - 2) + nib, into two exact tiles  B1 = (16 sc) (hi2 - 2)  and  B2 = sc * nib  (1/32 of each) that multiply
 //     the same activation fragment one after the other (a fragment read from LDS feeds two matrix instructions);
 //   * no min term; one scale per 16 elements;
 //   * a half super-block of a row is 64 bytes of ql and 32 of qh; lane (n, g) multiplies ql bytes 32 g .. 32 g + 31
@@ -877,14 +877,14 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
     const uint32_t hd[8] = {ha.x >> hs, ha.y >> hs, ha.z >> hs, ha.w >> hs, hc.x >> hs, hc.y >> hs, hc.z >> hs, hc.w >> hs};
     // scales 8 H + 2 g + t / 4 (low nibbles) and 8 H + 4 + 2 g + t / 4 (high nibbles)
     const uint32_t wlo = (H == 0 ? R.sc.x : R.sc.z) >> (16u * (uint32_t)g), whi = (H == 0 ? R.sc.y : R.sc.w) >> (16u * (uint32_t)g);
-    half2_t s2[2][2], s1[2][2];  // [k-step / 4][low, high]
+    half2_t sc[2][2];  // [k-step / 4][low, high]
 #pragma unroll
     for (int th = 0; th < 2; th++) {
-        const float fl = (float)(int)(int8_t)(wlo >> (8 * th)), fh = (float)(int)(int8_t)(whi >> (8 * th));
-        const _Float16 l2 = (_Float16)fl, h2 = (_Float16)fh, l1 = (_Float16)(16.0f * fl), h1 = (_Float16)(16.0f * fh);  // exact: |sc| <= 128
-        s2[th][0] = half2_t{l2, l2}, s2[th][1] = half2_t{h2, h2};
-        s1[th][0] = half2_t{l1, l1}, s1[th][1] = half2_t{h1, h1};
+        const _Float16 lo = (_Float16)(float)(int)(int8_t)(wlo >> (8 * th)), hi = (_Float16)(float)(int)(int8_t)(whi >> (8 * th));
+        sc[th][0] = half2_t{lo, lo}, sc[th][1] = half2_t{hi, hi};
     }
+    Q6Scales sv;
+    sv.set(sc[0][0], sc[0][1]);
 
     // software pipeline in issue order, as in the Q4_K kernel; every fragment feeds two matrix instructions
     constexpr int kSlots = 2 * MB;
@@ -893,7 +893,7 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
 #pragma unroll
     for (int i = 0; i < MB; i++) af[0][i] = __builtin_bit_cast(half8_t, a_cur[g * BM + 32 * i + col]);
 #pragma unroll
-    for (int c = 0; c < 8; c++) dq6_chunk(c, qd[0], hd[0], s2[0], s1[0], dq);
+    for (int c = 0; c < 8; c++) dq6_chunk(c, qd[0], hd[0], sv, dq);
 #pragma unroll
     for (int t = 0; t < 8; t++) {
         const half8_t b1 = dq.b1(), b2 = dq.b2();
@@ -912,8 +912,10 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
             }
             if (t < 7) {
 #pragma unroll
-                for (int ch = slot * 8 / kSlots; ch < (slot + 1) * 8 / kSlots; ch++)
-                    dq6_chunk(ch, qd[t + 1], hd[t + 1], s2[(t + 1) >> 2], s1[(t + 1) >> 2], dq);
+                for (int ch = slot * 8 / kSlots; ch < (slot + 1) * 8 / kSlots; ch++) {
+                    if (t == 3 && ch == 0) sv.set(sc[1][0], sc[1][1]);
+                    dq6_chunk(ch, qd[t + 1], hd[t + 1], sv, dq);
+                }
                 if (slot == 0) {
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -925,7 +927,7 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
         }
     }
     if (H == 1) {
-        const float d = f16_bits_to_f32(R.d);
+        const float d = kQ6OperandScale * f16_bits_to_f32(R.d);
 #pragma unroll
         for (int i = 0; i < MB; i++)
 #pragma unroll

@@ -109,29 +109,40 @@ struct Block16 {  // FMT 2: Q3_K, 3: Q2_K
 
 constexpr int kQ6Bytes = 210, kQ6Groups = 16, kQ6Stage = 192;  // LDS items of a wave's quant stage: 128 ql + 64 qh
 
-// The two operands of one k-step, built in eight pieces that are placed between matrix instructions.
+// The two operands of one k-step, built in eight pieces that are placed between matrix instructions: 1/32 of sc * nib and of
+// 16 sc * (hi2 - 2), so that every multiplier and offset of a packed f16 fma is a number f16 holds (the kernels multiply d by 32).
+// 0x6400 | nib is the f16 1024 + nib: times sc / 32, less 32 sc.  0x40 | hi2 as the upper byte is the f16 2 + hi2 / 2: times sc,
+// less 3 sc.  All of it exact for |sc| <= 128.  22 vector instructions a k-step; an addition and a multiplication a pair, with the
+// unscaled values, were 30.  The row kernel is bound by in-order issue at two waves a SIMD, the tile kernel by memory: us of a call, 30 -> 22,
+// 4096 x 14336 M = 2048 419 -> 407, 14336 x 4096 M = 512 116 -> 113, M = 128 51.8 -> 50.0, M = 64 30.0 -> 29.4.
 struct Dq6 {
     uint32_t nlo, nhi, hlo, hhi;
     half2_t r1[4], r2[4];
     __device__ __forceinline__ half8_t b1() const { return half8_t{r1[0][0], r1[0][1], r1[1][0], r1[1][1], r1[2][0], r1[2][1], r1[3][0], r1[3][1]}; }
     __device__ __forceinline__ half8_t b2() const { return half8_t{r2[0][0], r2[0][1], r2[1][0], r2[1][1], r2[2][0], r2[2][1], r2[3][0], r2[3][1]}; }
 };
-// qlw: the ql dword of the k-step; qhw: its qh dword already shifted by 2 g; s2 / s1: (sc, sc) and (16 sc, 16 sc)
-// of the low-nibble and of the high-nibble elements.  0x6400 | v is the f16 1024 + v; both steps of each value are exact.
-__device__ __forceinline__ void dq6_chunk(const int c, const uint32_t qlw, const uint32_t qhw, const half2_t (&s2)[2],
-                                          const half2_t (&s1)[2], Dq6 &d) {
-    const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f}, m1026 = {(_Float16)-1026.0f, (_Float16)-1026.0f};
-    const uint32_t sel = (c & 1) ? 0x04030402u : 0x04010400u;  // bytes (b0, b1) resp. (b2, b3) -> 0x64bb pairs
+constexpr float kQ6OperandScale = 32.0f;
+struct Q6Scales {  // of the low-nibble and of the high-nibble elements of four k-steps
+    half2_t sc[2], sc32[2], off[2], off3[2];
+    __device__ __forceinline__ void set(const half2_t lo, const half2_t hi) {
+        const half2_t c32 = {(_Float16)0.03125f, (_Float16)0.03125f}, m32 = {(_Float16)-32.0f, (_Float16)-32.0f}, m3 = {(_Float16)-3.0f, (_Float16)-3.0f};
+        sc[0] = lo, sc[1] = hi;
+#pragma unroll
+        for (int i = 0; i < 2; i++) sc32[i] = sc[i] * c32, off[i] = sc[i] * m32, off3[i] = sc[i] * m3;
+    }
+};
+// qlw: the ql dword of the k-step; qhw: its qh dword already shifted by 2 g
+__device__ __forceinline__ void dq6_chunk(const int c, const uint32_t qlw, const uint32_t qhw, const Q6Scales &s, Dq6 &d) {
     if (c == 0) d.nlo = qlw & 0x0F0F0F0Fu;
     if (c == 2) d.nhi = (qlw >> 4) & 0x0F0F0F0Fu;
-    if (c == 4) d.hlo = qhw & 0x03030303u;
-    if (c == 6) d.hhi = (qhw >> 4) & 0x03030303u;
-    if (c < 4) {
-        const uint32_t v = c < 2 ? d.nlo : d.nhi;
-        d.r2[c] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + m1024) * s2[c >> 1];
-    } else {
-        const uint32_t v = c < 6 ? d.hlo : d.hhi;
-        d.r1[c - 4] = (__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + m1026) * s1[(c - 4) >> 1];
+    if (c == 4) d.hlo = (qhw & 0x03030303u) | 0x40404040u;
+    if (c == 6) d.hhi = ((qhw >> 4) & 0x03030303u) | 0x40404040u;
+    if (c < 4) {  // bytes (b0, b1) resp. (b2, b3) -> 0x64bb pairs
+        const uint32_t v = __builtin_amdgcn_perm(0x64646464u, c < 2 ? d.nlo : d.nhi, (c & 1) ? 0x04030402u : 0x04010400u);
+        d.r2[c] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, v), s.sc32[c >> 1], s.off[c >> 1]);
+    } else {  // ... -> 0xbb00 pairs (selector 12 is a zero byte)
+        const uint32_t v = __builtin_amdgcn_perm(0u, c < 6 ? d.hlo : d.hhi, (c & 1) ? 0x030C020Cu : 0x010C000Cu);
+        d.r1[c - 4] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, v), s.sc[(c - 4) >> 1], s.off3[(c - 4) >> 1]);
     }
 }
 

@@ -126,21 +126,20 @@ struct KwQ6 {
     const uint4 *row_;
     int i_, g_;
     uint32_t q[4], h[4];  // of four k-steps
-    half2_t s2[2][2], s1[2][2];
+    half2_t sc[2][2];  // [k-step / 4][low, high]
+    Q6Scales s;
     float d;
     template <int H>
     __device__ __forceinline__ void load(const uint4 *st, const int row, const int g) {
         row_ = st, i_ = row, g_ = g;
         const uint4 sv = st[slot(6, row)];
-        d = f16_bits_to_f32(reinterpret_cast<const uint32_t *>(st + slot(7, row))[3] >> 16);
+        d = kQ6OperandScale * f16_bits_to_f32(reinterpret_cast<const uint32_t *>(st + slot(7, row))[3] >> 16);
         // scales 8 H + 2 g + t / 4 (low nibbles) and 8 H + 4 + 2 g + t / 4 (high nibbles)
         const uint32_t wlo = (H == 0 ? sv.x : sv.z) >> (16u * (uint32_t)g), whi = (H == 0 ? sv.y : sv.w) >> (16u * (uint32_t)g);
 #pragma unroll
         for (int th = 0; th < 2; th++) {
-            const float fl = (float)(int)(int8_t)(wlo >> (8 * th)), fh = (float)(int)(int8_t)(whi >> (8 * th));
-            const _Float16 l2 = (_Float16)fl, h2 = (_Float16)fh, l1 = (_Float16)(16.0f * fl), h1 = (_Float16)(16.0f * fh);  // exact: |sc| <= 128
-            s2[th][0] = half2_t{l2, l2}, s2[th][1] = half2_t{h2, h2};
-            s1[th][0] = half2_t{l1, l1}, s1[th][1] = half2_t{h1, h1};
+            const _Float16 lo = (_Float16)(float)(int)(int8_t)(wlo >> (8 * th)), hi = (_Float16)(float)(int)(int8_t)(whi >> (8 * th));
+            sc[th][0] = half2_t{lo, lo}, sc[th][1] = half2_t{hi, hi};
         }
     }
     template <int H>
@@ -150,10 +149,11 @@ struct KwQ6 {
             const uint32_t hs = 2u * (uint32_t)g_;
             q[0] = v.x, q[1] = v.y, q[2] = v.z, q[3] = v.w;
             h[0] = w.x >> hs, h[1] = w.y >> hs, h[2] = w.z >> hs, h[3] = w.w >> hs;
+            s.set(sc[t >> 2][0], sc[t >> 2][1]);
         }
         Dq6 v;
 #pragma unroll
-        for (int c = 0; c < 8; c++) dq6_chunk(c, q[t % 4], h[t % 4], s2[t >> 2], s1[t >> 2], v);
+        for (int c = 0; c < 8; c++) dq6_chunk(c, q[t % 4], h[t % 4], s, v);
         b[0] = v.b1(), b[1] = v.b2();
     }
     __device__ __forceinline__ half8_t sums(int) const { return half8_t{0, 0, 0, 0, 0, 0, 0, 0}; }
