@@ -4,9 +4,10 @@
 // The kernels of gemm.hip give every wave its own weight rows and fill the machine with a K split over workgroups, whose
 // partial tiles a second launch adds: at M = 64 their loop has 0.5 us of matrix work per step and waits for memory in each,
 // and prepare + multiply + add are three dependent launches.  Here a workgroup owns a tile of 32 MB activation rows x 32 NR
-// weight rows for the whole of K.  Its (up to) eight waves take consecutive runs of super-blocks, run without a barrier from
+// weight rows for the whole of K.  Its (up to) eight waves take every eighth super-block each, run without a barrier from
 // start to end, and their fp32 tiles are added through LDS in wave order: no partial tiles in memory, no third launch, and
-// the result does not depend on scheduling.
+// the result does not depend on scheduling.  (Consecutive runs of super-blocks, which is what the waves took before, lie far apart in
+// a row: 1 to 5 % slower, two Q4_K weights of 14336 x 4096 M = 64 38.6 -> 36.8 us, Q5_K 8192 x 4096 M = 100 24.6 -> 23.4.)
 //   * Weights: a wave copies a unit of its rows (one or half a super-block of 32 NR rows) directly global -> LDS, one unit
 //     ahead, into LDS of its own; a lane (row n = lane % 32, half g = lane / 32) reads its quants and scales back and
 //     makes the exact f16 operands of gemm_common.hpp.
@@ -16,7 +17,10 @@
 //     unit is never longer than that for its first fragments.
 //   * The operands of k-step s + 1 are made between the matrix instructions of step s.
 //
-// What bounds it: no one unit.  The time goes in whole rounds of 256 workgroups, each as long as its share of the row: 7 us, launch and
+// What bounds it: a compute unit's path to memory, through which weights and activations come in the order of their requests.  By time stamps
+// (Q4_K 14336 x 4096 M = 64, 224 workgroups of 64 x 64), a wave's first requests are all issued 1.1 to 8.7 us after its start and its loop ends
+// 8.8 to 15.2 us after it: what waits for weights from HBM holds up the activations behind it, 0.74 MB a workgroup at 26
+// bytes a clock.  Adding the tiles takes 1.2 us of it.  The time goes in whole rounds of 256 workgroups, each as long as its share of the row: 7 us, launch and
 // pre-pass included, and per round and eight super-blocks of a row 2.9 (Q2_K), 3.5 (Q4_K, Q3_K), 4.6 (Q5_K), 4.9 us (Q8_0, Q6_K) with 32 x
 // 32 tiles (up to 32 activation rows, rows of 32 super-blocks and more); 0.6 to 0.8 of that where fewer than 64 workgroups run.  Inside, by
 // counters (share of the waves' time that they issue / are ready and cannot issue / wait for memory, LDS or each other; share of the
@@ -41,6 +45,12 @@ __device__ __forceinline__ const uint8_t *at(const uint8_t *p, uint32_t off) {
     asm("" : "+v"(off));
     return p + off;
 }
+
+// Neighbouring results of a row, which may begin at any of them.
+template <class T, int ALIGN, int COUNT>
+struct __attribute__((packed, aligned(ALIGN))) RowPiece {
+    T v[COUNT > 0 ? COUNT : 1];
+};
 
 // 16 bytes per lane from a buffer to LDS (lane l lands at dst + 16 l).  The buffer form and not dma16(): the compiler takes a
 // global load into LDS for an access to either memory and waits for everything outstanding at the next use of any load.
@@ -269,6 +279,10 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
 
 // ------------------------------------------------------------------------------------------------
 constexpr int kKwWaves = 8;
+// A wave's accumulators lie in LDS as the 64 lanes' 16-byte slots (four rows of one column), lane l at tile_slot(l): a thread that
+// reads four neighbouring columns back and one that writes its slot meet 64 different banks with the 15 beside them.
+constexpr int kTileRun = 76;
+__device__ __forceinline__ int tile_slot(const int l) { return 20 * (l & 3) + (l >> 2); }
 
 template <class F, int MB, int NR>
 struct Kw {
@@ -276,9 +290,9 @@ struct Kw {
     static constexpr int kSteps = 8 + F::kSums;                                        // k-steps and sum steps of a half
     // k-steps of activation fragments in flight: a divisor of the steps of a super-block
     static constexpr int kDepth = F::kSums == 1 ? 6 : F::kSums == 2 ? (MB * NR == 4 ? 4 : 5) : (MB * NR == 4 ? 2 : 4);
-    static constexpr int kTile = MB * NR * 4 * 64;                                     // 16-byte slots of a wave's fp32 tile
+    static constexpr int kTile = MB * NR * 4 * kTileRun;                               // 16-byte slots of a wave's fp32 tile
     static_assert((2 * kSteps) % kDepth == 0, "the ring's slots are picked at compile time");
-    static_assert(kDepth <= 8, "a unit's copies must be older than the fragments in flight when it is used");
+    static_assert(kDepth <= kSteps, "a unit's copies must be older than the fragments in flight when it is used");
 };
 
 template <class F, int MB, int NR>
@@ -303,10 +317,11 @@ struct KwCopy {  // a wave's copies of one unit
 };
 
 // Half H of a super-block.  cur: the staged unit; nxt: where the copies of the next unit go (half HN of the super-block at
-// sb_next of every row); xa: the items of the k-step whose fragments are requested next.
+// sb_next of every row); xa: the items of the k-step whose fragments are requested next; jump: from the end of this super-block's
+// items to the wave's next ones.
 template <class F, int MB, int NR, int H, bool NEXT>
 __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__restrict__ nxt, const __amdgpu_buffer_rsrc_t r, const uint32_t sb_next,
-                                        const KwCopy<F, MB, NR> &C, const uint8_t *__restrict__ &xa, const uint32_t step, const uint32_t a_off,
+                                        const KwCopy<F, MB, NR> &C, const uint8_t *__restrict__ &xa, const uint32_t step, const uint32_t jump, const uint32_t a_off,
                                         half8_t (&af)[Kw<F, MB, NR>::kDepth][MB], const int lane, float16_t (&acc)[NR][MB], float16_t (&part)[NR][MB]) {
     using K = Kw<F, MB, NR>;
     const int col = lane & 31, g = lane >> 5;
@@ -356,6 +371,7 @@ __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__
                 }
             }
         // the slot takes the fragments of kDepth steps on (past the last step: items of another wave, or the slack behind them)
+        if (H == 1 && s == K::kSteps - K::kDepth) xa += jump;
 #pragma unroll
         for (int i = 0; i < MB; i++) af[slot][i] = *reinterpret_cast<const half8_t *>(at(xa, a_off) + 512 * i);
         xa += step;
@@ -387,14 +403,69 @@ __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__
     }
 }
 
-// grid (8, inner x splits of K, outer / 8), up to eight waves; wave w of split z takes super-blocks [z * chunk + w * per, + per)
-// below min(spr, (z + 1) * chunk).  Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the
-// blocks of activation rows, otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of
-// the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
+// Adds the waves' tiles in wave order and stores the sums.  Run (rg, block i, quarter q) of a tile: lane l = 32 g + c left rows 8 q + 4 g
+// .. + 3 of block i and column c of row group rg at tile_slot(l).  A thread takes COLS neighbouring columns of four rows, as many
+// as leave every thread something to do: with four a row of the result leaves in 8 or 16 bytes a lane, with one in 2 or 4.
+// (One column a thread throughout, stores of 2 bytes a lane: a workgroup of four waves and a 64 x 64 tile took 2.9 us from its loop's end to
+// its last store, 1.5 now; 14336 x 4096 M = 64 with four waves 23.4 -> 22.3 us a call, Q8_0 4999 x 3584 M = 203 34.3 -> 32.9.)
+template <int TILE, int MB, int NR, int COLS, int WAVES>
+__device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, const int nwaves, const int m0, const int n0, const int M, const int Mp,
+                                          const int N, const int z, const int ybf16, void *__restrict__ yg, float *__restrict__ partial) {
+    constexpr int kPer = 32 / COLS;  // threads of a row
+    for (int u = (int)threadIdx.x; u < MB * NR * 8 * kPer; u += (int)blockDim.x) {
+        const int j = u % kPer, g = u / kPer & 1, rg = u / (2 * kPer) % NR, q = u / (2 * kPer * NR) & 3, i = u / (8 * kPer * NR);
+        const int n = n0 + 32 * rg + COLS * j, ml = 32 * i + 8 * q + 4 * g, m = m0 + ml;
+        const float4_t *src = red + ((rg * MB + i) * 4 + q) * kTileRun + tile_slot(32 * g + COLS * j);
+        float4_t t[WAVES][COLS];  // (all asked for at once)
+#pragma unroll
+        for (int w = 0; w < WAVES; w++)
+#pragma unroll
+            for (int c = 0; c < COLS; c++) t[w][c] = src[(w < nwaves ? w : 0) * TILE + 20 * c];
+        const float4_t scale = partial ? float4_t{1.0f, 1.0f, 1.0f, 1.0f} : *reinterpret_cast<const float4_t *>(rs + ml);
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+#pragma unroll
+            for (int w = 1; w < WAVES; w++)
+                if (w < nwaves) t[0][c] += t[w][c];
+            t[0][c] *= scale;
+        }
+        const bool bf = !partial && ybf16;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (m + e >= M) break;
+            float *to = partial ? partial + ((size_t)z * Mp + m + e) * N + n : reinterpret_cast<float *>(yg) + (size_t)(m + e) * N + n;
+            uint16_t *to16 = reinterpret_cast<uint16_t *>(yg) + (size_t)(m + e) * N + n;
+            if (COLS > 1 && n + COLS <= N) {
+                if (bf) {
+                    RowPiece<uint32_t, 2, COLS / 2> v;
+#pragma unroll
+                    for (int c = 0; c < COLS / 2; c++) v.v[c] = bf16_rne_bits(t[0][2 * c][e]) | bf16_rne_bits(t[0][2 * c + (COLS > 1 ? 1 : 0)][e]) << 16;
+                    *reinterpret_cast<RowPiece<uint32_t, 2, COLS / 2> *>(to16) = v;
+                } else {
+                    RowPiece<float, 4, COLS> v;
+#pragma unroll
+                    for (int c = 0; c < COLS; c++) v.v[c] = t[0][c][e];
+                    *reinterpret_cast<RowPiece<float, 4, COLS> *>(to) = v;
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < COLS; c++) {
+                    if (n + c >= N) break;
+                    if (bf) to16[c] = (uint16_t)bf16_rne_bits(t[0][c][e]);
+                    else to[c] = t[0][c][e];
+                }
+            }
+        }
+    }
+}
+
+// grid (8, inner x splits of K, outer / 8), up to eight waves; split z has super-blocks [z * chunk, min(spr, (z + 1) * chunk)).
+// Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the blocks of activation rows,
+// otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
 template <class F, int MB, int NR>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
-                                                             int spr, int per, int chunk, int inner, int outer, int by_m, int ybf16,
+                                                             int spr, int chunk, int inner, int outer, int by_m, int ybf16,
                                                              float *__restrict__ partial, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
     extern __shared__ uint4 smem[];
@@ -406,9 +477,10 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     take_weight(second, ybf16, nt, W, yg, N);
     const int m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
-    int sb0 = z * chunk + wave * per, cnt = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - sb0;
-    const bool idle = cnt < 1;  // the last split is the shortest: a wave left without work multiplies one super-block for nothing
-    sb0 = idle ? 0 : sb0, cnt = idle ? 1 : cnt < per ? cnt : per;
+    // wave w takes every nwaves'th super-block of the split from the w'th on: what the workgroup reads at a time lies side by side
+    const int own = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - z * chunk - wave;
+    const bool idle = own < 1;  // the last split is the shortest: a wave left without work multiplies one super-block for nothing
+    const int sb0 = idle ? 0 : z * chunk + wave, cnt = idle ? 1 : (own + nwaves - 1) / nwaves;
     const uint32_t row_bytes = (uint32_t)spr * F::kBytes;
     KwCopy<F, MB, NR> C;
 #pragma unroll
@@ -446,23 +518,23 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         for (int i = 0; i < MB; i++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[rg][i][e] = 0.0f, part[rg][i][e] = 0.0f;
+    const uint32_t jump = (uint32_t)(nwaves - 1) * (2 * K::kSteps) * step;
     for (int s = 0; s + 1 < cnt; s++) {
         if (F::kUnitHalves == 1) {
-            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
-            sb_off += F::kBytes;
-            kw_half<F, MB, NR, 1, true>(st1, st0, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
+            sb_off += (uint32_t)nwaves * F::kBytes;
+            kw_half<F, MB, NR, 1, true>(st1, st0, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
         } else {
-            sb_off += F::kBytes;
-            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
-            kw_half<F, MB, NR, 1, true>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+            sb_off += (uint32_t)nwaves * F::kBytes;
+            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
+            kw_half<F, MB, NR, 1, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
             uint4 *t = st0;
             st0 = st1, st1 = t;
         }
     }
-    kw_half<F, MB, NR, 0, F::kUnitHalves == 1>(st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
-    kw_half<F, MB, NR, 1, false>(F::kUnitHalves == 1 ? st1 : st0, st1, r, sb_off, C, xa, step, a_off, af, lane, acc, part);
+    kw_half<F, MB, NR, 0, F::kUnitHalves == 1>(st0, st1, r, sb_off, C, xa, step, 0, a_off, af, lane, acc, part);
+    kw_half<F, MB, NR, 1, false>(F::kUnitHalves == 1 ? st1 : st0, st1, r, sb_off, C, xa, step, 0, a_off, af, lane, acc, part);
 
-    // The waves' tiles are added in wave order: slot (rg, block i, quarter q, lane) holds rows 8 q + 4 g .. + 3 of block i
     wait_vm<0>();
     __syncthreads();
     float4_t *red = reinterpret_cast<float4_t *>(smem);
@@ -473,38 +545,13 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         for (int i = 0; i < MB; i++)
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                red[wave * K::kTile + ((rg * MB + i) * 4 + q) * 64 + lane] =
+                red[wave * K::kTile + ((rg * MB + i) * 4 + q) * kTileRun + tile_slot(lane)] =
                     idle ? float4_t{0.0f, 0.0f, 0.0f, 0.0f}
                          : float4_t{acc[rg][i][4 * q], acc[rg][i][4 * q + 1], acc[rg][i][4 * q + 2], acc[rg][i][4 * q + 3]};
     if (wave == 0 && lane < 32 * MB) rs[lane] = rs_mine;
     __syncthreads();
-    constexpr int kTrips = (K::kTile + 64 * kKwWaves - 1) / (64 * kKwWaves);  // with all eight waves
-    for (int base = tid; base < K::kTile; base += kTrips * (int)blockDim.x) {
-#pragma unroll
-        for (int j = 0; j < kTrips; j++) {
-            const int idx = base + j * (int)blockDim.x;
-            if (idx >= K::kTile) break;
-            const int l = idx & 63, t = idx >> 6, q = t & 3, i = (t >> 2) % MB, rg = (t >> 2) / MB;
-            const int n = n0 + 32 * rg + (l & 31), ml = 32 * i + 8 * q + 4 * (l >> 5), m = m0 + ml;
-            float4_t u[kKwWaves];
-#pragma unroll
-            for (int w = 0; w < kKwWaves; w++) u[w] = red[(w < nwaves ? w : 0) * K::kTile + idx];
-            float4_t v = u[0];
-#pragma unroll
-            for (int w = 1; w < kKwWaves; w++)
-                if (w < nwaves) v += u[w];
-            if (!partial) v *= *reinterpret_cast<const float4_t *>(rs + ml);
-            if (n < N) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    if (m + e >= M) continue;
-                    if (partial) partial[((size_t)z * Mp + m + e) * N + n] = v[e];
-                    else if (ybf16) reinterpret_cast<uint16_t *>(yg)[(size_t)(m + e) * N + n] = (uint16_t)bf16_rne_bits(v[e]);
-                    else reinterpret_cast<float *>(yg)[(size_t)(m + e) * N + n] = v[e];
-                }
-            }
-        }
-    }
+    if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
+    else add_tiles<K::kTile, MB, NR, MB * NR, 4>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
 }
 
 }  // namespace
@@ -516,7 +563,7 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
                             float *partial, GemmSecond second, hipStream_t s) {
     using K = Kw<F, MB, NR>;
     auto kern = k_qgemm_kw<F, MB, NR>;
-    const int per = (p.chunk + kKwWaves - 1) / kKwWaves, nwaves = (p.chunk + per - 1) / per;
+    const int nwaves = p.chunk < p.nw ? p.chunk : p.nw;
     const size_t stage = (size_t)nwaves * 2 * K::kItems * 16, red = (size_t)nwaves * K::kTile * 16 + 32 * MB * 4, lds = stage > red ? stage : red;
     static_assert((size_t)kKwWaves * 2 * K::kItems * 16 <= 160 * 1024 && (size_t)kKwWaves * K::kTile * 16 + 32 * MB * 4 <= 160 * 1024, "LDS");
     if (lds > 64 * 1024) {
@@ -528,7 +575,7 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
     const bool by_m = mblocks >= 8 && (int64_t)mblocks * MB * 2 * 256 > (int64_t)tiles * NR * F::kBytes;
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, per, p.chunk, inner, outer, by_m ? 1 : 0,
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer, by_m ? 1 : 0,
                        (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond : 0), p.splits > 1 ? partial : nullptr, second);
     return hipGetLastError();
 }
