@@ -2384,19 +2384,42 @@ bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
     return (type == kTypeQ4K || type == kTypeQ5K || type == kTypeQ6K || type == kTypeQ8_0 || type == kTypeQ3K || type == kTypeQ2K) && m >= 1 && m <= (int64_t)1 << 22 && n >= 1 && k >= 256 && k % 256 == 0 && k <= (int64_t)1 << 22 && n <= 0x7FFFFF00;
 }
 
+// Waves of a workgroup of the tile kernel: eight while the tiles fill the machine at most once, four, two workgroups to a compute unit, above.  Two
+// workgroups are at different places of their tiles, so that one multiplies while the other waits for its first weights, adds its
+// waves' tiles or stores; alone on a compute unit four waves wait longer for memory than eight.  Four against eight, times
+// as long over 1400 drawn shapes, by tile and rounds of 256 workgroups:
+//   32 x 32: 1.02 up to half a round (Q6_K, Q8_0 and Q2_K 1.05), 1.01 up to one, 0.98 up to two, 0.95 above
+//   64 x 32: 0.98 to 0.99 up to one, 0.88 above (16 waves of it fit a compute unit)
+//   64 x 64: 1.02 up to 0.8, 0.99 up to one (Q6_K and Q8_0 1.00 and, with rows of 12 to 40 super-blocks, up to 1.17), 0.92 up to
+//     two, 0.89 up to three, 0.84 above; 32 x 64 alike
+// They decide the order in which a result is summed: a launch of two weights has the waves that either has alone.
+static int kw_waves(int mb, int nr, double rounds, uint32_t type) {
+    if (mb == 2 && nr == 1) return 4;
+    const bool late = mb * nr < 4 || type == kTypeQ6K || type == kTypeQ8_0;
+    return rounds <= (late ? 1.0 : 0.8) ? 8 : 4;
+}
+// Workgroups eight apart are on one die, whose cache holds an eighth of the larger operand's tiles and all of the other's.
+bool kw_by_m(int64_t mblocks, int64_t tiles, int mb, int nr, int64_t block_bytes) {
+    return mblocks >= 8 && mblocks * mb * 2 * 256 > tiles * nr * block_bytes;
+}
+static int64_t block_bytes(uint32_t type) {  // of a super-block of 256 elements
+    return type == kTypeQ4K ? 144 : type == kTypeQ5K ? 176 : type == kTypeQ6K ? 210 : type == kTypeQ8_0 ? 272 : type == kTypeQ3K ? 110 : 84;
+}
+
 // The tile kernel's best tile and K split for a shape, and the microseconds it is expected to take behind the pre-pass, the gap in front
-// of its launch (2.7 us) included.  Fitted to times of 1500 shapes (rms 12 %; 14 % over 150 others, drawn from 2 to 700 activation
-// rows and timed by kernel trace): per round of 256 workgroups a wave's super-blocks cost 1/124 us per KB of activations and
+// of its launch (2.7 us) included, with eight waves.  Fitted to times of 1500 shapes (rms 12 %; 14 % over 150 others, drawn from 2 to 700 activation
+// rows and timed by kernel trace; with the waves that it gets, the tile chosen is within 2 % of the best one on average over 1380 drawn shapes of more
+// than 32 rows): per round of 256 workgroups a wave's super-blocks cost 1/124 us per KB of activations and
 // 1/34 us per KB of weights the workgroup takes in, plus 0.8 us per 32 x 32 tile (Q6_K has twice the matrix instructions).
 struct KwChoice {
-    int mb, nr, splits;
+    int mb, nr, splits, nw;
     double us, rounds;
 };
 static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
-    const double block = type == kTypeQ4K ? 144 : type == kTypeQ5K ? 176 : type == kTypeQ6K ? 210 : type == kTypeQ8_0 ? 272 : type == kTypeQ3K ? 110 : 84;
+    const double block = (double)block_bytes(type);
     const double items = type == kTypeQ3K || type == kTypeQ2K ? 40 : type == kTypeQ6K || type == kTypeQ8_0 ? 32 : 36;  // per row and super-block
     const double cost = type == kTypeQ6K ? 1.35 : 0.79;
-    KwChoice best = {1, 1, 1, 0.0, 0.0};
+    KwChoice best = {1, 1, 1, 8, 0.0, 0.0};
     bool have = false;
     for (int mb = 1; mb <= (m <= 32 ? 1 : 2); mb++)
         for (int nr = 1; nr <= 2; nr++) {
@@ -2409,7 +2432,7 @@ static KwChoice kw_choice(int64_t m, int64_t n, int64_t spr, uint32_t type) {
                 const double nwaves = m <= kSmallMaxM2 && spr < 8 ? (double)spr : 8.0;  // (a short row's workgroup has a wave per super-block)
                 const double one = (double)per * nwaves * (mb * 32 * items * 16 / 1e3 / 124.0 + nr * 32 * block / 1e3 / 34.0) + cost * mb * nr * per;
                 const double us = 5.9 + (1.0 + (rounds - 1.0) * 0.78) * one + (splits > 1 ? 2.5 + splits * (double)m * (double)n * 8.0 * 0.7 / 4.0e6 : 0.0);
-                if (!have || us < best.us) best = {mb, nr, splits, us, (double)wgs / 256.0}, have = true;
+                if (!have || us < best.us) best = {mb, nr, splits, kw_waves(mb, nr, (double)wgs / 256.0, type), us, (double)wgs / 256.0}, have = true;
             }
         }
     return best;
@@ -2421,6 +2444,38 @@ static double rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
     const int64_t wgs = (n + 255) / 256 * (p.mp / (32 * p.mb)) * p.splits;
     return 9.6 + (double)((wgs + 255) / 256) * 2.0 * p.chunk * half * (p.mb == 4 ? 1.45 : 1.0) +
            (p.splits > 1 ? 5.5 + (double)p.splits * (double)m * (double)n * 8.0 * 0.32 / 4.0e6 : 0.0);
+}
+
+// Both again for calls of more than 64 activation rows of three super-blocks or more, the pre-pass included, fitted to 1380 drawn shapes (33 to 2048
+// rows, 400 to 20000 weight rows of 2 to 56 super-blocks; rms 8 to 10 %, row kernels 11 %).  A round of 256 workgroups costs a
+// tile's start and end and so much a super-block; what the last round lacks saves `part` of its share, and a machine less than
+// half full saves up to `few` of the round.
+struct KwFit {
+    double call, round, part, few, split, split_us;  // (split_us: per million partial sums)
+    double sb[6];                                    // Q4_K, Q5_K, Q6_K, Q8_0, Q3_K, Q2_K
+};
+constexpr KwFit kKwFits[3] = {{7.93, 0.0, 0.41, 0.25, 2.96, 3.61, {0.334, 0.407, 0.477, 0.415, 0.406, 0.341}},    // 32 x 32
+                              {7.90, 0.13, 0.29, 0.22, 2.58, 4.52, {0.528, 0.603, 0.679, 0.621, 0.615, 0.564}},   // 64 x 32
+                              {8.24, 1.33, 0.39, 0.26, 2.44, 3.66, {0.740, 0.881, 1.166, 0.974, 0.896, 0.767}}};  // 64 x 64
+constexpr double kRowsFit[6] = {1.312, 1.460, 1.966, 2.444, 1.672, 1.472};  // half a super-block
+static int fit_index(uint32_t type) {
+    return type == kTypeQ4K ? 0 : type == kTypeQ5K ? 1 : type == kTypeQ6K ? 2 : type == kTypeQ8_0 ? 3 : type == kTypeQ3K ? 4 : 5;
+}
+static double many_tiles_us(const KwChoice &kw, int64_t m, int64_t n, int64_t spr, uint32_t type) {
+    const KwFit &f = kKwFits[kw.mb + kw.nr - 2];
+    const double r = kw.rounds, whole = __builtin_ceil(r);
+    const double rounds = r > 1.0 ? f.part * r + (1.0 - f.part) * whole : r < 0.5 ? 1.0 - f.few * (1.0 - 2.0 * r) : 1.0;
+    const double us = f.call + rounds * (f.round + f.sb[fit_index(type)] * (double)((spr + kw.splits - 1) / kw.splits)) +
+                      (kw.splits > 1 ? f.split + f.split_us * 1e-6 * kw.splits * (double)m * (double)n : 0.0);
+    // more activations than a die's cache holds, all of which its workgroups read at a time (Q4_K 14336 x 4096: M = 1024, 8 MB, 185
+    // us as expected, M = 2048 590 for 377)
+    const int64_t mt = (m + 32 * kw.mb - 1) / (32 * kw.mb), nt = (n + 32 * kw.nr - 1) / (32 * kw.nr);
+    return m * spr * 512 > (int64_t)12 << 20 && !kw_by_m(mt, nt, kw.mb, kw.nr, block_bytes(type)) ? us * 1.5 : us;
+}
+static double many_rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
+    const int64_t wgs = (n + 255) / 256 * (p.mp / (32 * p.mb)) * p.splits;
+    return 10.25 + (double)((wgs + 255) / 256) * (1.84 + 2.0 * p.chunk * kRowsFit[fit_index(type)] * (p.mb == 4 ? 1.53 : 1.0)) +
+           (p.splits > 1 ? 1.31 + 2.04e-6 * p.splits * (double)m * (double)n : 0.0);
 }
 
 // 17 to 32 activation rows, Q4_K, Q5_K and Q8_0: microseconds of a whole call with the tile kernel and with the short-batch kernel's
@@ -2524,7 +2579,7 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         // for two, Q6_K 9465 x 5632 56.6 -> 45.5.
         if (spr > 8 && spr <= 12) {
             waves = n <= (spr == 9 ? 7168 : 4096);
-            if (waves) kw.splits = 1, kw.nr = 1;
+            if (waves) kw.splits = 1, kw.nr = 1, kw.nw = kw_waves(1, 1, (double)((n + 31) / 32) / 256.0, type);
         } else if (spr > 16 && spr <= 20) {
             waves = n <= 14336;
         } else {
@@ -2554,6 +2609,11 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         // fifth) the row kernels, which read the activations once per 256 weight rows, are ahead
         const double t_rows = rows_us(p, m, n, type);
         waves = kw.rounds <= (type == kTypeQ6K ? 1.9 : type == kTypeQ8_0 ? 4.0 : type == kTypeQ3K || type == kTypeQ5K ? 2.1 : 2.6) && kw.us < t_rows;
+        // With four waves to a workgroup the tiles stay ahead for longer: over the 1380 shapes 0.945 of the time that the line above
+        // gives.  us of a call, rows -> tiles: Q4_K 4096 x 4096 M = 512 40 -> 35, 1024 x 4096 M = 2048 45 -> 37, Q8_0 14336 x 4096 M = 512
+        // 143 -> 116; 14336 x 4096 Q4_K M = 512, 1792 tiles, stays with the rows, 79 to 94.  Not one block of rows, where the row
+        // kernels read nothing twice, either, and not rows of one or two super-blocks, which leave half of the waves without work.
+        if (!waves && m > 64 && spr > 2) waves = many_tiles_us(kw, m, n, spr, type) < 0.97 * many_rows_us(p, m, n, type);
     }
     if (small) {
         // short batches: rows longer than a run are cut into runs of 16 (or 8) super-blocks, these kernels' K split
@@ -2563,9 +2623,9 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
     if (waves && n <= kKwMaxRows) {
         GemmPlan t = p;
         t.kernel = GemmKernel::kWaves;
-        t.mb = kw.mb, t.nr = kw.nr, t.splits = kw.splits, t.chunk = (int)((spr + kw.splits - 1) / kw.splits);
-        // (one padding for both block heights, so that weights of one batch share their converted activations)
-        t.mp = (int)(m <= 32 ? 32 : (m + 63) / 64 * 64);
+        t.mb = kw.mb, t.nr = kw.nr, t.nw = kw.nw, t.splits = kw.splits, t.chunk = (int)((spr + kw.splits - 1) / kw.splits);
+        // (one padding for both block heights and for the row kernels of the batch's wider weights: they share their converted activations)
+        t.mp = (int)(m <= 32 ? 32 : m <= 192 ? (m + 63) / 64 * 64 : (m + 127) / 128 * 128);
         // its items past the end (and now and then more splits) take more scratch: not where only the other kernel's fits the array of
         // the entry point that allocates nothing
         if (plan_bytes(t, type, n, k) <= PMETAL_HIP_NOALLOC_SCRATCH_BYTES || plan_bytes(p, type, n, k) > PMETAL_HIP_NOALLOC_SCRATCH_BYTES) p = t;
@@ -2594,6 +2654,7 @@ bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type
     if (p.kernel == GemmKernel::kWaves) {
         if (n0 + n1 > kKwMaxRows) return false;
         const KwChoice kw = kw_choice(m, n0 + n1, k / 256, type);
+        if (p.nw != q.nw) return false;
         if (kw.splits == 1) plan->mb = kw.mb, plan->nr = kw.nr;
     }
     return true;

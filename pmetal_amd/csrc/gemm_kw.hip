@@ -572,7 +572,7 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
     }
     second.first = (int)((n + 32 * NR - 1) / (32 * NR));
     const int tiles = second.first + (second.n + 32 * NR - 1) / (32 * NR), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
-    const bool by_m = mblocks >= 8 && (int64_t)mblocks * MB * 2 * 256 > (int64_t)tiles * NR * F::kBytes;
+    const bool by_m = kw_by_m(mblocks, tiles, MB, NR, F::kBytes);
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
     hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer, by_m ? 1 : 0,

@@ -95,10 +95,12 @@ struct GemmPlan {
     int mb;      // 32-row activation blocks per workgroup (kRows: 1, 2 or 4; kWaves: 1 or 2)
     int nr;      // kWaves: 32-row blocks of weights per workgroup (1 or 2)
     int mp;      // padded activation rows, a multiple of 32 mb
-    int nw;      // kRows: waves per workgroup
+    int nw;      // waves per workgroup (kWaves: at most; a short row has fewer)
     int splits;  // workgroups along K (more than one: partial tiles plus a reduction kernel)
     int chunk;   // super-blocks per split
 };
+// Which operand's tiles the dies share among them in the tile kernel (true: the blocks of activation rows)
+bool kw_by_m(int64_t mblocks, int64_t tiles, int mb, int nr, int64_t block_bytes);
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k);
 // (the padded row count mp does not depend on the type; the K split does)
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type = kTypeQ4K);

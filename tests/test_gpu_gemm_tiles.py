@@ -158,6 +158,22 @@ def test_each_tile(oracle, t, mb, nr, m, n, k):
     test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k)
 
 
+# ... with four and with eight waves, which decide how many columns a thread takes where the tiles are added: odd weight row counts (rows of
+# results that begin at any of them, a last piece of one to three columns), rows of 3, 4, 5, 6 and 8 super-blocks (fewer than the waves, as
+# many, and a wave with one more than the others), the last activation row of a tile alone in its block; and two weights in
+# one launch, to the bit what each is alone.
+@pytest.mark.parametrize("mb,nr,nw,m,n,k", [(1, 1, 4, 81, 9837, 1280), (1, 1, 8, 47, 3529, 2048), (1, 1, 4, 20, 17001, 768), (2, 1, 4, 35, 7427, 1024),
+                                            (2, 1, 4, 304, 1591, 1536), (2, 2, 4, 97, 14829, 1024), (2, 2, 4, 399, 3967, 1280), (2, 2, 8, 49, 12359, 1024)])
+@pytest.mark.parametrize("t", TYPES)
+def test_each_tile_with_either_wave_count(oracle, t, mb, nr, nw, m, n, k):
+    p = gemm_plan(t, m, n, k)
+    assert (p.kernel, p.mb, p.nr, p.splits, p.nw) == (WAVES, mb, nr, 1, nw), p
+    test_tiles_match_dequantize_then_matmul(oracle, t, m, n, k)
+    if (mb, nr) == (2, 2):
+        assert gemm_pair_plan(t, m, n, n - 128, k).nw == nw
+        test_pairs_match_separate_calls(oracle, t, m, k, (n, n - 128))
+
+
 # ... and with K split over workgroups, which the plan does for long rows; the last split is shorter than the others (69, 73 and 17
 # super-blocks in four, 73 in two)
 @pytest.mark.parametrize("t,mb,nr,splits,m,n,k", [(Q4K, 2, 1, 4, 161, 321, 18688), (Q6K, 2, 1, 4, 33, 1025, 4352), (Q8_0, 2, 1, 4, 33, 1025, 4352),
