@@ -345,28 +345,42 @@ __device__ __forceinline__ void rw_half(const uint4 *__restrict__ a_cur, uint4 *
             }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the headers are in registers before their buffer is refilled
-#pragma unroll
-        for (int rg = 0; rg < NR; rg++) {
-            dma16(wh_nxt + L.h_off[rg], hb + rg * 64);
-            if (FMT == 1) dma16(wh_nxt + L.qh_off[rg], qhs + rg * 64);
-        }
     }
-    // copies for the next half super-block
+    // The copies for the next half super-block in five steps, of which 128 rows take one behind each of the first k-steps: all at the start of
+    // a half they held its waves up for 610 to 970 of 3930 cycles (a copy passes the address unit in 16, and a workgroup issues 56), and no matrix
+    // instruction ran meanwhile.  Fewer rows have no k-steps to spare behind which the copies could come back.  The quant copies must be the newest
+    // requests of this half: the barrier at its end waits for all but them.
+    auto copies = [&](const int step) __attribute__((always_inline)) {
+        if (step < 3) {
 #pragma unroll
-    for (int i = 0; i < Lane<MB, NR, NW>::kARounds; i++)
-        if (i * kThreads + L.wave * 64 < kGroups * BM) dma16(xs_nxt + L.a_off[i], a_nxt + i * kThreads + L.wave * 64);
-    // the quant copies must be the newest requests of this half: the barrier at its end waits for all but them
-    __builtin_amdgcn_sched_barrier(0);
+            for (int i = 2 * step; i < 2 * step + 2; i++)
+                if (i < Lane<MB, NR, NW>::kARounds && i * kThreads + L.wave * 64 < kGroups * BM) dma16(xs_nxt + L.a_off[i], a_nxt + i * kThreads + L.wave * 64);
+        }
+        if (H == 0 && step == 2) {
 #pragma unroll
-    for (int rg = 0; rg < NR; rg++)
+            for (int rg = 0; rg < NR; rg++) {
+                dma16(wh_nxt + L.h_off[rg], hb + rg * 64);
+                if (FMT == 1) dma16(wh_nxt + L.qh_off[rg], qhs + rg * 64);
+            }
+        }
+        if (step >= 3) {
 #pragma unroll
-        for (int r = 0; r < 2; r++) dma16(wq_nxt + L.q_off[rg][r], q_nxt + rg * 128 + r * 64);
-    __builtin_amdgcn_sched_barrier(0);  // the copies are requested before anything else of this half
+            for (int rg = 0; rg < NR; rg++) dma16(wq_nxt + L.q_off[rg][step - 3], q_nxt + rg * 128 + (step - 3) * 64);
+        }
+    };
+    static_assert(Lane<MB, NR, NW>::kARounds <= 6, "two rounds of activation copies a step");
+    if (MB < 4) {
+#pragma unroll
+        for (int step = 0; step < 5; step++) copies(step);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
-    // scales and mins of sub-blocks j0 = 4 H + 2 g and j0 + 1 (6-bit fields, crates/pmetal/src/commands/quantize.rs:844-855)
-    const uint32_t sh = 16u * (uint32_t)g;
+    // Scales and mins of sub-blocks j0 = 4 H + 2 g and j0 + 1.  The min term: (-h, -h, -l, -l) against the activations' (H, L, H, L), all four cross products of the exact head + tail
+    // splits, straight into the accumulators (after the eight k-steps).
+    const uint32_t pick = g ? 0x04030402u : 0x04010400u;
+    const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
     half2_t sc2[NR][2], off2[NR][2];
-    uint32_t mn[NR][2];
+    half8_t br[NR];
     uint32_t qd[NR][8];
     // this lane's 32 quant bytes per row group: pieces 2g and 2g+1 of row col (the copy swizzles the four pieces of
     // a row by (row / 4) % 4 so that 16 consecutive rows read conflict-free)
@@ -376,20 +390,11 @@ __device__ __forceinline__ void rw_half(const uint4 *__restrict__ a_cur, uint4 *
         const uint4 qa = q_cur[rg * 128 + col * 4 + ((2 * g) ^ sw)], qb = q_cur[rg * 128 + col * 4 + ((2 * g + 1) ^ sw)];
         qd[rg][0] = qa.x, qd[rg][1] = qa.y, qd[rg][2] = qa.z, qd[rg][3] = qa.w;
         qd[rg][4] = qb.x, qd[rg][5] = qb.y, qd[rg][6] = qb.z, qd[rg][7] = qb.w;
-        uint32_t sc0, sc1;
-        if (H == 0) {
-            const uint32_t yv = R.hdr[rg].y >> sh, zv = R.hdr[rg].z >> sh;
-            sc0 = yv & 63u, sc1 = (yv >> 8) & 63u;
-            mn[rg][0] = zv & 63u, mn[rg][1] = (zv >> 8) & 63u;
-        } else {
-            const uint32_t wv = R.hdr[rg].w >> sh, yv = R.hdr[rg].y >> sh, zv = R.hdr[rg].z >> sh;
-            sc0 = (wv & 0xFu) | ((yv >> 2) & 0x30u), sc1 = ((wv >> 8) & 0xFu) | ((yv >> 10) & 0x30u);
-            mn[rg][0] = ((wv >> 4) & 0xFu) | ((zv >> 2) & 0x30u), mn[rg][1] = ((wv >> 12) & 0xFu) | ((zv >> 10) & 0x30u);
-        }
-        const _Float16 s0 = (_Float16)(float)sc0, s1 = (_Float16)(float)sc1;
-        const _Float16 o0 = (_Float16)(-1024.0f * (float)sc0), o1 = (_Float16)(-1024.0f * (float)sc1);  // exact: sc <= 63
-        sc2[rg][0] = half2_t{s0, s0}, sc2[rg][1] = half2_t{s1, s1};
-        off2[rg][0] = half2_t{o0, o0}, off2[rg][1] = half2_t{o1, o1};
+        const u32x4 h = R.hdr[rg];
+        const half2_t sc = byte_pair(scale_bytes<H>(h.y, h.w), pick), mn = byte_pair(min_bytes<H>(h.z, h.w), pick);
+        sc2[rg][0] = half2_t{sc[0], sc[0]}, sc2[rg][1] = half2_t{sc[1], sc[1]};
+        off2[rg][0] = sc2[rg][0] * m1024, off2[rg][1] = sc2[rg][1] * m1024;  // exact: sc <= 63
+        br[rg] = heads_and_tails(mn, -f16_twice(h.x >> 16));
     }
 
     // Q5_K: where k-step t finds its fifth bits.  GGML order: qh dword t (the same four bytes as quant dword t), bits
@@ -400,18 +405,6 @@ __device__ __forceinline__ void rw_half(const uint4 *__restrict__ a_cur, uint4 *
         const uint32_t dw = g ? R.qh[rg][4 * H + 2 + (t >> 2)] : R.qh[rg][4 * H + (t >> 2)];
         return dw >> (8 * (t & 3));  // (the decoder masks the byte)
     };
-
-    // min term of sub-blocks j0, j0 + 1: (-h, -h, -l, -l) against the activations' (H, L, H, L): all four cross
-    // products of the exact head + tail splits, straight into the accumulators (after the eight k-steps)
-    half8_t br[NR];
-#pragma unroll
-    for (int rg = 0; rg < NR; rg++) {
-        const float dmin = f16_bits_to_f32(R.hdr[rg].x >> 16);
-        _Float16 h0, l0, h1, l1;
-        neg_min_split(dmin, mn[rg][0], h0, l0);
-        neg_min_split(dmin, mn[rg][1], h1, l1);
-        br[rg] = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
-    }
 
     // Software pipeline, written in issue order (a wave issues in order, so the order here is the schedule):
     // the activation fragments of k-step t + 1 are requested before the products of k-step t, and the weights of
@@ -458,6 +451,7 @@ __device__ __forceinline__ void rw_half(const uint4 *__restrict__ a_cur, uint4 *
                     for (int ii = 0; ii < MB; ii++)
                         af[(t + 1) & 1][ii] = __builtin_bit_cast(half8_t, a_cur[(t < 7 ? (t + 1) * 2 + g : 16 + g) * BM + 32 * ii + col]);
                 }
+                if (MB >= 4 && i == MB - 1 && rg == NR - 1 && t < 5) copies(t);
                 __builtin_amdgcn_sched_barrier(0);
             }
     }
@@ -620,43 +614,50 @@ __device__ __forceinline__ void rw16_half(const uint4 *__restrict__ a_cur, uint4
             dbits = sd.w >> 16;
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-#pragma unroll
-        for (int r = 0; r < B::kHdrRounds; r++) dma16(wh_nxt + h_off[r], hs + 64 * r);
     }
+    // in steps behind k-steps or all at the start, as in the Q4_K kernel; the quant copy must be the newest request of this half
+    auto copies = [&](const int step) __attribute__((always_inline)) {
+        if (step < 3) {
 #pragma unroll
-    for (int i = 0; i < kARounds; i++)
-        if (i * kThreads + wave * 64 < kGroups16 * BM) dma16(xs_nxt + a_off[i], a_nxt + i * kThreads + wave * 64);
-    // the quant copy must be the newest request of this half: the barrier at its end waits for all but it
-    __builtin_amdgcn_sched_barrier(0);
-    dma16(wq_nxt + q_off, q_nxt);
-    __builtin_amdgcn_sched_barrier(0);
+            for (int i = 2 * step; i < 2 * step + 2; i++)
+                if (i < kARounds && i * kThreads + wave * 64 < kGroups16 * BM) dma16(xs_nxt + a_off[i], a_nxt + i * kThreads + wave * 64);
+        }
+        if (H == 0 && step == 2) {
+#pragma unroll
+            for (int r = 0; r < B::kHdrRounds; r++) dma16(wh_nxt + h_off[r], hs + 64 * r);
+        }
+        if (step == 3) dma16(wq_nxt + q_off, q_nxt);
+    };
+    static_assert(kARounds <= 6, "two rounds of activation copies a step");
+    if (MB < 4) {
+#pragma unroll
+        for (int step = 0; step < 4; step++) copies(step);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
     // this lane's 16 quant bytes: piece g of row col
     const uint4 qv = q_cur[col * 2 + g];
     const uint32_t qd[4] = {qv.x, qv.y, qv.z, qv.w};
     // scales (and mins) of the lane's four sub-blocks j = 8 H + 4 sp + 2 lh + g, index 2 sp + lh
     half2_t sc2[4], off2[4];
-    float nm[4];  // what a sub-block subtracts per unit of its activation sum, negated: -dmin m (Q2_K), -4 d s' (Q3_K); exact in fp32
+    half8_t br[2];  // what a sub-block subtracts per unit of its activation sum, negated: -dmin m (Q2_K), -4 d s' (Q3_K)
+    const uint32_t pick = g ? 0x04030401u : 0x04020400u;  // bytes g and g + 2
+    const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f}, m4 = {(_Float16)-4.0f, (_Float16)-4.0f};
 #pragma unroll
-    for (int sp = 0; sp < 2; sp++)
-#pragma unroll
-        for (int lh = 0; lh < 2; lh++) {
-            float scf;
-            if (FMT == 3) {  // byte j of the sixteen: low nibble scale, high nibble min
-                const uint32_t b = (hdr[2 * H + sp] >> (8u * (uint32_t)g + 16u * lh)) & 0xFFu;
-                scf = (float)(b & 15u);
-                nm[2 * sp + lh] = -(f16_bits_to_f32(dbits >> 16) * (float)(b >> 4));
-            } else {
-                // sc6 of sub-block j: low nibble (j < 8) or high nibble (j >= 8) of byte j % 8, bits 4..5 = bits
-                // 2 (j / 4) of byte 8 + j % 4
-                const uint32_t lo4 = (hdr[sp] >> (8u * (uint32_t)g + 16u * lh + 4u * H)) & 15u;
-                const uint32_t hi2 = (hdr[2] >> (8u * (uint32_t)g + 16u * lh + 2u * (2 * H + sp))) & 3u;
-                scf = (float)((int)(lo4 | (hi2 << 4)) - 32);
-                nm[2 * sp + lh] = -(f16_bits_to_f32(dbits & 0xFFFFu) * (4.0f * scf));
-            }
-            const _Float16 sh = (_Float16)scf, oh = (_Float16)(-1024.0f * scf);  // exact: |sc| <= 32
-            sc2[2 * sp + lh] = half2_t{sh, sh}, off2[2 * sp + lh] = half2_t{oh, oh};
+    for (int sp = 0; sp < 2; sp++) {
+        half2_t sc;
+        if (FMT == 3) {  // byte j of the sixteen: low nibble scale, high nibble min
+            sc = byte_pair(hdr[2 * H + sp] & 0x0F0F0F0Fu, pick);
+            br[sp] = heads_and_tails(byte_pair((hdr[2 * H + sp] >> 4) & 0x0F0F0F0Fu, pick), -f16_twice(dbits >> 16));
+        } else {
+            // sc6 of sub-block j: low nibble (j < 8) or high nibble (j >= 8) of byte j % 8, bits 4..5 = bits
+            // 2 (j / 4) of byte 8 + j % 4
+            sc = byte_pair(((hdr[sp] >> (4 * H)) & 0x0F0F0F0Fu) | (((hdr[2] >> (2 * (2 * H + sp))) & 0x03030303u) << 4), pick, -1056.0f);
+            br[sp] = heads_and_tails(sc * m4, f16_twice(dbits));
         }
+        sc2[2 * sp] = half2_t{sc[0], sc[0]}, sc2[2 * sp + 1] = half2_t{sc[1], sc[1]};
+        off2[2 * sp] = sc2[2 * sp] * m1024, off2[2 * sp + 1] = sc2[2 * sp + 1] * m1024;  // exact: |sc| <= 32
+    }
     // operand of k-step t: dword t / 2, the two-bit fields at 4 (t % 2) and 4 (t % 2) + 2 (Q3_K: bit 2 from hmask)
     auto operand = [&](int t) -> half8_t {
         const int dw = t >> 1, sp = t & 1;
@@ -698,6 +699,7 @@ __device__ __forceinline__ void rw16_half(const uint4 *__restrict__ a_cur, uint4
                     af[(t + 1) & 1][ii] = __builtin_bit_cast(half8_t, a_cur[(t < 7 ? (t + 1) * 2 + g : 16 + g) * BM + 32 * ii + col]);
                 if (t < 7) b = operand(t + 1);
             }
+            if (MB >= 4 && i == MB - 1 && t < 4) copies(t);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -706,13 +708,10 @@ __device__ __forceinline__ void rw16_half(const uint4 *__restrict__ a_cur, uint4
         // (sp, 0), (sp, 1)
 #pragma unroll
         for (int sp = 0; sp < 2; sp++) {
-            const _Float16 h0 = (_Float16)nm[2 * sp], h1 = (_Float16)nm[2 * sp + 1];
-            const _Float16 l0 = (_Float16)(nm[2 * sp] - (float)h0), l1 = (_Float16)(nm[2 * sp + 1] - (float)h1);
-            const half8_t br = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
 #pragma unroll
             for (int i = 0; i < MB; i++) {
                 const half8_t a = sp == 0 ? af[0][i] : __builtin_bit_cast(half8_t, a_cur[(18 + g) * BM + 32 * i + col]);
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, br, acc[i], 0, 0, 0);
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, br[sp], acc[i], 0, 0, 0);
             }
         }
     }
@@ -857,16 +856,25 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
         R.sc = u32x4{sv.x, sv.y, sv.z, sv.w};
         R.d = dv.w >> 16;
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the header is in registers before its buffer is refilled
-        dma16(wh_nxt + L.h_off, hb);
     }
+    // In steps behind k-steps or all at the start, as in the Q4_K kernel.  The three quant copies, two half super-blocks ahead (ql bytes
+    // 64 H .., qh bytes 128 + 32 H .. of that super-block), stay the newest requests (see barrier_keep).
+    auto copies = [&](const int step) __attribute__((always_inline)) {
+        if (step < 2) {
 #pragma unroll
-    for (int i = 0; i < LaneQ6<MB>::kARounds; i++) dma16(xs_nxt + L.a_off[i], a_nxt + i * kThreads + L.wave * 64);
-    __builtin_amdgcn_sched_barrier(0);  // the three quant copies stay the newest requests (see barrier_keep)
-    // quant pieces two half super-blocks ahead: ql bytes 64 H .., qh bytes 128 + 32 H .. of that super-block
+            for (int i = 2 * step; i < 2 * step + 2; i++)
+                if (i < LaneQ6<MB>::kARounds) dma16(xs_nxt + L.a_off[i], a_nxt + i * kThreads + L.wave * 64);
+        }
+        if (H == 0 && step == 2) dma16(wh_nxt + L.h_off, hb);
+        if (step == 3 || step == 4) dma16(wq_nxt + 64 * H + L.ql_off[step - 3], q_nxt + (step - 3) * 64);
+        if (step == 5) dma16(wq_nxt + 32 * H + L.qh_off, q_nxt + 128);
+    };
+    static_assert(LaneQ6<MB>::kARounds <= 4, "two rounds of activation copies a step");
+    if (MB < 4) {
 #pragma unroll
-    for (int r = 0; r < 2; r++) dma16(wq_nxt + 64 * H + L.ql_off[r], q_nxt + r * 64);
-    dma16(wq_nxt + 32 * H + L.qh_off, q_nxt + 128);
-    __builtin_amdgcn_sched_barrier(0);  // the copies are requested before anything else of this half
+        for (int step = 0; step < 6; step++) copies(step);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
     // this lane's 32 ql bytes and the 32 qh bytes of its row (pieces swizzled by the copy for conflict-free reads)
     const int sw = (col >> 2) & 3, sw2 = (col >> 3) & 1;
@@ -923,6 +931,7 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
                         af[(t + 1) & 1][ii] = __builtin_bit_cast(half8_t, a_cur[((t + 1) * 2 + g) * BM + 32 * ii + col]);
                 }
             }
+            if (MB >= 4 && slot == kSlots - 1 && t < 6) copies(t);
             __builtin_amdgcn_sched_barrier(0);
         }
     }

@@ -97,6 +97,34 @@ __device__ __forceinline__ void neg_min_split(const float dmin, const uint32_t m
     l = (_Float16)(p - (float)h);
 }
 
+// Integers below 64, a byte each, as the f16 pair of the two that `pick` names: 0x64bb is 1024 + bb, so `bias` is -1024 (- 32: signed).
+// The compiler reads halves of a pair by operand selection, so a scale for all lanes of a packed operation costs no move.
+__device__ __forceinline__ half2_t byte_pair(const uint32_t bytes, const uint32_t pick, const float bias = -1024.0f) {
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, bytes, pick)) + half2_t{(_Float16)bias, (_Float16)bias};
+}
+// m0 k and m1 k as f16 heads and tails (h0, h0, l0, l0, h1, h1, l1, l1), the operand that meets the activations' (H, L, H, L).  Exact: k has
+// eleven bits and |m| at most seven, and what the head leaves is a multiple of k's last bit, which the fma keeps.
+__device__ __forceinline__ half8_t heads_and_tails(const half2_t m, const half2_t k) {
+    const half2_t h = m * k, l = __builtin_elementwise_fma(m, k, -h);
+    return half8_t{h[0], h[0], l[0], l[0], h[1], h[1], l[1], l[1]};
+}
+__device__ __forceinline__ half2_t f16_twice(const uint32_t bits16) {  // of the low half
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(bits16, bits16, 0x01000100u));
+}
+// (Decoding a lane's two scales and mins one by one in f32 took some 45 vector instructions a half super-block and row group, this takes
+// 16: with the copies of a half spread over its k-steps the row kernels' 128-row forms take, us of a call at 14336 x 4096 M = 2048 before ->
+// after, Q4_K 290 -> 280, Q5_K 318 -> 300, Q3_K 349 -> 325, Q2_K 316 -> 302; of the two the copies are 5 of Q4_K's 10.)
+// Q4_K and Q5_K: the scales and mins of four sub-blocks (half H of the super-block), a byte each, from the twelve bytes y, z, w
+// (6-bit fields, crates/pmetal/src/commands/quantize.rs:844-855).
+template <int H>
+__device__ __forceinline__ uint32_t scale_bytes(const uint32_t y, const uint32_t w) {
+    return H == 0 ? y & 0x3F3F3F3Fu : (w & 0x0F0F0F0Fu) | ((y >> 2) & 0x30303030u);
+}
+template <int H>
+__device__ __forceinline__ uint32_t min_bytes(const uint32_t z, const uint32_t w) {
+    return H == 0 ? z & 0x3F3F3F3Fu : ((w >> 4) & 0x0F0F0F0Fu) | ((z >> 2) & 0x30303030u);
+}
+
 constexpr int kGroups16 = 20;  // activation items per row and half super-block: 16 operands and four of sub-block sums
 template <int FMT>
 struct Block16 {  // FMT 2: Q3_K, 3: Q2_K

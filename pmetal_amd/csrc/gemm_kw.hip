@@ -75,34 +75,18 @@ struct KwQ45 {  // FMT 0: Q4_K, 1: Q5_K
     const uint4 *row_;
     int g_;
     uint32_t q[4], qh[4];  // of four k-steps
-    half2_t sc2[2], off2[2];
-    half8_t br;
-    float d;
+    half2_t scs, offs, mns;  // of the lane's two sub-blocks: scale, -1024 scale, min
+    uint32_t dd;             // d | dmin << 16
     template <int H>
     __device__ __forceinline__ void load(const uint4 *st, int, const int g) {
         row_ = st, g_ = g;
         const uint4 hdr = st[0];
-        // scales and mins of sub-blocks j0 = 4 H + 2 g and j0 + 1 (6-bit fields, crates/pmetal/src/commands/quantize.rs:844-855)
-        const uint32_t sh = 16u * (uint32_t)g;
-        const uint32_t yv = hdr.y >> sh, zv = hdr.z >> sh, wv = hdr.w >> sh;
-        uint32_t sc0, sc1, mn0, mn1;
-        if (H == 0) {
-            sc0 = yv & 63u, sc1 = (yv >> 8) & 63u;
-            mn0 = zv & 63u, mn1 = (zv >> 8) & 63u;
-        } else {
-            sc0 = (wv & 0xFu) | ((yv >> 2) & 0x30u), sc1 = ((wv >> 8) & 0xFu) | ((yv >> 10) & 0x30u);
-            mn0 = ((wv >> 4) & 0xFu) | ((zv >> 2) & 0x30u), mn1 = ((wv >> 12) & 0xFu) | ((zv >> 10) & 0x30u);
-        }
-        const _Float16 s0 = (_Float16)(float)sc0, s1 = (_Float16)(float)sc1;
-        const _Float16 o0 = (_Float16)(-1024.0f * (float)sc0), o1 = (_Float16)(-1024.0f * (float)sc1);  // exact: sc <= 63
-        sc2[0] = half2_t{s0, s0}, sc2[1] = half2_t{s1, s1};
-        off2[0] = half2_t{o0, o0}, off2[1] = half2_t{o1, o1};
-        d = f16_bits_to_f32(hdr.x & 0xFFFFu);
-        const float dmin = f16_bits_to_f32(hdr.x >> 16);
-        _Float16 h0, l0, h1, l1;
-        neg_min_split(dmin, mn0, h0, l0);
-        neg_min_split(dmin, mn1, h1, l1);
-        br = half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
+        // scales and mins of sub-blocks 4 H + 2 g and the next one
+        const uint32_t pick = g ? 0x04030402u : 0x04010400u;
+        const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+        scs = byte_pair(scale_bytes<H>(hdr.y, hdr.w), pick), mns = byte_pair(min_bytes<H>(hdr.z, hdr.w), pick);
+        offs = scs * m1024;  // exact: sc <= 63
+        dd = hdr.x;
     }
     template <int H>
     __device__ __forceinline__ void operands(const int t, half8_t (&b)[1]) {
@@ -118,13 +102,15 @@ struct KwQ45 {  // FMT 0: Q4_K, 1: Q5_K
             }
         }
         const uint32_t hq = !FMT ? 0u : ORDER ? qh[t % 4] : qh[0] >> (8 * (t & 3));
+        const half2_t sc2[2] = {half2_t{scs[0], scs[0]}, half2_t{scs[1], scs[1]}}, off2[2] = {half2_t{offs[0], offs[0]}, half2_t{offs[1], offs[1]}};
         Dq v;
 #pragma unroll
         for (int c = 0; c < 4; c++) dq_chunk<ORDER, FMT>(c, t, q[t % 4], sc2, off2, v, hq);
         b[0] = v.value();
     }
-    __device__ __forceinline__ half8_t sums(int) const { return br; }
-    __device__ __forceinline__ float scale(int) const { return d; }
+    // (made where they are used: the 64 x 64 tile has no registers to hold them over the half)
+    __device__ __forceinline__ half8_t sums(int) const { return heads_and_tails(mns, -f16_twice(dd >> 16)); }
+    __device__ __forceinline__ float scale(int) const { return f16_bits_to_f32(dd & 0xFFFFu); }
 };
 
 struct KwQ6 {
@@ -204,6 +190,7 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
     uint32_t qd[4], hm[4];
     half2_t sc2[4], off2[4];
     half8_t br[FMT == 3 ? 2 : 1];  // Q2_K's mins
+    half2_t dk;                     // Q3_K: d
     float d;
     template <int H>
     __device__ __forceinline__ void load(const uint4 *st, int, const int g) {
@@ -223,26 +210,22 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
             dbits = sd.w >> 16;
         }
         d = f16_bits_to_f32(dbits & 0xFFFFu);
-        // scales (Q2_K: and what a sub-block subtracts per unit of its activation sum) of sub-blocks 8 H + 4 sp + 2 lh + g
-        float nm[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // (Q2_K)
+        // scales (Q2_K: and what a sub-block subtracts per unit of its activation sum) of sub-blocks 8 H + 4 sp + 2 lh + g, index 2 sp + lh
+        const uint32_t pick = g ? 0x04030401u : 0x04020400u;  // bytes g and g + 2
+        const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+        if constexpr (FMT == 2) dk = f16_twice(dbits);
 #pragma unroll
-        for (int sp = 0; sp < 2; sp++)
-#pragma unroll
-            for (int lh = 0; lh < 2; lh++) {
-                float scf;
-                if (FMT == 3) {
-                    const uint32_t b = (hdr[2 * H + sp] >> (8u * (uint32_t)g + 16u * lh)) & 0xFFu;
-                    scf = (float)(b & 15u);
-                    nm[2 * sp + lh] = -(f16_bits_to_f32(dbits >> 16) * (float)(b >> 4));
-                } else {
-                    const uint32_t lo4 = (hdr[sp] >> (8u * (uint32_t)g + 16u * lh + 4u * H)) & 15u;
-                    const uint32_t hi2 = (hdr[2] >> (8u * (uint32_t)g + 16u * lh + 2u * (2 * H + sp))) & 3u;
-                    scf = (float)((int)(lo4 | (hi2 << 4)) - 32);
-                }
-                const _Float16 sh = (_Float16)scf, oh = (_Float16)(-1024.0f * scf);  // exact: |sc| <= 32
-                sc2[2 * sp + lh] = half2_t{sh, sh}, off2[2 * sp + lh] = half2_t{oh, oh};
+        for (int sp = 0; sp < 2; sp++) {
+            half2_t sc;
+            if constexpr (FMT == 3) {
+                sc = byte_pair(hdr[2 * H + sp] & 0x0F0F0F0Fu, pick);
+                br[sp] = heads_and_tails(byte_pair((hdr[2 * H + sp] >> 4) & 0x0F0F0F0Fu, pick), -f16_twice(dbits >> 16));
+            } else {
+                sc = byte_pair(((hdr[sp] >> (4 * H)) & 0x0F0F0F0Fu) | (((hdr[2] >> (2 * (2 * H + sp))) & 0x03030303u) << 4), pick, -1056.0f);
             }
-        if constexpr (FMT == 3) br[0] = split(nm[0], nm[1]), br[1] = split(nm[2], nm[3]);
+            sc2[2 * sp] = half2_t{sc[0], sc[0]}, sc2[2 * sp + 1] = half2_t{sc[1], sc[1]};
+            off2[2 * sp] = sc2[2 * sp] * m1024, off2[2 * sp + 1] = sc2[2 * sp + 1] * m1024;  // exact: |sc| <= 32
+        }
         if (FMT == 2) {
 #pragma unroll
             for (int i = 0; i < 4; i++) hm[i] >>= 4 * H;
@@ -262,17 +245,11 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
         const half2_t r3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u)), sc2[2 * sp + 1], off2[2 * sp + 1]);
         b[0] = half8_t{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
     }
-    // the two values as f16 heads and tails
-    static __device__ __forceinline__ half8_t split(const float m0, const float m1) {
-        const _Float16 h0 = (_Float16)m0, h1 = (_Float16)m1;
-        const _Float16 l0 = (_Float16)(m0 - (float)h0), l1 = (_Float16)(m1 - (float)h1);
-        return half8_t{h0, h0, l0, l0, h1, h1, l1, l1};
-    }
     // (Q3_K subtracts 4 d sc: made from the scales where it is used.  Held over the half it took the 64 x 64 tile past 256 registers
     // and one of them to scratch memory)
     __device__ __forceinline__ half8_t sums(int i) const {
         if constexpr (FMT == 3) return br[i];
-        else return split(-(d * (4.0f * (float)sc2[2 * i][0])), -(d * (4.0f * (float)sc2[2 * i + 1][0])));
+        else return heads_and_tails(half2_t{sc2[2 * i][0], sc2[2 * i + 1][0]} * half2_t{(_Float16)-4.0f, (_Float16)-4.0f}, dk);
     }
     __device__ __forceinline__ float scale(int) const { return d; }
 };
