@@ -248,11 +248,13 @@ int32_t scratch_of_current_device(NoAllocScratch **out) {
 }
 
 // ---- host-to-host codec calls on large tensors ----
-// A tensor of at least kPipeMinElems elements in pageable host memory goes through chunks (a quarter of the tensor, at
-// most kPipeElems elements; smaller tensors take one allocate-copy-run-copy round): a few host threads copy a chunk into a
-// pinned staging buffer, a copy engine moves it, the kernel runs, and the result comes back the same way, each chunk on
-// the stream of its slot, so that the host copies, both transfer directions and the kernels of neighbouring chunks
-// overlap.  The slots (pinned and device buffers, streams, events) are made on first use, per device, and kept until
+// A tensor of at least kPipeMinElems elements in pageable host memory goes through chunks (a third of the tensor, at
+// most kPipeElems elements; smaller tensors take one allocate-copy-run-copy round): a few host threads, the call's own, copy a chunk into a
+// pinned staging buffer, the kernel runs, and the result is copied out of another one, each chunk on the stream of its slot, so that the
+// host copies, both transfer directions and the kernels of neighbouring chunks overlap.  A copy engine moves the f32 side; the blocks, a
+// quarter of the bytes or less, the kernel itself reads from pinned memory or writes there, each once: a copy of them is a command, a
+// trip over the bus and a wait more in each chunk (us of a call on 3 Mi elements with the copy / so, quantize and dequantize: Q8_0 551, 595 / 473, 479,
+// Q4_K 510, 499 / 399, 426, Q6_K 558, 540 / 402, 453; f32 read or written that way too is slower, 488 and 561 for Q4_K).  The slots (pinned and device buffers, streams, events) are made on first use, per device, and kept until
 // the process ends; calls take turns (one mutex).
 constexpr size_t kPipeElems = (size_t)4 << 20;  // 16 MiB of f32; a multiple of every block size
 constexpr size_t kPipeQBytes = kPipeElems / 256 * 292;  // the largest encoded chunk (Q8_K)
@@ -261,7 +263,7 @@ constexpr int kPipeSlots = 3;
 
 struct PipeSlot {
     float *h_f32 = nullptr, *d_f32 = nullptr;
-    uint8_t *h_q = nullptr, *d_q = nullptr;
+    uint8_t *h_q = nullptr;
     hipStream_t st = nullptr;
     hipEvent_t done = nullptr;
 };
@@ -279,9 +281,8 @@ int32_t host_pipe(HostPipe **out) {  // caller holds g_pipe_mutex
     if (!p.ready) {
         for (PipeSlot &sl : p.slot) {  // (a call that failed half way left what it had: only the missing pieces are made)
             if (!sl.h_f32) HIP_TRY(hipHostMalloc((void **)&sl.h_f32, kPipeElems * sizeof(float), hipHostMallocDefault));
-            if (!sl.h_q) HIP_TRY(hipHostMalloc((void **)&sl.h_q, kPipeQBytes, hipHostMallocDefault));
+            if (!sl.h_q) HIP_TRY(hipHostMalloc((void **)&sl.h_q, kPipeQBytes, hipHostMallocMapped | hipHostMallocCoherent));
             if (!sl.d_f32) HIP_TRY(hipMalloc((void **)&sl.d_f32, kPipeElems * sizeof(float)));
-            if (!sl.d_q) HIP_TRY(hipMalloc((void **)&sl.d_q, kPipeQBytes));
             if (!sl.st) HIP_TRY(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking));
             if (!sl.done) HIP_TRY(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
         }
@@ -748,31 +749,31 @@ int32_t codec_pipelined(bool quantize, uint32_t t, float *plain, uint8_t *packed
     std::lock_guard<std::mutex> lock(g_pipe_mutex);
     HostPipe *p = nullptr;
     if (int32_t rc = host_pipe(&p)) return rc;
-    // chunk: a quarter of the tensor (so that the stages of neighbouring chunks overlap), at most what a slot holds
-    size_t chunk = ((n / 4 + kPipeGrain - 1) / kPipeGrain) * kPipeGrain;
+    // chunk: a third of the tensor (so that the stages of neighbouring chunks overlap; four or more are slower, each costs some 20 us), at
+    // most what a slot holds
+    size_t chunk = ((n / 3 + kPipeGrain - 1) / kPipeGrain) * kPipeGrain;
     chunk = chunk < kPipeMinElems ? kPipeMinElems : (chunk > kPipeElems ? kPipeElems : chunk);
     const size_t chunks = (n + chunk - 1) / chunk, q_chunk = pmetal_hip_tensor_size(t, chunk);
     auto elems_of = [&](size_t i) { return i + 1 < chunks ? chunk : n - i * chunk; };
+    pmh::CopyTeam team;
     int32_t rc = PMETAL_HIP_OK;
     auto retire = [&](size_t i) -> int32_t {  // chunk i's result: staging buffer -> caller's memory
         PipeSlot &sl = p->slot[i % kPipeSlots];
         HIP_TRY(hipEventSynchronize(sl.done));
-        if (quantize) pmh::par_copy(packed + i * q_chunk, sl.h_q, pmetal_hip_tensor_size(t, elems_of(i)));
-        else pmh::par_copy(plain + i * chunk, sl.h_f32, elems_of(i) * sizeof(float));
+        if (quantize) team.copy(packed + i * q_chunk, sl.h_q, pmetal_hip_tensor_size(t, elems_of(i)));
+        else team.copy(plain + i * chunk, sl.h_f32, elems_of(i) * sizeof(float));
         return PMETAL_HIP_OK;
     };
     auto submit = [&](size_t i) -> int32_t {
         PipeSlot &sl = p->slot[i % kPipeSlots];
         const size_t elems = elems_of(i), qb = pmetal_hip_tensor_size(t, elems);
         if (quantize) {
-            pmh::par_copy(sl.h_f32, plain + i * chunk, elems * sizeof(float));
+            team.copy(sl.h_f32, plain + i * chunk, elems * sizeof(float));
             HIP_TRY(hipMemcpyAsync(sl.d_f32, sl.h_f32, elems * sizeof(float), hipMemcpyHostToDevice, sl.st));
-            if (int32_t r = pmetal_hip_quantize_dev(t, sl.d_f32, elems, sl.d_q, qb, sl.st)) return r;
-            HIP_TRY(hipMemcpyAsync(sl.h_q, sl.d_q, qb, hipMemcpyDeviceToHost, sl.st));
+            if (int32_t r = pmetal_hip_quantize_dev(t, sl.d_f32, elems, sl.h_q, qb, sl.st)) return r;
         } else {
-            pmh::par_copy(sl.h_q, packed + i * q_chunk, qb);
-            HIP_TRY(hipMemcpyAsync(sl.d_q, sl.h_q, qb, hipMemcpyHostToDevice, sl.st));
-            if (int32_t r = pmetal_hip_dequantize_dev(t, sl.d_q, qb, sl.d_f32, elems, order, sl.st)) return r;
+            team.copy(sl.h_q, packed + i * q_chunk, qb);
+            if (int32_t r = pmetal_hip_dequantize_dev(t, sl.h_q, qb, sl.d_f32, elems, order, sl.st)) return r;
             HIP_TRY(hipMemcpyAsync(sl.h_f32, sl.d_f32, elems * sizeof(float), hipMemcpyDeviceToHost, sl.st));
         }
         HIP_TRY(hipEventRecord(sl.done, sl.st));

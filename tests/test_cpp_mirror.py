@@ -39,3 +39,12 @@ def test_host_copy_without_threads(tmp_path):
                     "-static-libstdc++", "-pthread", "-Wl,--wrap=pthread_create"], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_copy_team_over_many_copies(tmp_path):
+    """The threads of one codec call, used for copy after copy: every byte of each, asleep or not, however many can be made."""
+    exe = str(tmp_path / "test_copy_team")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", os.path.join(ROOT, "tests", "cpp", "test_copy_team.cpp"), "-o", exe,
+                    "-static-libstdc++", "-pthread", "-Wl,--wrap=pthread_create"], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
