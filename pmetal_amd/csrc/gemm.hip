@@ -1103,7 +1103,7 @@ __device__ __forceinline__ void rw_half_q8(const uint4 *__restrict__ a_cur, uint
                 }
             }
         }
-        const float d = f16_bits_to_f32(cur.d[b]);
+        const float d = tile_scale(f16_bits_to_f32(cur.d[b]));
 #pragma unroll
         for (int i = 0; i < MB; i++)
 #pragma unroll

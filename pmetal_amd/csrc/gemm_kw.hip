@@ -175,7 +175,7 @@ struct KwQ8 {  // eight 34-byte blocks stand for a super-block; a half (136 byte
         else b[0] = q8_operand(__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16));
     }
     __device__ __forceinline__ half8_t sums(int) const { return half8_t{0, 0, 0, 0, 0, 0, 0, 0}; }
-    __device__ __forceinline__ float scale(int t) const { return ds[(t >> 1) % 2]; }
+    __device__ __forceinline__ float scale(int t) const { return tile_scale(ds[(t >> 1) % 2]); }
 };
 
 template <int FMT>
