@@ -64,13 +64,15 @@ struct PrepRaw {  // the eight elements of an item as they lie in memory
 // NI > 0: k <= 8 NI NT / R; a thread's items stay in registers between the row maximum and the conversion.  NI = 0: any k.
 template <bool XF32, int ORDER, int R, int NI>
 __global__ __launch_bounds__(R == 1 ? 512 : 1024) void k_prep_rw(const void *__restrict__ xg, int64_t k, int M, int Mp,
-                                                                  float *__restrict__ rowscale, uint4 *__restrict__ xs) {
+                                                                  float *__restrict__ rowscale, uint4 *__restrict__ xs, uint32_t *__restrict__ clear,
+                                                                  int n_clear) {  // (n_clear: at most 512 words)
     constexpr int NT = R == 1 ? 512 : 1024, JN = NT / R, NWV = NT / 64;
     constexpr int kGroups = ORDER == 5 ? 20 : (ORDER == 2 || ORDER == 3 ? 16 : 18);  // items per half super-block and row (shadows the Q4_K constant)
     const int tid = threadIdx.x, lane = tid & 63, r = tid % R, j = tid / R;
     const int m = blockIdx.x * R + r;
     const bool live = m < M;
     const int64_t items = k / 8;
+    if (blockIdx.x == 0 && tid < n_clear) clear[tid] = 0;
     // an item's two runs of four elements (lo, hi), its half super-block and its operand group
     auto place = [&](const int64_t q, int64_t &lo, int64_t &hi, int64_t &half, int &t, int &g) __attribute__((always_inline)) {
         if (ORDER == 2 || ORDER == 3) {  // half = 128 elements, 16 items
@@ -2782,7 +2784,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     const int64_t ni = (k / 8 * per_wg + (per_wg == 1 ? 511 : 1023)) / (per_wg == 1 ? 512 : 1024);
 #define PMH_PREP_N(F, O, R, NI)                                                                                              \
     hipLaunchKernelGGL((k_prep_rw<F, O, R, NI>), dim3((unsigned)p.mp / (R)), dim3((R) == 1 ? 512 : 1024), 0, s, x, k, (int)m, \
-                       (int)p.mp, rowscale, xs)
+                       (int)p.mp, rowscale, xs, arrived, n_arrived)
 #define PMH_PREP_R(F, O, R)                       \
     do {                                          \
         if (ni <= 1) PMH_PREP_N(F, O, R, 1);      \
@@ -2799,6 +2801,12 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
         else if (per_wg == 2) PMH_PREP_R(F, O, 2); \
         else PMH_PREP_R(F, O, 1);               \
     } while (0)
+    // The tile kernel adds the splits of K itself where this call's pre-pass has cleared its counters, at most 256 of them: they lie in the slack
+    // behind the partial tiles, 8 KiB and more.
+    const int64_t kw_tiles = ((n + 32 * p.nr - 1) / (32 * p.nr)) * ((m + 32 * p.mb - 1) / (32 * p.mb));
+    const bool joined = p.kernel == GemmKernel::kWaves && p.splits > 1 && joins_splits(p.mb, p.nr) && !reuse_prepass && kw_tiles <= 256;
+    uint32_t *const arrived = joined ? reinterpret_cast<uint32_t *>(ws + plan_bytes(p, type, n, k) - kw_slack(p)) : nullptr;
+    const int n_arrived = joined ? (int)kw_tiles : 0;
     const bool own = qgemm_converts_itself(p, type, m, n, second.n, k, x_dtype, shared);
     if (own) {
         // Every wave converts what it multiplies.  Results over the activations would race with other workgroups' reads of them.
@@ -2851,8 +2859,8 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     if (e != hipSuccess) return e;
     const bool ybf = y_dtype == kDtypeBf16;
     if (p.kernel == GemmKernel::kWaves) {
-        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, second, s);
-        if (e != hipSuccess || p.splits == 1) return e;
+        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, arrived, second, s);
+        if (e != hipSuccess || p.splits == 1 || joined) return e;
     } else if (p.kernel == GemmKernel::kSmall) {
         const int nwaves = spr < kSmallWaves ? spr : kSmallWaves;
         const int tiles = (int)((n + 15) / 16);

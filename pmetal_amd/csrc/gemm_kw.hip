@@ -255,7 +255,7 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
 };
 
 // ------------------------------------------------------------------------------------------------
-constexpr int kKwWaves = 8;
+constexpr int kKwWaves = 8, kMostSplits = 4;  // (as the plan makes them)
 // A wave's accumulators lie in LDS as the 64 lanes' 16-byte slots (four rows of one column), lane l at tile_slot(l): a thread that
 // reads four neighbouring columns back and one that writes its slot meet 64 different banks with the 15 beside them.
 constexpr int kTileRun = 76;
@@ -380,12 +380,18 @@ __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__
     }
 }
 
+// Partial sums go from one workgroup to another inside a launch: stores and loads that every die sees (relaxed, agent scope), so that
+// no cache has to be written back or emptied for them.  (A release and an acquire in their place, a write-back of the die's whole L2 for
+// each workgroup, made a call 2 to 11 us longer: Q6_K 4096 x 14336 at 27 rows 26.8 -> 36.0.)
+__device__ __forceinline__ void put_shared(float *to, const float v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float get_shared(const float *from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 // Adds the waves' tiles in wave order and stores the sums.  Run (rg, block i, quarter q) of a tile: lane l = 32 g + c left rows 8 q + 4 g
 // .. + 3 of block i and column c of row group rg at tile_slot(l).  A thread takes COLS neighbouring columns of four rows, as many
 // as leave every thread something to do: with four a row of the result leaves in 8 or 16 bytes a lane, with one in 2 or 4.
 // (One column a thread throughout, stores of 2 bytes a lane: a workgroup of four waves and a 64 x 64 tile took 2.9 us from its loop's end to
 // its last store, 1.5 now; 14336 x 4096 M = 64 with four waves 23.4 -> 22.3 us a call, Q8_0 4999 x 3584 M = 203 34.3 -> 32.9.)
-template <int TILE, int MB, int NR, int COLS, int WAVES>
+template <int TILE, int MB, int NR, int COLS, int WAVES, bool SHARED>
 __device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, const int nwaves, const int m0, const int n0, const int M, const int Mp,
                                           const int N, const int z, const int ybf16, void *__restrict__ yg, float *__restrict__ partial) {
     constexpr int kPer = 32 / COLS;  // threads of a row
@@ -412,7 +418,11 @@ __device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, 
             if (m + e >= M) break;
             float *to = partial ? partial + ((size_t)z * Mp + m + e) * N + n : reinterpret_cast<float *>(yg) + (size_t)(m + e) * N + n;
             uint16_t *to16 = reinterpret_cast<uint16_t *>(yg) + (size_t)(m + e) * N + n;
-            if (COLS > 1 && n + COLS <= N) {
+            if (SHARED) {
+#pragma unroll
+                for (int c = 0; c < COLS; c++)
+                    if (n + c < N) put_shared(to + c, t[0][c][e]);
+            } else if (COLS > 1 && n + COLS <= N) {
                 if (bf) {
                     RowPiece<uint32_t, 2, COLS / 2> v;
 #pragma unroll
@@ -436,14 +446,57 @@ __device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, 
     }
 }
 
+// The splits of K of a tile, each of which has left its partial sums: the workgroup that comes last adds them in split order, as k_rw_reduce
+// does, whose launch it saves: us of a call at 27 rows with that launch / so, Q4_K 4096 x 14336 19.6 / 18.6, 2560 x 9728 14.7 / 13.9, Q6_K 25.4 /
+// 24.4, 17.9 / 17.1, Q8_0 24.0 / 23.2; four splits of 64 x 32 tiles 1 to 2 %.  (Who is last does not change the result.  Nobody waits for
+// anybody: `arrived` counts, and the pre-pass has cleared it.)
+template <int MB, int NR>
+__device__ __forceinline__ void join_splits(uint32_t *arrived, const int splits, const int m0, const int n0, const int M, const int Mp, const int N,
+                                            const float *__restrict__ rowscale, const int ybf16, void *__restrict__ yg, const float *partial) {
+    __shared__ uint32_t before;
+    wait_vm<0>();  // this wave's partial sums have arrived where every die sees them; behind the barrier, everyone's
+    __syncthreads();
+    if (threadIdx.x == 0) before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (before + 1 != (uint32_t)splits) return;
+    constexpr int kAtATime = MB * NR == 1 ? 2 : 8;  // outputs a thread asks for together: a trip to memory each otherwise
+    const size_t plane = (size_t)Mp * N;
+    for (int u0 = (int)threadIdx.x; u0 < 1024 * MB * NR; u0 += kAtATime * (int)blockDim.x) {
+        float t[kAtATime][kMostSplits], rs[kAtATime];
+#pragma unroll
+        for (int e = 0; e < kAtATime; e++) {
+            const int u = u0 + e * (int)blockDim.x, m = m0 + u / (32 * NR), n = n0 + u % (32 * NR);
+            const bool in = u < 1024 * MB * NR && m < M && n < N;
+            const float *src = partial + (in ? (size_t)m * N + n : 0);
+            rs[e] = rowscale[in ? m : 0];
+#pragma unroll
+            for (int z = 0; z < kMostSplits; z++) t[e][z] = get_shared(src + (z < splits ? z : 0) * plane);
+        }
+#pragma unroll
+        for (int e = 0; e < kAtATime; e++) {
+            const int u = u0 + e * (int)blockDim.x, m = m0 + u / (32 * NR), n = n0 + u % (32 * NR);
+            if (u >= 1024 * MB * NR || m >= M || n >= N) continue;
+            float v = t[e][0];
+#pragma unroll
+            for (int z = 1; z < kMostSplits; z++)
+                if (z < splits) v += t[e][z];
+            v *= rs[e];
+            if (ybf16) reinterpret_cast<uint16_t *>(yg)[(size_t)m * N + n] = (uint16_t)bf16_rne_bits(v);
+            else reinterpret_cast<float *>(yg)[(size_t)m * N + n] = v;
+        }
+    }
+}
+
+// SPLIT: with a K split; then there is no second weight, and second.y is the tiles' counters, or NULL where k_rw_reduce adds the splits.
+// (One kernel for both is 0.1 us slower without a split.)
 // grid (8, inner x splits of K, outer / 8), up to eight waves; split z has super-blocks [z * chunk, min(spr, (z + 1) * chunk)).
 // Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the blocks of activation rows,
 // otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
-template <class F, int MB, int NR>
+template <class F, int MB, int NR, bool SPLIT>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
                                                              int spr, int chunk, int inner, int outer, int by_m, int ybf16,
-                                                             float *__restrict__ partial, const pmh::GemmSecond second) {
+                                                             float *partial, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
     extern __shared__ uint4 smem[];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, g = lane >> 5;
@@ -451,7 +504,10 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     const int out = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / inner, in = (int)blockIdx.y - z * inner;
     if (out >= outer) return;  // (the whole workgroup)
     int nt = by_m ? in : out;
-    take_weight(second, ybf16, nt, W, yg, N);
+    if (!SPLIT) {
+        take_weight(second, ybf16, nt, W, yg, N);
+        partial = nullptr;
+    }
     const int m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
     // wave w takes every nwaves'th super-block of the split from the w'th on: what the workgroup reads at a time lies side by side
@@ -527,8 +583,13 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
                          : float4_t{acc[rg][i][4 * q], acc[rg][i][4 * q + 1], acc[rg][i][4 * q + 2], acc[rg][i][4 * q + 3]};
     if (wave == 0 && lane < 32 * MB) rs[lane] = rs_mine;
     __syncthreads();
-    if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
-    else add_tiles<K::kTile, MB, NR, MB * NR, 4>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
+    constexpr bool kJoins = SPLIT && pmh::joins_splits(MB, NR);
+    if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves, kJoins>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
+    else add_tiles<K::kTile, MB, NR, MB * NR, 4, kJoins>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
+    if constexpr (kJoins) {
+        if (second.y)  // (in the place of a second weight's result: the counters)
+            join_splits<MB, NR>(reinterpret_cast<uint32_t *>(second.y) + out * inner + in, (int)gridDim.y / inner, m0, n0, M, Mp, N, rowscale, ybf16, yg, partial);
+    }
 }
 
 }  // namespace
@@ -537,9 +598,9 @@ namespace pmh {
 
 template <class F, int MB, int NR>
 static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n, int spr,
-                            float *partial, GemmSecond second, hipStream_t s) {
+                            float *partial, uint32_t *arrived, GemmSecond second, hipStream_t s) {
     using K = Kw<F, MB, NR>;
-    auto kern = k_qgemm_kw<F, MB, NR>;
+    auto kern = p.splits > 1 ? k_qgemm_kw<F, MB, NR, true> : k_qgemm_kw<F, MB, NR, false>;
     const int nwaves = p.chunk < p.nw ? p.chunk : p.nw;
     const size_t stage = (size_t)nwaves * 2 * K::kItems * 16, red = (size_t)nwaves * K::kTile * 16 + 32 * MB * 4, lds = stage > red ? stage : red;
     static_assert((size_t)kKwWaves * 2 * K::kItems * 16 <= 160 * 1024 && (size_t)kKwWaves * K::kTile * 16 + 32 * MB * 4 <= 160 * 1024, "LDS");
@@ -551,6 +612,7 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
     const int tiles = second.first + (second.n + 32 * NR - 1) / (32 * NR), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
     const bool by_m = kw_by_m(mblocks, tiles, MB, NR, F::kBytes);
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
+    if (p.splits > 1) second.y = arrived;  // (a K split has no second weight)
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
     hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer, by_m ? 1 : 0,
                        (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond : 0), p.splits > 1 ? partial : nullptr, second);
@@ -559,18 +621,18 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
 
 template <class F>
 static hipError_t launch_kw_tile(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n,
-                                 int spr, float *partial, GemmSecond second, hipStream_t s) {
-    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
-    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
-    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
-    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, second, s);
+                                 int spr, float *partial, uint32_t *arrived, GemmSecond second, hipStream_t s) {
+    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
+    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
+    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
+    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
 }
 
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &p, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
-                           int64_t n, int spr, uint32_t order, float *partial, const GemmSecond &second, hipStream_t s) {
+                           int64_t n, int spr, uint32_t order, float *partial, uint32_t *arrived, const GemmSecond &second, hipStream_t s) {
     const uint4 *x4 = reinterpret_cast<const uint4 *>(xs);
     const bool ref = order == kOrderRef;
-    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, second, s); };
+    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s); };
     switch (type) {
     case kTypeQ4K: return ref ? go(KwQ45<0, 0>{}) : go(KwQ45<1, 0>{});
     case kTypeQ5K: return ref ? go(KwQ45<0, 1>{}) : go(KwQ45<1, 1>{});

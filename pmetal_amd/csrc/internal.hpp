@@ -124,9 +124,13 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
                         int64_t m, void *y, uint32_t y_dtype, uint32_t order, void *workspace, hipStream_t s,
                         bool reuse_prepass = false, const GemmSecond &second = GemmSecond{}, bool shared = false);
 
-// gemm_kw.hip (spr: super-blocks per row; partial: fp32 tiles [splits][mp][n] when plan.splits > 1, not scaled by rowscale)
+// Which tiles of the tile kernel's launch add their splits of K themselves (gemm_kw.hip).  Not 64 x 64 ones: four waves take in up to 64 KiB of
+// partial sums then, which the launch behind reads with the whole machine (Q4_K 2048 x 8192 M = 120 21.2 us a call, 24.8 without it).
+constexpr bool joins_splits(int mb, int nr) { return mb * nr < 4; }
+// gemm_kw.hip (spr: super-blocks per row; partial: fp32 tiles [splits][mp][n] when plan.splits > 1, not scaled by rowscale; arrived: a
+// cleared counter per tile of Y, where the launch adds the splits itself)
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &plan, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
-                           int64_t n, int spr, uint32_t order, float *partial, const GemmSecond &second, hipStream_t s);
+                           int64_t n, int spr, uint32_t order, float *partial, uint32_t *arrived, const GemmSecond &second, hipStream_t s);
 
 // ---- q8k.hip: Q8_K activation blocks and the integer dot products over them ----
 hipError_t launch_quantize_q8k(const float *x, size_t n, uint8_t *dst, hipStream_t s);

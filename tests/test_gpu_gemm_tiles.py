@@ -446,3 +446,54 @@ def test_short_batches_with_infinities(oracle, t, k, dtype):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
     assert np.max(np.abs(got[15] - want[15])) <= bound(k) * np.max(np.abs(want[15]))
+
+
+# Splits of K of a tile, added by the workgroup that comes last (a call of its own, the first weight of a batch) or by a launch behind (the
+# other weights, whose call has no pre-pass to clear the counters): the same bits.  Two and four splits, the last one shorter or without
+# work; one row and column past a tile and short of it; 32 x 32, 64 x 32 and 64 x 64 tiles, up to 128 of them.
+SPLIT_CASES = [(17, 8448, (1, 33)), (31, 8192, (70, 4096)), (32, 9728, (2560, 31)), (64, 8192, (97, 1000)), (63, 14336, (65, 2048)),
+               (100, 8192, (1023, 130)), (200, 14336, (1000, 64)), (500, 8192, (700, 129))]
+
+
+@pytest.mark.parametrize("m,k,ns", SPLIT_CASES)
+@pytest.mark.parametrize("t", [Q4K, Q6K, Q8_0, 13, 11, 10])
+def test_splits_of_a_tile(oracle, t, m, k, ns):
+    for n in ns:
+        p = gemm_plan(t, m, n, k)
+        if p.kernel == WAVES and p.splits > 1:
+            break
+    else:
+        pytest.skip("no K split of tiles")
+    test_pairs_match_separate_calls(oracle, t, m, k, ns)
+
+
+@pytest.mark.parametrize("m,n,k,y_dtype", [(27, 4096, 14336, pm.DTYPE_F32), (100, 1001, 8192, pm.DTYPE_BF16)])
+def test_splits_of_a_tile_replayed(m, n, k, y_dtype):
+    p = gemm_plan(Q6K, m, n, k)
+    assert p.kernel == WAVES and p.splits > 1
+    lib, size = _lib.load(), m * n * (4 if y_dtype == pm.DTYPE_F32 else 2)
+    rng = np.random.default_rng(m)
+    dw, dx, dy = pm.DeviceBuffer.from_host(random_blocks(rng, Q6K, n, k)), pm.DeviceBuffer.from_host(rng.standard_normal((m, k)).astype(np.float32)), pm.DeviceBuffer(size)
+    stream = lib.pmetal_hip_stream_create()
+
+    def call():
+        pm.check(lib.pmetal_hip_qgemm(Q6K, dw.ptr, n, k, dx.ptr, pm.DTYPE_F32, m, dy.ptr, y_dtype, 0, stream))
+
+    try:
+        call()
+        pm.check(lib.pmetal_hip_sync(stream))
+        want = dy.to_host(np.uint8)
+        pm.check(lib.pmetal_hip_record_begin(stream))
+        for _ in range(2):
+            call()
+        rec = lib.pmetal_hip_record_end(stream)
+        assert rec, lib.pmetal_hip_last_error_message()
+        for rep in range(4):
+            pm.check(lib.pmetal_hip_memset(dy.ptr, 0xFF, size, None))
+            pm.check(lib.pmetal_hip_sync(None))
+            pm.check(lib.pmetal_hip_replay(rec, stream))
+            pm.check(lib.pmetal_hip_sync(stream))
+            assert np.array_equal(dy.to_host(np.uint8), want), rep
+        lib.pmetal_hip_recording_destroy(rec)
+    finally:
+        lib.pmetal_hip_stream_destroy(stream)
