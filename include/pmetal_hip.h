@@ -137,9 +137,9 @@ int32_t pmetal_hip_event_destroy(void *event);
  * pmetal_hip_tensor_size(type, n).  A trailing partial 256-super-block is emitted as
  * zero bytes (k_quants.rs:890-892); Q8_0 zero-pads inside its last block.
  * The host variants (here and of dequantize) are synchronous; tensors of 256 Ki elements
- * or more stream through pinned staging buffers that the library keeps (3 x 21 MiB of
- * pinned host and of device memory per device, made on first use), and such calls take
- * turns across threads.                                                                */
+ * or more stream through staging buffers that the library keeps (3 x 21 MiB of pinned
+ * host and 3 x 16 MiB of device memory per device, made on first use), and such calls
+ * take turns across threads.                                                           */
 int32_t pmetal_hip_quantize(uint32_t ggml_type, const float *src_host, size_t n, uint8_t *dst_host,
                             size_t dst_len);
 int32_t pmetal_hip_quantize_dev(uint32_t ggml_type, const float *src_dev, size_t n, uint8_t *dst_dev,

@@ -24,7 +24,8 @@
 // pre-pass included, and per round and eight super-blocks of a row 2.9 (Q2_K), 3.5 (Q4_K, Q3_K), 4.6 (Q5_K), 4.9 us (Q8_0, Q6_K) with 32 x
 // 32 tiles (up to 32 activation rows, rows of 32 super-blocks and more); 0.6 to 0.8 of that where fewer than 64 workgroups run.  Inside, by
 // counters (share of the waves' time that they issue / are ready and cannot issue / wait for memory, LDS or each other; share of the
-// time that the matrix cores work):
+// time that the matrix cores work; all with eight waves a workgroup and the splits added by a launch behind: as they are 29.2, 24.8 and, the sum of
+// the splits in it, 21.5 us):
 //   Q4_K, two of 14336 x 4096, M = 64 (64 x 64, 448 workgroups)       34.0 us  28 / 50 / 22 %, matrix cores 25 %
 //   Q8_0, 4999 x 3584, M = 203 (64 x 32, 628 workgroups)              28.8 us  37 / 29 / 34 %, 17 % (LDS bank conflicts 15 %: rows of 144 bytes)
 //   Q6_K, 4096 x 14336, M = 27 (32 x 32, two splits, 256 workgroups)  21.7 us  33 / 36 / 32 %, 17 %
