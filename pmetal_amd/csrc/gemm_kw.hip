@@ -299,7 +299,7 @@ struct KwCopy {  // a wave's copies of one unit
 // items to the wave's next ones.
 template <class F, int MB, int NR, int H, bool NEXT>
 __device__ __forceinline__ void kw_half(const uint4 *__restrict__ cur, uint4 *__restrict__ nxt, const __amdgpu_buffer_rsrc_t r, const uint32_t sb_next,
-                                        const KwCopy<F, MB, NR> &C, const uint8_t *__restrict__ &xa, const uint32_t step, const uint32_t jump, const uint32_t a_off,
+                                        const KwCopy<F, MB, NR> &C, const uint8_t *__restrict__ &xa, const uint32_t step, const size_t jump, const uint32_t a_off,
                                         half8_t (&af)[Kw<F, MB, NR>::kDepth][MB], const int lane, float16_t (&acc)[NR][MB], float16_t (&part)[NR][MB]) {
     using K = Kw<F, MB, NR>;
     const int col = lane & 31, g = lane >> 5;
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         for (int i = 0; i < MB; i++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[rg][i][e] = 0.0f, part[rg][i][e] = 0.0f;
-    const uint32_t jump = (uint32_t)(nwaves - 1) * (2 * K::kSteps) * step;
+    const size_t jump = (size_t)(nwaves - 1) * (2 * K::kSteps) * step;  // (past 4 GiB from 2.2 million activation rows on)
     for (int s = 0; s + 1 < cnt; s++) {
         if (F::kUnitHalves == 1) {
             kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);

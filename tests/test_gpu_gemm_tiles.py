@@ -497,3 +497,33 @@ def test_splits_of_a_tile_replayed(m, n, k, y_dtype):
         lib.pmetal_hip_recording_destroy(rec)
     finally:
         lib.pmetal_hip_stream_destroy(stream)
+
+
+# So many activation rows that a wave's way from one of its super-blocks to the next is more than 4 GiB of items (1920 bytes a row for Q2_K, 1728
+# for Q4_K, with four waves): rows from every part of them, the last one among them.
+@pytest.mark.parametrize("t,m", [(10, 2300001), (Q4K, 2560001)])
+def test_millions_of_activation_rows(oracle, t, m):
+    n, k, chunk = 64, 1280, 100000
+    p = gemm_plan(t, m, n, k)
+    assert (p.kernel, p.nw) == (WAVES, 4) and 3 * {10: 640, Q4K: 576}[t] * p.mp > 1 << 32
+    lib, stream = _lib.load(), _lib.load().pmetal_hip_stream_create()  # (its workspace goes with it)
+    rng = np.random.default_rng(m)
+    raw = random_blocks(rng, t, n, k)
+    dw, dx, df, dy = pm.DeviceBuffer.from_host(raw), pm.DeviceBuffer(2 * m * k), pm.DeviceBuffer(4 * chunk * k), pm.DeviceBuffer(4 * m * n)
+    try:
+        for r in range(0, m, chunk):
+            elems = min(chunk, m - r) * k
+            pm.check(lib.pmetal_hip_fill_normal_f32(df.ptr, elems, r + 1, 1.0, 0.0, 0.0, stream))
+            pm.check(lib.pmetal_hip_f32_to_bf16_dev(df.ptr, dx.ptr + 2 * r * k, elems, stream))
+        pm.check(lib.pmetal_hip_memset(dy.ptr, 0xFF, 4 * m * n, stream))
+        pm.check(lib.pmetal_hip_qgemm(t, dw.ptr, n, k, dx.ptr, pm.DTYPE_BF16, m, dy.ptr, pm.DTYPE_F32, 0, stream))
+        pm.check(lib.pmetal_hip_sync(stream))
+        rows = np.concatenate([np.arange(4), rng.integers(0, m, 40), np.arange(m - 4, m)])
+        x, got = np.empty((rows.size, k), np.uint16), np.empty((rows.size, n), np.float32)
+        for i, r in enumerate(rows):
+            pm.check(lib.pmetal_hip_d2h(x[i].ctypes.data, dx.ptr + 2 * int(r) * k, 2 * k))
+            pm.check(lib.pmetal_hip_d2h(got[i].ctypes.data, dy.ptr + 4 * int(r) * n, 4 * n))
+    finally:
+        pm.check(lib.pmetal_hip_stream_destroy(stream))
+    want = reference(oracle, t, raw, n, k, oracle.bf16_bits_to_f32(x.reshape(-1)).reshape(rows.size, k), 0)
+    assert np.max(np.abs(got - want)) <= (k / 16 + 16) * 2.0 ** -24 * 4 * np.max(np.abs(want))  # (the bound of the other tiles)
