@@ -2637,8 +2637,9 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         t.mb = kw.mb, t.nr = kw.nr, t.nw = kw.nw, t.splits = kw.splits, t.chunk = (int)((spr + kw.splits - 1) / kw.splits);
         // (one padding for both block heights and for the row kernels of the batch's wider weights: they share their converted activations)
         t.mp = (int)(m <= 32 ? 32 : m <= 192 ? (m + 63) / 64 * 64 : (m + 127) / 128 * 128);
-        // its items past the end (and now and then more splits) take more scratch: not where only the other kernel's fits the array of
-        // the entry point that allocates nothing
+        // ... where that fits the array of the entry point that allocates nothing; the tiles themselves need whole blocks of 64
+        if (m > 192 && plan_bytes(t, type, n, k) > PMETAL_HIP_NOALLOC_SCRATCH_BYTES) t.mp = (int)((m + 63) / 64 * 64);
+        // its items past the end (and now and then more splits) take more scratch: not where only the other kernel's fits that array
         if (plan_bytes(t, type, n, k) <= PMETAL_HIP_NOALLOC_SCRATCH_BYTES || plan_bytes(p, type, n, k) > PMETAL_HIP_NOALLOC_SCRATCH_BYTES) p = t;
     }
     return p;

@@ -102,7 +102,7 @@ struct GemmPlan {
 // Which operand's tiles the dies share among them in the tile kernel (true: the blocks of activation rows)
 bool kw_by_m(int64_t mblocks, int64_t tiles, int mb, int nr, int64_t block_bytes);
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k);
-// (the padded row count mp does not depend on the type; the K split does)
+// (the padded row count mp follows m and the kernel, and the type and n only where the entry point that allocates nothing would be short of scratch)
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type = kTypeQ4K);
 // Bytes of device workspace qgemm needs for a weight of `type` at (m, n, k); the caller provides it.
 size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k);

@@ -43,6 +43,15 @@ def test_workspace_holds_what_is_written(t, m, n, k):
     assert gemm_workspace_bytes(t, m, n, k) == need + (256 * p.mp if p.kernel == WAVES else 0)
 
 
+# Calls of the entry point that allocates nothing: what its 32 MiB of scratch hold with activations padded to whole tiles fits, also where the
+# padding to 128 rows that a batch's weights share would not.
+@pytest.mark.parametrize("t,m,n,k", [(Q6K, 1040, 125, 13568), (Q4K, 814, 67, 16128), (Q3K, 677, 68, 17920), (Q8_0, 1040, 125, 13568), (Q5K, 814, 67, 16128)])
+def test_scratch_that_whole_tiles_fit(t, m, n, k):
+    p = gemm_plan(t, m, n, k)
+    assert p.kernel == WAVES and p.mp % 128 == 64, p
+    assert gemm_workspace_bytes(t, m, n, k) <= 32 << 20
+
+
 # Few activation rows: the kernel that measured faster (us with the short-batch kernel, with the tile kernel), clear cases of either.
 @pytest.mark.parametrize("t,m,n,k,kernel", [
     (Q5K, 19, 17096, 19712, SMALL),  # 84, 135: long rows in three rounds of tiles
