@@ -373,7 +373,10 @@ __device__ __forceinline__ void rw_half(const uint4 *__restrict__ a_cur, uint4 *
     static_assert(Lane<MB, NR, NW>::kARounds <= 6, "two rounds of activation copies a step");
     if (MB < 4) {
 #pragma unroll
-        for (int step = 0; step < 5; step++) copies(step);
+        for (int step = 0; step < 5; step++) {
+            if (step == 3) __builtin_amdgcn_sched_barrier(0);  // (what follows is quant copies)
+            copies(step);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -633,7 +636,10 @@ __device__ __forceinline__ void rw16_half(const uint4 *__restrict__ a_cur, uint4
     static_assert(kARounds <= 6, "two rounds of activation copies a step");
     if (MB < 4) {
 #pragma unroll
-        for (int step = 0; step < 4; step++) copies(step);
+        for (int step = 0; step < 4; step++) {
+            if (step == 3) __builtin_amdgcn_sched_barrier(0);  // (what follows is quant copies)
+            copies(step);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -874,7 +880,10 @@ __device__ __forceinline__ void rw_half_q6(const uint4 *__restrict__ a_cur, uint
     static_assert(LaneQ6<MB>::kARounds <= 4, "two rounds of activation copies a step");
     if (MB < 4) {
 #pragma unroll
-        for (int step = 0; step < 6; step++) copies(step);
+        for (int step = 0; step < 6; step++) {
+            if (step == 3) __builtin_amdgcn_sched_barrier(0);  // (what follows is quant copies)
+            copies(step);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 
