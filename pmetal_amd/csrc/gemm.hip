@@ -2656,12 +2656,12 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
 
 size_t qgemm_workspace_bytes(uint32_t type, int64_t m, int64_t n, int64_t k) { return plan_bytes(qgemm_plan(m, n, k, type), type, n, k); }
 
-bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan) {
+static bool pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan, int *second_nw) {
     if (!qgemm_fits(type, m, n0 + n1, k)) return false;
     const GemmPlan p = qgemm_plan(m, n0, k, type), q = qgemm_plan(m, n1, k, type);
     // the same kernel for both and no K split: every result is then the sum, in the same order, that it is in a call of its own
     if (p.kernel != q.kernel || p.mp != q.mp || p.splits > 1 || q.splits > 1) return false;
-    *plan = p;
+    *plan = p, *second_nw = q.nw;
     // Short batches and wave tiles gain the second launch's start and the idle end of the first (us for two weights sharing their
     // activations, apart -> together: Q4_K 14336 x 4096 M = 16 27.2 -> 21.7, M = 64 41.9 -> 41.0; Q6_K 4096 x 4096 M = 16 21.9 ->
     // 13.4).  Row kernels, one workgroup per compute unit, only where a round of workgroups that neither weight fills goes
@@ -2675,10 +2675,19 @@ bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type
     if (p.kernel == GemmKernel::kWaves) {
         if (n0 + n1 > kKwMaxRows) return false;
         const KwChoice kw = kw_choice(m, n0 + n1, k / 256, type);
-        if (p.nw != q.nw) return false;
         if (kw.splits == 1) plan->mb = kw.mb, plan->nr = kw.nr;
+        // One weight's tiles have four waves, the other's eight: a launch of its own for each costs 4 to 6 us more, workgroups of eight waves
+        // for both what two workgroups of four on a compute unit gain. us, together / apart: Q4_K 4096 and 1024 x 4096, M = 100 17.6 / 20.9, Q6_K M = 96 20.1 /
+        // 28.0, Q8_0 2048 and 512 x 2048 M = 160 11.3 / 16.2, two and a half rounds of 64 x 32 tiles of Q8_0 2560 and 1280 x 2560 M = 300 30.6 / 26.9.
+        const int64_t spr = k / 256, tiles = ((n0 + 32 * plan->nr - 1) / (32 * plan->nr) + (n1 + 32 * plan->nr - 1) / (32 * plan->nr)) * ((m + 32 * plan->mb - 1) / (32 * plan->mb));
+        if (p.nw != q.nw && spr > 8 && tiles > (plan->mb * plan->nr == 1 ? 1024 : 512)) return false;
     }
     return true;
+}
+
+bool qgemm_pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t type, GemmPlan *plan) {
+    int second_nw;
+    return pair_plan(m, n0, n1, k, type, plan, &second_nw);
 }
 
 // Tiles of `rows` weight rows along the grid; with a second weight also where its tiles begin and the bit that says so.
@@ -2775,7 +2784,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     GemmSecond second = second_weight;
     GemmPlan p;
     if (second.n == 0) p = qgemm_plan(m, n, k, type);
-    else if (!qgemm_pair_plan(m, n, second.n, k, type, &p)) return hipErrorInvalidValue;
+    else if (!pair_plan(m, n, second.n, k, type, &p, &second.nw)) return hipErrorInvalidValue;
     const int spr = (int)(k / 256);
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
     uint4 *xs = reinterpret_cast<uint4 *>(ws);

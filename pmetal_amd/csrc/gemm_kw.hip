@@ -257,6 +257,8 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
 
 // ------------------------------------------------------------------------------------------------
 constexpr int kKwWaves = 8, kMostSplits = 4;  // (as the plan makes them)
+// Bits beside kHasSecond: the tiles of the first, of the second weight have four waves of the workgroup's eight; they go two to a workgroup (see launch_kw)
+constexpr int kFirstOfFour = 2, kSecondOfFour = 4, kByTwos = 8;
 // A wave's accumulators lie in LDS as the 64 lanes' 16-byte slots (four rows of one column), lane l at tile_slot(l): a thread that
 // reads four neighbouring columns back and one that writes its slot meet 64 different banks with the 15 beside them.
 constexpr int kTileRun = 76;
@@ -393,10 +395,10 @@ __device__ __forceinline__ float get_shared(const float *from) { return __hip_at
 // (One column a thread throughout, stores of 2 bytes a lane: a workgroup of four waves and a 64 x 64 tile took 2.9 us from its loop's end to
 // its last store, 1.5 now; 14336 x 4096 M = 64 with four waves 23.4 -> 22.3 us a call, Q8_0 4999 x 3584 M = 203 34.3 -> 32.9.)
 template <int TILE, int MB, int NR, int COLS, int WAVES, bool SHARED>
-__device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, const int nwaves, const int m0, const int n0, const int M, const int Mp,
-                                          const int N, const int z, const int ybf16, void *__restrict__ yg, float *__restrict__ partial) {
+__device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, const int tid, const int threads, const int nwaves, const int m0,
+                                          const int n0, const int M, const int Mp, const int N, const int z, const int ybf16, void *__restrict__ yg, float *__restrict__ partial) {
     constexpr int kPer = 32 / COLS;  // threads of a row
-    for (int u = (int)threadIdx.x; u < MB * NR * 8 * kPer; u += (int)blockDim.x) {
+    for (int u = tid; u < MB * NR * 8 * kPer; u += threads) {
         const int j = u % kPer, g = u / kPer & 1, rg = u / (2 * kPer) % NR, q = u / (2 * kPer * NR) & 3, i = u / (8 * kPer * NR);
         const int n = n0 + 32 * rg + COLS * j, ml = 32 * i + 8 * q + 4 * g, m = m0 + ml;
         const float4_t *src = red + ((rg * MB + i) * 4 + q) * kTileRun + tile_slot(32 * g + COLS * j);
@@ -501,20 +503,30 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     using K = Kw<F, MB, NR>;
     extern __shared__ uint4 smem[];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, g = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = (int)(blockDim.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block_waves = (int)(blockDim.x >> 6);
     const int out = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / inner, in = (int)blockIdx.y - z * inner;
     if (out >= outer) return;  // (the whole workgroup)
-    int nt = by_m ? in : out;
+    int nt = by_m ? in : out, nwaves = block_waves, tile_wave = wave, which = 0, tile_threads = (int)blockDim.x;
     if (!SPLIT) {
-        take_weight(second, ybf16, nt, W, yg, N);
+        if (ybf16 & kHasSecond) {
+            const bool of_four = ybf16 & (nt >= second.first ? kSecondOfFour : kFirstOfFour), by_twos = of_four && (ybf16 & kByTwos);
+            take_weight(second, ybf16, nt, W, yg, N);
+            ybf16 &= 1;
+            nwaves = of_four ? 4 : nwaves;
+            if (by_twos) {
+                tile_threads = 256, which = wave >> 2, tile_wave = wave & 3, nt = 2 * nt + which;
+                if (nt * (32 * NR) >= N) nt--, M = 0;  // (an odd last tile has none beside it: once more, and not stored)
+            }
+            nwaves = spr < nwaves ? spr : nwaves;
+        }
         partial = nullptr;
     }
     const int m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
     // wave w takes every nwaves'th super-block of the split from the w'th on: what the workgroup reads at a time lies side by side
-    const int own = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - z * chunk - wave;
+    const int own = (spr < (z + 1) * chunk ? spr : (z + 1) * chunk) - z * chunk - tile_wave;
     const bool idle = own < 1;  // the last split is the shortest: a wave left without work multiplies one super-block for nothing
-    const int sb0 = idle ? 0 : z * chunk + wave, cnt = idle ? 1 : (own + nwaves - 1) / nwaves;
+    const int sb0 = idle ? 0 : z * chunk + tile_wave, cnt = idle ? 1 : (own + nwaves - 1) / nwaves;
     const uint32_t row_bytes = (uint32_t)spr * F::kBytes;
     KwCopy<F, MB, NR> C;
 #pragma unroll
@@ -534,17 +546,9 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W + (size_t)n0 * row_bytes), 0, (int)(left < 0xFFFFFFF0u ? left : 0xFFFFFFF0u), 0x00027000);
     const uint32_t step = 32u * (uint32_t)Mp, a_off = (uint32_t)(g * Mp + m0 + col) * 16u;
     const uint8_t *xa = reinterpret_cast<const uint8_t *>(xs) + (size_t)(sb0 * 2 * K::kSteps) * step;
-    C.template issue<0>(r, sb_off, st0, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    half8_t af[Kw<F, MB, NR>::kDepth][MB];
-#pragma unroll
-    for (int s = 0; s < K::kDepth; s++) {
-#pragma unroll
-        for (int i = 0; i < MB; i++) af[s][i] = *reinterpret_cast<const half8_t *>(at(xa, a_off) + 512 * i);
-        xa += step;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    const float rs_mine = lane < 32 * MB ? rowscale[m0 + lane] : 0.0f;
+    // (beside a weight of eight waves a tile of four may have four more in its workgroup, which wait and store)
+    const bool works = SPLIT || tile_wave < nwaves;
+    float rs_mine = 0.0f;
     float16_t acc[NR][MB], part[NR][MB];
 #pragma unroll
     for (int rg = 0; rg < NR; rg++)
@@ -552,41 +556,57 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         for (int i = 0; i < MB; i++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[rg][i][e] = 0.0f, part[rg][i][e] = 0.0f;
-    const size_t jump = (size_t)(nwaves - 1) * (2 * K::kSteps) * step;  // (past 4 GiB from 2.2 million activation rows on)
-    for (int s = 0; s + 1 < cnt; s++) {
-        if (F::kUnitHalves == 1) {
-            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
-            sb_off += (uint32_t)nwaves * F::kBytes;
-            kw_half<F, MB, NR, 1, true>(st1, st0, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
-        } else {
-            sb_off += (uint32_t)nwaves * F::kBytes;
-            kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
-            kw_half<F, MB, NR, 1, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
-            uint4 *t = st0;
-            st0 = st1, st1 = t;
+    if (works) {
+        C.template issue<0>(r, sb_off, st0, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        half8_t af[Kw<F, MB, NR>::kDepth][MB];
+#pragma unroll
+        for (int s = 0; s < K::kDepth; s++) {
+#pragma unroll
+            for (int i = 0; i < MB; i++) af[s][i] = *reinterpret_cast<const half8_t *>(at(xa, a_off) + 512 * i);
+            xa += step;
         }
+        __builtin_amdgcn_sched_barrier(0);
+        rs_mine = lane < 32 * MB ? rowscale[m0 + lane] : 0.0f;
+        const size_t jump = (size_t)(nwaves - 1) * (2 * K::kSteps) * step;  // (past 4 GiB from 2.2 million activation rows on)
+        for (int s = 0; s + 1 < cnt; s++) {
+            if (F::kUnitHalves == 1) {
+                kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
+                sb_off += (uint32_t)nwaves * F::kBytes;
+                kw_half<F, MB, NR, 1, true>(st1, st0, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
+            } else {
+                sb_off += (uint32_t)nwaves * F::kBytes;
+                kw_half<F, MB, NR, 0, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
+                kw_half<F, MB, NR, 1, true>(st0, st1, r, sb_off, C, xa, step, jump, a_off, af, lane, acc, part);
+                uint4 *t = st0;
+                st0 = st1, st1 = t;
+            }
+        }
+        kw_half<F, MB, NR, 0, F::kUnitHalves == 1>(st0, st1, r, sb_off, C, xa, step, 0, a_off, af, lane, acc, part);
+        kw_half<F, MB, NR, 1, false>(F::kUnitHalves == 1 ? st1 : st0, st1, r, sb_off, C, xa, step, 0, a_off, af, lane, acc, part);
     }
-    kw_half<F, MB, NR, 0, F::kUnitHalves == 1>(st0, st1, r, sb_off, C, xa, step, 0, a_off, af, lane, acc, part);
-    kw_half<F, MB, NR, 1, false>(F::kUnitHalves == 1 ? st1 : st0, st1, r, sb_off, C, xa, step, 0, a_off, af, lane, acc, part);
-
     wait_vm<0>();
     __syncthreads();
     float4_t *red = reinterpret_cast<float4_t *>(smem);
-    float *rs = reinterpret_cast<float *>(smem) + (size_t)nwaves * K::kTile * 4;
+    float *rs = reinterpret_cast<float *>(smem) + (size_t)block_waves * K::kTile * 4 + 32 * MB * which;
+    if (works) {
 #pragma unroll
-    for (int rg = 0; rg < NR; rg++)
+        for (int rg = 0; rg < NR; rg++)
 #pragma unroll
-        for (int i = 0; i < MB; i++)
+            for (int i = 0; i < MB; i++)
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                red[wave * K::kTile + ((rg * MB + i) * 4 + q) * kTileRun + tile_slot(lane)] =
-                    idle ? float4_t{0.0f, 0.0f, 0.0f, 0.0f}
-                         : float4_t{acc[rg][i][4 * q], acc[rg][i][4 * q + 1], acc[rg][i][4 * q + 2], acc[rg][i][4 * q + 3]};
-    if (wave == 0 && lane < 32 * MB) rs[lane] = rs_mine;
+                for (int q = 0; q < 4; q++)
+                    red[wave * K::kTile + ((rg * MB + i) * 4 + q) * kTileRun + tile_slot(lane)] =
+                        idle ? float4_t{0.0f, 0.0f, 0.0f, 0.0f}
+                             : float4_t{acc[rg][i][4 * q], acc[rg][i][4 * q + 1], acc[rg][i][4 * q + 2], acc[rg][i][4 * q + 3]};
+    }
+    if (tile_wave == 0 && lane < 32 * MB) rs[lane] = rs_mine;
     __syncthreads();
+    red += 4 * which * K::kTile;
+    const int tile_tid = SPLIT ? (int)threadIdx.x : tid - 256 * which, threads = SPLIT ? (int)blockDim.x : tile_threads;
     constexpr bool kJoins = SPLIT && pmh::joins_splits(MB, NR);
-    if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves, kJoins>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
-    else add_tiles<K::kTile, MB, NR, MB * NR, 4, kJoins>(red, rs, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
+    if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves, kJoins>(red, rs, tile_tid, threads, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
+    else add_tiles<K::kTile, MB, NR, MB * NR, 4, kJoins>(red, rs, tile_tid, threads, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
     if constexpr (kJoins) {
         if (second.y)  // (in the place of a second weight's result: the counters)
             join_splits<MB, NR>(reinterpret_cast<uint32_t *>(second.y) + out * inner + in, (int)gridDim.y / inner, m0, n0, M, Mp, N, rowscale, ybf16, yg, partial);
@@ -602,21 +622,33 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
                             float *partial, uint32_t *arrived, GemmSecond second, hipStream_t s) {
     using K = Kw<F, MB, NR>;
     auto kern = p.splits > 1 ? k_qgemm_kw<F, MB, NR, true> : k_qgemm_kw<F, MB, NR, false>;
-    const int nwaves = p.chunk < p.nw ? p.chunk : p.nw;
-    const size_t stage = (size_t)nwaves * 2 * K::kItems * 16, red = (size_t)nwaves * K::kTile * 16 + 32 * MB * 4, lds = stage > red ? stage : red;
-    static_assert((size_t)kKwWaves * 2 * K::kItems * 16 <= 160 * 1024 && (size_t)kKwWaves * K::kTile * 16 + 32 * MB * 4 <= 160 * 1024, "LDS");
+    auto waves_of = [&](int nw) { return p.chunk < nw ? p.chunk : nw; };
+    const int w0 = waves_of(p.nw), w1 = second.n > 0 ? waves_of(second.nw) : w0;
+    // Two weights, tiles of eight waves (or what a short row has of them) and of four: workgroups of eight for both, so that either result
+    // is the sum that it is alone.
+    const bool mixed = w0 != w1;
+    const int nwaves = mixed ? kKwWaves : w0;
+    const size_t stage = (size_t)nwaves * 2 * K::kItems * 16, red = (size_t)nwaves * K::kTile * 16 + (mixed ? 2 : 1) * 32 * MB * 4, lds = stage > red ? stage : red;
+    static_assert((size_t)kKwWaves * 2 * K::kItems * 16 <= 160 * 1024 && (size_t)kKwWaves * K::kTile * 16 + 2 * 32 * MB * 4 <= 160 * 1024, "LDS");
     if (lds > 64 * 1024) {
         hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (a != hipSuccess) return a;
     }
-    second.first = (int)((n + 32 * NR - 1) / (32 * NR));
-    const int tiles = second.first + (second.n + 32 * NR - 1) / (32 * NR), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
-    const bool by_m = kw_by_m(mblocks, tiles, MB, NR, F::kBytes);
+    const int t0 = (int)((n + 32 * NR - 1) / (32 * NR)), t1 = (second.n + 32 * NR - 1) / (32 * NR), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
+    const bool by_m = kw_by_m(mblocks, t0 + t1, MB, NR, F::kBytes);
+    // Tiles of four go two to a workgroup where that is fewer rounds of workgroups, of which a compute unit holds one, and two of 32 x 32 tiles.
+    // Otherwise a workgroup each, whose other four waves wait: a machine that is not full has more of it at work (us, by twos / alone: Q8_0
+    // 4096 and 2048 x 4096 M = 96 30.6 / 23.4, Q4_K 4096 and 1024 x 4096 M = 100 24.1 / 17.6).
+    auto rounds = [&](int64_t tiles) { return (tiles * mblocks + (MB * NR == 1 ? 511 : 255)) / (MB * NR == 1 ? 512 : 256); };
+    const bool by_twos = mixed && rounds(w0 == 4 ? (t0 + 1) / 2 + t1 : t0 + (t1 + 1) / 2) < rounds(t0 + t1);
+    const int of_four = !mixed ? 0 : (w0 == 4 ? kFirstOfFour : kSecondOfFour) | (by_twos ? kByTwos : 0);
+    second.first = by_twos && w0 == 4 ? (t0 + 1) / 2 : t0;
+    const int tiles = second.first + (by_twos && w1 == 4 ? (t1 + 1) / 2 : t1);  // (or pairs of them)
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
     if (p.splits > 1) second.y = arrived;  // (a K split has no second weight)
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
     hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer, by_m ? 1 : 0,
-                       (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond : 0), p.splits > 1 ? partial : nullptr, second);
+                       (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond | of_four : 0), p.splits > 1 ? partial : nullptr, second);
     return hipGetLastError();
 }
 

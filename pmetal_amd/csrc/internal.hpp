@@ -88,7 +88,8 @@ struct GemmSecond {
     const uint8_t *w;
     void *y;
     int n;      // weight rows; 0: no second weight
-    int first;  // its first workgroup along the grid's x dimension (kWaves: its first tile)
+    int first;  // its first workgroup along the grid's x dimension (kWaves: its first tile, or pair of tiles)
+    int nw;     // kWaves: the waves of its tiles, as its own plan has them
 };
 struct GemmPlan {
     GemmKernel kernel;

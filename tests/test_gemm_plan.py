@@ -52,6 +52,23 @@ def test_scratch_that_whole_tiles_fit(t, m, n, k):
     assert gemm_workspace_bytes(t, m, n, k) <= 32 << 20
 
 
+# Two weights of one batch of which one has tiles of four waves and the other of eight: one launch where that is faster (us: apart, together).
+@pytest.mark.parametrize("t,m,n0,n1,k,share", [
+    (Q4K, 100, 4096, 1024, 4096, True),    # 20.9, 17.6: q and k of a grouped-query attention
+    (Q4K, 128, 3072, 1024, 3072, True),    # 17.6, 12.9
+    (Q6K, 96, 4096, 1024, 4096, True),     # 28.0, 20.1
+    (Q8_0, 160, 2048, 512, 2048, True),    # 16.2, 11.3
+    (Q5K, 160, 2048, 512, 2048, True),     # 16.2, 11.1
+    (Q2K, 46, 504, 6528, 1280, True),      # 13.2, 8.8
+    (Q3K, 141, 1763, 348, 256, True),      # 12.9, 8.4: a row of one super-block has one wave either way
+    (Q8_0, 300, 2560, 1280, 2560, False),  # 26.9, 30.6
+    (Q8_0, 454, 318, 3869, 4096, False)])  # 46.2, 52.9
+def test_pairs_of_four_and_eight_waves(t, m, n0, n1, k, share):
+    a, b = gemm_plan(t, m, n0, k), gemm_plan(t, m, n1, k)
+    assert (a.kernel, b.kernel) == (WAVES, WAVES) and a.nw != b.nw
+    assert (gemm_pair_plan(t, m, n0, n1, k) is not None) == share
+
+
 # Few activation rows: the kernel that measured faster (us with the short-batch kernel, with the tile kernel), clear cases of either.
 @pytest.mark.parametrize("t,m,n,k,kernel", [
     (Q5K, 19, 17096, 19712, SMALL),  # 84, 135: long rows in three rounds of tiles

@@ -113,6 +113,23 @@ def test_pairs_match_separate_calls(oracle, t, m, k, ns):
             assert np.array_equal(got, gpu_qgemm(t, raw, n, k, bits, m, order=order)), order
 
 
+# ... of which one has tiles of four waves and the other of eight (or the five of a short row), in one launch.  Of each tile: the weight of four
+# waves in front and behind, its tiles one to a workgroup beside four waves that wait (the first two cases), two to a workgroup, an odd and an
+# even number of them, where that saves a round of workgroups.
+MIXED = [(1, 1, 193, 2048, (174, 1980)), (1, 1, 135, 1280, (2656, 68)), (1, 1, 213, 1280, (1665, 654)), (1, 1, 155, 2048, (35, 3227)), (1, 1, 130, 1280, (2210, 1048)),
+         (2, 1, 163, 2048, (177, 2310)), (2, 1, 161, 1280, (2386, 71)), (2, 1, 182, 1280, (2049, 656)), (2, 1, 190, 2048, (520, 2193)), (2, 1, 177, 2304, (49, 2661)),
+         (2, 2, 162, 2048, (551, 2193)), (2, 2, 231, 1280, (1695, 367)), (2, 2, 272, 1280, (1040, 2221)), (2, 2, 384, 2304, (1483, 1177)), (2, 2, 234, 1792, (1872, 2188))]
+MIXED = [(t, *c) for c in MIXED for t in (Q4K, Q6K, Q8_0, 13, 11, 10)] + [(Q6K, 1, 2, 31, 2304, (1003, 9001)), (Q8_0, 1, 2, 31, 1280, (8500, 6000))]
+
+
+@pytest.mark.parametrize("t,mb,nr,m,k,ns", MIXED)
+def test_pairs_of_four_and_eight_waves(oracle, t, mb, nr, m, k, ns):
+    p = gemm_pair_plan(t, m, *ns, k)
+    assert p is not None and (p.kernel, p.mb, p.nr) == (WAVES, mb, nr), p
+    assert {gemm_plan(t, m, n, k).nw for n in ns} == {4, 8}
+    test_pairs_match_separate_calls(oracle, t, m, k, ns)
+
+
 def test_results_in_one_place_are_not_paired(oracle):
     m, n, k = 64, 300, 512
     rng = np.random.default_rng(5)
