@@ -2481,16 +2481,18 @@ constexpr double kRowsFit[6] = {1.312, 1.460, 1.966, 2.444, 1.672, 1.472};  // h
 static int fit_index(uint32_t type) {
     return type == kTypeQ4K ? 0 : type == kTypeQ5K ? 1 : type == kTypeQ6K ? 2 : type == kTypeQ8_0 ? 3 : type == kTypeQ3K ? 4 : 5;
 }
+// Whether the dies do not share the activations among them and each reads more of them than its cache holds.
+static bool dies_read_all(int64_t m, int64_t spr, int mb, int nr, int64_t tiles, uint32_t type) {
+    return m * spr * 512 > (int64_t)12 << 20 && !kw_by_m((m + 32 * mb - 1) / (32 * mb), tiles, mb, nr, block_bytes(type));
+}
 static double many_tiles_us(const KwChoice &kw, int64_t m, int64_t n, int64_t spr, uint32_t type) {
     const KwFit &f = kKwFits[kw.mb + kw.nr - 2];
     const double r = kw.rounds, whole = __builtin_ceil(r);
     const double rounds = r > 1.0 ? f.part * r + (1.0 - f.part) * whole : r < 0.5 ? 1.0 - f.few * (1.0 - 2.0 * r) : 1.0;
     const double us = f.call + rounds * (f.round + f.sb[fit_index(type)] * (double)((spr + kw.splits - 1) / kw.splits)) +
                       (kw.splits > 1 ? f.split + f.split_us * 1e-6 * kw.splits * (double)m * (double)n : 0.0);
-    // more activations than a die's cache holds, all of which its workgroups read at a time (Q4_K 14336 x 4096: M = 1024, 8 MB, 185
-    // us as expected, M = 2048 590 for 377)
-    const int64_t mt = (m + 32 * kw.mb - 1) / (32 * kw.mb), nt = (n + 32 * kw.nr - 1) / (32 * kw.nr);
-    return m * spr * 512 > (int64_t)12 << 20 && !kw_by_m(mt, nt, kw.mb, kw.nr, block_bytes(type)) ? us * 1.5 : us;
+    // (Q4_K 14336 x 4096: M = 1024, 8 MB of activations, 185 us as expected, M = 2048 590 for 377)
+    return dies_read_all(m, spr, kw.mb, kw.nr, (n + 32 * kw.nr - 1) / (32 * kw.nr), type) ? us * 1.5 : us;
 }
 static double many_rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
     const int64_t wgs = (n + 255) / 256 * (p.mp / (32 * p.mb)) * p.splits;
@@ -2679,8 +2681,16 @@ static bool pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t typ
         // One weight's tiles have four waves, the other's eight: a launch of its own for each costs 4 to 6 us more, workgroups of eight waves
         // for both what two workgroups of four on a compute unit gain. us, together / apart: Q4_K 4096 and 1024 x 4096, M = 100 17.6 / 20.9, Q6_K M = 96 20.1 /
         // 28.0, Q8_0 2048 and 512 x 2048 M = 160 11.3 / 16.2, two and a half rounds of 64 x 32 tiles of Q8_0 2560 and 1280 x 2560 M = 300 30.6 / 26.9.
-        const int64_t spr = k / 256, tiles = ((n0 + 32 * plan->nr - 1) / (32 * plan->nr) + (n1 + 32 * plan->nr - 1) / (32 * plan->nr)) * ((m + 32 * plan->mb - 1) / (32 * plan->mb));
+        const int64_t spr = k / 256, nt = (n0 + 32 * plan->nr - 1) / (32 * plan->nr) + (n1 + 32 * plan->nr - 1) / (32 * plan->nr);
+        const int64_t tiles = nt * ((m + 32 * plan->mb - 1) / (32 * plan->mb));
         if (p.nw != q.nw && spr > 8 && tiles > (plan->mb * plan->nr == 1 ? 1024 : 512)) return false;
+        // Tiles of which alone the dies share the activations, and together, more weight rows than activation rows then, the weights. That
+        // costs from some 1300 activation rows on; Q8_0's tiles, which take longer, from 1900, Q6_K's nothing. us, together / apart, two
+        // weights: Q4_K 4600 x 4096 M = 2048 390 / 232, 3322 x 4864 M = 1487 206 / 155, 2352 x 5888 M = 1081 111 / 139, Q2_K 5502 x 9216 M = 1709 927 / 533,
+        // Q5_K 3032 and 1694 x 7168 M = 1456 224 / 193, Q8_0 2932 x 6912 M = 2004 373 / 329, 1891 x 7936 M = 1540 216 / 226, Q6_K 3366 x 4608 M = 2362 370 / 380.
+        auto alone = [&](const GemmPlan &a, int64_t n) { return dies_read_all(m, spr, a.mb, a.nr, (n + 32 * a.nr - 1) / (32 * a.nr), type); };
+        const int64_t most = type == kTypeQ6K ? m : type == kTypeQ8_0 ? 1900 : 1280;
+        if (m > most && dies_read_all(m, spr, plan->mb, plan->nr, nt, type) && !(alone(p, n0) && alone(q, n1))) return false;
     }
     return true;
 }

@@ -69,6 +69,23 @@ def test_pairs_of_four_and_eight_waves(t, m, n0, n1, k, share):
     assert (gemm_pair_plan(t, m, n0, n1, k) is not None) == share
 
 
+# Two weights whose tiles alone let the dies share the activations, and together do not: apart where each die would then read more of them than it
+# can hold, and that takes longer (us: together, apart).
+@pytest.mark.parametrize("t,m,n0,n1,k,share", [
+    (Q4K, 2048, 4600, 4600, 4096, False),  # 390, 232
+    (Q4K, 1487, 3322, 3322, 4864, False),  # 206, 155
+    (Q4K, 1081, 2352, 2352, 5888, True),   # 111, 139
+    (Q2K, 1709, 5502, 5502, 9216, False),  # 927, 533
+    (Q3K, 1848, 5305, 5305, 6400, False),  # 673, 430
+    (Q5K, 1456, 3032, 1694, 7168, False),  # 224, 193
+    (Q8_0, 2004, 2932, 2932, 6912, False), # 373, 329
+    (Q8_0, 1540, 1891, 1891, 7936, True),  # 216, 226
+    (Q6K, 2362, 3366, 3366, 4608, True)])  # 370, 380
+def test_pairs_of_many_activation_rows(t, m, n0, n1, k, share):
+    assert gemm_plan(t, m, n0, k).kernel == WAVES and gemm_plan(t, m, n1, k).kernel == WAVES
+    assert (gemm_pair_plan(t, m, n0, n1, k) is not None) == share
+
+
 # Few activation rows: the kernel that measured faster (us with the short-batch kernel, with the tile kernel), clear cases of either.
 @pytest.mark.parametrize("t,m,n,k,kernel", [
     (Q5K, 19, 17096, 19712, SMALL),  # 84, 135: long rows in three rounds of tiles
