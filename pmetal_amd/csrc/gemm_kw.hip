@@ -110,7 +110,11 @@ struct KwQ45 {  // FMT 0: Q4_K, 1: Q5_K
         b[0] = v.value();
     }
     // (made where they are used: the 64 x 64 tile has no registers to hold them over the half)
-    __device__ __forceinline__ half8_t sums(int) const { return heads_and_tails(mns, -f16_twice(dd >> 16)); }
+    __device__ __forceinline__ half8_t sums(int) const {
+        uint32_t w = dd;
+        asm("" : "+v"(w));  // (not earlier: 170 registers for Q4_K's 64 x 32 tile, two waves a SIMD, for 163, three, and a register of Q5_K's 64 x 64 in memory)
+        return heads_and_tails(mns, -f16_twice(w >> 16));
+    }
     __device__ __forceinline__ float scale(int) const { return f16_bits_to_f32(dd & 0xFFFFu); }
 };
 
