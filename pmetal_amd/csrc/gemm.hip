@@ -2485,14 +2485,20 @@ static int fit_index(uint32_t type) {
 static bool dies_read_all(int64_t m, int64_t spr, int mb, int nr, int64_t tiles, uint32_t type) {
     return m * spr * 512 > (int64_t)12 << 20 && !kw_by_m((m + 32 * mb - 1) / (32 * mb), tiles, mb, nr, block_bytes(type));
 }
-static double many_tiles_us(const KwChoice &kw, int64_t m, int64_t n, int64_t spr, uint32_t type) {
+// Rounds are counted half way from the whole machine's to the busiest die's (even: the whole machine's): of nine blocks of the operand that the
+// dies share one has two and the others one.  Without that 4 of 513 drawn shapes that went to the tiles took 1.27 to 1.33 times the rows'
+// time: Q4_K 1276 x 8704 M = 615, ten blocks of activation rows; Q6_K 5344 x 9472 M = 153 62 -> 82 us, four dies with 33 workgroups for 32 compute units.
+static double many_tiles_us(const KwChoice &kw, int64_t m, int64_t n, int64_t spr, uint32_t type, bool even = false) {
     const KwFit &f = kKwFits[kw.mb + kw.nr - 2];
-    const double r = kw.rounds, whole = __builtin_ceil(r);
+    const int64_t mt = (m + 32 * kw.mb - 1) / (32 * kw.mb), nt = (n + 32 * kw.nr - 1) / (32 * kw.nr);
+    const bool by_m = kw_by_m(mt, nt, kw.mb, kw.nr, block_bytes(type));
+    const double busiest = (double)(((by_m ? mt : nt) + 7) / 8 * (by_m ? nt : mt) * kw.splits) / 32.0;
+    const double r = even ? kw.rounds : (kw.rounds + busiest) / 2, whole = __builtin_ceil(r);
     const double rounds = r > 1.0 ? f.part * r + (1.0 - f.part) * whole : r < 0.5 ? 1.0 - f.few * (1.0 - 2.0 * r) : 1.0;
     const double us = f.call + rounds * (f.round + f.sb[fit_index(type)] * (double)((spr + kw.splits - 1) / kw.splits)) +
                       (kw.splits > 1 ? f.split + f.split_us * 1e-6 * kw.splits * (double)m * (double)n : 0.0);
     // (Q4_K 14336 x 4096: M = 1024, 8 MB of activations, 185 us as expected, M = 2048 590 for 377)
-    return dies_read_all(m, spr, kw.mb, kw.nr, (n + 32 * kw.nr - 1) / (32 * kw.nr), type) ? us * 1.5 : us;
+    return dies_read_all(m, spr, kw.mb, kw.nr, nt, type) ? us * 1.5 : us;
 }
 static double many_rows_us(const GemmPlan &p, int64_t m, int64_t n, uint32_t type) {
     const int64_t wgs = (n + 255) / 256 * (p.mp / (32 * p.mb)) * p.splits;
@@ -2635,7 +2641,13 @@ GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type) {
         // gives.  us of a call, rows -> tiles: Q4_K 4096 x 4096 M = 512 40 -> 35, 1024 x 4096 M = 2048 45 -> 37, Q8_0 14336 x 4096 M = 512
         // 143 -> 116; 14336 x 4096 Q4_K M = 512, 1792 tiles, stays with the rows, 79 to 94.  Not one block of rows, where the row
         // kernels read nothing twice, either, and not rows of one or two super-blocks, which leave half of the waves without work.
-        if (!waves && m > 64 && spr > 2) waves = many_tiles_us(kw, m, n, spr, type) < 0.97 * many_rows_us(p, m, n, type);
+        if (!waves && m > 64 && spr > 2) {
+            const double rows = 0.97 * many_rows_us(p, m, n, type);
+            waves = many_tiles_us(kw, m, n, spr, type) < rows;
+            // (but the tiles, if only uneven dies speak against them, where the rows' K split does not fit the scratch of the entry point that
+            // allocates nothing: Q4_K 1605 x 8448 M = 636 66.8 us, 50.1 with 41 MB of scratch)
+            if (!waves && plan_bytes(p, type, n, k) > PMETAL_HIP_NOALLOC_SCRATCH_BYTES) waves = many_tiles_us(kw, m, n, spr, type, true) < rows;
+        }
     }
     if (small) {
         // short batches: rows longer than a run are cut into runs of 16 (or 8) super-blocks, these kernels' K split

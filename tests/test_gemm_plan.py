@@ -1,7 +1,7 @@
 """The GEMM's launch plan (host code, no device needed): what it names can be launched."""
 import pytest
 
-from gpu_util import Q4K, Q6K, Q8_0, SMALL, WAVES, gemm_converts_itself, gemm_pair_plan, gemm_plan, gemm_small_lds, gemm_workspace_bytes
+from gpu_util import Q4K, Q6K, Q8_0, ROWS, SMALL, WAVES, gemm_converts_itself, gemm_pair_plan, gemm_plan, gemm_small_lds, gemm_workspace_bytes
 
 Q5K, Q3K, Q2K = 13, 11, 10
 TYPES = [Q4K, Q6K, Q8_0, Q5K, Q3K, Q2K]
@@ -84,6 +84,12 @@ def test_pairs_of_four_and_eight_waves(t, m, n0, n1, k, share):
 def test_pairs_of_many_activation_rows(t, m, n0, n1, k, share):
     assert gemm_plan(t, m, n0, k).kernel == WAVES and gemm_plan(t, m, n1, k).kernel == WAVES
     assert (gemm_pair_plan(t, m, n0, n1, k) is not None) == share
+
+
+# Tiles of which one die has twice the others' share, or a few more than it has compute units: the row kernels (1.28 and 1.33 times as fast).
+@pytest.mark.parametrize("t,m,n,k", [(Q4K, 615, 1276, 8704), (Q6K, 153, 5344, 9472)])
+def test_uneven_dies_take_the_rows(t, m, n, k):
+    assert gemm_plan(t, m, n, k).kernel == ROWS
 
 
 # Few activation rows: the kernel that measured faster (us with the short-batch kernel, with the tile kernel), clear cases of either.
