@@ -261,6 +261,9 @@ struct KwQ23 {  // FMT 2: Q3_K, 3: Q2_K
 
 // ------------------------------------------------------------------------------------------------
 constexpr int kKwWaves = 8, kMostSplits = 4;  // (as the plan makes them)
+// Forms of the kernel: without a K split, with one, and two weights of which one has tiles of four waves and the other of eight.  (One kernel for
+// all: 0.1 us a call without a split, and up to 2 % of calls with short rows.)
+constexpr int kPlain = 0, kSplit = 1, kMixed = 2;
 // Bits beside kHasSecond: the tiles of the first, of the second weight have four waves of the workgroup's eight; they go two to a workgroup (see launch_kw)
 constexpr int kFirstOfFour = 2, kSecondOfFour = 4, kByTwos = 8;
 // A wave's accumulators lie in LDS as the 64 lanes' 16-byte slots (four rows of one column), lane l at tile_slot(l): a thread that
@@ -494,17 +497,17 @@ __device__ __forceinline__ void join_splits(uint32_t *arrived, const int splits,
     }
 }
 
-// SPLIT: with a K split; then there is no second weight, and second.y is the tiles' counters, or NULL where k_rw_reduce adds the splits.
-// (One kernel for both is 0.1 us slower without a split.)
+// With a K split there is no second weight, and second.y is the tiles' counters, or NULL where k_rw_reduce adds the splits.
 // grid (8, inner x splits of K, outer / 8), up to eight waves; split z has super-blocks [z * chunk, min(spr, (z + 1) * chunk)).
 // Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the blocks of activation rows,
 // otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
-template <class F, int MB, int NR, bool SPLIT>
+template <class F, int MB, int NR, int FORM>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
                                                              int spr, int chunk, int inner, int outer, int by_m, int ybf16,
                                                              float *partial, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
+    constexpr bool SPLIT = FORM == kSplit, MIXED = FORM == kMixed;
     extern __shared__ uint4 smem[];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block_waves = (int)(blockDim.x >> 6);
@@ -512,16 +515,15 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     if (out >= outer) return;  // (the whole workgroup)
     int nt = by_m ? in : out, nwaves = block_waves, tile_wave = wave, which = 0, tile_threads = (int)blockDim.x;
     if (!SPLIT) {
-        if (ybf16 & kHasSecond) {
-            const bool of_four = ybf16 & (nt >= second.first ? kSecondOfFour : kFirstOfFour), by_twos = of_four && (ybf16 & kByTwos);
-            take_weight(second, ybf16, nt, W, yg, N);
+        const bool of_four = MIXED && (ybf16 & (nt >= second.first ? kSecondOfFour : kFirstOfFour)), by_twos = of_four && (ybf16 & kByTwos);
+        take_weight(second, ybf16, nt, W, yg, N);
+        if (MIXED) {
             ybf16 &= 1;
-            nwaves = of_four ? 4 : nwaves;
+            nwaves = of_four ? 4 : spr < nwaves ? spr : nwaves;
             if (by_twos) {
                 tile_threads = 256, which = wave >> 2, tile_wave = wave & 3, nt = 2 * nt + which;
                 if (nt * (32 * NR) >= N) nt--, M = 0;  // (an odd last tile has none beside it: once more, and not stored)
             }
-            nwaves = spr < nwaves ? spr : nwaves;
         }
         partial = nullptr;
     }
@@ -551,7 +553,7 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     const uint32_t step = 32u * (uint32_t)Mp, a_off = (uint32_t)(g * Mp + m0 + col) * 16u;
     const uint8_t *xa = reinterpret_cast<const uint8_t *>(xs) + (size_t)(sb0 * 2 * K::kSteps) * step;
     // (beside a weight of eight waves a tile of four may have four more in its workgroup, which wait and store)
-    const bool works = SPLIT || tile_wave < nwaves;
+    const bool works = !MIXED || tile_wave < nwaves;
     float rs_mine = 0.0f;
     float16_t acc[NR][MB], part[NR][MB];
 #pragma unroll
@@ -606,8 +608,8 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     }
     if (tile_wave == 0 && lane < 32 * MB) rs[lane] = rs_mine;
     __syncthreads();
-    red += 4 * which * K::kTile;
-    const int tile_tid = SPLIT ? (int)threadIdx.x : tid - 256 * which, threads = SPLIT ? (int)blockDim.x : tile_threads;
+    if (MIXED) red += 4 * which * K::kTile;
+    const int tile_tid = MIXED ? tid - 256 * which : (int)threadIdx.x, threads = MIXED ? tile_threads : (int)blockDim.x;
     constexpr bool kJoins = SPLIT && pmh::joins_splits(MB, NR);
     if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves, kJoins>(red, rs, tile_tid, threads, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
     else add_tiles<K::kTile, MB, NR, MB * NR, 4, kJoins>(red, rs, tile_tid, threads, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
@@ -625,13 +627,13 @@ template <class F, int MB, int NR>
 static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n, int spr,
                             float *partial, uint32_t *arrived, GemmSecond second, hipStream_t s) {
     using K = Kw<F, MB, NR>;
-    auto kern = p.splits > 1 ? k_qgemm_kw<F, MB, NR, true> : k_qgemm_kw<F, MB, NR, false>;
     auto waves_of = [&](int nw) { return p.chunk < nw ? p.chunk : nw; };
     const int w0 = waves_of(p.nw), w1 = second.n > 0 ? waves_of(second.nw) : w0;
     // Two weights, tiles of eight waves (or what a short row has of them) and of four: workgroups of eight for both, so that either result
     // is the sum that it is alone.
     const bool mixed = w0 != w1;
     const int nwaves = mixed ? kKwWaves : w0;
+    auto kern = p.splits > 1 ? k_qgemm_kw<F, MB, NR, kSplit> : mixed ? k_qgemm_kw<F, MB, NR, kMixed> : k_qgemm_kw<F, MB, NR, kPlain>;
     const size_t stage = (size_t)nwaves * 2 * K::kItems * 16, red = (size_t)nwaves * K::kTile * 16 + (mixed ? 2 : 1) * 32 * MB * 4, lds = stage > red ? stage : red;
     static_assert((size_t)kKwWaves * 2 * K::kItems * 16 <= 160 * 1024 && (size_t)kKwWaves * K::kTile * 16 + 2 * 32 * MB * 4 <= 160 * 1024, "LDS");
     if (lds > 64 * 1024) {
