@@ -459,7 +459,9 @@ __device__ __forceinline__ void add_tiles(const float4_t *red, const float *rs, 
 // The splits of K of a tile, each of which has left its partial sums: the workgroup that comes last adds them in split order, as k_rw_reduce
 // does, whose launch it saves: us of a call at 27 rows with that launch / so, Q4_K 4096 x 14336 19.6 / 18.6, 2560 x 9728 14.7 / 13.9, Q6_K 25.4 /
 // 24.4, 17.9 / 17.1, Q8_0 24.0 / 23.2; four splits of 64 x 32 tiles 1 to 2 %.  (Who is last does not change the result.  Nobody waits for
-// anybody: `arrived` counts, and the pre-pass has cleared it.)
+// anybody: `arrived` counts, and the pre-pass has cleared it.)  The counter is relaxed, too, and no release by the language's rules. What orders the
+// sums is the instruction set: a store at agent scope writes through to where every die sees it (sc1), s_waitcnt vmcnt(0) returns when
+// it has arrived there, the barrier holds the count back until all waves are that far, and the loads behind it (sc1) pass by the die's own copies.
 template <int MB, int NR>
 __device__ __forceinline__ void join_splits(uint32_t *arrived, const int splits, const int m0, const int n0, const int M, const int Mp, const int N,
                                             const float *__restrict__ rowscale, const int ybf16, void *__restrict__ yg, const float *partial) {
@@ -497,7 +499,7 @@ __device__ __forceinline__ void join_splits(uint32_t *arrived, const int splits,
     }
 }
 
-// With a K split there is no second weight, and second.y is the tiles' counters, or NULL where k_rw_reduce adds the splits.
+// With a K split there is no second weight, and `arrived` has a cleared counter a tile, or is NULL where k_rw_reduce adds the splits.
 // grid (8, inner x splits of K, outer / 8), up to eight waves; split z has super-blocks [z * chunk, min(spr, (z + 1) * chunk)).
 // Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the blocks of activation rows,
 // otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
@@ -505,7 +507,7 @@ template <class F, int MB, int NR, int FORM>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
                                                              int spr, int chunk, int inner, int outer, int by_m, int ybf16,
-                                                             float *partial, const pmh::GemmSecond second) {
+                                                             float *partial, uint32_t *arrived, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
     constexpr bool SPLIT = FORM == kSplit, MIXED = FORM == kMixed;
     extern __shared__ uint4 smem[];
@@ -614,8 +616,7 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     if (nwaves > 4) add_tiles<K::kTile, MB, NR, (MB * NR == 4 ? 2 : 1), kKwWaves, kJoins>(red, rs, tile_tid, threads, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
     else add_tiles<K::kTile, MB, NR, MB * NR, 4, kJoins>(red, rs, tile_tid, threads, nwaves, m0, n0, M, Mp, N, z, ybf16, yg, partial);
     if constexpr (kJoins) {
-        if (second.y)  // (in the place of a second weight's result: the counters)
-            join_splits<MB, NR>(reinterpret_cast<uint32_t *>(second.y) + out * inner + in, (int)gridDim.y / inner, m0, n0, M, Mp, N, rowscale, ybf16, yg, partial);
+        if (arrived) join_splits<MB, NR>(arrived + out * inner + in, (int)gridDim.y / inner, m0, n0, M, Mp, N, rowscale, ybf16, yg, partial);
     }
 }
 
@@ -651,10 +652,9 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
     second.first = by_twos && w0 == 4 ? (t0 + 1) / 2 : t0;
     const int tiles = second.first + (by_twos && w1 == 4 ? (t1 + 1) / 2 : t1);  // (or pairs of them)
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
-    if (p.splits > 1) second.y = arrived;  // (a K split has no second weight)
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
     hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer, by_m ? 1 : 0,
-                       (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond | of_four : 0), p.splits > 1 ? partial : nullptr, second);
+                       (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond | of_four : 0), p.splits > 1 ? partial : nullptr, arrived, second);
     return hipGetLastError();
 }
 
