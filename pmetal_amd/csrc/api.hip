@@ -744,15 +744,19 @@ int32_t pmetal_hip_dequantize(uint32_t t, const uint8_t *src, size_t src_len, co
 
 }  // extern "C"
 
+// A third of the tensor (so that the stages of neighbouring chunks overlap; four or more are slower, each costs some 20 us), at most what a
+// slot holds.
+size_t pmh::codec_chunk(size_t n) {
+    const size_t chunk = (n + 3 * kPipeGrain - 1) / (3 * kPipeGrain) * kPipeGrain;
+    return chunk < kPipeMinElems ? kPipeMinElems : chunk > kPipeElems ? kPipeElems : chunk;
+}
+
 namespace {
 int32_t codec_pipelined(bool quantize, uint32_t t, float *plain, uint8_t *packed, size_t n, uint32_t order) {
     std::lock_guard<std::mutex> lock(g_pipe_mutex);
     HostPipe *p = nullptr;
     if (int32_t rc = host_pipe(&p)) return rc;
-    // chunk: a third of the tensor (so that the stages of neighbouring chunks overlap; four or more are slower, each costs some 20 us), at
-    // most what a slot holds
-    size_t chunk = ((n / 3 + kPipeGrain - 1) / kPipeGrain) * kPipeGrain;
-    chunk = chunk < kPipeMinElems ? kPipeMinElems : (chunk > kPipeElems ? kPipeElems : chunk);
+    const size_t chunk = pmh::codec_chunk(n);
     const size_t chunks = (n + chunk - 1) / chunk, q_chunk = pmetal_hip_tensor_size(t, chunk);
     auto elems_of = [&](size_t i) { return i + 1 < chunks ? chunk : n - i * chunk; };
     pmh::CopyTeam team;

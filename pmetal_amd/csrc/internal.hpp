@@ -154,6 +154,9 @@ hipError_t launch_kl_sums_quantized(uint32_t type, const uint8_t *src, const flo
 // k a multiple of 256 and at most 32768 (the activation blocks live in LDS); type Q4_K or Q6_K
 hipError_t launch_qgemv_q8k(uint32_t type, const uint8_t *w, int64_t n, int64_t k, const uint8_t *xq, float *y, hipStream_t s);
 
+// ---- api.hip ----
+size_t codec_chunk(size_t n);  // elements of a staging chunk of the host codec
+
 // ---- util.hip ----
 hipError_t launch_fill_normal(float *dst, size_t n, uint64_t seed, float std, float outlier_rate,
                               float outlier_mag, hipStream_t s);

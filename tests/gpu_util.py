@@ -95,6 +95,13 @@ def gemm_workspace_bytes(t, m, n, k):
     return fn(t, m, n, k)
 
 
+def codec_chunk(n):
+    """Elements of a staging chunk of the host codec."""
+    fn = _lib.load()._ZN3pmh11codec_chunkEm
+    fn.restype, fn.argtypes = C.c_size_t, [C.c_size_t]
+    return fn(n)
+
+
 def gemm_small_lds(t, m, k, tiles_per_wg, own, xf32):
     fn = _lib.load()._ZN3pmh15qgemm_small_ldsEjllibb
     fn.restype, fn.argtypes = C.c_size_t, [C.c_uint32, C.c_int64, C.c_int64, C.c_int, C.c_bool, C.c_bool]

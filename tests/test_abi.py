@@ -9,6 +9,7 @@ import pytest
 
 import pmetal_amd as pm
 from pmetal_amd import _lib
+from gpu_util import codec_chunk
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 Q8_0, Q4K, Q6K = 8, 12, 14
@@ -20,6 +21,20 @@ def lib():
         from pmetal_amd import build
         build.build()
     return _lib.load()
+
+
+# Staging chunks of a host tensor of 256 Ki elements or more: whole 8 Ki of them, three while they fit their slots, also where a third of
+# the elements is a whole number of 8 Ki and one or two more.
+@pytest.mark.parametrize("n", [786432, 786433, 983041, 983042, 983043, 3 * 8192 * 512, 3 * 8192 * 512 - 1, 5_000_000])
+def test_host_codec_chunks(lib, n):
+    chunk = codec_chunk(n)
+    assert chunk % 8192 == 0 and 256 << 10 <= chunk <= 4 << 20
+    assert -(-n // chunk) == 3
+
+
+def test_host_codec_chunks_at_the_limits(lib):
+    assert [codec_chunk(n) for n in (1, 262144, 600000, 786432)] == [262144] * 4
+    assert [codec_chunk(n) for n in (12582912, 12582913, 1 << 40)] == [4 << 20] * 3
 
 
 def test_header_and_library_agree(lib):
