@@ -6,7 +6,7 @@ import pytest
 
 import pmetal_amd as pm
 from pmetal_amd import _lib
-from gpu_util import Q4K, Q6K, Q8_0, first_mismatch, gpu_dequantize_dev, gpu_quantize_dev, weights
+from gpu_util import Q4K, Q6K, Q8_0, codec_chunk, first_mismatch, gpu_dequantize_dev, gpu_quantize_dev, weights
 
 pytestmark = pytest.mark.gpu
 BLOCK = {Q8_0: 34, Q4K: 144, Q6K: 210}
@@ -280,12 +280,11 @@ def test_quantize_host_pointer_entry_point(oracle, t):
     assert np.array_equal(pm.quantize(x, t), oracle.quantize(t, x))
 
 
-@pytest.mark.parametrize("t,n", [(Q8_0, 4750880), (Q6K, 12548352)])
+@pytest.mark.parametrize("t,n", [(Q8_0, 5135904), (Q6K, 9410816)])
 def test_host_pointer_entry_points_copy_the_last_bytes(t, n):
     """The last staging chunk's blocks are two bytes more than a multiple of 16 KiB, which the copy threads share out."""
     lib = _lib.load()
-    chunk = min(max((n // 4 + 8191) // 8192 * 8192, 256 << 10), 4 << 20)
-    last = lib.pmetal_hip_tensor_size(t, n - 3 * chunk)
+    last = lib.pmetal_hip_tensor_size(t, n - (n - 1) // codec_chunk(n) * codec_chunk(n))
     assert last >= 1 << 20 and last % 16384 == 2
     x = weights(t, n)
     want = gpu_quantize_dev(t, x)
@@ -302,7 +301,7 @@ def test_host_pointer_entry_points_copy_the_last_bytes(t, n):
 @pytest.mark.parametrize("n", [11_000_000 + 123, 20_000_000 + 7, 1_500_000 + 31, 262_144])
 @pytest.mark.parametrize("t", [Q8_0, Q4K, Q6K, 13, 11, 10, 15])
 def test_host_pointer_entry_points_on_a_tensor_of_several_staging_chunks(oracle, t, n):
-    """Host tensors of 256 Ki elements or more go through pinned staging chunks (a quarter of the tensor rounded up to
+    """Host tensors of 256 Ki elements or more go through pinned staging chunks (a third of the tensor rounded up to
     8192 elements, between 256 Ki and 4 Mi elements).  Ragged tails: the bytes equal those of the one-launch device
     path, and the super-blocks on both sides of chunk boundaries, the first and the last ones equal the oracle's; the
     same for the way back."""
@@ -310,7 +309,7 @@ def test_host_pointer_entry_points_on_a_tensor_of_several_staging_chunks(oracle,
     got = pm.quantize(x, t)
     assert np.array_equal(got, gpu_quantize_dev(t, x))
     bs, ts = (32, 34) if t == Q8_0 else (256, {Q4K: 144, Q6K: 210, 13: 176, 11: 110, 10: 84, 15: 292}[t])
-    chunk = min(max((n // 4 + 8191) // 8192 * 8192, 256 << 10), 4 << 20)
+    chunk = codec_chunk(n)
     spots = [0] + [c * chunk - 2 * bs for c in (1, 2) if c * chunk + 2 * bs < n] + [(n // bs - 3) * bs]
     for e0 in spots:
         e1 = min(n, e0 + 4 * bs)
