@@ -101,10 +101,4 @@ public:
     }
 };
 
-// One copy by threads of its own.
-inline void par_copy(void *dst, const void *src, size_t bytes) noexcept {
-    CopyTeam team;
-    team.copy(dst, src, bytes);
-}
-
 }  // namespace pmh

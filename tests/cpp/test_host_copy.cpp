@@ -18,7 +18,7 @@ int main() {
             std::vector<unsigned char> src(bytes + 1), dst(bytes + 64, 0xA5);
             for (size_t i = 0; i < bytes; i++) src[i] = (unsigned char)(i * 2654435761u >> 13);
             g_left = threads;
-            pmh::par_copy(dst.data(), src.data(), bytes);
+            pmh::CopyTeam().copy(dst.data(), src.data(), bytes);
             for (size_t i = 0; i < bytes; i++)
                 if (dst[i] != src[i]) return std::printf("threads %d bytes %zu: differs at %zu\n", threads, bytes, i), 1;
             for (size_t i = bytes; i < dst.size(); i++)
