@@ -2805,8 +2805,9 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     if (!qgemm_fits(type, m, n, k)) return hipErrorInvalidValue;
     GemmSecond second = second_weight;
     GemmPlan p;
+    int second_nw = 0;  // kWaves: the waves of the second weight's tiles, as its own plan has them
     if (second.n == 0) p = qgemm_plan(m, n, k, type);
-    else if (!pair_plan(m, n, second.n, k, type, &p, &second.nw)) return hipErrorInvalidValue;
+    else if (!pair_plan(m, n, second.n, k, type, &p, &second_nw)) return hipErrorInvalidValue;
     const int spr = (int)(k / 256);
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
     uint4 *xs = reinterpret_cast<uint4 *>(ws);
@@ -2900,7 +2901,7 @@ hipError_t launch_qgemm(uint32_t type, const uint8_t *w, int64_t n, int64_t k, c
     if (e != hipSuccess) return e;
     const bool ybf = y_dtype == kDtypeBf16;
     if (p.kernel == GemmKernel::kWaves) {
-        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, arrived, second, s);
+        e = launch_qgemm_kw(type, p, w, xs, rowscale, y, ybf, m, n, spr, order, partial, arrived, second, second_nw, s);
         if (e != hipSuccess || p.splits == 1 || joined) return e;
     } else if (p.kernel == GemmKernel::kSmall) {
         const int nwaves = spr < kSmallWaves ? spr : kSmallWaves;

@@ -264,8 +264,9 @@ constexpr int kKwWaves = 8, kMostSplits = 4;  // (as the plan makes them)
 // Forms of the kernel: without a K split, with one, and two weights of which one has tiles of four waves and the other of eight.  (One kernel for
 // all: 0.1 us a call without a split, and up to 2 % of calls with short rows.)
 constexpr int kPlain = 0, kSplit = 1, kMixed = 2;
-// Bits beside kHasSecond: the tiles of the first, of the second weight have four waves of the workgroup's eight; they go two to a workgroup (see launch_kw)
-constexpr int kFirstOfFour = 2, kSecondOfFour = 4, kByTwos = 8;
+// Bits beside kHasSecond: the tiles of the first, of the second weight have four waves of the workgroup's eight; they go two to a workgroup (see launch_kw);
+// `outer` counts the blocks of activation rows
+constexpr int kFirstOfFour = 2, kSecondOfFour = 4, kByTwos = 8, kByM = 16;
 // A wave's accumulators lie in LDS as the 64 lanes' 16-byte slots (four rows of one column), lane l at tile_slot(l): a thread that
 // reads four neighbouring columns back and one that writes its slot meet 64 different banks with the 15 beside them.
 constexpr int kTileRun = 76;
@@ -503,10 +504,13 @@ __device__ __forceinline__ void join_splits(uint32_t *arrived, const int splits,
 // grid (8, inner x splits of K, outer / 8), up to eight waves; split z has super-blocks [z * chunk, min(spr, (z + 1) * chunk)).
 // Workgroups eight apart are on one die: `outer` counts the tiles of the larger operand (by_m: the blocks of activation rows,
 // otherwise the tiles of weight rows), so each die's cache holds an eighth of that one and all of the other (M = 2048, 1024 x 4096 Q4_K with the activations, 19 MB, read by every die: 60.6 us; by an eighth each: 39.1).
+// The first 64 bytes of arguments arrive with the wave. The others, and the number and size of the workgroups behind them, are fetched from one piece of 128
+// bytes: with 18 bytes past it a call took 0.2 to 0.6 us longer (Q2_K 1326 x 768 M = 63 7.18 -> 7.39, on another machine Q6_K 430 x 512 M = 418 8.2 -> 8.9).
+static_assert(64 + 16 + sizeof(pmh::GemmSecond) + 18 <= 128, "arguments in one piece");
 template <class F, int MB, int NR, int FORM>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
-                                                             int spr, int chunk, int inner, int outer, int by_m, int ybf16,
+                                                             int spr, int chunk, int inner, int outer, int ybf16,
                                                              float *partial, uint32_t *arrived, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
     constexpr bool SPLIT = FORM == kSplit, MIXED = FORM == kMixed;
@@ -515,12 +519,12 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block_waves = (int)(blockDim.x >> 6);
     const int out = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / inner, in = (int)blockIdx.y - z * inner;
     if (out >= outer) return;  // (the whole workgroup)
+    const bool by_m = ybf16 & kByM;
     int nt = by_m ? in : out, nwaves = block_waves, tile_wave = wave, which = 0, tile_threads = (int)blockDim.x;
     if (!SPLIT) {
         const bool of_four = MIXED && (ybf16 & (nt >= second.first ? kSecondOfFour : kFirstOfFour)), by_twos = of_four && (ybf16 & kByTwos);
         take_weight(second, ybf16, nt, W, yg, N);
         if (MIXED) {
-            ybf16 &= 1;
             nwaves = of_four ? 4 : spr < nwaves ? spr : nwaves;
             if (by_twos) {
                 tile_threads = 256, which = wave >> 2, tile_wave = wave & 3, nt = 2 * nt + which;
@@ -529,6 +533,7 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         }
         partial = nullptr;
     }
+    ybf16 &= 1;
     const int m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
     // wave w takes every nwaves'th super-block of the split from the w'th on: what the workgroup reads at a time lies side by side
@@ -558,12 +563,6 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     const bool works = !MIXED || tile_wave < nwaves;
     float rs_mine = 0.0f;
     float16_t acc[NR][MB], part[NR][MB];
-#pragma unroll
-    for (int rg = 0; rg < NR; rg++)
-#pragma unroll
-        for (int i = 0; i < MB; i++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[rg][i][e] = 0.0f, part[rg][i][e] = 0.0f;
     if (works) {
         C.template issue<0>(r, sb_off, st0, lane);
         __builtin_amdgcn_sched_barrier(0);
@@ -576,6 +575,12 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         }
         __builtin_amdgcn_sched_barrier(0);
         rs_mine = lane < 32 * MB ? rowscale[m0 + lane] : 0.0f;
+#pragma unroll
+        for (int rg = 0; rg < NR; rg++)
+#pragma unroll
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[rg][i][e] = 0.0f, part[rg][i][e] = 0.0f;
         const size_t jump = (size_t)(nwaves - 1) * (2 * K::kSteps) * step;  // (past 4 GiB from 2.2 million activation rows on)
         for (int s = 0; s + 1 < cnt; s++) {
             if (F::kUnitHalves == 1) {
@@ -626,10 +631,10 @@ namespace pmh {
 
 template <class F, int MB, int NR>
 static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n, int spr,
-                            float *partial, uint32_t *arrived, GemmSecond second, hipStream_t s) {
+                            float *partial, uint32_t *arrived, GemmSecond second, int second_nw, hipStream_t s) {
     using K = Kw<F, MB, NR>;
     auto waves_of = [&](int nw) { return p.chunk < nw ? p.chunk : nw; };
-    const int w0 = waves_of(p.nw), w1 = second.n > 0 ? waves_of(second.nw) : w0;
+    const int w0 = waves_of(p.nw), w1 = second.n > 0 ? waves_of(second_nw) : w0;
     // Two weights, tiles of eight waves (or what a short row has of them) and of four: workgroups of eight for both, so that either result
     // is the sum that it is alone.
     const bool mixed = w0 != w1;
@@ -653,25 +658,25 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
     const int tiles = second.first + (by_twos && w1 == 4 ? (t1 + 1) / 2 : t1);  // (or pairs of them)
     const int inner = by_m ? tiles : mblocks, outer = by_m ? mblocks : tiles;
     const dim3 grid(8, (unsigned)(inner * p.splits), (unsigned)((outer + 7) / 8));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer, by_m ? 1 : 0,
-                       (y_bf16 ? 1 : 0) | (second.n > 0 ? kHasSecond | of_four : 0), p.splits > 1 ? partial : nullptr, arrived, second);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nwaves), lds, s, w, xs, rowscale, y, (int)m, p.mp, (int)n, spr, p.chunk, inner, outer,
+                       (y_bf16 ? 1 : 0) | (by_m ? kByM : 0) | (second.n > 0 ? kHasSecond | of_four : 0), p.splits > 1 ? partial : nullptr, arrived, second);
     return hipGetLastError();
 }
 
 template <class F>
 static hipError_t launch_kw_tile(const GemmPlan &p, const uint8_t *w, const uint4 *xs, const float *rowscale, void *y, bool y_bf16, int64_t m, int64_t n,
-                                 int spr, float *partial, uint32_t *arrived, GemmSecond second, hipStream_t s) {
-    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
-    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
-    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
-    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s);
+                                 int spr, float *partial, uint32_t *arrived, GemmSecond second, int second_nw, hipStream_t s) {
+    if (p.mb == 1 && p.nr == 1) return launch_kw<F, 1, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, second_nw, s);
+    if (p.mb == 1) return launch_kw<F, 1, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, second_nw, s);
+    if (p.nr == 1) return launch_kw<F, 2, 1>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, second_nw, s);
+    return launch_kw<F, 2, 2>(p, w, xs, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, second_nw, s);
 }
 
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &p, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
-                           int64_t n, int spr, uint32_t order, float *partial, uint32_t *arrived, const GemmSecond &second, hipStream_t s) {
+                           int64_t n, int spr, uint32_t order, float *partial, uint32_t *arrived, const GemmSecond &second, int second_nw, hipStream_t s) {
     const uint4 *x4 = reinterpret_cast<const uint4 *>(xs);
     const bool ref = order == kOrderRef;
-    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, s); };
+    auto go = [&](auto format) { return launch_kw_tile<decltype(format)>(p, w, x4, rowscale, y, y_bf16, m, n, spr, partial, arrived, second, second_nw, s); };
     switch (type) {
     case kTypeQ4K: return ref ? go(KwQ45<0, 0>{}) : go(KwQ45<1, 0>{});
     case kTypeQ5K: return ref ? go(KwQ45<0, 1>{}) : go(KwQ45<1, 1>{});

@@ -89,7 +89,6 @@ struct GemmSecond {
     void *y;
     int n;      // weight rows; 0: no second weight
     int first;  // its first workgroup along the grid's x dimension (kWaves: its first tile, or pair of tiles)
-    int nw;     // kWaves: the waves of its tiles, as its own plan has them
 };
 struct GemmPlan {
     GemmKernel kernel;
@@ -131,7 +130,7 @@ constexpr bool joins_splits(int mb, int nr) { return mb * nr < 4; }
 // gemm_kw.hip (spr: super-blocks per row; partial: fp32 tiles [splits][mp][n] when plan.splits > 1, not scaled by rowscale; arrived: a
 // cleared counter per tile of Y, where the launch adds the splits itself)
 hipError_t launch_qgemm_kw(uint32_t type, const GemmPlan &plan, const uint8_t *w, const void *xs, const float *rowscale, void *y, bool y_bf16, int64_t m,
-                           int64_t n, int spr, uint32_t order, float *partial, uint32_t *arrived, const GemmSecond &second, hipStream_t s);
+                           int64_t n, int spr, uint32_t order, float *partial, uint32_t *arrived, const GemmSecond &second, int second_nw, hipStream_t s);
 
 // ---- q8k.hip: Q8_K activation blocks and the integer dot products over them ----
 hipError_t launch_quantize_q8k(const float *x, size_t n, uint8_t *dst, hipStream_t s);
