@@ -2409,7 +2409,7 @@ bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k) {
 // waves' tiles or stores; alone on a compute unit four waves wait longer for memory than eight.  Four against eight, times
 // as long over 1400 drawn shapes, by tile and rounds of 256 workgroups:
 //   32 x 32: 1.02 up to half a round (Q6_K, Q8_0 and Q2_K 1.05), 1.01 up to one, 0.98 up to two, 0.95 above
-//   64 x 32: 0.98 to 0.99 up to one, 0.88 above (16 waves of it fit a compute unit)
+//   64 x 32: 0.98 to 0.99 up to one, 0.88 above (by registers twelve waves of it fit a compute unit, three workgroups of four or one of eight)
 //   64 x 64: 1.02 up to 0.8, 0.99 up to one (Q6_K and Q8_0 1.00 and, with rows of 12 to 40 super-blocks, up to 1.17), 0.92 up to
 //     two, 0.89 up to three, 0.84 above; 32 x 64 alike
 // They decide the order in which a result is summed: a launch of two weights has the waves that either has alone.

@@ -4,9 +4,10 @@
 // The kernels of gemm.hip give every wave its own weight rows and fill the machine with a K split over workgroups, whose
 // partial tiles a second launch adds: at M = 64 their loop has 0.5 us of matrix work per step and waits for memory in each,
 // and prepare + multiply + add are three dependent launches.  Here a workgroup owns a tile of 32 MB activation rows x 32 NR
-// weight rows for the whole of K.  Its (up to) eight waves take every eighth super-block each, run without a barrier from
-// start to end, and their fp32 tiles are added through LDS in wave order: no partial tiles in memory, no third launch, and
-// the result does not depend on scheduling.  (Consecutive runs of super-blocks, which is what the waves took before, lie far apart in
+// weight rows for the whole of K.  Its waves, eight or four (the plan's kw_waves) and no more than there are super-blocks, take super-blocks in
+// turn, run without a barrier from start to end, and their fp32 tiles are added through LDS in wave order: the result does not depend on
+// scheduling, and there are no partial tiles in memory.  Only where a few long rows leave the machine empty does a tile have two or four
+// workgroups, the last of which, or a launch behind, adds their sums (join_splits).  (Consecutive runs of super-blocks, which is what the waves took before, lie far apart in
 // a row: 1 to 5 % slower, two Q4_K weights of 14336 x 4096 M = 64 38.6 -> 36.8 us, Q5_K 8192 x 4096 M = 100 24.6 -> 23.4.)
 //   * Weights: a wave copies a unit of its rows (one or half a super-block of 32 NR rows) directly global -> LDS, one unit
 //     ahead, into LDS of its own; a lane (row n = lane % 32, half g = lane / 32) reads its quants and scales back and
@@ -24,11 +25,10 @@
 // pre-pass included, and per round and eight super-blocks of a row 2.9 (Q2_K), 3.5 (Q4_K, Q3_K), 4.6 (Q5_K), 4.9 us (Q8_0, Q6_K) with 32 x
 // 32 tiles (up to 32 activation rows, rows of 32 super-blocks and more); 0.6 to 0.8 of that where fewer than 64 workgroups run.  Inside, by
 // counters (share of the waves' time that they issue / are ready and cannot issue / wait for memory, LDS or each other; share of the
-// time that the matrix cores work; all with eight waves a workgroup and the splits added by a launch behind: as they are 29.2, 24.8 and, the sum of
-// the splits in it, 21.5 us):
-//   Q4_K, two of 14336 x 4096, M = 64 (64 x 64, 448 workgroups)       34.0 us  28 / 50 / 22 %, matrix cores 25 %
-//   Q8_0, 4999 x 3584, M = 203 (64 x 32, 628 workgroups)              28.8 us  37 / 29 / 34 %, 17 % (LDS bank conflicts 15 %: rows of 144 bytes)
-//   Q6_K, 4096 x 14336, M = 27 (32 x 32, two splits, 256 workgroups)  21.7 us  33 / 36 / 32 %, 17 %
+// time that the matrix cores work):
+//   Q4_K, two of 14336 x 4096, M = 64 (64 x 64, 448 workgroups of four waves)     28.6 us  31 / 55 / 15 %, matrix cores 32 %
+//   Q8_0, 4999 x 3584, M = 203 (64 x 32, 628 of four)                             24.0 us  30 / 45 / 26 %, 23 % (LDS bank conflicts 22 %: rows of 144 bytes)
+//   Q6_K, 4096 x 14336, M = 27 (32 x 32, two splits joined, 256 of eight)         21.5 us  26 / 44 / 30 %, 17 %
 #include "gemm_common.hpp"
 
 namespace {

@@ -96,7 +96,7 @@ struct GemmPlan {
     int nr;      // kWaves: 32-row blocks of weights per workgroup (1 or 2)
     int mp;      // padded activation rows, a multiple of 32 mb
     int nw;      // waves per workgroup (kWaves: at most; a short row has fewer)
-    int splits;  // workgroups along K (more than one: partial tiles plus a reduction kernel)
+    int splits;  // workgroups along K (more than one: partial tiles, added by a reduction kernel or, kWaves, by the tile's last workgroup)
     int chunk;   // super-blocks per split
 };
 // Which operand's tiles the dies share among them in the tile kernel (true: the blocks of activation rows)
