@@ -2422,6 +2422,16 @@ static int kw_waves(int mb, int nr, double rounds, uint32_t type) {
 bool kw_by_m(int64_t mblocks, int64_t tiles, int mb, int nr, int64_t block_bytes) {
     return mblocks >= 8 && mblocks * mb * 2 * 256 > tiles * nr * block_bytes;
 }
+// Rounds are the busiest die's workgroups of eight waves by what its 32 compute units hold of them: one each, two of 32 x 32 tiles.
+KwMixed kw_mixed(int64_t mblocks, int64_t of_four, int64_t of_eight, bool by_m, int mb, int nr) {
+    auto rounds = [&](int64_t columns) {
+        const int64_t outer = by_m ? mblocks : columns, inner = by_m ? columns : mblocks;
+        return (double)((outer + 7) / 8 * inner) / (mb * nr == 1 ? 64.0 : 32.0);
+    };
+    const double alone = rounds(of_four + of_eight), twos = rounds((of_four + 1) / 2 + of_eight);
+    const bool by_twos = __builtin_ceil(twos) < __builtin_ceil(alone);
+    return {by_twos, by_twos ? twos : alone};
+}
 static int64_t block_bytes(uint32_t type) {  // of a super-block of 256 elements
     return type == kTypeQ4K ? 144 : type == kTypeQ5K ? 176 : type == kTypeQ6K ? 210 : type == kTypeQ8_0 ? 272 : type == kTypeQ3K ? 110 : 84;
 }
@@ -2692,10 +2702,17 @@ static bool pair_plan(int64_t m, int64_t n0, int64_t n1, int64_t k, uint32_t typ
         if (kw.splits == 1) plan->mb = kw.mb, plan->nr = kw.nr;
         // One weight's tiles have four waves, the other's eight: a launch of its own for each costs 4 to 6 us more, workgroups of eight waves
         // for both what two workgroups of four on a compute unit gain. us, together / apart: Q4_K 4096 and 1024 x 4096, M = 100 17.6 / 20.9, Q6_K M = 96 20.1 /
-        // 28.0, Q8_0 2048 and 512 x 2048 M = 160 11.3 / 16.2, two and a half rounds of 64 x 32 tiles of Q8_0 2560 and 1280 x 2560 M = 300 30.6 / 26.9.
-        const int64_t spr = k / 256, nt = (n0 + 32 * plan->nr - 1) / (32 * plan->nr) + (n1 + 32 * plan->nr - 1) / (32 * plan->nr);
-        const int64_t tiles = nt * ((m + 32 * plan->mb - 1) / (32 * plan->mb));
-        if (p.nw != q.nw && spr > 8 && tiles > (plan->mb * plan->nr == 1 ? 1024 : 512)) return false;
+        // 28.0, Q8_0 2048 and 512 x 2048 M = 160 11.3 / 16.2; two and a half rounds of 64 x 32 tiles of Q8_0 2560 and 1280 x 2560 M = 300 30.6 / 26.9, Q4_K
+        // 1008 and 504 x 5888 M = 720, twelve blocks of activation rows on eight dies, 51.1 / 39.3.
+        // Times as long together as apart, by rounds, over 1150 drawn pairs with rows of more than four super-blocks (shorter ones have as many waves
+        // either way): up to one 0.70 to 0.89; to one and a half 1.03 to 1.17, 32 x 32 tiles 0.88; to two 0.86 to 0.94; above 1.00 to 1.09. Over 500 others so
+        // 0.83 (0.84 all together), ten of the 448 that are together 2 to 12 % longer.
+        const int64_t spr = k / 256, nt0 = (n0 + 32 * plan->nr - 1) / (32 * plan->nr), nt1 = (n1 + 32 * plan->nr - 1) / (32 * plan->nr), nt = nt0 + nt1;
+        if (p.nw != q.nw && spr > 4) {
+            const int64_t mt = (m + 32 * plan->mb - 1) / (32 * plan->mb);
+            const double rounds = kw_mixed(mt, p.nw == 4 ? nt0 : nt1, p.nw == 4 ? nt1 : nt0, kw_by_m(mt, nt, plan->mb, plan->nr, block_bytes(type)), plan->mb, plan->nr).rounds;
+            if (rounds > 2.0 || (rounds > 1.0 && rounds <= 1.5 && plan->mb * plan->nr > 1)) return false;
+        }
         // Tiles of which alone the dies share the activations, and together, more weight rows than activation rows then, the weights. That
         // costs from some 1300 activation rows on; Q8_0's tiles, which take longer, from 1900, Q6_K's nothing. us, together / apart, two
         // weights: Q4_K 4600 x 4096 M = 2048 390 / 232, 3322 x 4864 M = 1487 206 / 155, 2352 x 5888 M = 1081 111 / 139, Q2_K 5502 x 9216 M = 1709 927 / 533,

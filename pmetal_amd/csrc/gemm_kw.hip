@@ -648,11 +648,10 @@ static hipError_t launch_kw(const GemmPlan &p, const uint8_t *w, const uint4 *xs
     }
     const int t0 = (int)((n + 32 * NR - 1) / (32 * NR)), t1 = (second.n + 32 * NR - 1) / (32 * NR), mblocks = (int)((m + 32 * MB - 1) / (32 * MB));
     const bool by_m = kw_by_m(mblocks, t0 + t1, MB, NR, F::kBytes);
-    // Tiles of four go two to a workgroup where that is fewer rounds of workgroups, of which a compute unit holds one, and two of 32 x 32 tiles.
+    // Tiles of four go two to a workgroup where that is fewer rounds of the busiest die's compute units.
     // Otherwise a workgroup each, whose other four waves wait: a machine that is not full has more of it at work (us, by twos / alone: Q8_0
     // 4096 and 2048 x 4096 M = 96 30.6 / 23.4, Q4_K 4096 and 1024 x 4096 M = 100 24.1 / 17.6).
-    auto rounds = [&](int64_t tiles) { return (tiles * mblocks + (MB * NR == 1 ? 511 : 255)) / (MB * NR == 1 ? 512 : 256); };
-    const bool by_twos = mixed && rounds(w0 == 4 ? (t0 + 1) / 2 + t1 : t0 + (t1 + 1) / 2) < rounds(t0 + t1);
+    const bool by_twos = mixed && kw_mixed(mblocks, w0 == 4 ? t0 : t1, w0 == 4 ? t1 : t0, by_m, MB, NR).by_twos;
     const int of_four = !mixed ? 0 : (w0 == 4 ? kFirstOfFour : kSecondOfFour) | (by_twos ? kByTwos : 0);
     second.first = by_twos && w0 == 4 ? (t0 + 1) / 2 : t0;
     const int tiles = second.first + (by_twos && w1 == 4 ? (t1 + 1) / 2 : t1);  // (or pairs of them)

@@ -101,6 +101,13 @@ struct GemmPlan {
 };
 // Which operand's tiles the dies share among them in the tile kernel (true: the blocks of activation rows)
 bool kw_by_m(int64_t mblocks, int64_t tiles, int mb, int nr, int64_t block_bytes);
+// Two weights in one launch of the tile kernel, with workgroups of eight waves, tiles of four and of eight waves (columns of each): whether two tiles of four
+// share a workgroup, and the rounds of workgroups that the launch takes
+struct KwMixed {
+    bool by_twos;
+    double rounds;
+};
+KwMixed kw_mixed(int64_t mblocks, int64_t of_four, int64_t of_eight, bool by_m, int mb, int nr);
 bool qgemm_fits(uint32_t type, int64_t m, int64_t n, int64_t k);
 // (the padded row count mp follows m and the kernel, and the type and n only where the entry point that allocates nothing would be short of scratch)
 GemmPlan qgemm_plan(int64_t m, int64_t n, int64_t k, uint32_t type = kTypeQ4K);

@@ -61,7 +61,11 @@ def test_scratch_that_whole_tiles_fit(t, m, n, k):
     (Q5K, 160, 2048, 512, 2048, True),     # 16.2, 11.1
     (Q2K, 46, 504, 6528, 1280, True),      # 13.2, 8.8
     (Q3K, 141, 1763, 348, 256, True),      # 12.9, 8.4: a row of one super-block has one wave either way
+    (Q4K, 790, 1095, 273, 7680, True),     # 58.8, 44.2
     (Q8_0, 300, 2560, 1280, 2560, False),  # 26.9, 30.6
+    (Q4K, 720, 1008, 504, 5888, False),    # 39.3, 51.1: of 288 workgroups 48 on each of four dies
+    (Q8_0, 311, 5917, 463, 1280, False),   # 24.7, 31.6: 65 on one die
+    (Q2K, 560, 6724, 374, 1280, False),    # 34.3, 38.7
     (Q8_0, 454, 318, 3869, 4096, False)])  # 46.2, 52.9
 def test_pairs_of_four_and_eight_waves(t, m, n0, n1, k, share):
     a, b = gemm_plan(t, m, n0, k), gemm_plan(t, m, n1, k)

@@ -115,10 +115,12 @@ def test_pairs_match_separate_calls(oracle, t, m, k, ns):
 
 # ... of which one has tiles of four waves and the other of eight (or the five of a short row), in one launch.  Of each tile: the weight of four
 # waves in front and behind, its tiles one to a workgroup beside four waves that wait (the first two cases), two to a workgroup, an odd and an
-# even number of them, where that saves a round of workgroups.
+# even number of them, where that saves a round of workgroups.  The last seven: the dies share the blocks of activation rows.
 MIXED = [(1, 1, 193, 2048, (174, 1980)), (1, 1, 135, 1280, (2656, 68)), (1, 1, 213, 1280, (1665, 654)), (1, 1, 155, 2048, (35, 3227)), (1, 1, 130, 1280, (2210, 1048)),
          (2, 1, 163, 2048, (177, 2310)), (2, 1, 161, 1280, (2386, 71)), (2, 1, 182, 1280, (2049, 656)), (2, 1, 190, 2048, (520, 2193)), (2, 1, 177, 2304, (49, 2661)),
-         (2, 2, 162, 2048, (551, 2193)), (2, 2, 231, 1280, (1695, 367)), (2, 2, 272, 1280, (1040, 2221)), (2, 2, 384, 2304, (1483, 1177)), (2, 2, 234, 1792, (1872, 2188))]
+         (2, 2, 162, 2048, (551, 2193)), (2, 2, 231, 1280, (1695, 367)), (2, 2, 272, 1280, (1040, 2221)), (2, 2, 384, 2304, (1483, 1177)), (2, 2, 234, 1792, (1872, 2188)),
+         (1, 1, 531, 1280, (778, 132)), (1, 1, 544, 1792, (223, 720)), (2, 1, 620, 2048, (591, 125)), (2, 1, 551, 1536, (159, 654)),
+         (2, 2, 581, 1792, (687, 343)), (2, 2, 585, 1280, (225, 820)), (2, 2, 545, 1536, (416, 525))]
 MIXED = [(t, *c) for c in MIXED for t in (Q4K, Q6K, Q8_0, 13, 11, 10)] + [(Q6K, 1, 2, 31, 2304, (1003, 9001)), (Q8_0, 1, 2, 31, 1280, (8500, 6000))]
 
 
