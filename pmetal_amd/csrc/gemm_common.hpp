@@ -194,7 +194,7 @@ __device__ __forceinline__ half8_t q8_operand(const uint32_t w0, const uint32_t 
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 // Two weights in one launch: the workgroups from second.first on belong to the second one.  Whether there is one is a bit of an
-// argument that arrives with the wave (kHasSecond in `mode` or `ybf16`): the kernel of a single weight asks for nothing more.
+// argument that arrives with the wave (kHasSecond in `mode`, `flags` or `ybf16`): the kernel of a single weight asks for nothing more.
 constexpr int kHasSecond = 256;
 __device__ __forceinline__ void take_weight(const pmh::GemmSecond &second, int &flags, int &bx, const uint8_t *__restrict__ &W, void *__restrict__ &y,
                                             int &N) {

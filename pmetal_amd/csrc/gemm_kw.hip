@@ -510,7 +510,7 @@ static_assert(64 + 16 + sizeof(pmh::GemmSecond) + 18 <= 128, "arguments in one p
 template <class F, int MB, int NR, int FORM>
 __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__restrict__ W, const uint4 *__restrict__ xs,
                                                              const float *__restrict__ rowscale, void *__restrict__ yg, int M, int Mp, int N,
-                                                             int spr, int chunk, int inner, int outer, int ybf16,
+                                                             int spr, int chunk, int inner, int outer, int flags,
                                                              float *partial, uint32_t *arrived, const pmh::GemmSecond second) {
     using K = Kw<F, MB, NR>;
     constexpr bool SPLIT = FORM == kSplit, MIXED = FORM == kMixed;
@@ -519,11 +519,12 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block_waves = (int)(blockDim.x >> 6);
     const int out = (int)blockIdx.z * 8 + (int)blockIdx.x, z = (int)blockIdx.y / inner, in = (int)blockIdx.y - z * inner;
     if (out >= outer) return;  // (the whole workgroup)
-    const bool by_m = ybf16 & kByM;
+    const bool by_m = flags & kByM;
+    const int ybf16 = MIXED ? flags & 1 : flags & 7;  // (as a condition, & 1, it gave the tail of the other forms up to 100 instructions more)
     int nt = by_m ? in : out, nwaves = block_waves, tile_wave = wave, which = 0, tile_threads = (int)blockDim.x;
     if (!SPLIT) {
-        const bool of_four = MIXED && (ybf16 & (nt >= second.first ? kSecondOfFour : kFirstOfFour)), by_twos = of_four && (ybf16 & kByTwos);
-        take_weight(second, ybf16, nt, W, yg, N);
+        const bool of_four = MIXED && (flags & (nt >= second.first ? kSecondOfFour : kFirstOfFour)), by_twos = of_four && (flags & kByTwos);
+        take_weight(second, flags, nt, W, yg, N);
         if (MIXED) {
             nwaves = of_four ? 4 : spr < nwaves ? spr : nwaves;
             if (by_twos) {
@@ -533,7 +534,6 @@ __global__ __launch_bounds__(64 * kKwWaves) void k_qgemm_kw(const uint8_t *__res
         }
         partial = nullptr;
     }
-    ybf16 &= 1;
     const int m0 = (by_m ? out : in) * (32 * MB);
     const int n0 = nt * (32 * NR);
     // wave w takes every nwaves'th super-block of the split from the w'th on: what the workgroup reads at a time lies side by side
